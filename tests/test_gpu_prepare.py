@@ -1,0 +1,35 @@
+"""Weight preparation kernels against the oracle at the edges of their units: 32 rows x 128 bytes (rows of B^T), 8 squares
+of 8 x 8 bf16 or 16 x 16 bytes (rows of B)."""
+import numpy as np
+import pytest
+import torch
+
+import mm_amx_amd as mx
+from gpu_util import dev, dev_bf16, host_bits
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _init():
+    mx.init(0)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "int8", "uint8"])
+@pytest.mark.parametrize("K", [1, 63, 64, 65, 128, 511, 1025])
+@pytest.mark.parametrize("N", [1, 31, 64, 129, 257])
+def test_repack_unit_edges(po, dt, K, N):
+    rng = np.random.default_rng(K * 1000 + N)
+    if dt == "bf16":
+        B, up = rng.integers(1, 65536, (K, N)).astype(np.uint16), dev_bf16
+        want = po.repack(B, layout="mfma")
+    else:
+        B, up = rng.integers(-128, 128, (K, N)).astype(np.int8), dev
+        want = po.repack(B, layout="mfma")
+        if dt == "uint8":  # stored as u - 128
+            B = (B.astype(np.int16) + 128).astype(np.uint8)
+    assert np.array_equal(host_bits(mx.repack_b(up(B))).view(np.uint8), want.view(np.uint8))
+    # rows that start at any multiple of the element, inside a wider matrix
+    wide = torch.zeros((N, K + 3), dtype=up(B).dtype, device="cuda")
+    wide[:, 1:K + 1] = up(np.ascontiguousarray(B.T))
+    assert np.array_equal(host_bits(mx.repack_b(wide[:, 1:K + 1], transpose=True)).view(np.uint8), want.view(np.uint8))
