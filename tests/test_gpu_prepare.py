@@ -33,3 +33,19 @@ def test_repack_unit_edges(po, dt, K, N):
     wide = torch.zeros((N, K + 3), dtype=up(B).dtype, device="cuda")
     wide[:, 1:K + 1] = up(np.ascontiguousarray(B.T))
     assert np.array_equal(host_bits(mx.repack_b(wide[:, 1:K + 1], transpose=True)).view(np.uint8), want.view(np.uint8))
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 7), (5, 64), (33, 1029), (2, 70001), (700, 8)])
+@pytest.mark.parametrize("gap", [0, 5])
+def test_quantisers_row_ends_and_gaps(po, rows, cols, gap):
+    """Rows that end in the middle of a 16-byte load, with and without a gap behind them; the largest weight last."""
+    rng = np.random.default_rng(rows * 7 + cols)
+    W = po.f32_to_bf16((rng.standard_normal((rows, cols)) * 0.02).astype(np.float32))
+    W[-1, -1] = po.f32_to_bf16(np.array([-3.0], np.float32))[0]
+    wide = torch.full((rows, cols + gap), float("nan"), dtype=torch.bfloat16, device="cuda")  # (a gap takes no part)
+    wide[:, :cols] = dev_bf16(W)
+    got, scales = mx.quantize_weights(wide[:, :cols])
+    want, dq, q = po.quantize_weights(W)
+    assert np.array_equal(host_bits(got), want)
+    assert host_bits(scales).tolist() == [np.float32(q), np.float32(dq)]
+    assert np.array_equal(host_bits(mx.quantize_weights_scaled(wide[:, :cols], 1234.5)), po.quantize_scale_trunc(W, 1234.5))
