@@ -523,49 +523,136 @@ int launch_matvec(bool i8, const void* A, int64_t lda, const void* b, void* c, i
     return check_hip(hipGetLastError(), "matvec_kernel launch");
 }
 
-// ---- int4: per-column symmetric quantisation + packing in one pass per panel ---------------------------
-// One workgroup per 32-column panel.  Phase 1: column maxima of |w|; phase 2: every thread builds one dword
-// (8 values of one column) per fragment.  Not a hot path (done once per weight matrix).
+// ---- int4: per-column symmetric quantisation + packing, one workgroup per 32-column panel ----------------
+// The maxima of the panel's columns come first, so its weights are read twice (the second time mostly from the caches); both
+// passes move 16 bytes per lane, over whole lines, with the panel spread over 16 wavefronts.
+//   [N, K]: a column is a row.  Pass 1: half a wavefront per column would leave lines half used, so a wavefront walks one
+//   column at a time, 1 KiB per load.  Pass 2: a wavefront makes a fragment (32 columns x 64 of k) from 4 loads of 8 rows x
+//   128 bytes; a lane's 8 weights are one dword of slot (k half g, column), dword i = chunk % 4: a store is two lines.
+//   [K, N]: a row holds the panel's 32 columns in 64 bytes.  Pass 1: lane -> (row, 8 columns).  Pass 2: a lane reads 8 rows
+//   of 8 columns and builds the dword of each column from its own 8 x 8 square.
+// (4096 x 11008, [N, K] / [K, N]: two-byte loads by four wavefronts per panel took 261 / 360 us; now 45 / 70.)
+constexpr int QUANT4_WAVES = 16;
+
+__device__ __forceinline__ uint32_t int4_of(float w, float scale) {
+    float q = rintf(w * scale);
+    q = (q != q) ? 0.0f : q;  // a NaN weight, or an infinite one (its column's scale is then 0): quantised to 0
+    q = fminf(fmaxf(q, -7.0f), 7.0f);
+    return (uint32_t)(int)q & 0xfu;
+}
+
 template <bool TRANSPOSED>
-__global__ __launch_bounds__(256) void quant4_pack_kernel(const char* W, int64_t ldw, int K, int N, char* out, int nfrag,
-                                                          float* deq_out) {
-    __shared__ float smax[8][32];
+__global__ __launch_bounds__(QUANT4_WAVES * 64) void quant4_pack_kernel(const char* __restrict__ W, int64_t ldw, int K, int N,
+                                                                        char* __restrict__ out, int nfrag, float* deq_out) {
+    __shared__ float smax[32][QUANT4_WAVES];
     __shared__ float sscale[32];
-    const int t = threadIdx.x;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int n0 = blockIdx.x * 32;
-    auto wval = [&](int k, int n) -> float {
-        if (k >= K || n >= N) return 0.0f;
-        const char* p = TRANSPOSED ? W + (int64_t)n * ldw + (int64_t)k * 2 : W + (int64_t)k * ldw + (int64_t)n * 2;
-        return from_bf16(*reinterpret_cast<const uint16_t*>(p));
-    };
-    {
-        const int c = t & 31, kr = t >> 5;
-        float m = 0.0f;
-        for (int k = kr; k < K; k += 8) m = fmaxf(m, fabsf(wval(k, n0 + c)));
-        smax[kr][c] = m;
+    constexpr int UNR = 4;
+    // (fmaxf drops a NaN)
+    if constexpr (TRANSPOSED) {
+        for (int c = wave; c < 32; c += QUANT4_WAVES) {
+            float m = 0.0f;
+            if (n0 + c < N) {
+                const char* const row = W + (int64_t)(n0 + c) * ldw;
+                for (int k = lane * 8; k < K; k += 512 * UNR) {
+                    u32x4 v[UNR];
+                    if (k + 512 * (UNR - 1) + 8 <= K) {
+#pragma unroll
+                        for (int u = 0; u < UNR; u++) v[u] = load16_tail<2>(row + (int64_t)(k + 512 * u) * 2, 16);
+                    } else {
+#pragma unroll
+                        for (int u = 0; u < UNR; u++) v[u] = load16_tail<2>(row + (int64_t)(k + 512 * u) * 2, (int64_t)(K - k - 512 * u) * 2);
+                    }
+#pragma unroll
+                    for (int u = 0; u < UNR; u++)
+#pragma unroll
+                        for (int d = 0; d < 4; d++) m = fmaxf(fmaxf(m, fabsf(u2f(v[u][d] << 16))), fabsf(u2f(v[u][d] & 0xffff0000u)));
+                }
+            }
+            for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
+            if (lane < QUANT4_WAVES) smax[c][lane] = m;
+        }
+    } else {
+        const int ng = lane & 3;  // columns 8 ng .. 8 ng + 7 of the panel
+        const int64_t left = (int64_t)(N - n0 - 8 * ng) * 2;
+        float m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        for (int k = wave * 16 + (lane >> 2); k < K; k += QUANT4_WAVES * 16 * UNR) {
+            u32x4 v[UNR];
+#pragma unroll
+            for (int u = 0; u < UNR; u++) {
+                const int ku = k + QUANT4_WAVES * 16 * u;
+                v[u] = load16_tail<2>(W + (int64_t)ku * ldw + (int64_t)(n0 + 8 * ng) * 2, ku < K ? left : 0);
+            }
+#pragma unroll
+            for (int u = 0; u < UNR; u++)
+#pragma unroll
+                for (int d = 0; d < 4; d++) {
+                    m[2 * d] = fmaxf(m[2 * d], fabsf(u2f(v[u][d] << 16)));
+                    m[2 * d + 1] = fmaxf(m[2 * d + 1], fabsf(u2f(v[u][d] & 0xffff0000u)));
+                }
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            for (int off = 4; off < 64; off <<= 1) m[e] = fmaxf(m[e], __shfl_xor(m[e], off));
+            if (lane < 4) smax[8 * ng + e][wave] = m[e];
+        }
     }
     __syncthreads();
     if (t < 32) {
         float a = 0.0f;
 #pragma unroll
-        for (int r = 0; r < 8; r++) a = fmaxf(a, smax[r][t]);
+        for (int r = 0; r < QUANT4_WAVES; r++) a = fmaxf(a, smax[t][r]);
         sscale[t] = a > 0.0f ? 7.0f / a : 0.0f;
         if (n0 + t < N) deq_out[n0 + t] = a / 7.0f;
     }
     __syncthreads();
-    const int i = t & 3, c = (t >> 2) & 31, g = t >> 7;
-    const float qs = sscale[c];
-    for (int f = 0; f < nfrag; f++) {
-        const int k0 = 64 * f + 32 * g + 8 * i;
-        uint32_t d = 0;
+    char* const o = out + (int64_t)blockIdx.x * nfrag * 1024;
+    if constexpr (TRANSPOSED) {
+        const int r8 = lane >> 3, c = lane & 7;
+        float qs[4];
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-            float q = rintf(wval(k0 + e, n0 + c) * qs);
-            q = (q != q) ? 0.0f : q;  // a NaN weight, or an infinite one (its column's scale is then 0): quantised to 0
-            q = fminf(fmaxf(q, -7.0f), 7.0f);
-            d |= ((uint32_t)(int)q & 0xfu) << (4 * e);
+        for (int i = 0; i < 4; i++) qs[i] = sscale[8 * i + r8];
+        for (int f = wave; f < nfrag; f += QUANT4_WAVES) {
+            const int k = 64 * f + 8 * c;
+            u32x4 v[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int n = n0 + 8 * i + r8;
+                v[i] = load16_tail<2>(W + (int64_t)n * ldw + (int64_t)k * 2, n < N ? (int64_t)(K - k) * 2 : 0);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                uint32_t d = 0;
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    d |= (int4_of(u2f(v[i][e] << 16), qs[i]) | int4_of(u2f(v[i][e] & 0xffff0000u), qs[i]) << 4) << (8 * e);
+                *reinterpret_cast<uint32_t*>(o + (int64_t)f * 1024 + ((c >> 2) * 32 + 8 * i + r8) * 16 + (c & 3) * 4) = d;
+            }
         }
-        *reinterpret_cast<uint32_t*>(out + ((int64_t)blockIdx.x * nfrag + f) * 1024 + t * 4) = d;
+    } else {
+        // lane -> (columns 8 ng .., chunk of 8 k); 16 chunks = two fragments per wavefront
+        const int ng = lane & 3, kc = lane >> 2;
+        const int64_t left = (int64_t)(N - n0 - 8 * ng) * 2;
+        float qs[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) qs[e] = sscale[8 * ng + e];
+        for (int f2 = wave; f2 * 2 < nfrag; f2 += QUANT4_WAVES) {
+            const int k = 128 * f2 + 8 * kc;
+            u32x4 v[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                v[e] = load16_tail<2>(W + (int64_t)(k + e) * ldw + (int64_t)(n0 + 8 * ng) * 2, k + e < K ? left : 0);
+            char* const slot = o + (int64_t)(2 * f2 + (kc >> 3)) * 1024 + (((kc >> 2) & 1) * 32 + 8 * ng) * 16 + (kc & 3) * 4;
+#pragma unroll
+            for (int n = 0; n < 8; n++) {
+                uint32_t d = 0;
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+                    d |= int4_of(n & 1 ? u2f(v[e][n >> 1] & 0xffff0000u) : u2f(v[e][n >> 1] << 16), qs[n]) << (4 * e);
+                *reinterpret_cast<uint32_t*>(slot + n * 16) = d;
+            }
+        }
     }
 }
 
@@ -573,11 +660,12 @@ int launch_quantize_pack_int4(const void* W, int64_t ldw, int K, int N, int tran
                               hipStream_t st) {
     const int nfrag = (K + 255) / 256 * 4;
     const int npanels = (N + 31) / 32;
+    const dim3 threads(QUANT4_WAVES * 64);
     if (transpose)
-        hipLaunchKernelGGL(quant4_pack_kernel<true>, dim3(npanels), dim3(256), 0, st, static_cast<const char*>(W), ldw, K, N,
+        hipLaunchKernelGGL(quant4_pack_kernel<true>, dim3(npanels), threads, 0, st, static_cast<const char*>(W), ldw, K, N,
                            static_cast<char*>(packed), nfrag, deq_out);
     else
-        hipLaunchKernelGGL(quant4_pack_kernel<false>, dim3(npanels), dim3(256), 0, st, static_cast<const char*>(W), ldw, K, N,
+        hipLaunchKernelGGL(quant4_pack_kernel<false>, dim3(npanels), threads, 0, st, static_cast<const char*>(W), ldw, K, N,
                            static_cast<char*>(packed), nfrag, deq_out);
     return check_hip(hipGetLastError(), "quant4_pack_kernel launch");
 }

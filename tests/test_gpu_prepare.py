@@ -49,3 +49,18 @@ def test_quantisers_row_ends_and_gaps(po, rows, cols, gap):
     assert np.array_equal(host_bits(got), want)
     assert host_bits(scales).tolist() == [np.float32(q), np.float32(dq)]
     assert np.array_equal(host_bits(mx.quantize_weights_scaled(wide[:, :cols], 1234.5)), po.quantize_scale_trunc(W, 1234.5))
+
+
+@pytest.mark.parametrize("K", [1, 64, 255, 513, 2056])
+@pytest.mark.parametrize("N", [1, 33, 96])
+def test_int4_pack_unit_edges(po, K, N):
+    rng = np.random.default_rng(K * 31 + N)
+    W = po.f32_to_bf16((rng.standard_normal((K, N)) * 0.02).astype(np.float32))
+    q, deq = po.quantize_int4(W)
+    want = po.pack_int4(q)
+    for W_, trans in ((W, False), (np.ascontiguousarray(W.T), True)):
+        wide = torch.full((W_.shape[0], W_.shape[1] + 3), float("nan"), dtype=torch.bfloat16, device="cuda")
+        wide[:, 1:1 + W_.shape[1]] = dev_bf16(W_)
+        packed, d = mx.quantize_pack_int4(wide[:, 1:1 + W_.shape[1]], transpose=trans)
+        assert np.array_equal(host_bits(packed), np.ascontiguousarray(want).view(np.uint8).reshape(-1))
+        assert np.array_equal(host_bits(d), deq)
