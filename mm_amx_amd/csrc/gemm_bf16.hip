@@ -25,10 +25,10 @@ int launch_gemm_tiles_bf16(const void* A, int64_t lda, const void* Bp, int M, in
 // Bytes of workspace the plan for this shape would use (0: no K split), assuming operands the ring pipeline takes.
 size_t plan_workspace_bytes(int elesz, bool w8, int M, int K, int Ncols, uint32_t steps, int k_splits) {
     const int64_t kbytes = (int64_t)K * elesz;
-    if (kbytes % 128) return 0;
+    if (kbytes % 16 || (kbytes % 128 && (k_splits > 1 || kbytes < 128))) return 0;  // (rows of A that are not aligned, or a forced split of a K with a tail)
     const SplitRequest rq = {k_splits, reinterpret_cast<char*>(256), ~(size_t)0};
     if (steps & MMX_PP_SILU_GATE) return 0;
-    const Plan p = choose_plan(M, Ncols, (int)(kbytes / 128), false, w8, 2, rq, elesz == 1);
+    const Plan p = choose_plan(M, Ncols, (int)(kbytes / 128), false, w8, kbytes % 128 ? 4 : 2, rq, elesz == 1);
     if (p.S <= 1) return 0;
     const size_t tiles = (size_t)((M + p.t.bm - 1) / p.t.bm) * ((Ncols + p.t.bn - 1) / p.t.bn);
     return WS_COUNTER_BYTES + tiles * p.S * p.t.bm * p.t.bn * 4;

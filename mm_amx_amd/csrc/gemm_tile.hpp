@@ -18,12 +18,14 @@
 //           issued from inline asm into rings of LDS slots (A in whole 128-byte lines per row, B in
 //           half-stages of two fragments per panel), hand-scheduled against the MFMAs (see the
 //           comment at the pipeline);
+//   MODE 4  MODE 2 for a K that does not fill its last 128 bytes: whole k-iterations as there, the rest in a step of its own;
 //   MODE 0  global -> VGPR -> LDS with 16-byte loads, two LDS stages, rows past M clamped to the
 //           last row: the fallback when A or the packed weights are too large for the 32-bit
 //           offsets MODE 2 addresses with, and a tested alternative;
-//   MODE 3  MODE 0 with per-element masking: the general path for K tails (K*sizeof(T) not a
-//           multiple of 128) and for A rows that are not 16-byte aligned.  Rows past M and
-//           elements past K are read as zero, never touched in memory.
+//   MODE 3  MODE 0 for A rows of any alignment and any K: 16-byte loads from wherever the row starts,
+//           masked in the last k-iteration only (elements past K are read as zero, never touched in memory).
+//           (Masked element by element it was 4-10 times slower: 391 x 1001 x 3001 bf16 108 -> 25 us,
+//           2000 x 8001 x 8000 4322 -> 452.)
 #pragma once
 #include <atomic>
 #include <type_traits>
@@ -123,14 +125,25 @@ __device__ __forceinline__ int8_t cvt_out<int8_t>(float r) { return to_s8_sat(r)
 template <>
 __device__ __forceinline__ int32_t cvt_out<int32_t>(float r) { return (int32_t)r; }
 
-__device__ __forceinline__ u32x4 load_a_chunk_masked(const char* rowptr, int kbyte, int kbytes, bool vec_ok) {
+// The 16 bytes at byte kb of a row of kbytes, whatever the row's alignment (the hardware takes 16-byte loads from any
+// address); what lies past the row is zero and not touched: the last 16 bytes of the row are fetched instead and shifted.
+__device__ __forceinline__ u32x4 load_a_chunk_tail(const char* rowptr, int kb, int kbytes) {
     u32x4 v = u32x4{0u, 0u, 0u, 0u};
-    if (kbyte >= kbytes) return v;
-    if (vec_ok && kbyte + 16 <= kbytes) return *reinterpret_cast<const u32x4*>(rowptr + kbyte);
+    if (kb >= kbytes) return v;
+    if (kbytes >= 16) {
+        const int over = kb + 16 > kbytes ? kb + 16 - kbytes : 0;
+        uint64_t h[2];
+        __builtin_memcpy(h, __builtin_assume_aligned(rowptr + kb - over, 1), 16);
+        const int s = 8 * (over & 7);
+        if (over >= 8) h[0] = h[1], h[1] = 0;
+        if (s) h[0] = (h[0] >> s) | (h[1] << (64 - s)), h[1] >>= s;
+        v = u32x4{(uint32_t)h[0], (uint32_t)(h[0] >> 32), (uint32_t)h[1], (uint32_t)(h[1] >> 32)};
+        return v;
+    }
     uint32_t w[4] = {0, 0, 0, 0};
 #pragma unroll
     for (int b = 0; b < 16; b++) {
-        if (kbyte + b < kbytes) w[b >> 2] |= (uint32_t)(uint8_t)rowptr[kbyte + b] << (8 * (b & 3));
+        if (kb + b < kbytes) w[b >> 2] |= (uint32_t)(uint8_t)rowptr[kb + b] << (8 * (b & 3));
     }
     return u32x4{w[0], w[1], w[2], w[3]};
 }
@@ -188,6 +201,7 @@ template <typename TIn, int BM, int BN, int MODE, typename TOut, int SMAX, int N
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4, NW / 4))) void gemm_kernel(const GemmArgs g) {
     static_assert(NW == 4 || (NW == 8 && MODE == 2), "eight wavefronts exist for the ring pipeline only");
     constexpr int NT = NW * 64;  // threads
+    constexpr bool RING = MODE == 2 || MODE == 4;
     using MF = Mfma<TIn>;
     using frag = typename MF::frag;
     using accv = typename MF::accv;
@@ -245,7 +259,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
     // go into LDS behind the operand buffers, straight from memory (global_load_lds_dword: 64 columns per
     // instruction, no registers) and ahead of every operand load, so they have long landed when the epilogue
     // reads them: fetched at the point of use, each column block paid a trip to memory with the matrix pipe idle.
-    constexpr int OC_OFF = MODE == 2 ? Ring<BM, BN, W8>::BYTES : 2 * STAGE;
+    constexpr int OC_OFF = RING ? Ring<BM, BN, W8>::BYTES : 2 * STAGE;
     {
         const Epilogue& e0 = g.ep;
         const float* const src_of[3] = {(e0.steps & MMX_PP_BIAS) ? e0.bias : nullptr,
@@ -275,7 +289,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
         gelu_c[c] = u2f(bits);
     }
 
-    u32x4 ra[MODE == 2 ? 1 : A_IT], rb[MODE == 2 ? 1 : B_IT];  // staging registers of modes 0 and 3
+    u32x4 ra[RING ? 1 : A_IT], rb[RING ? 1 : B_IT];  // staging registers of modes 0 and 3
 
     auto fetch = [&](int kt) {
 #pragma unroll
@@ -289,10 +303,12 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
                 const char* src = g.A + (int64_t)grow * g.lda + kt * 128 + chunk * 16;
                 ra[it] = *reinterpret_cast<const u32x4*>(src);
             } else {
-                ra[it] = u32x4{0u, 0u, 0u, 0u};
-                if (grow < g.M)
-                    ra[it] = load_a_chunk_masked(g.A + (int64_t)grow * g.lda, kt * 128 + chunk * 16, g.kbytes,
-                                                 g.a_vec_ok);
+                const char* row = g.A + (int64_t)(grow < g.M ? grow : g.M - 1) * g.lda;
+                if ((kt + 1) * 128 <= g.kbytes) {  // (uniform: only the last k-iteration has anything to mask)
+                    __builtin_memcpy(&ra[it], __builtin_assume_aligned(row + kt * 128 + chunk * 16, 1), 16);
+                } else {
+                    ra[it] = load_a_chunk_tail(row, kt * 128 + chunk * 16, g.kbytes);
+                }
             }
         }
 #pragma unroll
@@ -345,7 +361,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
             for (int j = 0; j < NJ; j++) acc[i][j] = MF::run(b[j], a[i], acc[i][j]);
     };
 
-    if constexpr (MODE == 2) {
+    if constexpr (RING) {
         // ---- hand-scheduled ring pipeline -------------------------------------------------------------
         // One wave per SIMD means nothing hides a stall, and a wave issues in order: a burst of LDS
         // reads or of global loads in front of the MFMAs leaves the matrix pipe idle while the burst
@@ -619,6 +635,59 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
         } else {
             if (wave_u < NCLS0) ring(std::integral_constant<int, 0>{});
             else ring(std::integral_constant<int, 1>{});
+        }
+        // MODE 4: the part of K behind the last whole k-iteration, once: A through registers (its rows end inside the 128
+        // bytes) and the weights, whose padding is there, into the first slots of the rings; then four k-steps.  The trip to
+        // memory is not hidden behind anything, but it is one: the masked pipeline, which this replaces for aligned rows,
+        // waits for one per k-iteration (bf16 1064 x 3544 x 786 62 -> 31 us, 64 x 4104 x 4096 52 -> 14).  (A mode of its own: behind this branch the compiler keeps the accumulators twice,
+        // which the largest tiles have no registers for.)
+        if constexpr (MODE == 4) {
+        if (SMAX == 1 || kt0 + nk == g.nk) {
+            constexpr int AC = BM * 8 / NT, BC = (BN / 32) * (BP_IT / 16);
+            u32x4 ta[AC], tb[(BC + NT - 1) / NT];
+#pragma unroll
+            for (int it = 0; it < AC; it++) {
+                const int row = (it * NT + tid) >> 3, chunk = (tid & 7) ^ ((row >> 1) & 7);
+                const int grow = m0 + row < g.M ? m0 + row : g.M - 1;
+                ta[it] = load_a_chunk_tail(g.A + (int64_t)grow * g.lda, g.nk * 128 + chunk * 16, g.kbytes);
+            }
+#pragma unroll
+            for (int it = 0; it < (BC + NT - 1) / NT; it++) {
+                const int c = it * NT + tid;
+                int panel = panel0 + c / (BP_IT / 16);
+                panel = panel < g.npanels ? panel : g.npanels - 1;
+                if (BC % NT == 0 || c < BC)
+                    tb[it] = *reinterpret_cast<const u32x4*>(g.Bp + (int64_t)panel * g.panel_stride + (int64_t)g.nk * BP_IT + (c % (BP_IT / 16)) * 16);
+            }
+            __syncthreads();  // every wave has finished with the rings (and its own re-fetched slots have landed)
+#pragma unroll
+            for (int it = 0; it < AC; it++) *reinterpret_cast<u32x4*>(smem + (it * NT + tid) * 16) = ta[it];
+#pragma unroll
+            for (int it = 0; it < (BC + NT - 1) / NT; it++) {
+                const int c = it * NT + tid, in = c % (BP_IT / 16);
+                if (BC % NT == 0 || c < BC)
+                    *reinterpret_cast<u32x4*>(smem + B0 + (in / (BP_HS / 16)) * BH + (c / (BP_IT / 16)) * BP_HS + (in % (BP_HS / 16)) * 16) = tb[it];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const int chunk = W8 ? 4 * (s >> 1) + 2 * g32 + (s & 1) : 2 * s + g32;
+                const char* sA = smem + (wm * WM + l32) * 128 + ((chunk ^ ((l32 >> 1) & 7)) * 16);
+                const char* sB = smem + B0 + (s >> 1) * BH + wn * NJ * BP_HS + lane * 16;
+#pragma unroll
+                for (int i = 0; i < MI; i++) fa[0][i] = *reinterpret_cast<const frag*>(sA + i * 32 * 128);
+#pragma unroll
+                for (int j = 0; j < NJ; j++) {
+                    if constexpr (W8) {
+                        const u32x4 raw = *reinterpret_cast<const u32x4*>(sB + j * BP_HS);
+                        fb[0][j] = (s & 1) ? s8x8_to_bf16(raw[2], raw[3]) : s8x8_to_bf16(raw[0], raw[1]);
+                    } else {
+                        fb[0][j] = *reinterpret_cast<const frag*>(sB + j * BP_HS + (s & 1) * 1024);
+                    }
+                }
+                mma(fa[0], fb[0]);
+            }
+        }
         }
     } else {
     fetch(kt0);
@@ -1019,12 +1088,14 @@ static inline Plan choose_plan(int M, int Ncols, int nk, bool need_pairs, bool w
         if (wide_only && c.bn == 64) continue;                      // (no 64-column tile for int8 weights under bf16 A)
         if (need_pairs && c.bm == 64) continue;                     // (the 64-row tile stores no gate/up pairs)
         if (mode == 3 && !(c.bm == 128 && c.bn == 128)) continue;   // the masked path exists for one tile shape
-        if (mode != 2 && (c.bn == 64 || c.bm == 64)) continue;      // the 64-wide and 64-row tiles exist for the ring pipeline only
+        if (mode == 4 && !((c.bm == 256 && c.bn == 192) || (c.bm <= 128 && c.bn <= 128))) continue;  // (the tiles of MODE 4)
+        if (mode == 4 && c.bm == 256 && rq.k_splits > 1) continue;
+        if (mode != 2 && mode != 4 && (c.bn == 64 || c.bm == 64)) continue;      // the 64-wide and 64-row tiles exist for the ring pipeline only
         const int tiles = ((M + c.bm - 1) / c.bm) * ((Ncols + c.bn - 1) / c.bn);
         for (int S = 1; S <= KSPLIT_MAX; S++) {
             if (rq.k_splits > 0 && S != rq.k_splits) continue;
             if (S > 1) {
-                if (need_pairs || c.bn == 64 || !rq.ws || tiles > WS_MAX_TILES) break;
+                if (need_pairs || c.bn == 64 || !rq.ws || tiles > WS_MAX_TILES || (mode == 4 && c.bm == 256)) break;
                 const int kq = slice_kiters(nk, S);
                 if ((S - 1) * kq >= nk) continue;  // an empty last slice
                 if (WS_COUNTER_BYTES + (size_t)tiles * S * c.bm * c.bn * 4 > rq.ws_bytes) continue;
@@ -1067,13 +1138,13 @@ template <typename TIn, int BM, int BN, int MODE, typename TOut, int SMAX, int N
 static int launch_cfg(const GemmArgs& g, int grid, hipStream_t st) {
     constexpr bool W8 = Mfma<TIn>::W8;
     // operand buffers, then three arrays of BN per-column post-op operands
-    constexpr int lds = (MODE == 2 ? Ring<BM, BN, W8>::BYTES : 2 * (BM * 128 + BN * (W8 ? 64 : 128))) + 3 * BN * 4;
+    constexpr int lds = (MODE == 2 || MODE == 4 ? Ring<BM, BN, W8>::BYTES : 2 * (BM * 128 + BN * (W8 ? 64 : 128))) + 3 * BN * 4;
     static_assert(lds <= 160 * 1024, "LDS of a CU");
     auto kern = gemm_kernel<TIn, BM, BN, MODE, TOut, SMAX, NW>;
     static std::atomic<uint64_t> attr_done{0};  // one per instantiation: the devices whose LDS limit has been raised
     int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds, attr_done);
     if (rc) return rc;
-    static const char* const loads[] = {"regs", "", "ring", "masked"};
+    static const char* const loads[] = {"regs", "", "ring", "masked", "ring"};
     char name[96];
     snprintf(name, sizeof name, "gemm_%s_%dx%d_%s%s_out_%s%s", type_tag<TIn>(), BM, BN, loads[MODE], NW == 8 ? "8w" : "", type_tag<TOut>(),
              g.ksplit == 2 ? "_ksplit2" : g.ksplit == 3 ? "_ksplit3" : g.ksplit == 4 ? "_ksplit4" : "");
@@ -1091,8 +1162,16 @@ static int launch_cfg(const GemmArgs& g, int grid, hipStream_t st) {
 
 template <typename TIn, typename TOut>
 static int launch_tiles(const GemmArgs& g, TileCfg t, int mode, int grid, hipStream_t st) {
-    if (g.ksplit > 1 && mode != 2) return set_error(MMX_E_UNSUPPORTED, "the K split needs the ring pipeline (aligned A, K a multiple of 128 bytes)");
+    if (g.ksplit > 1 && mode != 2 && mode != 4) return set_error(MMX_E_UNSUPPORTED, "the K split needs the ring pipeline (aligned A, K a multiple of 128 bytes)");
     if (mode == 3) return MMX_LAUNCH(TIn, 128, 128, 3, TOut, 1);  // the masked path exists for one tile shape
+    if (mode == 4) {  // a K tail: four tiles cover the range (the K split's code costs an unsplit launch nothing measurable)
+        if (t.bm == 256 && t.bn == 192) return MMX_LAUNCH(TIn, 256, 192, 4, TOut, 1);
+        if (t.bm == 64 && t.bn == 128) return MMX_LAUNCH(TIn, 64, 128, 4, TOut, KSPLIT_MAX);
+        if constexpr (!Mfma<TIn>::W8) {
+            if (t.bm == 128 && t.bn == 64) return MMX_LAUNCH(TIn, 128, 64, 4, TOut, 1);
+        }
+        return MMX_LAUNCH(TIn, 128, 128, 4, TOut, KSPLIT_MAX);
+    }
     if (t.bm == 256 && t.bn == 256) {
         // two waves per SIMD (a 64x128 block each): MLP gate/up at M = 2048 325 -> 312 us, same bits
         // (not over int8 weights: there the four-wavefront forms are as fast or faster, 91.5 against 98.2 us for 256x192)
@@ -1137,13 +1216,15 @@ static inline int prepare_gemm(GemmArgs& g, TileCfg& t, int& mode, int elesz, co
     g.a_vec_ok = ((reinterpret_cast<uintptr_t>(A) & 15) == 0) && ((lda & 15) == 0);
     g.ep = ep;
     const bool pairs = (ep.steps & MMX_PP_SILU_GATE) != 0;
-    // the unmasked loads need aligned rows and a K that fills whole k-iterations
-    const bool fast_ok = g.a_vec_ok && (g.kbytes % 128 == 0);
+    // the unmasked loads need aligned rows; the ring pipeline finishes a K that does not fill its last k-iteration by itself
+    const bool fast_ok = g.a_vec_ok && (g.kbytes % 128 == 0 || (load_mode() == 2 && g.kbytes > 128));
     mode = fast_ok ? load_mode() : 3;
-    // mode 2 addresses A through 32-bit per-thread offsets
-    if (mode == 2 && ((int64_t)M * lda >= ((int64_t)1 << 32) - 4096 || g.panel_stride >= ((int64_t)1 << 28))) mode = 0;
+    if (mode == 2 && g.kbytes % 128) mode = 4;
+    // modes 2 and 4 address A through 32-bit per-thread offsets
+    if ((mode == 2 || mode == 4) && ((int64_t)M * lda >= ((int64_t)1 << 32) - 4096 || g.panel_stride >= ((int64_t)1 << 28))) mode = mode == 4 ? 3 : 0;
+    if (mode == 4) g.nk = g.kbytes / 128;
     SplitRequest use = rq;
-    if (mode != 2 || pairs) {
+    if ((mode != 2 && mode != 4) || pairs || (mode == 4 && rq.k_splits > 1)) {
         if (rq.k_splits > 1)
             return set_error(MMX_E_UNSUPPORTED, "a K split needs 16-byte aligned rows of A, K a multiple of 128 bytes and no SILU_GATE");
         use.k_splits = 1;

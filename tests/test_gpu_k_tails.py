@@ -1,0 +1,83 @@
+"""The tile kernels at a K that does not fill its last 128 bytes (aligned rows: the ring pipeline's last step; rows of any
+alignment: the masked pipeline), against the oracle: remainders of 2 to 126 bytes, one whole k-iteration in front or many,
+every tile that takes a tail, the K split, the gate/up store."""
+import numpy as np
+import pytest
+import torch
+
+import mm_amx_amd as mx
+from gpu_util import check_float_parity, dev, dev_bf16, host_bits
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _init():
+    mx.init(0)
+    yield
+    mx.set_tile("")
+
+
+def _in_nan(t, pad):
+    """t inside a wider matrix of NaN (bf16) or 77 (int8): what lies behind a row must not enter the result."""
+    wide = torch.full((t.shape[0], t.shape[1] + pad), float("nan") if t.dtype == torch.bfloat16 else 77, dtype=t.dtype, device="cuda")
+    wide[:, :t.shape[1]] = t
+    return wide[:, :t.shape[1]]
+
+
+@pytest.mark.parametrize("tile", ["", "256x192", "128x128", "128x64", "64x128"])
+@pytest.mark.parametrize("K", [65, 72, 127, 200, 1089])
+@pytest.mark.parametrize("kind", ["bf16", "w8", "i8"])
+def test_k_tail(po, kind, K, tile):
+    M, N = (300, 200) if tile == "" else (131, 97)
+    if kind == "i8":
+        K *= 2
+    rng = np.random.default_rng(K)
+    W = rng.integers(-127, 128, (K, N)).astype(np.int8)
+    if kind == "i8":
+        A = rng.integers(-127, 128, (M, K)).astype(np.int8)
+        up, ref, kw, odt = dev, po.gemm_i8(A, W), {}, torch.int32
+    else:
+        A = po.f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32))
+        if kind == "bf16":
+            W = po.f32_to_bf16((rng.standard_normal((K, N)) * 0.05).astype(np.float32))
+        ref = po.gemm_bf16(A, W if kind == "bf16" else po.f32_to_bf16(W.astype(np.float32)))
+        up, kw, odt = dev_bf16, ({} if kind == "bf16" else {"b_dtype": mx.I8}), torch.float32
+    packed = mx.repack_b((dev_bf16 if kind == "bf16" else dev)(W))
+    es = 1 if kind == "i8" else 2
+    mx.set_tile(tile)
+    for pad in ((-K * es % 16) // es + 16 // es, 3):   # rows 16-byte aligned, and not
+        C = torch.zeros((M, N), dtype=odt, device="cuda")
+        mx.gemm(_in_nan(up(A), pad), packed, N, mx.Epilogue(C), **kw)
+        if kind == "i8":
+            assert np.array_equal(host_bits(C), ref), mx.last_kernel()
+        else:
+            check_float_parity(host_bits(C), ref, f"{kind} K={K} pad={pad} {mx.last_kernel()}")
+    mx.set_tile("")
+
+
+@pytest.mark.parametrize("K", [4104, 4400])
+def test_k_tail_behind_a_k_split(po, K):
+    """Few tiles and a long K: the last slice, and it alone, takes the tail (8 and 48 elements)."""
+    M, N = 64, 256
+    rng = np.random.default_rng(K)
+    A = po.f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32))
+    B = po.f32_to_bf16((rng.standard_normal((K, N)) * 0.05).astype(np.float32))
+    C = torch.zeros((M, N), dtype=torch.float32, device="cuda")
+    mx.gemm(dev_bf16(A), mx.repack_b(dev_bf16(B)), N, mx.Epilogue(C))
+    assert "ksplit" in mx.last_kernel(), mx.last_kernel()
+    check_float_parity(host_bits(C), po.gemm_bf16(A, B), mx.last_kernel())
+
+
+def test_k_tail_gate_up(po):
+    M, K, N = 70, 200, 96
+    rng = np.random.default_rng(5)
+    x = po.f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32))
+    wg, wu = (po.f32_to_bf16((rng.standard_normal((N, K)) * 0.05).astype(np.float32)) for _ in range(2))
+    h = torch.zeros((M, N), dtype=torch.float32, device="cuda")
+    mx.gemm(dev_bf16(x), mx.repack_gate_up(dev_bf16(wg), dev_bf16(wu)), 2 * N, mx.Epilogue(h, mx.PP_SILU_GATE))
+    g, u = (po.gemm_bf16(x, np.ascontiguousarray(w.T)) for w in (wg, wu))
+    # silu is a 2^-14 approximation of g / (1 + exp(-g)); twice that for the roundings around it
+    want = g / (1.0 + np.exp(-g.astype(np.float64))) * u
+    got = host_bits(h).astype(np.float64)
+    assert np.linalg.norm(got - want) <= 2.0 ** -13 * np.linalg.norm(want), mx.last_kernel()
