@@ -158,7 +158,6 @@ static int make_epilogue(const mmx_epilogue* in, int a_dtype, int b_dtype, int M
     out->deq_oc = in->deq_scale_per_oc;
     out->q = in->q_scale;
     out->q_oc = in->q_scale_per_oc;
-    out->c_vec_ok = ((reinterpret_cast<uintptr_t>(in->C) & 15) == 0) && ((in->ldc_bytes & 15) == 0);
     return MMX_OK;
 }
 

@@ -39,7 +39,6 @@ struct Epilogue {
     const float* deq_oc;
     float q;
     const float* q_oc;
-    int c_vec_ok;  // C and ldc are 16-byte aligned
 };
 
 // A caller's request for a split of K over several workgroups per tile, and the memory for its partial sums.

@@ -125,6 +125,12 @@ __device__ __forceinline__ int8_t cvt_out<int8_t>(float r) { return to_s8_sat(r)
 template <>
 __device__ __forceinline__ int32_t cvt_out<int32_t>(float r) { return (int32_t)r; }
 
+// 16 bytes to an address that is aligned to an element of SZ bytes only: the hardware takes such stores whole.  (Rows of C
+// that are not 16-byte aligned used to be written element by element: 391 x 1024 x 3001 bf16 14.4 -> 8.8 us,
+// 1024 x 4096 x 10999 115 -> 76.)
+template <int SZ>
+__device__ __forceinline__ void store16(char* p, u32x4 v) { __builtin_memcpy(__builtin_assume_aligned(p, SZ), &v, 16); }
+
 // The 16 bytes at byte kb of a row of kbytes, whatever the row's alignment (the hardware takes 16-byte loads from any
 // address); what lies past the row is zero and not touched: the last 16 bytes of the row are fetched instead and shifted.
 __device__ __forceinline__ u32x4 load_a_chunk_tail(const char* rowptr, int kb, int kbytes) {
@@ -921,22 +927,21 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
                     lo = b1 ? recv : lo;
                     hi = b1 ? hi : recv;
                 }
-            if (ep.c_vec_ok && c0 + 16 <= out_n1) {
+            if (c0 + 16 <= out_n1) {
                 const int row0 = grow - (l32 & 3);  // first row of the quad
                 char* qdst = ep.C + (int64_t)row0 * ep.ldc + (int64_t)(c0 + 4 * (l32 & 3)) * SZ;
 #pragma unroll
                 for (int t = 0; t < 4; t++)
                     if (row0 + t < g.M)
-                        *reinterpret_cast<u32x4*>(qdst + (int64_t)t * ep.ldc) = u32x4{tr[4 * t], tr[4 * t + 1], tr[4 * t + 2], tr[4 * t + 3]};
+                        store16<SZ>(qdst + (int64_t)t * ep.ldc, u32x4{tr[4 * t], tr[4 * t + 1], tr[4 * t + 2], tr[4 * t + 3]});
                 return;
             }
         }
         if (grow >= g.M || c0 >= out_n1) return;
         char* dst = ep.C + (int64_t)grow * ep.ldc + (int64_t)c0 * SZ;
-        if (ep.c_vec_ok && c0 + 16 <= out_n1) {
+        if (c0 + 16 <= out_n1) {
 #pragma unroll
-            for (int t = 0; t < DW; t++)
-                *reinterpret_cast<u32x4*>(dst + 16 * t) = u32x4{o[4 * t], o[4 * t + 1], o[4 * t + 2], o[4 * t + 3]};
+            for (int t = 0; t < DW; t++) store16<SZ>(dst + 16 * t, u32x4{o[4 * t], o[4 * t + 1], o[4 * t + 2], o[4 * t + 3]});
         } else {
 #pragma unroll
             for (int e = 0; e < 16; e++) {
