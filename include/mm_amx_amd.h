@@ -192,6 +192,17 @@ size_t mmx_gemm_workspace_bytes(int a_dtype, int b_dtype, int M, int K, int N, i
 int mmx_gemm_splitk_static(int a_dtype, int b_dtype, const void* A, int64_t lda_bytes, const void* Bpacked, int M,
                            int K, int N, int n0, int n1, const mmx_epilogue* ep, int k_splits, void* stream);
 
+/* ---- C = PP(A · B) straight from a row-major B that is used once: amx_kernel::Matmul with constB = false
+ * (include/kernels_amx.hpp:1188-1192), without packing B first.  dtype MMX_BF16; B is [K, N], or [N, K] with transpose, row
+ * stride ldb_bytes; the post-op as in mmx_gemm (SILU_GATE excepted).
+ * K must be a multiple of 32, N of 8 (with transpose: at least 8), rows of A and B at most 16 and 8 MiB apart
+ * (MMX_E_UNSUPPORTED otherwise).  mmx_gemm_unpacked_workspace_bytes() says whether this is the faster way: -1 = no, or
+ * not possible: use mmx_repack_b and mmx_gemm; 0 = yes, no workspace used; otherwise the bytes of workspace with which K is
+ * split (same layout and rules as mmx_gemm_splitk's; with less, or NULL, fewer slices or none).  Call mmx_init first. */
+int64_t mmx_gemm_unpacked_workspace_bytes(int dtype, int M, int K, int N, int64_t lda_bytes, int64_t ldb_bytes, int transpose);
+int mmx_gemm_unpacked(int dtype, const void* A, int64_t lda_bytes, const void* B, int64_t ldb_bytes, int transpose, int M, int K,
+                      int N, const mmx_epilogue* ep, void* workspace, size_t workspace_bytes, void* stream);
+
 /* ---- c[M] = A[M, K] · b[K]: amx_kernel::MatmulVector::operator() (include/kernels_amx.hpp:959)
  * and amx_kernel::GemAvB::operator() (:1534).  dtype MMX_BF16 (c fp32) or MMX_I8 (c int32). */
 int mmx_matvec(int dtype, const void* A, int64_t lda_bytes, const void* b, void* c, int M, int K, void* stream);

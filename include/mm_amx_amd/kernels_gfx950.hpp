@@ -414,8 +414,19 @@ struct Matmul {
         require(K == matB.dims[transposeB ? 1 : 0], "Matmul: K of A and B differ");
         require(K >= kStep, "Matmul: K must be at least kStep");  // include/kernels_amx.hpp:1183
         require(ppkernel.out_rows() >= M && ppkernel.out_cols() >= n1, "Matmul: C is smaller than M x n1");
-        if (!constB || !internalB) internalB = repackB_1x2(matB, transposeB, stream);
         const mmx_epilogue e = ppkernel.descriptor();
+        if (!constB && k_splits == 0 && n0 == 0 && n1 == N && std::is_same<TA, bfloat16>::value && std::is_same<TB, bfloat16>::value) {
+            const int64_t need = mmx_gemm_unpacked_workspace_bytes(MMX_BF16, M, K, N, matA.stride, matB.stride, transposeB ? 1 : 0);
+            if (need >= 0) {  // B is read where it lies
+                const Workspace ws = need ? workspace_for(stream, (size_t)need) : Workspace();
+                check(mmx_gemm_unpacked(MMX_BF16, matA.data, matA.stride, matB.data, matB.stride, transposeB ? 1 : 0, M, K, N, &e, ws.data,
+                                        ws.bytes, stream),
+                      "Matmul (B not packed)");
+                internalB = PackedB<TB>();
+                return;
+            }
+        }
+        if (!constB || !internalB) internalB = repackB_1x2(matB, transposeB, stream);
         if (is_u8_mode) {  // tdpbusd / tdpbsud / tdpbuud: mmx_gemm_u8 (three passes, exact)
             const size_t need = mmx_gemm_u8_scratch_bytes(dtype_of<TA>::value, dtype_of<TB>::value, M, K, N, n0, n1);
             if (need > u8_scratch_bytes) {

@@ -17,7 +17,8 @@ _LIB_PATH = os.environ.get("MMX_LIB_PATH") or os.path.join(_HERE, "libmm_amx_amd
 
 EXPORTS = ["mmx_last_error", "mmx_init", "mmx_packed_b_bytes", "mmx_repack_b", "mmx_repack_gate_up",
            "mmx_quantize_weights", "mmx_quantize_weights_scaled", "mmx_quantize_pack_int4", "mmx_dequant_packed", "mmx_gemm", "mmx_gemm_splitk",
-           "mmx_gemm_splitk_static", "mmx_gemm_workspace_bytes", "mmx_gemm_u8_scratch_bytes", "mmx_gemm_u8", "mmx_matvec_u8", "mmx_matvec", "mmx_mlp", "mmx_mlp_splitk", "mmx_set_tile",
+           "mmx_gemm_splitk_static", "mmx_gemm_workspace_bytes", "mmx_gemm_unpacked_workspace_bytes", "mmx_gemm_unpacked",
+           "mmx_gemm_u8_scratch_bytes", "mmx_gemm_u8", "mmx_matvec_u8", "mmx_matvec", "mmx_mlp", "mmx_mlp_splitk", "mmx_set_tile",
            "mmx_set_option", "mmx_last_kernel"]
 # measurement aids (include/mm_amx_amd_bench.h)
 BENCH_EXPORTS = ["mmx_time_gemm", "mmx_probe_mfma", "mmx_probe_read"]
@@ -74,6 +75,10 @@ def lib():
                                              C.c_int, C.c_int, C.POINTER(_Epilogue), C.c_int, C.c_void_p]
         l.mmx_gemm_workspace_bytes.restype = C.c_size_t
         l.mmx_gemm_workspace_bytes.argtypes = [C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_uint32, C.c_int]
+        l.mmx_gemm_unpacked_workspace_bytes.restype = C.c_int64
+        l.mmx_gemm_unpacked_workspace_bytes.argtypes = [C.c_int, C.c_int, C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int]
+        l.mmx_gemm_unpacked.argtypes = [C.c_int, C.c_void_p, C.c_int64, C.c_void_p, C.c_int64, C.c_int, C.c_int, C.c_int, C.c_int,
+                                        C.POINTER(_Epilogue), C.c_void_p, C.c_size_t, C.c_void_p]
         l.mmx_gemm_u8_scratch_bytes.restype = C.c_size_t
         l.mmx_gemm_u8_scratch_bytes.argtypes = [C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int]
         l.mmx_gemm_u8.argtypes = [C.c_int, C.c_int, C.c_void_p, C.c_int64, C.c_void_p, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int,
@@ -282,6 +287,11 @@ def _check_gemm_args(A, Bpacked, N, ep, b_dt, n0, n1):
     need = _packed_bytes_host(b_dt, K, N)
     if Bpacked.numel() < need:
         raise MmxError(f"Bpacked holds {Bpacked.numel()} bytes, a packed [{K}, {N}] matrix takes {need}")
+    _check_result_args(ep, M, n1)
+    return M, K, a_dt
+
+
+def _check_result_args(ep, M, n1):
     Cout = ep.C
     _is_2d(Cout, "C")
     ncols = n1 // 2 if ep.steps & PP_SILU_GATE else n1
@@ -290,7 +300,6 @@ def _check_gemm_args(A, Bpacked, N, ep, b_dt, n0, n1):
     for v, name in ((ep.bias, "bias"), (ep.deq_oc, "deq_scale_per_oc"), (ep.q_oc, "q_scale_per_oc")):
         if v is not None and v.numel() < n1:
             raise MmxError(f"{name} holds {v.numel()} values, columns up to {n1} are computed")
-    return M, K, a_dt
 
 
 def _packed_bytes_host(dtype, K, N):
@@ -349,6 +358,29 @@ def gemm_static(A, Bpacked, N, ep, b_dtype=None, n0=0, n1=None, k_splits=0):
     s = ep.struct()
     _check(lib().mmx_gemm_splitk_static(a_dt, b_dt, A.data_ptr(), _row_stride_bytes(A), Bpacked.data_ptr(), M, K, N, n0, n1,
                                         C.byref(s), k_splits, _stream()))
+
+
+def gemm_unpacked(A, B, transpose, ep):
+    """C = PP(A · B) straight from a row-major bf16 B ([K,N], or [N,K] with transpose) that is used once.  Returns False,
+    and does nothing, where packing B first is faster or the only way (repack_b, gemm)."""
+    _is_2d(A, "A"), _is_2d(B, "B")
+    if A.dtype != torch.bfloat16 or B.dtype != torch.bfloat16:
+        return False
+    _dev(A, "A"), _dev(B, "B")
+    M, K = A.shape
+    N = B.shape[0] if transpose else B.shape[1]
+    if B.shape[1 if transpose else 0] != K:
+        raise MmxError(f"K of A ({K}) and B ({B.shape[1 if transpose else 0]}) differ")
+    lda, ldb = _row_stride_bytes(A), _row_stride_bytes(B)
+    need = lib().mmx_gemm_unpacked_workspace_bytes(BF16, M, K, N, lda, ldb, int(transpose))
+    if need < 0:
+        return False
+    _check_result_args(ep, M, N)
+    s = ep.struct()
+    ws = workspace(A.device, need) if need else None
+    _check(lib().mmx_gemm_unpacked(BF16, A.data_ptr(), lda, B.data_ptr(), ldb, int(transpose), M, K, N, C.byref(s),
+                                   None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), _stream()))
+    return True
 
 
 def gemm_u8(A, Bpacked, N, ep, b_unsigned, n0=0, n1=None, scratch=None):

@@ -73,6 +73,11 @@ size_t plan_workspace_bytes(int elesz, bool w8, int M, int K, int Ncols, uint32_
 bool skinny_i8_eligible(const void* x, int64_t ldx, int M, int K);
 int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int K, int N, int n0, int n1,
                   const Epilogue& ep, hipStream_t st, const SplitRequest* rq);
+bool unpacked_can(int M, int K, int N, int64_t lda, int64_t ldb, int transpose);
+bool unpacked_takes(int M, int K, int N, int64_t lda, int64_t ldb, int transpose);
+size_t unpacked_workspace_bytes(int M, int K, int N, int transpose);
+int launch_unpacked(const void* A, int64_t lda, const void* B, int64_t ldb, int transpose, int M, int K, int N, const Epilogue& ep, char* ws,
+                    size_t ws_bytes, hipStream_t st);
 int launch_repack(int elesz, const void* B, int64_t ldb, int K, int N, int transpose, void* out, hipStream_t st, int flip);
 size_t u8_scratch_bytes(bool a_unsigned, int M, int K, int n1);
 int launch_gemm_x8(bool a_unsigned, bool b_unsigned, const void* A, int64_t lda, const void* Bp, int M, int K, int N, int n0, int n1,
@@ -347,6 +352,31 @@ size_t mmx_gemm_workspace_bytes(int a_dtype, int b_dtype, int M, int K, int N, i
         return k_splits == 0 && !(steps & MMX_PP_SILU_GATE) ? skinny_workspace_bytes(i8 ? 3 : (w4 ? 2 : (w8 ? 1 : 0)), M, K, n0, n1) : 0;
     if ((!bf && !i8 && !w8) || M <= 32 || K <= 0 || N <= 0 || n0 < 0 || n1 > N || n0 >= n1 || k_splits < 0) return 0;
     return plan_workspace_bytes(i8 ? 1 : 2, w8, M, K, n1 - n0, steps, k_splits);
+}
+
+int64_t mmx_gemm_unpacked_workspace_bytes(int dtype, int M, int K, int N, int64_t lda_bytes, int64_t ldb_bytes, int transpose) {
+    // a forced tile asks for the tile kernels, which take packed weights
+    if (dtype != MMX_BF16 || forced_tile().bm != 0 || !unpacked_takes(M, K, N, lda_bytes, ldb_bytes, transpose)) return -1;
+    return (int64_t)unpacked_workspace_bytes(M, K, N, transpose);
+}
+
+int mmx_gemm_unpacked(int dtype, const void* A, int64_t lda_bytes, const void* B, int64_t ldb_bytes, int transpose, int M, int K, int N,
+                      const mmx_epilogue* ep_in, void* workspace, size_t workspace_bytes, void* stream) {
+    if (!A || !B) return set_error(MMX_E_INVALID, "mmx_gemm_unpacked: NULL operand");
+    if (M <= 0 || K <= 0 || N <= 0) return set_error(MMX_E_INVALID, "mmx_gemm_unpacked: M, K, N must be positive (got %d, %d, %d)", M, K, N);
+    if (dtype != MMX_BF16 || !unpacked_can(M, K, N, lda_bytes, ldb_bytes, transpose))
+        return set_error(MMX_E_UNSUPPORTED, "mmx_gemm_unpacked: this shape or type takes packed weights (mmx_repack_b, mmx_gemm)");
+    if (lda_bytes < (int64_t)K * 2) return set_error(MMX_E_INVALID, "mmx_gemm_unpacked: lda_bytes %lld smaller than a row of A", (long long)lda_bytes);
+    if (ldb_bytes < (int64_t)(transpose ? K : N) * 2) return set_error(MMX_E_INVALID, "mmx_gemm_unpacked: ldb_bytes %lld smaller than a row of B", (long long)ldb_bytes);
+    if ((lda_bytes | ldb_bytes) % 2 || (reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) % 2)
+        return set_error(MMX_E_INVALID, "mmx_gemm_unpacked: A or B is not aligned to its element size");
+    if (reinterpret_cast<uintptr_t>(workspace) & 255) return set_error(MMX_E_INVALID, "mmx_gemm_unpacked: the workspace must be 256-byte aligned");
+    Epilogue ep;
+    int rc = make_epilogue(ep_in, MMX_BF16, MMX_BF16, M, 0, N, &ep);
+    if (rc) return rc;
+    if (ep.steps & MMX_PP_SILU_GATE) return set_error(MMX_E_INVALID, "mmx_gemm_unpacked: SILU_GATE needs gate and up panels packed in turn");
+    return launch_unpacked(A, lda_bytes, B, ldb_bytes, transpose, M, K, N, ep, static_cast<char*>(workspace), workspace_bytes,
+                           static_cast<hipStream_t>(stream));
 }
 
 int mmx_matvec(int dtype, const void* A, int64_t lda_bytes, const void* b, void* c, int M, int K, void* stream) {

@@ -99,8 +99,8 @@ class Matmul:
     main.cpp:32-80.  ``weight_int8=True`` gives Matmul<bf16,int8,float> (:1319-1516): the bf16 B is
     compressed to int8 per tensor on first use and the op sets the post-op's dequant scale.
 
-    The packed weights are cached when ``constB`` (as :1188-1192); otherwise B is repacked on
-    every call.  Not thread-safe, like the reference; calls are ordered on the current stream."""
+    The packed weights are cached when ``constB`` (as :1188-1192); otherwise B is used where it lies (bf16, few rows
+    of A) or repacked on every call.  Not thread-safe, like the reference; calls are ordered on the current stream."""
 
     def __init__(self, constB=False, transposeB=False, weight_int8=False):
         self.constB, self.transposeB, self.weight_int8 = constB, transposeB, weight_int8
@@ -119,6 +119,9 @@ class Matmul:
             raise L.MmxError(f"Matmul: K = {K} must be at least {kstep}")
         n0 = 0 if n0 is None else n0
         n1 = N if n1 is None else n1
+        if not self.constB and not self.weight_int8 and n0 == 0 and n1 == N and L.gemm_unpacked(matA, matB, self.transposeB, ppkernel.descriptor()):
+            self.internalB = None  # read where it lay: nothing was packed
+            return
         if not self.constB or self.internalB is None:
             if self.weight_int8:
                 if matB.dtype != torch.bfloat16:

@@ -1,0 +1,141 @@
+"""Matmul with a second operand that is used once (constB = False): read where it lies, without packing.  Operands are small
+integers, so that every order of fp32 summation gives the same sums and results have to equal the packed form's, and the
+64-bit product, exactly."""
+import ctypes
+
+import pytest
+import torch
+
+import mm_amx_amd as mx
+from mm_amx_amd import _lib as L
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _init():
+    mx.init(0)
+
+
+def _ints(shape, seed, pad=0):
+    """Integers of [-8, 8] as bf16, inside a wider matrix of NaN when pad > 0 (rows of any alignment)."""
+    t = torch.randint(-8, 9, shape, generator=torch.Generator().manual_seed(seed)).to(torch.bfloat16).cuda()
+    if not pad:
+        return t
+    wide = torch.full((shape[0] + 1, shape[1] + pad), float("nan"), dtype=torch.bfloat16, device="cuda")
+    wide[:-1, pad // 2:pad // 2 + shape[1]] = t
+    return wide[:-1, pad // 2:pad // 2 + shape[1]]
+
+
+def _run(const, trans, A, B, C, **kw):
+    pp = mx.BiasGeluStore(C, kw.get("steps", mx.Steps.NONE), kw.get("bias"))
+    if "q" in kw:
+        pp.set_q_scale(kw["q"])
+    mx.Matmul(const, trans)(A, B, ppkernel=pp)
+    return C
+
+
+def _entry(trans, A, B, C):
+    """The C entry itself, which also takes the shapes for which packing first is the faster way."""
+    (M, K), N = A.shape, C.shape[1]
+    s, ws = L.Epilogue(C).struct(), L.workspace()
+    L._check(L.lib().mmx_gemm_unpacked(L.BF16, A.data_ptr(), L._row_stride_bytes(A), B.data_ptr(), L._row_stride_bytes(B), int(trans), M, K, N,
+                                       ctypes.byref(s), ws.data_ptr(), ws.numel(), L._stream()))
+
+
+# one step of k for one wavefront, shares with and without a remainder, a K split and none; rows on both sides of a block
+# of 16, 32 and 64; a strip of 128 columns with 8 of them live, full, and one more
+@pytest.mark.parametrize("trans", [False, True])
+@pytest.mark.parametrize("M,K,N", [(1, 32, 8), (15, 288, 128), (16, 4096, 136), (17, 1056, 264), (32, 8192, 256), (33, 96, 640),
+                                   (64, 2080, 384), (65, 4096, 128), (130, 640, 1000), (256, 1024, 1024), (300, 4128, 200)])
+@pytest.mark.parametrize("pad", [0, 5])
+def test_exact_sums(M, K, N, trans, pad):
+    A, B = _ints((M, K), 1, pad), _ints((N, K) if trans else (K, N), 2, pad)
+    wide = torch.full((M + 1, N + 3), -7.0, device="cuda")
+    _entry(trans, A, B, wide[:M, :N])
+    assert mx.last_kernel().startswith("unpacked_" + ("nk" if trans else "kn")), mx.last_kernel()
+    ref = A.double() @ (B.double().t() if trans else B.double())
+    assert torch.equal(wide[:M, :N].double(), ref)
+    assert (wide[M] == -7.0).all() and (wide[:, N:] == -7.0).all()  # nothing beyond the result is written
+    again = torch.empty((M, N), device="cuda")
+    for _ in range(3):  # (the arrival counters are back at zero)
+        _entry(trans, A, B, again)
+    assert torch.equal(again.double(), ref)
+    assert torch.equal(_run(False, trans, A, B, again.zero_()).double(), ref)  # whichever way the rule takes
+
+
+@pytest.mark.parametrize("N", [8, 131, 250])
+def test_any_column_count_from_rows_of_k(N):
+    A, B = _ints((24, 96), 3), _ints((N, 96), 4)
+    C = _run(False, True, A, B, torch.empty((24, N), device="cuda"))
+    assert mx.last_kernel().startswith("unpacked_nk")
+    assert torch.equal(C.double(), A.double() @ B.double().t())
+
+
+@pytest.mark.parametrize("out", [torch.float32, torch.bfloat16, torch.int8])
+@pytest.mark.parametrize("steps", [mx.Steps.NONE, mx.Steps.BIAS, mx.Steps.BIAS_GELU, mx.Steps.DEQUANT_BIAS_GELU_QUANT])
+def test_post_ops_equal_the_packed_form(out, steps):
+    M, K, N = 19, 2048, 264
+    A, B = _ints((M, K), 5), _ints((K, N), 6)
+    kw = {"steps": steps, "bias": torch.linspace(-3, 3, N, device="cuda") if steps & mx.Steps.BIAS else None}
+    if steps & mx.Steps.QUANT:
+        kw["q"] = torch.linspace(0.01, 0.1, N, device="cuda")
+    got = _run(False, False, A, B, torch.empty((M, N), dtype=out, device="cuda"), **kw)
+    assert mx.last_kernel().startswith("unpacked_kn")
+    want = _run(True, False, A, B, torch.empty((M, N), dtype=out, device="cuda"), **kw)
+    assert torch.equal(got, want)
+
+
+def test_infinities_stay_in_their_column_and_row():
+    M, K, N = 20, 320, 200
+    A, B = _ints((M, K), 7), _ints((N, K), 8)
+    B[5, 0], A[3, 1] = float("inf"), float("nan")
+    got = _run(False, True, A, B, torch.empty((M, N), device="cuda"))
+    want = _run(True, True, A, B, torch.empty((M, N), device="cuda"))
+    assert torch.equal(torch.isfinite(got), torch.isfinite(want))
+    ok = torch.isfinite(want)
+    assert torch.equal(got[ok], want[ok])
+
+
+def test_what_it_does_not_take_is_packed():
+    for (M, K, N), trans in [((4, 40, 64), False), ((4, 64, 63), False), ((2000, 256, 256), False), ((4, 33, 64), True)]:
+        A, B = _ints((M, K), 9), _ints((N, K) if trans else (K, N), 10)
+        C = _run(False, trans, A, B, torch.empty((M, N), device="cuda"))
+        assert not mx.last_kernel().startswith("unpacked")
+        assert torch.equal(C.double(), A.double() @ (B.double().t() if trans else B.double()))
+
+
+def test_column_ranges_are_packed():
+    A, B = _ints((4, 64), 11), _ints((64, 96), 12)
+    C = torch.zeros((4, 96), device="cuda")
+    mx.Matmul(False, False)(A, B, 32, 64, mx.BiasGeluStore(C))
+    assert torch.equal(C[:, 32:64].double(), (A.double() @ B.double())[:, 32:64]) and not C[:, :32].any() and not C[:, 64:].any()
+
+
+def test_replays_from_a_hip_graph():
+    M, K, N = 24, 8192, 256
+    A, B, C = _ints((M, K), 13), _ints((K, N), 14), torch.empty((M, N), device="cuda")
+    op, pp = mx.Matmul(False, False), mx.BiasGeluStore(C)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        op(A, B, ppkernel=pp)
+        side.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            op(A, B, ppkernel=pp)
+    for seed in range(15, 19):
+        A.copy_(_ints((M, K), seed))
+        C.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(C.double(), A.double() @ B.double())
+
+
+def test_errors_of_the_c_entry():
+    A, B, C = _ints((4, 64), 1), _ints((64, 64), 2), torch.empty((4, 64), device="cuda")
+    s = L.Epilogue(C).struct()
+    call = lambda dt, lda, ldb, st: L.lib().mmx_gemm_unpacked(dt, A.data_ptr(), lda, B.data_ptr(), ldb, 0, 4, 64, 64, ctypes.byref(st), None, 0, L._stream())
+    assert call(L.BF16, 128, 128, s) == 0
+    assert call(L.I8, 128, 128, s) != 0 and call(L.BF16, 126, 128, s) != 0 and call(L.BF16, 128, 126, s) != 0 and call(L.BF16, 129, 128, s) != 0
+    s.steps = L.PP_SILU_GATE
+    assert call(L.BF16, 128, 128, s) != 0
