@@ -112,14 +112,19 @@ def init(device=0):
         _initialised.add(device)
 
 
+# What a call costs before its launch is what bounds the small shapes (256 x 256 x 256: 12.4 us a call, 6 us of them on the
+# device), so the helpers that every call passes are kept to plain attribute reads: the raw stream handle instead of a
+# Stream object, one stride() instead of several, no query of the library whose answer the call does not need.
 def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _dev(t, what):
     if not (isinstance(t, torch.Tensor) and t.is_cuda):
         raise MmxError(f"{what} must be a tensor on the GPU")
-    init(t.device.index or 0)
+    d = t.get_device()
+    if d not in _initialised:
+        init(d)
     return t
 
 
@@ -136,11 +141,11 @@ def dtype_code(t):
 def _row_stride_bytes(t):
     # torch leaves the stride of a dimension of size 1 arbitrary: a single column is contiguous whatever
     # stride(1) says, and a single row has no row stride to speak of
-    if t.dim() != 2 or (t.stride(1) != 1 and t.shape[1] != 1):
+    st = t.stride()
+    if len(st) != 2 or (st[1] != 1 and t.shape[1] != 1):
         raise MmxError("expected a 2-D tensor with unit stride in its last dimension")
-    if t.shape[0] == 1:
-        return t.shape[1] * t.element_size()
-    return t.stride(0) * t.element_size()
+    rows, cols = t.shape
+    return (cols if rows == 1 else st[0]) * t.element_size()
 
 
 class Epilogue:
@@ -152,14 +157,22 @@ class Epilogue:
         self.steps = int(steps)
         self.bias, self.deq_oc, self.q_oc = bias, deq_scale_per_oc, q_scale_per_oc
         self.deq, self.q = float(deq_scale), float(q_scale)
-        for v, name in ((bias, "bias"), (deq_scale_per_oc, "deq_scale_per_oc"), (q_scale_per_oc, "q_scale_per_oc")):
-            if v is not None and not (v.is_cuda and v.dtype == torch.float32 and v.is_contiguous()):
-                raise MmxError(f"{name} must be a contiguous fp32 tensor on the GPU")
+        if bias is not None:
+            _column_operand(bias, "bias")
+        if deq_scale_per_oc is not None:
+            _column_operand(deq_scale_per_oc, "deq_scale_per_oc")
+        if q_scale_per_oc is not None:
+            _column_operand(q_scale_per_oc, "q_scale_per_oc")
 
     def struct(self):
-        p = lambda t: None if t is None else t.data_ptr()
-        return _Epilogue(self.steps, dtype_code(self.C), self.C.data_ptr(), _row_stride_bytes(self.C), p(self.bias),
-                         self.deq, p(self.deq_oc), self.q, p(self.q_oc))
+        out, bias, deq_oc, q_oc = self.C, self.bias, self.deq_oc, self.q_oc
+        return _Epilogue(self.steps, dtype_code(out), out.data_ptr(), _row_stride_bytes(out), None if bias is None else bias.data_ptr(),
+                         self.deq, None if deq_oc is None else deq_oc.data_ptr(), self.q, None if q_oc is None else q_oc.data_ptr())
+
+
+def _column_operand(v, name):
+    if not (v.is_cuda and v.dtype == torch.float32 and v.is_contiguous()):
+        raise MmxError(f"{name} must be a contiguous fp32 tensor on the GPU")
 
 
 def packed_b_bytes(dtype, K, N):
@@ -248,7 +261,7 @@ def workspace(device=None, nbytes=WORKSPACE_BYTES):
     being captured into a graph and has no workspace of that size yet (an allocation there would be captured
     too).  At most _MAX_WORKSPACES are kept (the oldest is dropped); release_workspaces() drops them all."""
     dev_index = torch.cuda.current_device() if device is None else (device.index or 0)
-    key = (dev_index, torch.cuda.current_stream(dev_index).cuda_stream)
+    key = (dev_index, torch._C._cuda_getCurrentRawStream(dev_index))
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
         if torch.cuda.is_current_stream_capturing():
@@ -292,14 +305,16 @@ def _check_gemm_args(A, Bpacked, N, ep, b_dt, n0, n1):
 
 
 def _check_result_args(ep, M, n1):
-    Cout = ep.C
-    _is_2d(Cout, "C")
+    _is_2d(ep.C, "C")
     ncols = n1 // 2 if ep.steps & PP_SILU_GATE else n1
-    if Cout.shape[0] < M or Cout.shape[1] < ncols:
-        raise MmxError(f"C is {tuple(Cout.shape)}, the result needs at least [{M}, {ncols}]")
-    for v, name in ((ep.bias, "bias"), (ep.deq_oc, "deq_scale_per_oc"), (ep.q_oc, "q_scale_per_oc")):
-        if v is not None and v.numel() < n1:
-            raise MmxError(f"{name} holds {v.numel()} values, columns up to {n1} are computed")
+    rows, cols = ep.C.shape
+    if rows < M or cols < ncols:
+        raise MmxError(f"C is {(rows, cols)}, the result needs at least [{M}, {ncols}]")
+    if (ep.bias is not None and ep.bias.numel() < n1) or (ep.deq_oc is not None and ep.deq_oc.numel() < n1) or \
+            (ep.q_oc is not None and ep.q_oc.numel() < n1):
+        for v, name in ((ep.bias, "bias"), (ep.deq_oc, "deq_scale_per_oc"), (ep.q_oc, "q_scale_per_oc")):
+            if v is not None and v.numel() < n1:
+                raise MmxError(f"{name} holds {v.numel()} values, columns up to {n1} are computed")
 
 
 def _packed_bytes_host(dtype, K, N):
@@ -308,7 +323,7 @@ def _packed_bytes_host(dtype, K, N):
         return 0
     if dtype == I4:
         return ((N + 31) // 32) * ((K + 255) // 256 * 4) * 1024
-    es = {BF16: 2, I8: 1, U8: 1}.get(dtype, 0)
+    es = 2 if dtype == BF16 else 1 if dtype in (I8, U8) else 0
     return ((N + 31) // 32) * 32 * ((K * es + 127) // 128 * 128)
 
 
@@ -316,9 +331,15 @@ def _split_args(A, k_splits, ws, need):
     """(k_splits, workspace pointer, bytes).  Without an explicit workspace the stream's own one is used, and it is
     only created when the library says the call can use one (`need` = mmx_gemm_workspace_bytes of the call, a
     callable): a shape that never splits allocates nothing."""
-    if k_splits == 1 and ws is None:
-        return 1, None, 0
     if ws is None:
+        if k_splits == 1:
+            return 1, None, 0
+        if k_splits == 0:
+            # the workspace this stream already has serves every choice of the library's own, which then need not be asked
+            device = A.get_device()
+            ws = _workspaces.get((device, torch._C._cuda_getCurrentRawStream(device)))
+            if ws is not None:
+                return 0, ws.data_ptr(), ws.numel()
         nbytes = need()
         if nbytes == 0 and k_splits == 0:
             return 1, None, 0

@@ -45,7 +45,7 @@ class BiasGeluStore:
         self.bias = bias
 
     def set_deq_scale(self, scale=1.0):
-        if not self.steps & Steps.DEQUANT:
+        if not int(self.steps) & L.PP_DEQUANT:  # (plain integers: an IntFlag's & costs half a microsecond, and Matmul calls this)
             raise L.MmxError("set_deq_scale: DEQUANT step not enabled")
         if isinstance(scale, torch.Tensor):
             self.deq_scale, self.deq_scale_per_oc = 1.0, scale
