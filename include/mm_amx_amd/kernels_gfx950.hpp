@@ -417,7 +417,11 @@ struct Matmul {
         const mmx_epilogue e = ppkernel.descriptor();
         if (!constB && k_splits == 0 && n0 == 0 && n1 == N && std::is_same<TA, bfloat16>::value && std::is_same<TB, bfloat16>::value) {
             const int64_t need = mmx_gemm_unpacked_workspace_bytes(MMX_BF16, M, K, N, matA.stride, matB.stride, transposeB ? 1 : 0);
-            if (need >= 0) {  // B is read where it lies
+            // a result that is written over B: other workgroups may still be reading it, a packed copy is safe
+            const uintptr_t b0 = reinterpret_cast<uintptr_t>(matB.data), c0 = reinterpret_cast<uintptr_t>(e.C);
+            const uintptr_t b_end = b0 + (size_t)matB.dims[0] * matB.stride;
+            const uintptr_t c_end = c0 + (size_t)M * e.ldc_bytes;
+            if (need >= 0 && (c0 >= b_end || b0 >= c_end)) {  // B is read where it lies
                 const Workspace ws = need ? workspace_for(stream, (size_t)need) : Workspace();
                 check(mmx_gemm_unpacked(MMX_BF16, matA.data, matA.stride, matB.data, matB.stride, transposeB ? 1 : 0, M, K, N, &e, ws.data,
                                         ws.bytes, stream),

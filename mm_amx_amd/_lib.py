@@ -398,6 +398,10 @@ def gemm_unpacked(A, B, transpose, ep):
         return False
     _check_result_args(ep, M, N)
     s = ep.struct()
+    # a result that is written over B: other workgroups may still be reading it, a packed copy is safe
+    b0, c0 = B.data_ptr(), s.C
+    if c0 < b0 + (B.shape[0] - 1) * ldb + 2 * B.shape[1] and b0 < c0 + (M - 1) * s.ldc_bytes + N * ep.C.element_size():
+        return False
     ws = workspace(A.device, need) if need else None
     _check(lib().mmx_gemm_unpacked(BF16, A.data_ptr(), lda, B.data_ptr(), ldb, int(transpose), M, K, N, C.byref(s),
                                    None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), _stream()))

@@ -112,6 +112,22 @@ def test_column_ranges_are_packed():
     assert torch.equal(C[:, 32:64].double(), (A.double() @ B.double())[:, 32:64]) and not C[:, :32].any() and not C[:, 64:].any()
 
 
+@pytest.mark.parametrize("trans", [False, True])
+def test_a_result_over_b_is_packed(trans):
+    M, K, N = 24, 512, 512
+    A, B = _ints((M, K), 16), _ints((K, N), 17)
+    ref = A.double() @ (B.double().t() if trans else B.double())
+    for rows in (slice(0, M), slice(K - M, K)):
+        over = B.clone()
+        C = over[rows]  # the first and the last rows of B itself
+        _run(False, trans, A, over, C)
+        assert not mx.last_kernel().startswith("unpacked")
+        assert torch.equal(C, ref.to(torch.bfloat16))
+    both = torch.cat([B, B[:M]])  # right behind B: no overlap
+    _run(False, trans, A, both[:K], both[K:])
+    assert mx.last_kernel().startswith("unpacked") and torch.equal(both[K:], ref.to(torch.bfloat16))
+
+
 def test_replays_from_a_hip_graph():
     M, K, N = 24, 8192, 256
     A, B, C = _ints((M, K), 13), _ints((K, N), 14), torch.empty((M, N), device="cuda")
