@@ -33,6 +33,10 @@ constexpr int RED_ROW = STRIP + 4;   // floats; the pad spreads 16 rows over the
 constexpr int MAX_SLICES = 16;
 constexpr int MAX_TILES = 4096;      // counters at the head of a workspace
 constexpr size_t COUNTER_BYTES = (size_t)MAX_TILES * 4;
+// What the front ends allocate once per stream.  No launch asks for more or uses more: a larger answer would replace the
+// stream's buffer, which a graph captured earlier may still write to, and the slices of a call would depend on its history.
+// (It takes slices from wide results only, where the CUs have strips enough: 128 x 8192 x 50304 334 us unsplit, 338 in four.)
+constexpr size_t STANDARD_WORKSPACE_BYTES = ((size_t)64 << 20) + ((size_t)16 << 10);
 
 // 16 bytes from any even address (the hardware takes them at any)
 typedef u32x4 __attribute__((aligned(2))) u32x4_any;
@@ -299,6 +303,7 @@ static size_t workspace_for_slices(int M, int N, int S) { return COUNTER_BYTES +
 // step is twice as long and comes in pieces of 64 bytes; the chip as a whole
 // does not take B in faster than 5.5 TB/s; each slice adds to the combination.
 static int choose_slices(int M, int K, int N, int transpose, size_t ws_bytes) {
+    if (ws_bytes > STANDARD_WORKSPACE_BYTES) ws_bytes = STANDARD_WORKSPACE_BYTES;
     const int mb = row_blocks(M), nw = mb == 4 ? 4 : 8;
     const int tiles = tile_count(M, N);
     const int steps = transpose ? (K + 63) / 64 : K / 32, cus = num_cus();
@@ -337,7 +342,7 @@ bool unpacked_takes(int M, int K, int N, int64_t lda, int64_t ldb, int transpose
 }
 
 size_t unpacked_workspace_bytes(int M, int K, int N, int transpose) {
-    const int S = choose_slices(M, K, N, transpose, ~(size_t)0);
+    const int S = choose_slices(M, K, N, transpose, STANDARD_WORKSPACE_BYTES);
     return S > 1 ? workspace_for_slices(M, N, S) : 0;
 }
 

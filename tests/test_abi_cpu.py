@@ -82,6 +82,26 @@ def test_sizes_and_argument_validation(lib):
     assert lib.mmx_gemm_u8_scratch_bytes(2, 2, 4, 64, 64, 0, 64) == 0 and lib.mmx_gemm_u8_scratch_bytes(5, 2, 4, 64, 64, 0, 64) > 0
 
 
+def test_no_automatic_workspace_is_larger_than_the_standard_one(lib):
+    """What the library asks for when it chooses the number of K slices itself fits the buffer that both front ends make
+    once per stream (64 MiB + 16 KiB): a larger answer would replace that buffer, which a captured graph may still use."""
+    import mm_amx_amd._lib as L
+    unpacked, packed = lib.mmx_gemm_unpacked_workspace_bytes, lib.mmx_gemm_workspace_bytes
+    unpacked.restype, packed.restype = C.c_int64, C.c_size_t
+    unpacked.argtypes = [C.c_int, C.c_int, C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int]
+    split = 0
+    for M in (1, 16, 17, 32, 33, 64, 65, 96, 128, 129, 192, 256):
+        for N in (8, 256, 1024, 4096, 8192, 13312, 16640, 34816, 50304, 100352, 151936, 200000):
+            for K in (32, 512, 2048, 4096, 6656, 8192, 11008, 14080, 16384, 65536):
+                for trans in (0, 1):
+                    need = unpacked(L.BF16, M, K, N, K * 2, (K if trans else N) * 2, trans)
+                    assert need <= L.WORKSPACE_BYTES, (M, K, N, trans, need)
+                    split += need > 0
+                for a, b in ((L.BF16, L.BF16), (L.BF16, L.I8), (L.I8, L.I8)):
+                    assert packed(a, b, M, K, N, 0, N, 0, 0) <= L.WORKSPACE_BYTES, (a, b, M, K, N)
+    assert split > 500  # (the walk meets shapes that are split)
+
+
 def test_package_fails_loudly_without_the_library(monkeypatch):
     import mm_amx_amd._lib as L
     monkeypatch.setattr(L, "_lib", None)
