@@ -348,9 +348,11 @@ size_t mmx_gemm_workspace_bytes(int a_dtype, int b_dtype, int M, int K, int N, i
     const bool bf = a_dtype == MMX_BF16 && b_dtype == MMX_BF16, i8 = a_dtype == MMX_I8 && b_dtype == MMX_I8;
     const bool w8 = a_dtype == MMX_BF16 && b_dtype == MMX_I8;
     const bool w4 = a_dtype == MMX_BF16 && b_dtype == MMX_I4;
-    if (M > 0 && M <= 32 && (bf || w8 || i8 || w4) && K > 0 && N > 0 && n0 >= 0 && n1 <= N && n0 < n1)
+    // int8 activations that the decode kernels do not take, by K or by a forced tile, go to the tile kernels at any M
+    const bool i8_tiles = i8 && M > 0 && K > 0 && (forced_tile().bm != 0 || !skinny_i8_eligible(nullptr, 0, M, K));
+    if (M > 0 && M <= 32 && !i8_tiles && (bf || w8 || i8 || w4) && K > 0 && N > 0 && n0 >= 0 && n1 <= N && n0 < n1)
         return k_splits == 0 && !(steps & MMX_PP_SILU_GATE) ? skinny_workspace_bytes(i8 ? 3 : (w4 ? 2 : (w8 ? 1 : 0)), M, K, n0, n1) : 0;
-    if ((!bf && !i8 && !w8) || M <= 32 || K <= 0 || N <= 0 || n0 < 0 || n1 > N || n0 >= n1 || k_splits < 0) return 0;
+    if ((!bf && !i8 && !w8) || (M <= 32 && !i8_tiles) || K <= 0 || N <= 0 || n0 < 0 || n1 > N || n0 >= n1 || k_splits < 0) return 0;
     return plan_workspace_bytes(i8 ? 1 : 2, w8, M, K, n1 - n0, steps, k_splits);
 }
 

@@ -22,10 +22,11 @@ int launch_gemm_tiles_bf16(const void* A, int64_t lda, const void* Bp, int M, in
     }
 }
 
-// Bytes of workspace the plan for this shape would use (0: no K split), assuming operands the ring pipeline takes.
+// Bytes of workspace the plan for this shape would use (0: no K split), assuming operands the ring pipeline takes: rows of
+// any K can be aligned through their stride, so this is an upper bound for those that are not.
 size_t plan_workspace_bytes(int elesz, bool w8, int M, int K, int Ncols, uint32_t steps, int k_splits) {
     const int64_t kbytes = (int64_t)K * elesz;
-    if (kbytes % 16 || (kbytes % 128 && (k_splits > 1 || kbytes < 128))) return 0;  // (rows of A that are not aligned, or a forced split of a K with a tail)
+    if (kbytes % 128 && (k_splits > 1 || kbytes < 128)) return 0;  // (a forced split of a K with a tail is refused)
     const SplitRequest rq = {k_splits, reinterpret_cast<char*>(256), ~(size_t)0};
     if (steps & MMX_PP_SILU_GATE) return 0;
     const Plan p = choose_plan(M, Ncols, (int)(kbytes / 128), false, w8, kbytes % 128 ? 4 : 2, rq, elesz == 1);

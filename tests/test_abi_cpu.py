@@ -102,6 +102,17 @@ def test_no_automatic_workspace_is_larger_than_the_standard_one(lib):
     assert split > 500  # (the walk meets shapes that are split)
 
 
+def test_the_workspace_query_covers_every_call_that_splits(lib):
+    """The query knows K but not the stride of A's rows: rows of any K can be 16-byte aligned, and such rows are split."""
+    import mm_amx_amd._lib as L
+    need = lib.mmx_gemm_workspace_bytes
+    need.restype = C.c_size_t
+    for a, b, K in ((L.BF16, L.BF16, 4100), (L.BF16, L.I8, 4099), (L.I8, L.I8, 8199)):
+        assert need(a, b, 64, K, 256, 0, 256, 0, 0) == need(a, b, 64, K + 16 - K % 16, 256, 0, 256, 0, 0) > 0
+    # int8 rows that the decode kernels do not take (K no multiple of 128) go to the tile kernels at any M
+    assert need(L.I8, L.I8, 16, 8256, 256, 0, 256, 0, 0) == need(L.I8, L.I8, 33, 8256, 256, 0, 256, 0, 0) > 0
+
+
 def test_package_fails_loudly_without_the_library(monkeypatch):
     import mm_amx_amd._lib as L
     monkeypatch.setattr(L, "_lib", None)

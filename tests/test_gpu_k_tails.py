@@ -69,6 +69,28 @@ def test_k_tail_behind_a_k_split(po, K):
     check_float_parity(host_bits(C), po.gemm_bf16(A, B), mx.last_kernel())
 
 
+@pytest.mark.parametrize("kind,M,K,pad", [("bf16", 64, 4100, 4), ("bf16", 64, 4100, 0), ("w8", 64, 4100, 4), ("i8", 64, 8201, 7),
+                                          ("i8", 16, 8256, 0), ("i8", 16, 8320, 0), ("bf16", 16, 8200, 0)])
+def test_the_plan_does_not_depend_on_earlier_calls(kind, M, K, pad):
+    """The first call of a stream and a call that finds the stream's workspace: the same kernel, the same bits."""
+    N = 256
+    g = torch.Generator(device="cuda").manual_seed(K)
+    A = torch.randn((M, K + pad), device="cuda", generator=g)[:, :K] if kind != "i8" else \
+        torch.randint(-127, 128, (M, K + pad), device="cuda", generator=g, dtype=torch.int8)[:, :K]
+    A = A if kind == "i8" else _in_nan(A.to(torch.bfloat16), pad)
+    W = torch.randint(-127, 128, (K, N), device="cuda", generator=g, dtype=torch.int8)
+    packed = mx.repack_b(W.to(torch.bfloat16) if kind == "bf16" else W)
+    kw = {"b_dtype": mx.I8} if kind == "w8" else {}
+    out = torch.zeros((2, M, N), dtype=torch.float32, device="cuda")
+    mx.release_workspaces()
+    mx.gemm(A, packed, N, mx.Epilogue(out[0]), **kw)
+    first = mx.last_kernel()
+    mx.workspace()
+    mx.gemm(A, packed, N, mx.Epilogue(out[1]), **kw)
+    assert mx.last_kernel() == first
+    assert torch.equal(out[0], out[1])
+
+
 def test_k_tail_gate_up(po):
     M, K, N = 70, 200, 96
     rng = np.random.default_rng(5)
