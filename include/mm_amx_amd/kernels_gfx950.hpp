@@ -421,6 +421,8 @@ struct Matmul {
             const uintptr_t b0 = reinterpret_cast<uintptr_t>(matB.data), c0 = reinterpret_cast<uintptr_t>(e.C);
             const uintptr_t b_end = b0 + (size_t)matB.dims[0] * matB.stride;
             const uintptr_t c_end = c0 + (size_t)M * e.ldc_bytes;
+            // (a stream under capture that has no workspace runs unsplit, which is slow for few columns and a long K, and whose
+            // sums can differ in the last bits: call the shape once before capturing.  Packing would need an allocation.)
             if (need >= 0 && (c0 >= b_end || b0 >= c_end)) {  // B is read where it lies
                 const Workspace ws = need ? workspace_for(stream, (size_t)need) : Workspace();
                 check(mmx_gemm_unpacked(MMX_BF16, matA.data, matA.stride, matB.data, matB.stride, transposeB ? 1 : 0, M, K, N, &e, ws.data,

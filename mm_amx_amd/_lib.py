@@ -383,7 +383,9 @@ def gemm_static(A, Bpacked, N, ep, b_dtype=None, n0=0, n1=None, k_splits=0):
 
 def gemm_unpacked(A, B, transpose, ep):
     """C = PP(A · B) straight from a row-major bf16 B ([K,N], or [N,K] with transpose) that is used once.  Returns False,
-    and does nothing, where packing B first is faster or the only way (repack_b, gemm)."""
+    and does nothing, where packing B first is faster or the only way (repack_b, gemm): also for a call that wants K slices
+    while the stream is being captured into a graph and has no workspace.  Such a first call is packed and not split, so its
+    sums can differ in the last bits from an eager call's; call the shape once eagerly before capturing to have the same."""
     _is_2d(A, "A"), _is_2d(B, "B")
     if A.dtype != torch.bfloat16 or B.dtype != torch.bfloat16:
         return False
@@ -403,6 +405,8 @@ def gemm_unpacked(A, B, transpose, ep):
     if c0 < b0 + (B.shape[0] - 1) * ldb + 2 * B.shape[1] and b0 < c0 + (M - 1) * s.ldc_bytes + N * ep.C.element_size():
         return False
     ws = workspace(A.device, need) if need else None
+    if need and ws is None:
+        return False
     _check(lib().mmx_gemm_unpacked(BF16, A.data_ptr(), lda, B.data_ptr(), ldb, int(transpose), M, K, N, C.byref(s),
                                    None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), _stream()))
     return True

@@ -100,7 +100,8 @@ class Matmul:
     compressed to int8 per tensor on first use and the op sets the post-op's dequant scale.
 
     The packed weights are cached when ``constB`` (as :1188-1192); otherwise B is used where it lies (bf16, few rows
-    of A) or repacked on every call.  Not thread-safe, like the reference; calls are ordered on the current stream."""
+    of A) or repacked on every call.  Not thread-safe, like the reference; calls are ordered on the current stream.
+    Under capture into a graph a stream without a workspace splits no K: call a shape once eagerly before capturing it."""
 
     def __init__(self, constB=False, transposeB=False, weight_int8=False):
         self.constB, self.transposeB, self.weight_int8 = constB, transposeB, weight_int8
