@@ -415,7 +415,8 @@ struct Matmul {
         require(K >= kStep, "Matmul: K must be at least kStep");  // include/kernels_amx.hpp:1183
         require(ppkernel.out_rows() >= M && ppkernel.out_cols() >= n1, "Matmul: C is smaller than M x n1");
         const mmx_epilogue e = ppkernel.descriptor();
-        if (!constB && k_splits == 0 && n0 == 0 && n1 == N && std::is_same<TA, bfloat16>::value && std::is_same<TB, bfloat16>::value) {
+        if (!constB && k_splits == 0 && n0 == 0 && n1 == N && std::is_same<TA, bfloat16>::value && std::is_same<TB, bfloat16>::value &&
+            !(e.steps & MMX_PP_SILU_GATE)) {
             const int64_t need = mmx_gemm_unpacked_workspace_bytes(MMX_BF16, M, K, N, matA.stride, matB.stride, transposeB ? 1 : 0);
             // a result that is written over B: other workgroups may still be reading it, a packed copy is safe
             const uintptr_t b0 = reinterpret_cast<uintptr_t>(matB.data), c0 = reinterpret_cast<uintptr_t>(e.C);

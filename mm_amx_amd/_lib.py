@@ -387,7 +387,7 @@ def gemm_unpacked(A, B, transpose, ep):
     while the stream is being captured into a graph and has no workspace.  Such a first call is packed and not split, so its
     sums can differ in the last bits from an eager call's; call the shape once eagerly before capturing to have the same."""
     _is_2d(A, "A"), _is_2d(B, "B")
-    if A.dtype != torch.bfloat16 or B.dtype != torch.bfloat16:
+    if A.dtype != torch.bfloat16 or B.dtype != torch.bfloat16 or ep.steps & PP_SILU_GATE:
         return False
     _dev(A, "A"), _dev(B, "B")
     M, K = A.shape

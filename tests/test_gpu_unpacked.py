@@ -168,6 +168,24 @@ def test_a_first_call_under_capture_packs(trans):
         assert torch.equal(C.double(), A.double() @ (B.double().t() if trans else B.double()))
 
 
+def test_gate_and_up_in_turn_are_packed():
+    """A post-op of the caller's own may ask for SILU_GATE over a B whose panels alternate already."""
+    M, K, N = 8, 256, 128
+    A, B = _ints((M, K), 26), _ints((K, 2 * N), 27)
+
+    class GateStore:
+        def __init__(self, C):
+            self.C = C
+
+        def descriptor(self):
+            return L.Epilogue(self.C, L.PP_SILU_GATE)
+
+    got, want = (torch.empty((M, N), device="cuda") for _ in range(2))
+    mx.Matmul(False, False)(A, B, ppkernel=GateStore(got))
+    mx.Matmul(True, False)(A, B, ppkernel=GateStore(want))
+    assert torch.equal(got, want)
+
+
 def test_errors_of_the_c_entry():
     A, B, C = _ints((4, 64), 1), _ints((64, 64), 2), torch.empty((4, 64), device="cuda")
     s = L.Epilogue(C).struct()
