@@ -421,7 +421,8 @@ struct Matmul {
             // a result that is written over B: other workgroups may still be reading it, a packed copy is safe
             const uintptr_t b0 = reinterpret_cast<uintptr_t>(matB.data), c0 = reinterpret_cast<uintptr_t>(e.C);
             const uintptr_t b_end = b0 + (size_t)matB.dims[0] * matB.stride;
-            const uintptr_t c_end = c0 + (size_t)M * e.ldc_bytes;
+            const size_t c_size = e.out_dtype == MMX_BF16 ? 2 : (e.out_dtype == MMX_I8 ? 1 : 4);
+            const uintptr_t c_end = c0 + (size_t)(M - 1) * e.ldc_bytes + (size_t)N * c_size;  // (a single row has no stride to speak of)
             // (a stream under capture that has no workspace runs unsplit, which is slow for few columns and a long K, and whose
             // sums can differ in the last bits: call the shape once before capturing.  Packing would need an allocation.)
             if (need >= 0 && (c0 >= b_end || b0 >= c_end)) {  // B is read where it lies

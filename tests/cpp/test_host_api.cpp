@@ -441,6 +441,40 @@ static void test_two_threads_first_call() {
     }
 }
 
+// ---- Matmul with constB = false: a result over B needs the packed copy, whatever the stride of a single row says ----
+static std::vector<bfloat16> small_ints(size_t n) {
+    std::uniform_int_distribution<int> d(-8, 8);
+    std::vector<bfloat16> v(n);
+    for (auto& x : v) x = bfloat16(static_cast<float>(d(rng)));
+    return v;
+}
+static std::vector<float> int_product(const std::vector<bfloat16>& A, const std::vector<bfloat16>& B, int M, int K, int N, bool transB) {
+    std::vector<float> r(static_cast<size_t>(M) * N, 0.0f);
+    for (int m = 0; m < M; m++)
+        for (int k = 0; k < K; k++)
+            for (int n = 0; n < N; n++)
+                r[static_cast<size_t>(m) * N + n] += static_cast<float>(A[static_cast<size_t>(m) * K + k]) *
+                                                     static_cast<float>(B[transB ? static_cast<size_t>(n) * K + k : static_cast<size_t>(k) * N + n]);
+    return r;
+}
+static void test_one_row_over_b(int K, int N) {
+    std::printf("  Matmul<bf16,bf16>, constB = false, one row of C reaching into B K=%d N=%d\n", K, N);
+    const auto hA = small_ints(K), hB = small_ints(static_cast<size_t>(K) * N);
+    tensor2D<bfloat16> A(1, K), room(K + 1, N, true);  // C starts one (bf16) row before B and is two of them long
+    A.upload(hA.data());
+    tensor2D<bfloat16> B(K, N, room.data + N, N * 2);
+    B.upload(hB.data());
+    tensor2D<float> C(1, N, reinterpret_cast<float*>(room.data), 0);
+    Matmul<bfloat16, bfloat16> mm;
+    mm(A, B, PP::BiasGeluStore<float, PP::NONE>(C));
+    const std::string kernel = mmx_last_kernel();
+    check_hip(hipDeviceSynchronize(), "sync");
+    EXPECT(kernel.find("unpacked") == std::string::npos, "ran %s over a B that the result overwrites", kernel.c_str());
+    std::vector<float> got(N);
+    check_hip(hipMemcpy(got.data(), C.data, N * sizeof(float), hipMemcpyDeviceToHost), "download");
+    EXPECT(got == int_product(hA, hB, 1, K, N, false), "wrong sums");
+}
+
 // ---- preconditions raise where the reference asserts ----
 static bool throws(const std::function<void()>& f) {
     try {
@@ -495,6 +529,7 @@ int main() {
         test_mlp(24, 512, 8192);    // decode: the down projection (K = 8192, 16 panels) takes its own K split
         test_mlp(96, 512, 1024, 2);  // the reference's do_splitK for the down projection (tests/amx-mlp.cpp:768)
         test_matmul_i8_requant(160, 2048, 320);  // long enough K for the two-way K split
+        test_one_row_over_b(512, 1024);
         test_two_threads_first_call();
         test_errors();
     } catch (const std::exception& e) {
