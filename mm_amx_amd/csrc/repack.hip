@@ -202,28 +202,48 @@ int launch_repack_gate_up(const void* wg, const void* wu, int64_t ldw, int K, in
 __global__ void zero_u32_kernel(uint32_t* p) { *p = 0u; }
 
 // All three kernels of this section stream bf16 and are bound by memory: a lane takes 16 bytes (8 weights) at a time, four
-// such loads in flight.  A matrix whose rows follow each other without a gap is walked as one row (the host passes rows = 1),
-// otherwise blockIdx.y walks the rows; weights past the last whole 8 of a row are taken one by one by load16_tail.
+// such loads in flight; weights past the last whole 8 of a row are taken one by one by load16_tail.  A matrix whose rows
+// follow each other without a gap is walked as one row (the host passes rows = 1).
 // (11008 x 4096 weights: two bytes per load and a 64-bit division per weight took 217 us for the maxima and 65 for the
 // quantisation; now 18 us, 5.1 TB/s read, and 25 us, 5.5 TB/s read and written; the scaled form 68 -> 30.)
+//   ROWS = false: blockIdx.y walks the rows, a lane's four loads lie along a row.
+//   ROWS = true, for rows with gaps that are too short to fill the four loads of a workgroup: 2^row_log2 lanes share a row, a
+//   lane's four loads are of four rows.  (Maxima and quantisation of rows with gaps, a row at a time -> shared out: 1000000 x 8
+//   4252 -> 17 us, 131072 x 128 518 -> 20, 16384 x 1024 67 -> 19, 4096 x 4096 31 -> 20, 4096 x 8192 46 -> 31.)
 constexpr int QUANT_UNR = 4;
 
-template <int THREADS, typename F>
-__device__ __forceinline__ void for_each_8_weights(const char* __restrict__ W, int64_t ldw, int rows, int64_t cols, F&& f) {
-    const int64_t step = (int64_t)gridDim.x * THREADS;
-    for (int r = blockIdx.y; r < rows; r += gridDim.y) {
-        const char* const row = W + (int64_t)r * ldw;
-        for (int64_t i0 = (int64_t)blockIdx.x * THREADS + threadIdx.x; i0 * 8 < cols; i0 += step * QUANT_UNR) {
-            u32x4 v[QUANT_UNR];
-            if ((i0 + (QUANT_UNR - 1) * step) * 8 + 8 <= cols) {
+template <int THREADS, bool ROWS, typename F>
+__device__ __forceinline__ void for_each_8_weights(const char* __restrict__ W, int64_t ldw, int rows, int64_t cols, int row_log2, F&& f) {
+    if constexpr (ROWS) {
+        const int per_block = THREADS >> row_log2;
+        const int64_t step = (int64_t)gridDim.x * per_block, r0 = (int64_t)blockIdx.x * per_block + (threadIdx.x >> row_log2);
+        for (int64_t r = r0; r < rows; r += step * QUANT_UNR) {
+            for (int64_t c = (int64_t)(threadIdx.x & ((1 << row_log2) - 1)) * 8; c < cols; c += (int64_t)8 << row_log2) {
+                u32x4 v[QUANT_UNR];
 #pragma unroll
-                for (int u = 0; u < QUANT_UNR; u++) v[u] = load16_tail<2>(row + (i0 + u * step) * 16, 16);
-            } else {
+                for (int u = 0; u < QUANT_UNR; u++)
+                    v[u] = load16_tail<2>(W + (r + u * step) * ldw + c * 2, r + u * step < rows ? (cols - c) * 2 : 0);
 #pragma unroll
-                for (int u = 0; u < QUANT_UNR; u++) v[u] = load16_tail<2>(row + (i0 + u * step) * 16, (cols - (i0 + u * step) * 8) * 2);
+                for (int u = 0; u < QUANT_UNR; u++)
+                    if (r + u * step < rows) f(r + u * step, c, v[u]);
             }
+        }
+    } else {
+        const int64_t step = (int64_t)gridDim.x * THREADS;
+        for (int r = blockIdx.y; r < rows; r += gridDim.y) {
+            const char* const row = W + (int64_t)r * ldw;
+            for (int64_t i0 = (int64_t)blockIdx.x * THREADS + threadIdx.x; i0 * 8 < cols; i0 += step * QUANT_UNR) {
+                u32x4 v[QUANT_UNR];
+                if ((i0 + (QUANT_UNR - 1) * step) * 8 + 8 <= cols) {
 #pragma unroll
-            for (int u = 0; u < QUANT_UNR; u++) f(r, (i0 + u * step) * 8, v[u]);
+                    for (int u = 0; u < QUANT_UNR; u++) v[u] = load16_tail<2>(row + (i0 + u * step) * 16, 16);
+                } else {
+#pragma unroll
+                    for (int u = 0; u < QUANT_UNR; u++) v[u] = load16_tail<2>(row + (i0 + u * step) * 16, (cols - (i0 + u * step) * 8) * 2);
+                }
+#pragma unroll
+                for (int u = 0; u < QUANT_UNR; u++) f(r, (i0 + u * step) * 8, v[u]);
+            }
         }
     }
 }
@@ -244,9 +264,11 @@ __device__ __forceinline__ void store_8_bytes(char* row, int64_t c, int64_t cols
 // atomics all meet at one address and take 10 ns each there, so there is one workgroup per CU, of 16 wavefronts (2048
 // workgroups of four: 4096 x 4096 weights in 27 us instead of 10).
 constexpr int ABSMAX_THREADS = 1024;
-__global__ __launch_bounds__(ABSMAX_THREADS) void absmax_kernel(const char* __restrict__ W, int64_t ldw, int rows, int64_t cols, uint32_t* out) {
+template <bool ROWS>
+__global__ __launch_bounds__(ABSMAX_THREADS) void absmax_kernel(const char* __restrict__ W, int64_t ldw, int rows, int64_t cols, int row_log2,
+                                                                uint32_t* out) {
     uint32_t m = 0;
-    for_each_8_weights<ABSMAX_THREADS>(W, ldw, rows, cols, [&](int, int64_t, const u32x4& v) __attribute__((always_inline)) {
+    for_each_8_weights<ABSMAX_THREADS, ROWS>(W, ldw, rows, cols, row_log2, [&](int64_t, int64_t, const u32x4& v) __attribute__((always_inline)) {
 #pragma unroll
         for (int d = 0; d < 4; d++) {
             const uint32_t lo = (v[d] << 16) & 0x7fffffffu, hi = v[d] & 0x7fff0000u;
@@ -269,21 +291,22 @@ __global__ __launch_bounds__(ABSMAX_THREADS) void absmax_kernel(const char* __re
 }
 
 // q = sat8(rne(w * (127/max))) (include/kernels_amx.hpp:508-523); scales_out = {127/max, max/127}
-__global__ __launch_bounds__(256) void quantize_kernel(const char* __restrict__ W, int64_t ldw, int rows, int64_t cols, char* __restrict__ Wq,
-                                                       int64_t ldq, const uint32_t* absmax_bits, float* scales_out) {
+template <bool ROWS>
+__global__ __launch_bounds__(256) void quantize_kernel(const char* __restrict__ W, int64_t ldw, int rows, int64_t cols, int row_log2,
+                                                       char* __restrict__ Wq, int64_t ldq, const uint32_t* absmax_bits, float* scales_out) {
     const float amax = u2f(*absmax_bits);
     const float q = 127 / amax;
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
         scales_out[0] = q;
         scales_out[1] = amax / 127;
     }
-    for_each_8_weights<256>(W, ldw, rows, cols, [&](int r, int64_t c, const u32x4& v) __attribute__((always_inline)) {
+    for_each_8_weights<256, ROWS>(W, ldw, rows, cols, row_log2, [&](int64_t r, int64_t c, const u32x4& v) __attribute__((always_inline)) {
         uint32_t o[2];
 #pragma unroll
         for (int h = 0; h < 2; h++)
             o[h] = to_s8_sat_x4(u2f(v[2 * h] << 16) * q, u2f(v[2 * h] & 0xffff0000u) * q, u2f(v[2 * h + 1] << 16) * q,
                                 u2f(v[2 * h + 1] & 0xffff0000u) * q);
-        if (c < cols) store_8_bytes(Wq + (int64_t)r * ldq, c, cols, o[0], o[1]);
+        if (c < cols) store_8_bytes(Wq + r * ldq, c, cols, o[0], o[1]);
     });
 }
 
@@ -292,22 +315,36 @@ static void one_row(int64_t ldw, int64_t ldq, int& rows, int64_t& cols) {
     if (ldw == cols * 2 && ldq == cols) cols *= rows, rows = 1;
 }
 
-// at most `most` workgroups, each taking QUANT_UNR loads per lane at a time
-static dim3 quantize_grid(int rows, int64_t cols, int threads, int most) {
-    const int64_t per_block = (int64_t)threads * 8 * QUANT_UNR, x = (cols + per_block - 1) / per_block;
+// How the kernels above walk a matrix: at most `most` workgroups, each taking QUANT_UNR loads per lane at a time.  Rows that
+// do not fill those of one workgroup are shared out (ROWS): the fewest lanes, a power of two, that cover a row.
+struct QuantWalk {
+    bool by_rows;
+    int row_log2;
+    dim3 grid;
+};
+static QuantWalk quantize_walk(int rows, int64_t cols, int threads, int most) {
+    const int64_t per_block = (int64_t)threads * 8 * QUANT_UNR;
+    if (rows > 1 && cols < per_block) {
+        int log2 = 0;
+        while ((8 << log2) < cols && (1 << log2) < threads) log2++;
+        const int64_t rows_per_block = (int64_t)(threads >> log2) * QUANT_UNR, x = (rows + rows_per_block - 1) / rows_per_block;
+        return {true, log2, dim3((unsigned)(x < most ? x : most))};
+    }
+    const int64_t x = (cols + per_block - 1) / per_block;
     const int gx = x < most ? (int)x : most, gy = most / gx;
-    return dim3((unsigned)gx, (unsigned)(rows < gy ? rows : gy));
+    return {false, 0, dim3((unsigned)gx, (unsigned)(rows < gy ? rows : gy))};
 }
 
 int launch_quantize(const void* W, int64_t ldw, int rows, int cols_in, void* Wq, int64_t ldq, float* scales_out,
                     uint32_t* scratch, hipStream_t st) {
     int64_t cols = cols_in;
     one_row(ldw, ldq, rows, cols);
-    const dim3 grid = quantize_grid(rows, cols, 256, 2048);
+    const QuantWalk m = quantize_walk(rows, cols, ABSMAX_THREADS, num_cus()), q = quantize_walk(rows, cols, 256, 2048);
     hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, st, scratch);
-    hipLaunchKernelGGL(absmax_kernel, quantize_grid(rows, cols, ABSMAX_THREADS, num_cus()), dim3(ABSMAX_THREADS), 0, st, static_cast<const char*>(W), ldw, rows, cols, scratch);
-    hipLaunchKernelGGL(quantize_kernel, grid, dim3(256), 0, st, static_cast<const char*>(W), ldw, rows, cols,
-                       static_cast<char*>(Wq), ldq, scratch, scales_out);
+    hipLaunchKernelGGL(m.by_rows ? absmax_kernel<true> : absmax_kernel<false>, m.grid, dim3(ABSMAX_THREADS), 0, st, static_cast<const char*>(W),
+                       ldw, rows, cols, m.row_log2, scratch);
+    hipLaunchKernelGGL(q.by_rows ? quantize_kernel<true> : quantize_kernel<false>, q.grid, dim3(256), 0, st, static_cast<const char*>(W), ldw,
+                       rows, cols, q.row_log2, static_cast<char*>(Wq), ldq, scratch, scales_out);
     return check_hip(hipGetLastError(), "quantize kernels launch");
 }
 
@@ -323,23 +360,24 @@ __device__ __forceinline__ uint32_t scale_trunc(float w, float scale) {
     return (uint32_t)q & 0xffu;
 }
 
+template <bool ROWS>
 __global__ __launch_bounds__(256) void quantize_scale_trunc_kernel(const char* __restrict__ W, int64_t ldw, int rows, int64_t cols,
-                                                                   float scale, char* __restrict__ Wq, int64_t ldq) {
-    for_each_8_weights<256>(W, ldw, rows, cols, [&](int r, int64_t c, const u32x4& v) __attribute__((always_inline)) {
+                                                                   int row_log2, float scale, char* __restrict__ Wq, int64_t ldq) {
+    for_each_8_weights<256, ROWS>(W, ldw, rows, cols, row_log2, [&](int64_t r, int64_t c, const u32x4& v) __attribute__((always_inline)) {
         uint32_t o[2] = {0, 0};
 #pragma unroll
         for (int d = 0; d < 4; d++)
             o[d >> 1] |= (scale_trunc(u2f(v[d] << 16), scale) | scale_trunc(u2f(v[d] & 0xffff0000u), scale) << 8) << (16 * (d & 1));
-        if (c < cols) store_8_bytes(Wq + (int64_t)r * ldq, c, cols, o[0], o[1]);
+        if (c < cols) store_8_bytes(Wq + r * ldq, c, cols, o[0], o[1]);
     });
 }
 
 int launch_quantize_scale_trunc(const void* W, int64_t ldw, int rows, int cols_in, float scale, void* Wq, int64_t ldq, hipStream_t st) {
     int64_t cols = cols_in;
     one_row(ldw, ldq, rows, cols);
-    const dim3 grid = quantize_grid(rows, cols, 256, 2048);
-    hipLaunchKernelGGL(quantize_scale_trunc_kernel, grid, dim3(256), 0, st, static_cast<const char*>(W), ldw, rows, cols, scale,
-                       static_cast<char*>(Wq), ldq);
+    const QuantWalk q = quantize_walk(rows, cols, 256, 2048);
+    hipLaunchKernelGGL(q.by_rows ? quantize_scale_trunc_kernel<true> : quantize_scale_trunc_kernel<false>, q.grid, dim3(256), 0, st,
+                       static_cast<const char*>(W), ldw, rows, cols, q.row_log2, scale, static_cast<char*>(Wq), ldq);
     return check_hip(hipGetLastError(), "quantize_scale_trunc_kernel launch");
 }
 

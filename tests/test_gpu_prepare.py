@@ -35,7 +35,8 @@ def test_repack_unit_edges(po, dt, K, N):
     assert np.array_equal(host_bits(mx.repack_b(wide[:, 1:K + 1], transpose=True)).view(np.uint8), want.view(np.uint8))
 
 
-@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 7), (5, 64), (33, 1029), (2, 70001), (700, 8)])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (3, 7), (5, 64), (33, 1029), (2, 70001), (700, 8), (4100, 9), (1025, 130),
+                                       (70, 8193), (5, 32767), (5, 32768), (9, 2048)])
 @pytest.mark.parametrize("gap", [0, 5])
 def test_quantisers_row_ends_and_gaps(po, rows, cols, gap):
     """Rows that end in the middle of a 16-byte load, with and without a gap behind them; the largest weight last."""
@@ -49,6 +50,32 @@ def test_quantisers_row_ends_and_gaps(po, rows, cols, gap):
     assert np.array_equal(host_bits(got), want)
     assert host_bits(scales).tolist() == [np.float32(q), np.float32(dq)]
     assert np.array_equal(host_bits(mx.quantize_weights_scaled(wide[:, :cols], 1234.5)), po.quantize_scale_trunc(W, 1234.5))
+
+
+def _us(f, n=10):
+    """The least of three timings of n calls, per call."""
+    best = float("inf")
+    for _ in range(3):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        f()
+        torch.cuda.synchronize()
+        a.record()
+        for _ in range(n):
+            f()
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b) * 1e3 / n)
+    return best
+
+
+@pytest.mark.parametrize("rows,cols", [(1000000, 8), (131072, 128), (16384, 1024)])
+def test_gaps_between_short_rows_cost_little(rows, cols):
+    """With a gap as long as the row up to twice the lines are read.  A workgroup to a row took 25 times as long as without
+    gaps at 131072 x 128 and 250 times at 1000000 x 8; with the rows shared out it is less than twice."""
+    W = torch.randn((rows, 2 * cols), device="cuda").to(torch.bfloat16)
+    for f in (mx.quantize_weights, lambda w: mx.quantize_weights_scaled(w, 30.0)):
+        whole, gaps = W[:, :cols].contiguous(), W[:, :cols]
+        assert _us(lambda: f(gaps)) <= 6 * _us(lambda: f(whole))
 
 
 @pytest.mark.parametrize("K", [1, 64, 255, 513, 2056])
