@@ -579,6 +579,109 @@ __device__ __forceinline__ uint32_t int4_of(float w, float scale) {
     return (uint32_t)(int)q & 0xfu;
 }
 
+// [N, K], 64 of k from k0 on: 4 loads of 8 rows x 128 bytes; and the fragment they make, scaled by qs.
+__device__ __forceinline__ void load_fragment_rows(u32x4 (&v)[4], const char* W, int64_t ldw, int K, int N, int n0, int k0) {
+    const int lane = threadIdx.x & 63, r8 = lane >> 3, k = k0 + 8 * (lane & 7);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int n = n0 + 8 * i + r8;
+        v[i] = load16_tail<2>(W + (int64_t)n * ldw + (int64_t)k * 2, n < N ? (int64_t)(K - k) * 2 : 0);
+    }
+}
+__device__ __forceinline__ void store_fragment_rows(const u32x4 (&v)[4], const float (&qs)[4], char* fragment) {
+    const int lane = threadIdx.x & 63, r8 = lane >> 3, c = lane & 7;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        uint32_t d = 0;
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            d |= (int4_of(u2f(v[i][e] << 16), qs[i]) | int4_of(u2f(v[i][e] & 0xffff0000u), qs[i]) << 4) << (8 * e);
+        *reinterpret_cast<uint32_t*>(fragment + ((c >> 2) * 32 + 8 * i + r8) * 16 + (c & 3) * 4) = d;
+    }
+}
+
+// [K, N], 128 of k from k0 on: a lane takes 8 columns of 8 rows, 16 chunks of k to a wavefront; and their two fragments.
+__device__ __forceinline__ void load_fragments_cols(u32x4 (&v)[8], const char* W, int64_t ldw, int K, int N, int n0, int k0) {
+    const int lane = threadIdx.x & 63, n = n0 + 8 * (lane & 3), k = k0 + 8 * (lane >> 2);
+#pragma unroll
+    for (int e = 0; e < 8; e++)
+        v[e] = load16_tail<2>(W + (int64_t)(k + e) * ldw + (int64_t)n * 2, k + e < K ? (int64_t)(N - n) * 2 : 0);
+}
+__device__ __forceinline__ void store_fragments_cols(const u32x4 (&v)[8], const float (&qs)[8], char* fragments) {
+    const int lane = threadIdx.x & 63, ng = lane & 3, kc = lane >> 2;
+    char* const slot = fragments + (kc >> 3) * 1024 + (((kc >> 2) & 1) * 32 + 8 * ng) * 16 + (kc & 3) * 4;
+#pragma unroll
+    for (int n = 0; n < 8; n++) {
+        uint32_t d = 0;
+#pragma unroll
+        for (int e = 0; e < 8; e++) d |= int4_of(n & 1 ? u2f(v[e][n >> 1] & 0xffff0000u) : u2f(v[e][n >> 1] << 16), qs[n]) << (4 * e);
+        *reinterpret_cast<uint32_t*>(slot + n * 16) = d;
+    }
+}
+
+// The scale of a column and what undoes it, from the column's largest |w|.
+__device__ __forceinline__ float int4_scale(float amax, float* deq) {
+    *deq = amax / 7.0f;
+    return amax > 0.0f ? 7.0f / amax : 0.0f;
+}
+
+// K of at most 256 (the four fragments that every panel has): the panel stays in registers between the two passes, read once,
+// by as many wavefronts as that takes - 4 of one fragment each from [N, K], 2 of two from [K, N].  (Sixteen wavefronts on a
+// panel that short are mostly idle: [N, K] / [K, N], K = 32 x 1048576 296 / 314 -> 89 / 90 us, 64 x 262144 77 / 84 -> 24 / 27,
+// 256 x 65536 22 / 29 -> 9 / 16.)
+template <bool TRANSPOSED>
+__global__ __launch_bounds__(TRANSPOSED ? 256 : 128) void quant4_pack_short_kernel(const char* __restrict__ W, int64_t ldw, int K, int N,
+                                                                                   char* __restrict__ out, float* deq_out) {
+    constexpr int WAVES = TRANSPOSED ? 4 : 2;
+    __shared__ float smax[32][WAVES];
+    __shared__ float sscale[32];
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int n0 = blockIdx.x * 32;
+    char* const o = out + (int64_t)blockIdx.x * 4096;
+    u32x4 v[TRANSPOSED ? 4 : 8];
+    if constexpr (TRANSPOSED) {
+        load_fragment_rows(v, W, ldw, K, N, n0, 64 * wave);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            float m = 0.0f;  // (fmaxf drops a NaN)
+#pragma unroll
+            for (int d = 0; d < 4; d++) m = fmaxf(fmaxf(m, fabsf(u2f(v[i][d] << 16))), fabsf(u2f(v[i][d] & 0xffff0000u)));
+            for (int off = 1; off < 8; off <<= 1) m = fmaxf(m, __shfl_xor(m, off));
+            if ((lane & 7) == 0) smax[8 * i + (lane >> 3)][wave] = m;
+        }
+    } else {
+        load_fragments_cols(v, W, ldw, K, N, n0, 128 * wave);
+#pragma unroll
+        for (int n = 0; n < 8; n++) {
+            float m = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 8; e++) m = fmaxf(m, fabsf(n & 1 ? u2f(v[e][n >> 1] & 0xffff0000u) : u2f(v[e][n >> 1] << 16)));
+            for (int off = 4; off < 64; off <<= 1) m = fmaxf(m, __shfl_xor(m, off));
+            if (lane < 4) smax[8 * lane + n][wave] = m;
+        }
+    }
+    __syncthreads();
+    if (t < 32) {
+        float a = 0.0f, deq;
+#pragma unroll
+        for (int w = 0; w < WAVES; w++) a = fmaxf(a, smax[t][w]);
+        sscale[t] = int4_scale(a, &deq);
+        if (n0 + t < N) deq_out[n0 + t] = deq;
+    }
+    __syncthreads();
+    if constexpr (TRANSPOSED) {
+        float qs[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) qs[i] = sscale[8 * i + (lane >> 3)];
+        store_fragment_rows(v, qs, o + wave * 1024);
+    } else {
+        float qs[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) qs[e] = sscale[8 * (lane & 3) + e];
+        store_fragments_cols(v, qs, o + wave * 2048);
+    }
+}
+
 template <bool TRANSPOSED>
 __global__ __launch_bounds__(QUANT4_WAVES * 64) void quant4_pack_kernel(const char* __restrict__ W, int64_t ldw, int K, int N,
                                                                         char* __restrict__ out, int nfrag, float* deq_out) {
@@ -638,58 +741,31 @@ __global__ __launch_bounds__(QUANT4_WAVES * 64) void quant4_pack_kernel(const ch
     }
     __syncthreads();
     if (t < 32) {
-        float a = 0.0f;
+        float a = 0.0f, deq;
 #pragma unroll
         for (int r = 0; r < QUANT4_WAVES; r++) a = fmaxf(a, smax[t][r]);
-        sscale[t] = a > 0.0f ? 7.0f / a : 0.0f;
-        if (n0 + t < N) deq_out[n0 + t] = a / 7.0f;
+        sscale[t] = int4_scale(a, &deq);
+        if (n0 + t < N) deq_out[n0 + t] = deq;
     }
     __syncthreads();
     char* const o = out + (int64_t)blockIdx.x * nfrag * 1024;
     if constexpr (TRANSPOSED) {
-        const int r8 = lane >> 3, c = lane & 7;
         float qs[4];
 #pragma unroll
-        for (int i = 0; i < 4; i++) qs[i] = sscale[8 * i + r8];
+        for (int i = 0; i < 4; i++) qs[i] = sscale[8 * i + (lane >> 3)];
         for (int f = wave; f < nfrag; f += QUANT4_WAVES) {
-            const int k = 64 * f + 8 * c;
             u32x4 v[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int n = n0 + 8 * i + r8;
-                v[i] = load16_tail<2>(W + (int64_t)n * ldw + (int64_t)k * 2, n < N ? (int64_t)(K - k) * 2 : 0);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                uint32_t d = 0;
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    d |= (int4_of(u2f(v[i][e] << 16), qs[i]) | int4_of(u2f(v[i][e] & 0xffff0000u), qs[i]) << 4) << (8 * e);
-                *reinterpret_cast<uint32_t*>(o + (int64_t)f * 1024 + ((c >> 2) * 32 + 8 * i + r8) * 16 + (c & 3) * 4) = d;
-            }
+            load_fragment_rows(v, W, ldw, K, N, n0, 64 * f);
+            store_fragment_rows(v, qs, o + (int64_t)f * 1024);
         }
     } else {
-        // lane -> (columns 8 ng .., chunk of 8 k); 16 chunks = two fragments per wavefront
-        const int ng = lane & 3, kc = lane >> 2;
-        const int64_t left = (int64_t)(N - n0 - 8 * ng) * 2;
         float qs[8];
 #pragma unroll
-        for (int e = 0; e < 8; e++) qs[e] = sscale[8 * ng + e];
+        for (int e = 0; e < 8; e++) qs[e] = sscale[8 * (lane & 3) + e];
         for (int f2 = wave; f2 * 2 < nfrag; f2 += QUANT4_WAVES) {
-            const int k = 128 * f2 + 8 * kc;
             u32x4 v[8];
-#pragma unroll
-            for (int e = 0; e < 8; e++)
-                v[e] = load16_tail<2>(W + (int64_t)(k + e) * ldw + (int64_t)(n0 + 8 * ng) * 2, k + e < K ? left : 0);
-            char* const slot = o + (int64_t)(2 * f2 + (kc >> 3)) * 1024 + (((kc >> 2) & 1) * 32 + 8 * ng) * 16 + (kc & 3) * 4;
-#pragma unroll
-            for (int n = 0; n < 8; n++) {
-                uint32_t d = 0;
-#pragma unroll
-                for (int e = 0; e < 8; e++)
-                    d |= int4_of(n & 1 ? u2f(v[e][n >> 1] & 0xffff0000u) : u2f(v[e][n >> 1] << 16), qs[n]) << (4 * e);
-                *reinterpret_cast<uint32_t*>(slot + n * 16) = d;
-            }
+            load_fragments_cols(v, W, ldw, K, N, n0, 128 * f2);
+            store_fragments_cols(v, qs, o + (int64_t)f2 * 2048);
         }
     }
 }
@@ -698,6 +774,11 @@ int launch_quantize_pack_int4(const void* W, int64_t ldw, int K, int N, int tran
                               hipStream_t st) {
     const int nfrag = (K + 255) / 256 * 4;
     const int npanels = (N + 31) / 32;
+    if (nfrag == 4) {
+        hipLaunchKernelGGL(transpose ? quant4_pack_short_kernel<true> : quant4_pack_short_kernel<false>, dim3(npanels),
+                           dim3(transpose ? 256 : 128), 0, st, static_cast<const char*>(W), ldw, K, N, static_cast<char*>(packed), deq_out);
+        return check_hip(hipGetLastError(), "quant4_pack_short_kernel launch");
+    }
     const dim3 threads(QUANT4_WAVES * 64);
     if (transpose)
         hipLaunchKernelGGL(quant4_pack_kernel<true>, dim3(npanels), threads, 0, st, static_cast<const char*>(W), ldw, K, N,
