@@ -370,8 +370,9 @@ int mmx_gemm_unpacked(int dtype, const void* A, int64_t lda_bytes, const void* B
         return set_error(MMX_E_UNSUPPORTED, "mmx_gemm_unpacked: this shape or type takes packed weights (mmx_repack_b, mmx_gemm)");
     if (lda_bytes < (int64_t)K * 2) return set_error(MMX_E_INVALID, "mmx_gemm_unpacked: lda_bytes %lld smaller than a row of A", (long long)lda_bytes);
     if (ldb_bytes < (int64_t)(transpose ? K : N) * 2) return set_error(MMX_E_INVALID, "mmx_gemm_unpacked: ldb_bytes %lld smaller than a row of B", (long long)ldb_bytes);
-    if ((lda_bytes | ldb_bytes) % 2 || (reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(B)) % 2)
-        return set_error(MMX_E_INVALID, "mmx_gemm_unpacked: A or B is not aligned to its element size");
+    // (B may lie anywhere, as for mmx_repack_b)
+    if ((lda_bytes | ldb_bytes) % 2 || reinterpret_cast<uintptr_t>(A) % 2)
+        return set_error(MMX_E_INVALID, "mmx_gemm_unpacked: A or the rows of B are not aligned to their element size");
     if (reinterpret_cast<uintptr_t>(workspace) & 255) return set_error(MMX_E_INVALID, "mmx_gemm_unpacked: the workspace must be 256-byte aligned");
     Epilogue ep;
     int rc = make_epilogue(ep_in, MMX_BF16, MMX_BF16, M, 0, N, &ep);

@@ -38,8 +38,8 @@ constexpr size_t COUNTER_BYTES = (size_t)MAX_TILES * 4;
 // (It takes slices from wide results only, where the CUs have strips enough: 128 x 8192 x 50304 334 us unsplit, 338 in four.)
 constexpr size_t STANDARD_WORKSPACE_BYTES = ((size_t)64 << 20) + ((size_t)16 << 10);
 
-// 16 bytes from any even address (the hardware takes them at any)
-typedef u32x4 __attribute__((aligned(2))) u32x4_any;
+// 16 bytes from any address (the hardware takes them at any)
+typedef u32x4 __attribute__((aligned(1))) u32x4_any;
 __device__ __forceinline__ u32x4 load16(const char* base, uint32_t off) { return *reinterpret_cast<const u32x4_any*>(base + off); }
 __device__ __forceinline__ u32x4 stream16(const char* base, uint32_t off) {
     return __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(base + off));

@@ -64,6 +64,20 @@ def test_exact_sums(M, K, N, trans, pad):
     assert torch.equal(_run(False, trans, A, B, again.zero_()).double(), ref)  # whichever way the rule takes
 
 
+@pytest.mark.parametrize("trans", [False, True])
+def test_b_at_an_odd_address(trans):
+    """A caller of the C entry may hand over a B that is not aligned to its element, as it may to mmx_repack_b."""
+    M, K, N = 20, 160, 136
+    A, B = _ints((M, K), 28), _ints((N, K) if trans else (K, N), 29)
+    room = torch.zeros(B.numel() * 2 + 1, dtype=torch.uint8, device="cuda")
+    room[1:] = B.contiguous().view(torch.uint8).view(-1)
+    C = torch.empty((M, N), device="cuda")
+    s = L.Epilogue(C).struct()
+    L._check(L.lib().mmx_gemm_unpacked(L.BF16, A.data_ptr(), K * 2, room.data_ptr() + 1, B.shape[1] * 2, int(trans), M, K, N, ctypes.byref(s),
+                                       None, 0, L._stream()))
+    assert torch.equal(C.double(), A.double() @ (B.double().t() if trans else B.double()))
+
+
 @pytest.mark.parametrize("N", [8, 131, 250])
 def test_any_column_count_from_rows_of_k(N):
     A, B = _ints((24, 96), 3), _ints((N, 96), 4)
