@@ -20,6 +20,45 @@ typedef __attribute__((__vector_size__(16 * sizeof(int)))) int i32x16;
 // held in small arrays)
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
+// ---- 16 bytes out of a row of any alignment that may end before them -------------------------------------------
+// What lies past the row is zero and not touched: the last 16 bytes of the row are fetched instead and moved down.  There is
+// no branch in it, so a series of these keeps all its loads in flight (fetched behind a test each, or element by element,
+// every load waits for the one before it).  len: bytes of the row, at least 16; at: any byte from 0 on, past the end too.
+template <typename T>
+__device__ __forceinline__ u32x4 fetch16_in_row(const char* row, T at, T len) {
+    u32x4 v;
+    const T last = len - 16;
+    __builtin_memcpy(&v, __builtin_assume_aligned(row + (at < last ? at : last), 1), 16);  // (the hardware takes any address)
+    return v;
+}
+// the same bytes once they are there: moved down by what the fetch started early, all of them zero if nothing is left
+template <typename T>
+__device__ __forceinline__ u32x4 settle16_in_row(u32x4 v, T at, T len) {
+    const T last = len - 16;
+    const uint32_t over = at < last ? 0u : (at - last < 16 ? (uint32_t)(at - last) : 16u);
+    uint64_t lo = (uint64_t)v[0] | (uint64_t)v[1] << 32, hi = (uint64_t)v[2] | (uint64_t)v[3] << 32;
+    lo = over & 8 ? hi : lo;
+    hi = over & 8 ? 0 : hi;
+    const uint32_t s = 8 * (over & 7);
+    lo = lo >> s | (hi << 1) << (63 - s);
+    hi >>= s;
+    if (over & 16) lo = hi = 0;
+    return u32x4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+}
+// rows shorter than 16 bytes: ES bytes at a time, from inside the row
+template <int ES, typename T>
+__device__ __forceinline__ u32x4 fetch16_in_short_row(const char* row, T at, T len) {
+    uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < 16; i += ES) {
+        const T b = at + i, from = b < len ? b : len - ES;
+        uint32_t e = 0;
+        __builtin_memcpy(&e, row + from, ES);
+        w[i >> 2] |= (b < len ? e : 0u) << (8 * (i & 3));
+    }
+    return u32x4{w[0], w[1], w[2], w[3]};
+}
+
 // error plumbing (host)
 int set_error(int code, const char* fmt, ...);
 int check_hip(hipError_t e, const char* what);

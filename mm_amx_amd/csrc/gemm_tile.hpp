@@ -131,29 +131,6 @@ __device__ __forceinline__ int32_t cvt_out<int32_t>(float r) { return (int32_t)r
 template <int SZ>
 __device__ __forceinline__ void store16(char* p, u32x4 v) { __builtin_memcpy(__builtin_assume_aligned(p, SZ), &v, 16); }
 
-// The 16 bytes at byte kb of a row of kbytes, whatever the row's alignment (the hardware takes 16-byte loads from any
-// address); what lies past the row is zero and not touched: the last 16 bytes of the row are fetched instead and shifted.
-__device__ __forceinline__ u32x4 load_a_chunk_tail(const char* rowptr, int kb, int kbytes) {
-    u32x4 v = u32x4{0u, 0u, 0u, 0u};
-    if (kb >= kbytes) return v;
-    if (kbytes >= 16) {
-        const int over = kb + 16 > kbytes ? kb + 16 - kbytes : 0;
-        uint64_t h[2];
-        __builtin_memcpy(h, __builtin_assume_aligned(rowptr + kb - over, 1), 16);
-        const int s = 8 * (over & 7);
-        if (over >= 8) h[0] = h[1], h[1] = 0;
-        if (s) h[0] = (h[0] >> s) | (h[1] << (64 - s)), h[1] >>= s;
-        v = u32x4{(uint32_t)h[0], (uint32_t)(h[0] >> 32), (uint32_t)h[1], (uint32_t)(h[1] >> 32)};
-        return v;
-    }
-    uint32_t w[4] = {0, 0, 0, 0};
-#pragma unroll
-    for (int b = 0; b < 16; b++) {
-        if (kb + b < kbytes) w[b >> 2] |= (uint32_t)(uint8_t)rowptr[kb + b] << (8 * (b & 3));
-    }
-    return u32x4{w[0], w[1], w[2], w[3]};
-}
-
 // LDS ring of the hand-scheduled pipeline: RA stages of A (BM rows x 128 bytes) and R half-stages of B (BN columns
 // x 64 bytes).  The ring is as deep as 156 KiB of LDS allow (R <= 2 RA - 2, see the pipeline): the loads of R - 1
 // half-stages are in flight while one is multiplied, and a small tile multiplies a half-stage in far less time
@@ -298,23 +275,36 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
     u32x4 ra[RING ? 1 : A_IT], rb[RING ? 1 : B_IT];  // staging registers of modes 0 and 3
 
     auto fetch = [&](int kt) {
+        // the row of A that a thread's load `it` is from, and the first of its 16 bytes
+        auto source = [&](int it, int& byte) {
+            const int c = it * 256 + tid, row = c >> 3;
+            byte = kt * 128 + ((c & 7) ^ (row & 7)) * 16;
+            const int grow = m0 + row;
+            return g.A + (int64_t)(grow < g.M ? grow : g.M - 1) * g.lda;
+        };
+        int byte;
+        if (MODE != 3 || (kt + 1) * 128 <= g.kbytes) {  // (uniform: only the last k-iteration has anything to mask)
 #pragma unroll
-        for (int it = 0; it < A_IT; it++) {
-            const int c = it * 256 + tid;
-            const int row = c >> 3, slot = c & 7;
-            const int chunk = slot ^ (row & 7);
-            int grow = m0 + row;
-            if constexpr (MODE != 3) {
-                grow = grow < g.M ? grow : g.M - 1;
-                const char* src = g.A + (int64_t)grow * g.lda + kt * 128 + chunk * 16;
-                ra[it] = *reinterpret_cast<const u32x4*>(src);
-            } else {
-                const char* row = g.A + (int64_t)(grow < g.M ? grow : g.M - 1) * g.lda;
-                if ((kt + 1) * 128 <= g.kbytes) {  // (uniform: only the last k-iteration has anything to mask)
-                    __builtin_memcpy(&ra[it], __builtin_assume_aligned(row + kt * 128 + chunk * 16, 1), 16);
-                } else {
-                    ra[it] = load_a_chunk_tail(row, kt * 128 + chunk * 16, g.kbytes);
-                }
+            for (int it = 0; it < A_IT; it++) {
+                const char* row = source(it, byte);
+                __builtin_memcpy(&ra[it], __builtin_assume_aligned(row + byte, MODE == 3 ? 1 : 16), 16);
+            }
+        } else if (g.kbytes >= 16) {  // all the loads first: behind a test each they were a chain (33 x 32 x 65536 11.1 -> 9.0 us)
+#pragma unroll
+            for (int it = 0; it < A_IT; it++) {
+                const char* row = source(it, byte);
+                ra[it] = fetch16_in_row(row, byte, g.kbytes);
+            }
+#pragma unroll
+            for (int it = 0; it < A_IT; it++) {
+                source(it, byte);
+                ra[it] = settle16_in_row(ra[it], byte, g.kbytes);
+            }
+        } else {
+#pragma unroll
+            for (int it = 0; it < A_IT; it++) {
+                const char* row = source(it, byte);
+                ra[it] = fetch16_in_short_row<std::is_same<TIn, int8_t>::value ? 1 : 2>(row, byte, g.kbytes);
             }
         }
 #pragma unroll
@@ -655,7 +645,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
             for (int it = 0; it < AC; it++) {
                 const int row = (it * NT + tid) >> 3, chunk = (tid & 7) ^ ((row >> 1) & 7);
                 const int grow = m0 + row < g.M ? m0 + row : g.M - 1;
-                ta[it] = load_a_chunk_tail(g.A + (int64_t)grow * g.lda, g.nk * 128 + chunk * 16, g.kbytes);
+                ta[it] = fetch16_in_row(g.A + (int64_t)grow * g.lda, g.nk * 128 + chunk * 16, g.kbytes);
             }
 #pragma unroll
             for (int it = 0; it < (BC + NT - 1) / NT; it++) {
@@ -667,7 +657,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
             }
             __syncthreads();  // every wave has finished with the rings (and its own re-fetched slots have landed)
 #pragma unroll
-            for (int it = 0; it < AC; it++) *reinterpret_cast<u32x4*>(smem + (it * NT + tid) * 16) = ta[it];
+            for (int it = 0; it < AC; it++)
+                *reinterpret_cast<u32x4*>(smem + (it * NT + tid) * 16) =
+                    settle16_in_row(ta[it], g.nk * 128 + ((tid & 7) ^ ((((it * NT + tid) >> 3) >> 1) & 7)) * 16, g.kbytes);
 #pragma unroll
             for (int it = 0; it < (BC + NT - 1) / NT; it++) {
                 const int c = it * NT + tid, in = c % (BP_IT / 16);
@@ -716,7 +708,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
         // the last iteration re-fetches its own stage into the idle buffer: harmless, and it keeps
         // the loop body free of branches so that the schedule below is one straight block
         const int kt_next = (kt + 1 < nk) ? kt + 1 : kt;
-        fetch(kt0 + kt_next);
+        if (MODE != 3 || kt + 1 < nk) fetch(kt0 + kt_next);  // (masked loads branch anyway, and a tail is waited for where it is fetched)
         __builtin_amdgcn_sched_barrier(0);
         read_frags(stage, 1, fa[1], fb[1]);
         mma(fa[0], fb[0]);
@@ -731,7 +723,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
         // stage has had three k-steps to land: synchronise here, then start reading the next
         // stage while the last k-step of this one is multiplied.
         commit(stage ^ 1);
-            __syncthreads();
+        __syncthreads();
         __builtin_amdgcn_sched_barrier(0);
         read_frags(stage ^ 1, 0, fa[0], fb[0]);
         mma(fa[1], fb[1]);

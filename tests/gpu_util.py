@@ -71,3 +71,19 @@ def check_gelu_parity(got_bits, ref_bits, ref_preact, what, frac_all=0.0):
     assert frac_good >= 0.999, f"{what}: {frac_good * 100:.3f}% within 1 bf16 ulp where GELU is well conditioned"
     assert frac >= frac_all, f"{what}: {frac * 100:.3f}% within 1 bf16 ulp over all elements"
     return err, frac_good, frac
+
+
+def call_us(f, n=10):
+    """The least of three timings of n calls, per call."""
+    best = float("inf")
+    for _ in range(3):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        f()
+        torch.cuda.synchronize()
+        a.record()
+        for _ in range(n):
+            f()
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b) * 1e3 / n)
+    return best

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import mm_amx_amd as mx
-from gpu_util import dev, dev_bf16, host_bits
+from gpu_util import call_us, dev, dev_bf16, host_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -52,22 +52,6 @@ def test_quantisers_row_ends_and_gaps(po, rows, cols, gap):
     assert np.array_equal(host_bits(mx.quantize_weights_scaled(wide[:, :cols], 1234.5)), po.quantize_scale_trunc(W, 1234.5))
 
 
-def _us(f, n=10):
-    """The least of three timings of n calls, per call."""
-    best = float("inf")
-    for _ in range(3):
-        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        f()
-        torch.cuda.synchronize()
-        a.record()
-        for _ in range(n):
-            f()
-        b.record()
-        torch.cuda.synchronize()
-        best = min(best, a.elapsed_time(b) * 1e3 / n)
-    return best
-
-
 @pytest.mark.parametrize("rows,cols", [(1000000, 8), (131072, 128), (16384, 1024)])
 def test_gaps_between_short_rows_cost_little(rows, cols):
     """With a gap as long as the row up to twice the lines are read.  A workgroup to a row took 25 times as long as without
@@ -75,7 +59,7 @@ def test_gaps_between_short_rows_cost_little(rows, cols):
     W = torch.randn((rows, 2 * cols), device="cuda").to(torch.bfloat16)
     for f in (mx.quantize_weights, lambda w: mx.quantize_weights_scaled(w, 30.0)):
         whole, gaps = W[:, :cols].contiguous(), W[:, :cols]
-        assert _us(lambda: f(gaps)) <= 6 * _us(lambda: f(whole))
+        assert call_us(lambda: f(gaps)) <= 6 * call_us(lambda: f(whole))
 
 
 @pytest.mark.parametrize("K", [1, 64, 65, 129, 255, 256, 257, 513, 2056])
@@ -103,4 +87,4 @@ def test_int4_pack_of_a_short_k_costs_no_more_than_its_bytes(K):
     long, short = (torch.randn((N, k), device="cuda").to(torch.bfloat16) for k in (512, K))
     for trans in (True, False):
         a, b = (long, short) if trans else (long.t().contiguous(), short.t().contiguous())
-        assert _us(lambda: mx.quantize_pack_int4(b, transpose=trans)) <= 0.45 * _us(lambda: mx.quantize_pack_int4(a, transpose=trans))
+        assert call_us(lambda: mx.quantize_pack_int4(b, transpose=trans)) <= 0.45 * call_us(lambda: mx.quantize_pack_int4(a, transpose=trans))
