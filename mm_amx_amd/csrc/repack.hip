@@ -18,20 +18,64 @@ namespace mmx {
 // whole 128-byte lines and that enough of them are in flight.  (One thread per 16-byte slot, gathering its elements one
 // by one, asked for 32 bytes of a line per row and instruction from [N, K] and for two bytes per lane from [K, N].)
 
-// 16 bytes at `p` of a row of which `left` bytes from p on exist (none when left <= 0); what does not exist is zero
-// and not touched.  The alignment is the element's: the hardware takes 16-byte loads from any address.
-template <int ES>
-__device__ __forceinline__ u32x4 load16_tail(const char* p, int64_t left) {
-    typedef typename std::conditional<ES == 2, uint16_t, uint8_t>::type elem;
-    u32x4 v = u32x4{0u, 0u, 0u, 0u};
-    if (left >= 16) {
-        __builtin_memcpy(&v, __builtin_assume_aligned(p, ES), 16);
-    } else if (left > 0) {
-        alignas(16) elem e[16 / ES];
+// All of a row of W to 2 W - 1 bytes, by W bytes from either end; zero behind it.
+template <int W>
+__device__ __forceinline__ u32x4 load_short_row(const char* row, int len) {
+    uint64_t head = 0, tail = 0;
+    __builtin_memcpy(&head, __builtin_assume_aligned(row, 1), W);
+    __builtin_memcpy(&tail, __builtin_assume_aligned(row + len - W, 1), W);
+    tail = (tail >> (8 * (2 * W - len) - 1)) >> 1;  // what lies behind the first W bytes, if anything
+    const uint64_t lo = W == 8 ? head : head | tail << (8 * (W & 7)), hi = W == 8 ? tail : 0;
+    return u32x4{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+}
+
+// N times 16 bytes from byte `at` of the rows at row(0) ... row(N - 1), each of len bytes.  What lies past the end, and a row
+// that is not live(i), is zero and not touched.  No load waits for another; what moves the bytes down runs behind all of them,
+// and only where the rows end inside the 16.  (Element by element behind tests, each load waited for the one before it: bytes
+// from [K, N], K = 512, N = 3001 9.4 us against 4.5 for a thread per slot.)
+// RowLength: what the host knows of len (the code for rows shorter than 16 bytes takes registers).
+enum RowLength { ANY_ROW, SHORT_ROW, LONG_ROW };  // any, below 16 bytes, 16 and up
+template <int ES, RowLength LEN = ANY_ROW, int N, typename Row, typename Live>
+__device__ __forceinline__ void load16_rows(u32x4 (&v)[N], int64_t at, int64_t len, Row&& row, Live&& live) {
 #pragma unroll
-        for (int i = 0; i < 16 / ES; i++) e[i] = i * ES < left ? reinterpret_cast<const elem*>(p)[i] : (elem)0;
-        __builtin_memcpy(&v, e, 16);
+    for (int i = 0; i < N; i++) v[i] = u32x4{0u, 0u, 0u, 0u};
+    typedef typename std::conditional<ES == 2, uint16_t, uint8_t>::type elem;
+    if (at >= len) return;
+    if (LEN == LONG_ROW || (LEN == ANY_ROW && len >= 16)) {
+        const int64_t from = at < len - 16 ? at : len - 16;
+#pragma unroll
+        for (int i = 0; i < N; i++)
+            if (live(i)) __builtin_memcpy(&v[i], __builtin_assume_aligned(row(i) + from, ES), 16);
+        if (from < at) {
+#pragma unroll
+            for (int i = 0; i < N; i++) v[i] = settle16_in_row(v[i], (int)(at - from), 16);
+        }
+    } else if constexpr (LEN == SHORT_ROW) {
+        auto all = [&](auto w) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < N; i++)
+                if (live(i)) v[i] = load_short_row<decltype(w)::value>(row(i), (int)len);
+        };
+        if (len >= 8) all(std::integral_constant<int, 8>{});
+        else if (len >= 4) all(std::integral_constant<int, 4>{});
+        else if (len >= 2) all(std::integral_constant<int, 2>{});
+        else all(std::integral_constant<int, 1>{});
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; i++)
+            if (live(i)) {
+                alignas(16) elem e[16 / ES];
+#pragma unroll
+                for (int j = 0; j < 16 / ES; j++) e[j] = j * ES < len ? reinterpret_cast<const elem*>(row(i))[j] : (elem)0;
+                __builtin_memcpy(&v[i], e, 16);
+            }
     }
+}
+// the same where all of it is there
+template <int ES>
+__device__ __forceinline__ u32x4 load16(const char* p) {
+    u32x4 v;
+    __builtin_memcpy(&v, __builtin_assume_aligned(p, ES), 16);
     return v;
 }
 
@@ -41,7 +85,7 @@ __device__ __forceinline__ u32x4 load16_tail(const char* p, int64_t left) {
 // a store are 128 consecutive bytes, whole lines again.  UNR such units per wavefront keep 4 UNR loads in flight.
 // PAIR: gate and up interleaved by panel, panel 2p = gate columns [32p, 32p + 32), panel 2p + 1 = up's.
 // N = 11008, K = 4096, against a thread per slot: bf16 82 -> 31 us (5.8 TB/s moved), bytes 91 -> 16, gate and up 157 -> 67.
-template <int ES, int UNR, bool PAIR>
+template <int ES, int UNR, bool PAIR, RowLength LEN>
 __global__ __launch_bounds__(256) void repack_rows_kernel(const char* __restrict__ B0, const char* __restrict__ B1, int64_t ldb, int kbytes,
                                                           int N, char* __restrict__ out, int kunits, int groups, int flip) {
     const int lane = threadIdx.x & 63;
@@ -51,34 +95,40 @@ __global__ __launch_bounds__(256) void repack_rows_kernel(const char* __restrict
     const int n0 = (PAIR ? panel >> 1 : panel) * 32;
     const int r8 = lane >> 3, c = lane & 7;
     u32x4 v[UNR][4];
-    auto fetch = [&](bool whole) __attribute__((always_inline)) {
+    char* const o = out + ((int64_t)panel * kunits + ku0) * 4096 + (c >> 1) * 1024 + (32 * (c & 1) + r8) * 16;
+    auto store = [&](bool whole) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < UNR; u++) {
+            if (!whole && ku0 + u >= kunits) break;
             const int kb = (ku0 + u) * 128 + c * 16;
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                const int n = n0 + 8 * i + r8;
-                v[u][i] = load16_tail<ES>(B + (int64_t)n * ldb + kb, whole ? 16 : (n < N ? kbytes - kb : 0));
+                u32x4 w = v[u][i];
+                if (ES == 1 && flip && n0 + 8 * i + r8 < N) {  // (the padding stays zero)
+#pragma unroll
+                    for (int e = 0; e < 16; e++)
+                        if (kb + e < kbytes) w[e >> 2] ^= 0x80u << (8 * (e & 3));
+                }
+                *reinterpret_cast<u32x4*>(o + u * 4096 + i * 128) = w;
             }
         }
     };
-    if (n0 + 32 <= N && (ku0 + UNR) * 128 <= kbytes) fetch(true);
-    else fetch(false);
-    char* const o = out + ((int64_t)panel * kunits + ku0) * 4096 + (c >> 1) * 1024 + (32 * (c & 1) + r8) * 16;
+    // (the stores are in both branches, so that each waits for its own load only: behind the join they waited for all,
+    // 3001 x 8192 bf16 17.9 us against 16.5)
+    if (n0 + 32 <= N && (ku0 + UNR) * 128 <= kbytes) {
 #pragma unroll
-    for (int u = 0; u < UNR; u++) {
-        if (ku0 + u >= kunits) break;
-        const int kb = (ku0 + u) * 128 + c * 16;
+        for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            u32x4 w = v[u][i];
-            if (ES == 1 && flip && n0 + 8 * i + r8 < N) {  // (the padding stays zero)
+            for (int u = 0; u < UNR; u++) v[u][i] = load16<ES>(B + (int64_t)(n0 + 8 * i + r8) * ldb + (ku0 + u) * 128 + c * 16);
+        __builtin_amdgcn_sched_barrier(0);  // (neighbouring lines of a row one right behind the other: unaligned rows share one)
+        store(true);
+    } else {
 #pragma unroll
-                for (int e = 0; e < 16; e++)
-                    if (kb + e < kbytes) w[e >> 2] ^= 0x80u << (8 * (e & 3));
-            }
-            *reinterpret_cast<u32x4*>(o + u * 4096 + i * 128) = w;
-        }
+        for (int u = 0; u < UNR; u++)
+            if (ku0 + u < kunits)
+                load16_rows<ES, LEN>(v[u], (ku0 + u) * 128 + c * 16, kbytes, [&](int i) { return B + (int64_t)(n0 + 8 * i + r8) * ldb; },
+                                     [&](int i) { return n0 + 8 * i + r8 < N; });
+        store(false);
     }
 }
 
@@ -89,7 +139,7 @@ __global__ __launch_bounds__(256) void repack_rows_kernel(const char* __restrict
 // as whole fragments.  LDS positions are XORed with the bits above the low four, which spreads the lanes of a write over
 // the banks.
 // 10240 x 10240, against a thread per slot: bf16 99 -> 90 us (4.7 TB/s moved), bytes 122 -> 35.
-template <int ES>
+template <int ES, RowLength LEN>
 __global__ __launch_bounds__(ES == 2 ? 256 : 64) void repack_cols_kernel(const char* __restrict__ B, int64_t ldb, int K, int N,
                                                                          char* __restrict__ out, int kunits, int npanels, int flip) {
     constexpr int EL = 16 / ES;               // columns and k of a lane's square
@@ -103,11 +153,10 @@ __global__ __launch_bounds__(ES == 2 ? 256 : 64) void repack_cols_kernel(const c
     u32x4 row[EL];
     if ((pg + 1) * (8 * EL) <= N && (ku + 1) * (8 * EL) <= K) {
 #pragma unroll
-        for (int e = 0; e < EL; e++) row[e] = load16_tail<ES>(B + (int64_t)(k + e) * ldb + (int64_t)n * ES, 16);
+        for (int e = 0; e < EL; e++) row[e] = load16<ES>(B + (int64_t)(k + e) * ldb + (int64_t)n * ES);
     } else {
-#pragma unroll
-        for (int e = 0; e < EL; e++)
-            row[e] = load16_tail<ES>(B + (int64_t)(k + e) * ldb + (int64_t)n * ES, k + e < K ? (int64_t)(N - n) * ES : 0);
+        load16_rows<ES, LEN>(row, (int64_t)n * ES, (int64_t)N * ES, [&](int e) { return B + (int64_t)(k + e) * ldb; },
+                        [&](int e) { return k + e < K; });
     }
     if (ES == 1 && flip) {
 #pragma unroll
@@ -172,7 +221,8 @@ static int launch_repack_rows(const void* B0, const void* B1, int64_t ldb, int K
     const int kunits = (int)(((int64_t)K * ES + 127) / 128), groups = (kunits + 4 * UNR - 1) / (4 * UNR);
     const int64_t blocks = (int64_t)npanels * groups;
     if (blocks > 0x7fffffff) return set_error(MMX_E_INVALID, "weight matrix too large to repack in one launch");
-    hipLaunchKernelGGL((repack_rows_kernel<ES, UNR, PAIR>), dim3((unsigned)blocks), dim3(256), 0, st, static_cast<const char*>(B0),
+    const bool is_short = (int64_t)K * ES < 16;
+    hipLaunchKernelGGL((is_short ? repack_rows_kernel<ES, UNR, PAIR, SHORT_ROW> : repack_rows_kernel<ES, UNR, PAIR, LONG_ROW>), dim3((unsigned)blocks), dim3(256), 0, st, static_cast<const char*>(B0),
                        static_cast<const char*>(B1), ldb, K * ES, N, static_cast<char*>(out), kunits, groups, flip);
     return check_hip(hipGetLastError(), "repack_rows_kernel launch");
 }
@@ -183,7 +233,8 @@ static int launch_repack_cols(const void* B, int64_t ldb, int K, int N, void* ou
     constexpr int WAVES = ES == 2 ? 4 : 1, PER_BLOCK = WAVES * (ES == 2 ? 2 : 4);
     const int64_t blocks = (int64_t)((npanels + PER_BLOCK - 1) / PER_BLOCK) * kunits;
     if (blocks > 0x7fffffff) return set_error(MMX_E_INVALID, "weight matrix too large to repack in one launch");
-    hipLaunchKernelGGL((repack_cols_kernel<ES>), dim3((unsigned)blocks), dim3(64 * WAVES), 0, st, static_cast<const char*>(B), ldb, K, N,
+    const bool is_short = (int64_t)N * ES < 16;
+    hipLaunchKernelGGL((is_short ? repack_cols_kernel<ES, SHORT_ROW> : repack_cols_kernel<ES, LONG_ROW>), dim3((unsigned)blocks), dim3(64 * WAVES), 0, st, static_cast<const char*>(B), ldb, K, N,
                        static_cast<char*>(out), kunits, npanels, flip);
     return check_hip(hipGetLastError(), "repack_cols_kernel launch");
 }
@@ -202,7 +253,7 @@ int launch_repack_gate_up(const void* wg, const void* wu, int64_t ldw, int K, in
 __global__ void zero_u32_kernel(uint32_t* p) { *p = 0u; }
 
 // All three kernels of this section stream bf16 and are bound by memory: a lane takes 16 bytes (8 weights) at a time, four
-// such loads in flight; weights past the last whole 8 of a row are taken one by one by load16_tail.  A matrix whose rows
+// such loads in flight.  A matrix whose rows
 // follow each other without a gap is walked as one row (the host passes rows = 1).
 // (11008 x 4096 weights: two bytes per load and a 64-bit division per weight took 217 us for the maxima and 65 for the
 // quantisation; now 18 us, 5.1 TB/s read, and 25 us, 5.5 TB/s read and written; the scaled form 68 -> 30.)
@@ -220,9 +271,7 @@ __device__ __forceinline__ void for_each_8_weights(const char* __restrict__ W, i
         for (int64_t r = r0; r < rows; r += step * QUANT_UNR) {
             for (int64_t c = (int64_t)(threadIdx.x & ((1 << row_log2) - 1)) * 8; c < cols; c += (int64_t)8 << row_log2) {
                 u32x4 v[QUANT_UNR];
-#pragma unroll
-                for (int u = 0; u < QUANT_UNR; u++)
-                    v[u] = load16_tail<2>(W + (r + u * step) * ldw + c * 2, r + u * step < rows ? (cols - c) * 2 : 0);
+                load16_rows<2>(v, c * 2, cols * 2, [&](int u) { return W + (r + u * step) * ldw; }, [&](int u) { return r + u * step < rows; });
 #pragma unroll
                 for (int u = 0; u < QUANT_UNR; u++)
                     if (r + u * step < rows) f(r + u * step, c, v[u]);
@@ -236,13 +285,18 @@ __device__ __forceinline__ void for_each_8_weights(const char* __restrict__ W, i
                 u32x4 v[QUANT_UNR];
                 if ((i0 + (QUANT_UNR - 1) * step) * 8 + 8 <= cols) {
 #pragma unroll
-                    for (int u = 0; u < QUANT_UNR; u++) v[u] = load16_tail<2>(row + (i0 + u * step) * 16, 16);
+                    for (int u = 0; u < QUANT_UNR; u++) v[u] = load16<2>(row + (i0 + u * step) * 16);
+#pragma unroll
+                    for (int u = 0; u < QUANT_UNR; u++) f(r, (i0 + u * step) * 8, v[u]);
                 } else {
 #pragma unroll
-                    for (int u = 0; u < QUANT_UNR; u++) v[u] = load16_tail<2>(row + (i0 + u * step) * 16, (cols - (i0 + u * step) * 8) * 2);
+                    for (int u = 0; u < QUANT_UNR; u++) {
+                        if ((i0 + u * step) * 8 >= cols) break;
+                        u32x4 w[1];
+                        load16_rows<2>(w, (i0 + u * step) * 16, cols * 2, [&](int) { return row; }, [&](int) { return true; });
+                        f(r, (i0 + u * step) * 8, w[0]);
+                    }
                 }
-#pragma unroll
-                for (int u = 0; u < QUANT_UNR; u++) f(r, (i0 + u * step) * 8, v[u]);
             }
         }
     }
@@ -315,23 +369,26 @@ static void one_row(int64_t ldw, int64_t ldq, int& rows, int64_t& cols) {
     if (ldw == cols * 2 && ldq == cols) cols *= rows, rows = 1;
 }
 
-// How the kernels above walk a matrix: at most `most` workgroups, each taking QUANT_UNR loads per lane at a time.  Rows that
-// do not fill those of one workgroup are shared out (ROWS): the fewest lanes, a power of two, that cover a row.
+// How the kernels above walk a matrix: QUANT_UNR loads per lane at a time, by at most `most` workgroups; with `spread` one load
+// per lane while there are fewer than two workgroups for every CU (a lane that works through four runs of eight weights by itself took 3.8 us
+// for 300 x 100, 3.3 with one; not for the maxima, whose workgroups cost an atomic each).  Rows with gaps that do not fill the
+// loads of one workgroup are shared out (ROWS): the fewest lanes, a power of two, that cover a row.
 struct QuantWalk {
     bool by_rows;
     int row_log2;
     dim3 grid;
 };
-static QuantWalk quantize_walk(int rows, int64_t cols, int threads, int most) {
-    const int64_t per_block = (int64_t)threads * 8 * QUANT_UNR;
-    if (rows > 1 && cols < per_block) {
+static QuantWalk quantize_walk(int rows, int64_t cols, int threads, int most, bool spread) {
+    auto blocks = [&](int64_t n, int64_t per_load, int64_t others) {
+        const int64_t x = (n + per_load * QUANT_UNR - 1) / (per_load * QUANT_UNR), x1 = (n + per_load - 1) / per_load;
+        return spread && x * others < 2 * num_cus() ? (x1 < 2 * num_cus() ? x1 : 2 * num_cus()) : (x < most ? x : most);
+    };
+    if (rows > 1 && cols < (int64_t)threads * 8 * QUANT_UNR) {
         int log2 = 0;
         while ((8 << log2) < cols && (1 << log2) < threads) log2++;
-        const int64_t rows_per_block = (int64_t)(threads >> log2) * QUANT_UNR, x = (rows + rows_per_block - 1) / rows_per_block;
-        return {true, log2, dim3((unsigned)(x < most ? x : most))};
+        return {true, log2, dim3((unsigned)blocks(rows, threads >> log2, 1))};
     }
-    const int64_t x = (cols + per_block - 1) / per_block;
-    const int gx = x < most ? (int)x : most, gy = most / gx;
+    const int gx = (int)blocks(cols, threads * 8, rows), gy = most / gx;
     return {false, 0, dim3((unsigned)gx, (unsigned)(rows < gy ? rows : gy))};
 }
 
@@ -339,7 +396,7 @@ int launch_quantize(const void* W, int64_t ldw, int rows, int cols_in, void* Wq,
                     uint32_t* scratch, hipStream_t st) {
     int64_t cols = cols_in;
     one_row(ldw, ldq, rows, cols);
-    const QuantWalk m = quantize_walk(rows, cols, ABSMAX_THREADS, num_cus()), q = quantize_walk(rows, cols, 256, 2048);
+    const QuantWalk m = quantize_walk(rows, cols, ABSMAX_THREADS, num_cus(), false), q = quantize_walk(rows, cols, 256, 2048, true);
     hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, st, scratch);
     hipLaunchKernelGGL(m.by_rows ? absmax_kernel<true> : absmax_kernel<false>, m.grid, dim3(ABSMAX_THREADS), 0, st, static_cast<const char*>(W),
                        ldw, rows, cols, m.row_log2, scratch);
@@ -375,7 +432,7 @@ __global__ __launch_bounds__(256) void quantize_scale_trunc_kernel(const char* _
 int launch_quantize_scale_trunc(const void* W, int64_t ldw, int rows, int cols_in, float scale, void* Wq, int64_t ldq, hipStream_t st) {
     int64_t cols = cols_in;
     one_row(ldw, ldq, rows, cols);
-    const QuantWalk q = quantize_walk(rows, cols, 256, 2048);
+    const QuantWalk q = quantize_walk(rows, cols, 256, 2048, true);
     hipLaunchKernelGGL(q.by_rows ? quantize_scale_trunc_kernel<true> : quantize_scale_trunc_kernel<false>, q.grid, dim3(256), 0, st,
                        static_cast<const char*>(W), ldw, rows, cols, q.row_log2, scale, static_cast<char*>(Wq), ldq);
     return check_hip(hipGetLastError(), "quantize_scale_trunc_kernel launch");
@@ -582,10 +639,12 @@ __device__ __forceinline__ uint32_t int4_of(float w, float scale) {
 // [N, K], 64 of k from k0 on: 4 loads of 8 rows x 128 bytes; and the fragment they make, scaled by qs.
 __device__ __forceinline__ void load_fragment_rows(u32x4 (&v)[4], const char* W, int64_t ldw, int K, int N, int n0, int k0) {
     const int lane = threadIdx.x & 63, r8 = lane >> 3, k = k0 + 8 * (lane & 7);
+    if (n0 + 32 <= N && k0 + 64 <= K) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int n = n0 + 8 * i + r8;
-        v[i] = load16_tail<2>(W + (int64_t)n * ldw + (int64_t)k * 2, n < N ? (int64_t)(K - k) * 2 : 0);
+        for (int i = 0; i < 4; i++) v[i] = load16<2>(W + (int64_t)(n0 + 8 * i + r8) * ldw + (int64_t)k * 2);
+    } else {
+        load16_rows<2>(v, (int64_t)k * 2, (int64_t)K * 2, [&](int i) { return W + (int64_t)(n0 + 8 * i + r8) * ldw; },
+                       [&](int i) { return n0 + 8 * i + r8 < N; });
     }
 }
 __device__ __forceinline__ void store_fragment_rows(const u32x4 (&v)[4], const float (&qs)[4], char* fragment) {
@@ -603,9 +662,13 @@ __device__ __forceinline__ void store_fragment_rows(const u32x4 (&v)[4], const f
 // [K, N], 128 of k from k0 on: a lane takes 8 columns of 8 rows, 16 chunks of k to a wavefront; and their two fragments.
 __device__ __forceinline__ void load_fragments_cols(u32x4 (&v)[8], const char* W, int64_t ldw, int K, int N, int n0, int k0) {
     const int lane = threadIdx.x & 63, n = n0 + 8 * (lane & 3), k = k0 + 8 * (lane >> 2);
+    if (n0 + 32 <= N && k0 + 128 <= K) {
 #pragma unroll
-    for (int e = 0; e < 8; e++)
-        v[e] = load16_tail<2>(W + (int64_t)(k + e) * ldw + (int64_t)n * 2, k + e < K ? (int64_t)(N - n) * 2 : 0);
+        for (int e = 0; e < 8; e++) v[e] = load16<2>(W + (int64_t)(k + e) * ldw + (int64_t)n * 2);
+    } else {
+        load16_rows<2>(v, (int64_t)n * 2, (int64_t)N * 2, [&](int e) { return W + (int64_t)(k + e) * ldw; },
+                       [&](int e) { return k + e < K; });
+    }
 }
 __device__ __forceinline__ void store_fragments_cols(const u32x4 (&v)[8], const float (&qs)[8], char* fragments) {
     const int lane = threadIdx.x & 63, ng = lane & 3, kc = lane >> 2;
@@ -700,10 +763,20 @@ __global__ __launch_bounds__(QUANT4_WAVES * 64) void quant4_pack_kernel(const ch
                     u32x4 v[UNR];
                     if (k + 512 * (UNR - 1) + 8 <= K) {
 #pragma unroll
-                        for (int u = 0; u < UNR; u++) v[u] = load16_tail<2>(row + (int64_t)(k + 512 * u) * 2, 16);
+                        for (int u = 0; u < UNR; u++) v[u] = load16<2>(row + (int64_t)(k + 512 * u) * 2);
                     } else {
 #pragma unroll
-                        for (int u = 0; u < UNR; u++) v[u] = load16_tail<2>(row + (int64_t)(k + 512 * u) * 2, (int64_t)(K - k - 512 * u) * 2);
+                        for (int u = 0; u < UNR; u++) {
+                            v[u] = u32x4{0u, 0u, 0u, 0u};
+                            if (k + 512 * u + 8 <= K) v[u] = load16<2>(row + (int64_t)(k + 512 * u) * 2);
+                        }
+#pragma unroll
+                        for (int u = 0; u < UNR; u++)
+                            if (k + 512 * u < K && k + 512 * u + 8 > K) {
+                                u32x4 w[1];
+                                load16_rows<2>(w, (int64_t)(k + 512 * u) * 2, (int64_t)K * 2, [&](int) { return row; }, [&](int) { return true; });
+                                v[u] = w[0];
+                            }
                     }
 #pragma unroll
                     for (int u = 0; u < UNR; u++)
@@ -716,14 +789,16 @@ __global__ __launch_bounds__(QUANT4_WAVES * 64) void quant4_pack_kernel(const ch
         }
     } else {
         const int ng = lane & 3;  // columns 8 ng .. 8 ng + 7 of the panel
-        const int64_t left = (int64_t)(N - n0 - 8 * ng) * 2;
         float m[8] = {0, 0, 0, 0, 0, 0, 0, 0};
         for (int k = wave * 16 + (lane >> 2); k < K; k += QUANT4_WAVES * 16 * UNR) {
             u32x4 v[UNR];
+            auto ku = [&](int u) { return k + QUANT4_WAVES * 16 * u; };
+            if (n0 + 32 <= N && ku(UNR - 1) < K) {
 #pragma unroll
-            for (int u = 0; u < UNR; u++) {
-                const int ku = k + QUANT4_WAVES * 16 * u;
-                v[u] = load16_tail<2>(W + (int64_t)ku * ldw + (int64_t)(n0 + 8 * ng) * 2, ku < K ? left : 0);
+                for (int u = 0; u < UNR; u++) v[u] = load16<2>(W + (int64_t)ku(u) * ldw + (int64_t)(n0 + 8 * ng) * 2);
+            } else {
+                load16_rows<2>(v, (int64_t)(n0 + 8 * ng) * 2, (int64_t)N * 2, [&](int u) { return W + (int64_t)ku(u) * ldw; },
+                               [&](int u) { return ku(u) < K; });
             }
 #pragma unroll
             for (int u = 0; u < UNR; u++)

@@ -16,8 +16,8 @@ def _init():
 
 
 @pytest.mark.parametrize("dt", ["bf16", "int8", "uint8"])
-@pytest.mark.parametrize("K", [1, 63, 64, 65, 128, 511, 1025])
-@pytest.mark.parametrize("N", [1, 31, 64, 129, 257])
+@pytest.mark.parametrize("K", [1, 2, 3, 7, 9, 15, 16, 63, 64, 65, 128, 511, 1025])
+@pytest.mark.parametrize("N", [1, 2, 3, 5, 7, 8, 9, 15, 17, 31, 64, 129, 257])
 def test_repack_unit_edges(po, dt, K, N):
     rng = np.random.default_rng(K * 1000 + N)
     if dt == "bf16":
@@ -88,3 +88,15 @@ def test_int4_pack_of_a_short_k_costs_no_more_than_its_bytes(K):
     for trans in (True, False):
         a, b = (long, short) if trans else (long.t().contiguous(), short.t().contiguous())
         assert call_us(lambda: mx.quantize_pack_int4(b, transpose=trans)) <= 0.45 * call_us(lambda: mx.quantize_pack_int4(a, transpose=trans))
+
+
+def test_rows_that_end_inside_16_bytes_are_one_trip_to_memory():
+    """Bytes from [K, N], a square of 16 x 16 per lane: fetched element by element at the end of a row they took 3 times as
+    long at N = 3001 as at N = 3008."""
+    took = {}
+    for N in (3001, 3008):
+        B = torch.randint(-128, 128, (512, N), device="cuda", dtype=torch.int8)
+        out = torch.empty(mx.packed_b_bytes(mx.I8, 512, N), dtype=torch.uint8, device="cuda")
+        call = (mx.I8, B.data_ptr(), N, 512, N, 0, out.data_ptr(), torch.cuda.current_stream().cuda_stream)
+        took[N] = call_us(lambda: mx.lib().mmx_repack_b(*call), n=50)
+    assert took[3001] <= 1.7 * took[3008], took
