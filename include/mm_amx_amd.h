@@ -244,14 +244,17 @@ int mmx_mlp_splitk(const void* x, int64_t ldx_bytes, const void* w_gate_up, cons
 /* ---- introspection / tuning (no reference counterpart) --------------------------------------- */
 /* Force the MFMA tile shape ("256x256", "256x192", "128x256", "128x192", "128x128", "128x64", "64x128" (aligned
  * operands and no SILU_GATE only; otherwise 128x128 is used), "" = automatic)
- * for the calling thread's later calls. */
+ * for the calling thread's later calls.  A K that does not fill its last 128 bytes has 256x192, 128x128, 128x64 (not over
+ * int8-compressed weights) and 64x128; rows of A that are not 16-byte aligned, or with such a K shorter than 128 bytes,
+ * have 128x128: where the forced shape does not exist 128x128 is used. */
 int mmx_set_tile(const char* shape);
 /* Name of the kernel variant the last mmx_gemm call of this thread launched. */
 const char* mmx_last_kernel(void);
 /* Sets a kernel option.  "load_mode": how the MFMA tile kernel brings A and B tiles into LDS —
  * 2 (default) direct HBM->LDS loads in a hand-scheduled ring pipeline, 0 through registers (the
- * fallback for operands beyond 32-bit offsets).  Shapes whose K tail or alignment need masked
- * loads use a masked kernel whatever this is set to.  "decode_halves": whether the streaming decode
+ * fallback for operands beyond 32-bit offsets).  Rows of A that are not 16-byte aligned use a masked
+ * kernel whatever this is set to, as does a K that does not fill its last 128 bytes if this is 0 or K is shorter than
+ * that (otherwise the ring pipeline finishes it in a step of its own).  "decode_halves": whether the streaming decode
  * kernel for M <= 4 splits every 32-column panel over two workgroups — -1 (default) where that fills the
  * CUs better, 0 never, 1 always while x takes at most 46 KiB of LDS (the two forms add the partial sums in
  * different orders).  "waves": 8 (default) lets the 256x192 tile kernel run as eight wavefronts per

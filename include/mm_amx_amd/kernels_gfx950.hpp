@@ -378,8 +378,8 @@ inline void release_workspaces() {
 
 // ---- Matmul<TA,TB,TC> (include/kernels_amx.hpp:1045-1315) ---------------------------------------
 // C = PP(A · B[:, n0:n1]).  With constB the packed weights are made at the first call and kept
-// (1188-1192); otherwise B is repacked on every call.  One object is used by one thread at a time,
-// as in the reference; calls are ordered on the stream.
+// (1188-1192); otherwise B is used where it lies (bf16, few rows of A) or repacked on every call.  One object is used by
+// one thread at a time, as in the reference; calls are ordered on the stream.
 template <typename TA, typename TB, typename TC = typename acc_type<TA>::type>
 struct Matmul {
     PackedB<TB> internalB;

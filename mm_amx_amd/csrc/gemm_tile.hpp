@@ -126,8 +126,8 @@ template <>
 __device__ __forceinline__ int32_t cvt_out<int32_t>(float r) { return (int32_t)r; }
 
 // 16 bytes to an address that is aligned to an element of SZ bytes only: the hardware takes such stores whole.  (Rows of C
-// that are not 16-byte aligned used to be written element by element: 391 x 1024 x 3001 bf16 14.4 -> 8.8 us,
-// 1024 x 4096 x 10999 115 -> 76.)
+// that are not 16-byte aligned used to be written element by element: a call of 391 x 1024 x 3001 bf16 14.4 -> 9.4 us,
+// of 1024 x 4096 x 10999 115 -> 85.)
 template <int SZ>
 __device__ __forceinline__ void store16(char* p, u32x4 v) { __builtin_memcpy(__builtin_assume_aligned(p, SZ), &v, 16); }
 
@@ -635,57 +635,57 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
         // MODE 4: the part of K behind the last whole k-iteration, once: A through registers (its rows end inside the 128
         // bytes) and the weights, whose padding is there, into the first slots of the rings; then four k-steps.  The trip to
         // memory is not hidden behind anything, but it is one: the masked pipeline, which this replaces for aligned rows,
-        // waits for one per k-iteration (bf16 1064 x 3544 x 786 62 -> 31 us, 64 x 4104 x 4096 52 -> 14).  (A mode of its own: behind this branch the compiler keeps the accumulators twice,
-        // which the largest tiles have no registers for.)
+        // waits for one per k-iteration (bf16 1064 x 3544 x 786 62 -> 31 us, 64 x 4104 x 4096 52 -> 14).  (A mode of its own:
+        // behind this branch the compiler keeps the accumulators twice, which the largest tiles have no registers for.)
         if constexpr (MODE == 4) {
-        if (SMAX == 1 || kt0 + nk == g.nk) {
-            constexpr int AC = BM * 8 / NT, BC = (BN / 32) * (BP_IT / 16);
-            u32x4 ta[AC], tb[(BC + NT - 1) / NT];
+            if (SMAX == 1 || kt0 + nk == g.nk) {
+                constexpr int AC = BM * 8 / NT, BC = (BN / 32) * (BP_IT / 16);
+                u32x4 ta[AC], tb[(BC + NT - 1) / NT];
 #pragma unroll
-            for (int it = 0; it < AC; it++) {
-                const int row = (it * NT + tid) >> 3, chunk = (tid & 7) ^ ((row >> 1) & 7);
-                const int grow = m0 + row < g.M ? m0 + row : g.M - 1;
-                ta[it] = fetch16_in_row(g.A + (int64_t)grow * g.lda, g.nk * 128 + chunk * 16, g.kbytes);
-            }
-#pragma unroll
-            for (int it = 0; it < (BC + NT - 1) / NT; it++) {
-                const int c = it * NT + tid;
-                int panel = panel0 + c / (BP_IT / 16);
-                panel = panel < g.npanels ? panel : g.npanels - 1;
-                if (BC % NT == 0 || c < BC)
-                    tb[it] = *reinterpret_cast<const u32x4*>(g.Bp + (int64_t)panel * g.panel_stride + (int64_t)g.nk * BP_IT + (c % (BP_IT / 16)) * 16);
-            }
-            __syncthreads();  // every wave has finished with the rings (and its own re-fetched slots have landed)
-#pragma unroll
-            for (int it = 0; it < AC; it++)
-                *reinterpret_cast<u32x4*>(smem + (it * NT + tid) * 16) =
-                    settle16_in_row(ta[it], g.nk * 128 + ((tid & 7) ^ ((((it * NT + tid) >> 3) >> 1) & 7)) * 16, g.kbytes);
-#pragma unroll
-            for (int it = 0; it < (BC + NT - 1) / NT; it++) {
-                const int c = it * NT + tid, in = c % (BP_IT / 16);
-                if (BC % NT == 0 || c < BC)
-                    *reinterpret_cast<u32x4*>(smem + B0 + (in / (BP_HS / 16)) * BH + (c / (BP_IT / 16)) * BP_HS + (in % (BP_HS / 16)) * 16) = tb[it];
-            }
-            __syncthreads();
-#pragma unroll
-            for (int s = 0; s < 4; s++) {
-                const int chunk = W8 ? 4 * (s >> 1) + 2 * g32 + (s & 1) : 2 * s + g32;
-                const char* sA = smem + (wm * WM + l32) * 128 + ((chunk ^ ((l32 >> 1) & 7)) * 16);
-                const char* sB = smem + B0 + (s >> 1) * BH + wn * NJ * BP_HS + lane * 16;
-#pragma unroll
-                for (int i = 0; i < MI; i++) fa[0][i] = *reinterpret_cast<const frag*>(sA + i * 32 * 128);
-#pragma unroll
-                for (int j = 0; j < NJ; j++) {
-                    if constexpr (W8) {
-                        const u32x4 raw = *reinterpret_cast<const u32x4*>(sB + j * BP_HS);
-                        fb[0][j] = (s & 1) ? s8x8_to_bf16(raw[2], raw[3]) : s8x8_to_bf16(raw[0], raw[1]);
-                    } else {
-                        fb[0][j] = *reinterpret_cast<const frag*>(sB + j * BP_HS + (s & 1) * 1024);
-                    }
+                for (int it = 0; it < AC; it++) {
+                    const int row = (it * NT + tid) >> 3, chunk = (tid & 7) ^ ((row >> 1) & 7);
+                    const int grow = m0 + row < g.M ? m0 + row : g.M - 1;
+                    ta[it] = fetch16_in_row(g.A + (int64_t)grow * g.lda, g.nk * 128 + chunk * 16, g.kbytes);
                 }
-                mma(fa[0], fb[0]);
+#pragma unroll
+                for (int it = 0; it < (BC + NT - 1) / NT; it++) {
+                    const int c = it * NT + tid;
+                    int panel = panel0 + c / (BP_IT / 16);
+                    panel = panel < g.npanels ? panel : g.npanels - 1;
+                    if (BC % NT == 0 || c < BC)
+                        tb[it] = *reinterpret_cast<const u32x4*>(g.Bp + (int64_t)panel * g.panel_stride + (int64_t)g.nk * BP_IT + (c % (BP_IT / 16)) * 16);
+                }
+                __syncthreads();  // every wave has finished with the rings (and its own re-fetched slots have landed)
+#pragma unroll
+                for (int it = 0; it < AC; it++)
+                    *reinterpret_cast<u32x4*>(smem + (it * NT + tid) * 16) =
+                        settle16_in_row(ta[it], g.nk * 128 + ((tid & 7) ^ ((((it * NT + tid) >> 3) >> 1) & 7)) * 16, g.kbytes);
+#pragma unroll
+                for (int it = 0; it < (BC + NT - 1) / NT; it++) {
+                    const int c = it * NT + tid, in = c % (BP_IT / 16);
+                    if (BC % NT == 0 || c < BC)
+                        *reinterpret_cast<u32x4*>(smem + B0 + (in / (BP_HS / 16)) * BH + (c / (BP_IT / 16)) * BP_HS + (in % (BP_HS / 16)) * 16) = tb[it];
+                }
+                __syncthreads();
+#pragma unroll
+                for (int s = 0; s < 4; s++) {
+                    const int chunk = W8 ? 4 * (s >> 1) + 2 * g32 + (s & 1) : 2 * s + g32;
+                    const char* sA = smem + (wm * WM + l32) * 128 + ((chunk ^ ((l32 >> 1) & 7)) * 16);
+                    const char* sB = smem + B0 + (s >> 1) * BH + wn * NJ * BP_HS + lane * 16;
+#pragma unroll
+                    for (int i = 0; i < MI; i++) fa[0][i] = *reinterpret_cast<const frag*>(sA + i * 32 * 128);
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) {
+                        if constexpr (W8) {
+                            const u32x4 raw = *reinterpret_cast<const u32x4*>(sB + j * BP_HS);
+                            fb[0][j] = (s & 1) ? s8x8_to_bf16(raw[2], raw[3]) : s8x8_to_bf16(raw[0], raw[1]);
+                        } else {
+                            fb[0][j] = *reinterpret_cast<const frag*>(sB + j * BP_HS + (s & 1) * 1024);
+                        }
+                    }
+                    mma(fa[0], fb[0]);
+                }
             }
-        }
         }
     } else {
     fetch(kt0);
@@ -1086,8 +1086,7 @@ static inline Plan choose_plan(int M, int Ncols, int nk, bool need_pairs, bool w
         if (need_pairs && c.bm == 64) continue;                     // (the 64-row tile stores no gate/up pairs)
         if (mode == 3 && !(c.bm == 128 && c.bn == 128)) continue;   // the masked path exists for one tile shape
         if (mode == 4 && !((c.bm == 256 && c.bn == 192) || (c.bm <= 128 && c.bn <= 128))) continue;  // (the tiles of MODE 4)
-        if (mode == 4 && c.bm == 256 && rq.k_splits > 1) continue;
-        if (mode != 2 && mode != 4 && (c.bn == 64 || c.bm == 64)) continue;      // the 64-wide and 64-row tiles exist for the ring pipeline only
+        if (mode != 2 && mode != 4 && (c.bn == 64 || c.bm == 64)) continue;  // the 64-wide and 64-row tiles exist for the ring pipeline only
         const int tiles = ((M + c.bm - 1) / c.bm) * ((Ncols + c.bn - 1) / c.bn);
         for (int S = 1; S <= KSPLIT_MAX; S++) {
             if (rq.k_splits > 0 && S != rq.k_splits) continue;
@@ -1150,7 +1149,7 @@ static int launch_cfg(const GemmArgs& g, int grid, hipStream_t st) {
     return check_hip(hipGetLastError(), name);
 }
 
-// The K split exists for the ring pipeline (MODE 2) and tiles at least 128 columns wide.
+// The K split exists for the ring pipeline (MODE 2; MODE 4 on its 128-row and 64-row tiles) and tiles at least 128 columns wide.
 #define MMX_LAUNCH(TIn, BM, BN, MODE, TOut, SMAX) \
     launch_cfg<TIn, BM, BN, MODE, TOut, SMAX>(g, grid, st)
 #define MMX_LAUNCH_MODES(TIn, BM, BN, TOut)                                                  \
@@ -1159,7 +1158,7 @@ static int launch_cfg(const GemmArgs& g, int grid, hipStream_t st) {
 
 template <typename TIn, typename TOut>
 static int launch_tiles(const GemmArgs& g, TileCfg t, int mode, int grid, hipStream_t st) {
-    if (g.ksplit > 1 && mode != 2 && mode != 4) return set_error(MMX_E_UNSUPPORTED, "the K split needs the ring pipeline (aligned A, K a multiple of 128 bytes)");
+    if (g.ksplit > 1 && mode != 2 && mode != 4) return set_error(MMX_E_UNSUPPORTED, "the K split needs the ring pipeline (16-byte aligned rows of A)");
     if (mode == 3) return MMX_LAUNCH(TIn, 128, 128, 3, TOut, 1);  // the masked path exists for one tile shape
     if (mode == 4) {  // a K tail: four tiles cover the range (the K split's code costs an unsplit launch nothing measurable)
         if (t.bm == 256 && t.bn == 192) return MMX_LAUNCH(TIn, 256, 192, 4, TOut, 1);
