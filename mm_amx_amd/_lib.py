@@ -112,11 +112,22 @@ def init(device=0):
         _initialised.add(device)
 
 
+# Two of torch's own names stand for torch.cuda.current_stream(device).cuda_stream and torch.cuda.current_device(), which make
+# an object or look at the context on every call (see below); a torch without them is served by the public ones.
+try:
+    from torch._C import _cuda_getCurrentRawStream as _raw_stream, _cuda_getDevice as _current_device
+except ImportError:
+    _current_device = torch.cuda.current_device
+
+    def _raw_stream(device):
+        return torch.cuda.current_stream(device).cuda_stream
+
+
 # What a call costs before its launch is what bounds the small shapes (256 x 256 x 256: 12.4 us a call, 6 us of them on the
 # device), so the helpers that every call passes are kept to plain attribute reads: the raw stream handle instead of a
 # Stream object, one stride() instead of several, no query of the library whose answer the call does not need.
 def _stream():
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    return _raw_stream(_current_device())
 
 
 def _dev(t, what):
@@ -261,7 +272,7 @@ def workspace(device=None, nbytes=WORKSPACE_BYTES):
     being captured into a graph and has no workspace of that size yet (an allocation there would be captured
     too).  At most _MAX_WORKSPACES are kept (the oldest is dropped); release_workspaces() drops them all."""
     dev_index = torch.cuda.current_device() if device is None else (device.index or 0)
-    key = (dev_index, torch._C._cuda_getCurrentRawStream(dev_index))
+    key = (dev_index, _raw_stream(dev_index))
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < nbytes:
         if torch.cuda.is_current_stream_capturing():
@@ -337,7 +348,7 @@ def _split_args(A, k_splits, ws, need):
         if k_splits == 0:
             # the workspace this stream already has serves every choice of the library's own, which then need not be asked
             device = A.get_device()
-            ws = _workspaces.get((device, torch._C._cuda_getCurrentRawStream(device)))
+            ws = _workspaces.get((device, _raw_stream(device)))
             if ws is not None:
                 return 0, ws.data_ptr(), ws.numel()
         nbytes = need()
