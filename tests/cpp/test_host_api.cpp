@@ -475,6 +475,56 @@ static void test_one_row_over_b(int K, int N) {
     EXPECT(got == int_product(hA, hB, 1, K, N, false), "wrong sums");
 }
 
+// B used where it lies (with and without K slices), then the same object where it has to be packed: more rows, a range of
+// columns, a result over B.  Sums of small integers are exact in any order.
+static void test_matmul_b_used_once(bool transB) {
+    std::printf("  Matmul<bf16,bf16>, constB = false, transB=%d\n", transB);
+    const struct { int M, K, N; bool unpacked; } shapes[] = {{24, 8192, 520, true}, {3, 64, 136, true}, {600, 96, 136, false}, {24, 8192, 520, true}};
+    Matmul<bfloat16, bfloat16> mm(false, transB);
+    for (const auto& s : shapes) {
+        const auto hA = small_ints(static_cast<size_t>(s.M) * s.K), hB = small_ints(static_cast<size_t>(s.K) * s.N);
+        const auto want = int_product(hA, hB, s.M, s.K, s.N, transB);
+        tensor2D<bfloat16> A(s.M, s.K), B(transB ? s.N : s.K, transB ? s.K : s.N);
+        tensor2D<float> C(s.M, s.N);
+        A.upload(hA.data());
+        B.upload(hB.data());
+        std::vector<float> got(want.size());
+        auto run = [&](int n0, int n1, const char* what, bool unpacked) {
+            if (n1 == s.N && n0 == 0) mm(A, B, PP::BiasGeluStore<float, PP::NONE>(C));
+            else mm(A, B, n0, n1, PP::BiasGeluStore<float, PP::NONE>(C));
+            const std::string kernel = mmx_last_kernel();
+            check_hip(hipDeviceSynchronize(), "sync");
+            C.download(got.data());
+            bool same = true;
+            for (int m = 0; m < s.M; m++)
+                for (int n = n0; n < n1; n++) same = same && got[static_cast<size_t>(m) * s.N + n] == want[static_cast<size_t>(m) * s.N + n];
+            EXPECT(same, "M=%d K=%d N=%d, %s: wrong sums (%s)", s.M, s.K, s.N, what, kernel.c_str());
+            EXPECT((kernel.find("unpacked") == 0) == unpacked, "M=%d K=%d N=%d, %s: ran %s", s.M, s.K, s.N, what, kernel.c_str());
+            EXPECT(!mm.internalB == unpacked, "M=%d K=%d N=%d, %s: packed weights kept from another call, or lost", s.M, s.K, s.N, what);
+            if (unpacked) EXPECT(std::atoi(kernel.c_str() + kernel.find("ksplit") + 6) > (s.K > 4096 ? 1 : 0), "M=%d K=%d N=%d: ran %s", s.M, s.K, s.N, kernel.c_str());
+        };
+        run(0, s.N, "whole", s.unpacked);
+        run(32, 64, "a range of columns", false);
+        run(0, s.N, "whole again", s.unpacked);
+    }
+    const int M = 16, K = 256, N = 256;  // the result is the first rows of B itself
+    const auto hA = small_ints(static_cast<size_t>(M) * K), hB = small_ints(static_cast<size_t>(K) * N);
+    tensor2D<bfloat16> A(M, K), B(K, N);
+    A.upload(hA.data());
+    B.upload(hB.data());
+    tensor2D<bfloat16> C(M, N, B.data, N * 2);
+    mm(A, B, PP::BiasGeluStore<bfloat16, PP::NONE>(C));
+    const std::string kernel = mmx_last_kernel();
+    check_hip(hipDeviceSynchronize(), "sync");
+    EXPECT(kernel.find("unpacked") == std::string::npos, "ran %s over a B that the result overwrites", kernel.c_str());
+    std::vector<bfloat16> got(static_cast<size_t>(M) * N);
+    C.download(got.data());
+    const auto want = int_product(hA, hB, M, K, N, transB);
+    size_t wrong = 0;
+    for (size_t i = 0; i < want.size(); i++) wrong += got[i].bits != bfloat16(want[i]).bits;
+    EXPECT(wrong == 0, "a result over B: %zu wrong", wrong);
+}
+
 // ---- preconditions raise where the reference asserts ----
 static bool throws(const std::function<void()>& f) {
     try {
@@ -530,6 +580,8 @@ int main() {
         test_mlp(96, 512, 1024, 2);  // the reference's do_splitK for the down projection (tests/amx-mlp.cpp:768)
         test_matmul_i8_requant(160, 2048, 320);  // long enough K for the two-way K split
         test_one_row_over_b(512, 1024);
+        test_matmul_b_used_once(false);
+        test_matmul_b_used_once(true);
         test_two_threads_first_call();
         test_errors();
     } catch (const std::exception& e) {

@@ -1,6 +1,6 @@
 """The tile kernels at a K that does not fill its last 128 bytes (aligned rows: the ring pipeline's last step; rows of any
 alignment: the masked pipeline), against the oracle: remainders of 2 to 126 bytes, one whole k-iteration in front or many,
-every tile that takes a tail, the K split, the gate/up store."""
+every tile that takes a tail, the K split, the gate/up store; and that the kernel named is the one that ran."""
 import numpy as np
 import pytest
 import torch
@@ -49,6 +49,10 @@ def test_k_tail(po, kind, K, tile):
     for pad in ((-K * es % 16) // es + 16 // es, 3):   # rows 16-byte aligned, and not
         C = torch.zeros((M, N), dtype=odt, device="cuda")
         mx.gemm(_in_nan(up(A), pad), packed, N, mx.Epilogue(C), **kw)
+        if pad != 3 and K * es > 128:  # (no 128x64 tile over int8 weights)
+            assert (("128x128" if kind == "w8" and tile == "128x64" else tile) + "_ring") in mx.last_kernel(), mx.last_kernel()
+        else:
+            assert "128x128_masked" in mx.last_kernel(), mx.last_kernel()
         if kind == "i8":
             assert np.array_equal(host_bits(C), ref), mx.last_kernel()
         else:
@@ -57,16 +61,27 @@ def test_k_tail(po, kind, K, tile):
 
 
 @pytest.mark.parametrize("K", [4104, 4400])
-def test_k_tail_behind_a_k_split(po, K):
-    """Few tiles and a long K: the last slice, and it alone, takes the tail (8 and 48 elements)."""
+@pytest.mark.parametrize("kind", ["bf16", "w8", "i8"])
+def test_k_tail_behind_a_k_split(po, kind, K):
+    """Few tiles and a long K: the last slice, and it alone, takes the tail (16 and 96 bytes of A)."""
     M, N = 64, 256
     rng = np.random.default_rng(K)
-    A = po.f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32))
-    B = po.f32_to_bf16((rng.standard_normal((K, N)) * 0.05).astype(np.float32))
-    C = torch.zeros((M, N), dtype=torch.float32, device="cuda")
-    mx.gemm(dev_bf16(A), mx.repack_b(dev_bf16(B)), N, mx.Epilogue(C))
-    assert "ksplit" in mx.last_kernel(), mx.last_kernel()
-    check_float_parity(host_bits(C), po.gemm_bf16(A, B), mx.last_kernel())
+    if kind == "i8":
+        K *= 2
+        A, B = (rng.integers(-127, 128, shape).astype(np.int8) for shape in ((M, K), (K, N)))
+        C, up, ref = torch.zeros((M, N), dtype=torch.int32, device="cuda"), dev, po.gemm_i8(A, B)
+    else:
+        A = po.f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32))
+        B = po.f32_to_bf16((rng.standard_normal((K, N)) * 0.05).astype(np.float32)) if kind == "bf16" else \
+            rng.integers(-127, 128, (K, N)).astype(np.int8)
+        C, up = torch.zeros((M, N), dtype=torch.float32, device="cuda"), dev_bf16
+        ref = po.gemm_bf16(A, B if kind == "bf16" else po.f32_to_bf16(B.astype(np.float32)))
+    mx.gemm(up(A), mx.repack_b((dev_bf16 if kind == "bf16" else dev)(B)), N, mx.Epilogue(C), **({"b_dtype": mx.I8} if kind == "w8" else {}))
+    assert "ring" in mx.last_kernel() and "ksplit" in mx.last_kernel(), mx.last_kernel()
+    if kind == "i8":
+        assert np.array_equal(host_bits(C), ref), mx.last_kernel()
+    else:
+        check_float_parity(host_bits(C), ref, mx.last_kernel())
 
 
 @pytest.mark.parametrize("kind,M,K,pad", [("bf16", 64, 4100, 4), ("bf16", 64, 4100, 0), ("w8", 64, 4100, 4), ("i8", 64, 8201, 7),
@@ -91,14 +106,24 @@ def test_the_plan_does_not_depend_on_earlier_calls(kind, M, K, pad):
     assert torch.equal(out[0], out[1])
 
 
-def test_k_tail_gate_up(po):
+@pytest.mark.parametrize("kind", ["bf16", "w8"])
+def test_k_tail_gate_up(po, kind):
     M, K, N = 70, 200, 96
     rng = np.random.default_rng(5)
     x = po.f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32))
-    wg, wu = (po.f32_to_bf16((rng.standard_normal((N, K)) * 0.05).astype(np.float32)) for _ in range(2))
     h = torch.zeros((M, N), dtype=torch.float32, device="cuda")
-    mx.gemm(dev_bf16(x), mx.repack_gate_up(dev_bf16(wg), dev_bf16(wu)), 2 * N, mx.Epilogue(h, mx.PP_SILU_GATE))
-    g, u = (po.gemm_bf16(x, np.ascontiguousarray(w.T)) for w in (wg, wu))
+    if kind == "bf16":
+        wg, wu = (po.f32_to_bf16((rng.standard_normal((N, K)) * 0.05).astype(np.float32)) for _ in range(2))
+        mx.gemm(dev_bf16(x), mx.repack_gate_up(dev_bf16(wg), dev_bf16(wu)), 2 * N, mx.Epilogue(h, mx.PP_SILU_GATE))
+    else:  # (gate and up in turn, 32 columns each; the scale keeps silu where it bends)
+        wg, wu = (rng.integers(-127, 128, (N, K)).astype(np.int8) for _ in range(2))
+        both = np.concatenate([w[n:n + 32] for n in range(0, N, 32) for w in (wg, wu)])
+        mx.gemm(dev_bf16(x), mx.repack_b(dev(both), transpose=True), 2 * N,
+                mx.Epilogue(h, mx.PP_SILU_GATE | mx.PP_DEQUANT, deq_scale=2.0 ** -10), b_dtype=mx.I8)
+    assert "ring" in mx.last_kernel(), mx.last_kernel()
+    g, u = (po.gemm_bf16(x, np.ascontiguousarray((w if kind == "bf16" else po.f32_to_bf16(w.astype(np.float32))).T)) for w in (wg, wu))
+    if kind == "w8":
+        g, u = g * 2.0 ** -10, u * 2.0 ** -10
     # silu is a 2^-14 approximation of g / (1 + exp(-g)); twice that for the roundings around it
     want = g / (1.0 + np.exp(-g.astype(np.float64))) * u
     got = host_bits(h).astype(np.float64)
