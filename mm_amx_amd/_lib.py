@@ -415,9 +415,14 @@ def gemm_unpacked(A, B, transpose, ep):
     b0, c0 = B.data_ptr(), s.C
     if c0 < b0 + (B.shape[0] - 1) * ldb + 2 * B.shape[1] and b0 < c0 + (M - 1) * s.ldc_bytes + N * ep.C.element_size():
         return False
-    ws = workspace(A.device, need) if need else None
-    if need and ws is None:
-        return False
+    ws = None
+    if need:
+        device = A.get_device()
+        ws = _workspaces.get((device, _raw_stream(device)))
+        if ws is None or ws.numel() < need:
+            ws = workspace(A.device, need)
+            if ws is None:
+                return False
     _check(lib().mmx_gemm_unpacked(BF16, A.data_ptr(), lda, B.data_ptr(), ldb, int(transpose), M, K, N, C.byref(s),
                                    None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), _stream()))
     return True

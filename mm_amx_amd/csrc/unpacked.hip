@@ -4,8 +4,8 @@
 // gains nothing from being packed first: packing reads and writes all of it, and the GEMM behind it reads it again.
 //
 // What bounds it: HBM, as long as the rows of A are few.  A wavefront owns a strip of 128 columns and streams its share of
-// K through registers, 32 of k (8 KiB; from [N, K] 64 of k) at a time; nothing goes through LDS on the way.  From [K, N] a lane loads 16 bytes
-// (8 columns) of 8 consecutive rows, so that 16 lanes cover 256 contiguous bytes of a row, and turns the 8 x 8 square in
+// K through registers, 32 of k (8 KiB; from [N, K] 64 of k) at a time; nothing goes through LDS on the way.  From [K, N] a
+// lane loads 16 bytes (8 columns) of 8 consecutive rows, so that 16 lanes cover 256 contiguous bytes of a row, and turns the 8 x 8 square in
 // registers (32 v_perm per 8 KiB, everything else is the naming of registers): MFMA i then multiplies the columns
 // 8 r + i, r = 0 ... 15, of the strip.  From [N, K] a lane's 16 bytes are 8 of k of one column already and MFMA i takes
 // the columns 16 i + r.  B is the first operand of the 16x16x32 MFMA, 16 rows of A the second; rows of A come from the
@@ -105,9 +105,11 @@ __device__ __forceinline__ void multiply_step(const Step<TR, MB>& s, f32x4 (&acc
     }
 }
 
-// TR: B is [N, K]; MB: blocks of 16 rows of A per workgroup; NW: wavefronts
+// TR: B is [N, K]; MB: blocks of 16 rows of A per workgroup; NW: wavefronts.
+// (Two workgroups of 64 rows per CU from [K, N]: left to itself the compiler took 374 registers for one, 186 + 188; from [N, K]
+// it needs more than the 256 that two would have.  With the stores of four columns at once 65 x 64 x 65536 32 -> 16 us.)
 template <bool TR, int MB, int NW>
-__global__ __launch_bounds__(64 * NW, MB == 1 && !TR ? 4 : (NW == 8 ? 2 : 1)) void unpacked_kernel(const UnpackedArgs s) {
+__global__ __launch_bounds__(64 * NW, MB == 1 && !TR ? 4 : (NW == 8 || !TR ? 2 : 1)) void unpacked_kernel(const UnpackedArgs s) {
     __shared__ __attribute__((aligned(16))) float red[NW][16][RED_ROW];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, g = lane >> 4;
@@ -278,45 +280,72 @@ __global__ __launch_bounds__(64 * NW, MB == 1 && !TR ? 4 : (NW == 8 ? 2 : 1)) vo
             for (int e = 0; e < 4; e++) o[e] = o[e] * (ep.q_oc ? ep.q_oc[n + (e < live ? e : 0)] : ep.q);
         }
         char* row = ep.C + (int64_t)m * ep.ldc;
-        if (ep.out_dtype == MMX_F32 && live == 4) {
-            typedef f32x4 __attribute__((aligned(4))) f32x4_any;
-            *reinterpret_cast<f32x4_any*>(row + (int64_t)n * 4) = f32x4{o[0], o[1], o[2], o[3]};
+        if (live == 4) {  // one store, at whatever address a row of C has
+            if (ep.out_dtype == MMX_F32) {
+                __builtin_memcpy(__builtin_assume_aligned(row + (int64_t)n * 4, 4), o, 16);
+            } else if (ep.out_dtype == MMX_BF16) {
+                const uint32_t w[2] = {(uint32_t)to_bf16(o[0]) | (uint32_t)to_bf16(o[1]) << 16, (uint32_t)to_bf16(o[2]) | (uint32_t)to_bf16(o[3]) << 16};
+                __builtin_memcpy(__builtin_assume_aligned(row + (int64_t)n * 2, 2), w, 8);
+            } else {
+                const uint32_t w = to_s8_sat_x4(o[0], o[1], o[2], o[3]);
+                __builtin_memcpy(row + n, &w, 4);
+            }
             continue;
         }
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-            if (e < live) {
-                if (ep.out_dtype == MMX_BF16) reinterpret_cast<uint16_t*>(row)[n + e] = to_bf16(o[e]);
-                else if (ep.out_dtype == MMX_I8) reinterpret_cast<int8_t*>(row)[n + e] = to_s8_sat(o[e]);
-                else reinterpret_cast<float*>(row)[n + e] = o[e];
-            }
+#pragma unroll 1
+        for (int e = 0; e < live; e++) {
+            if (ep.out_dtype == MMX_BF16) reinterpret_cast<uint16_t*>(row)[n + e] = to_bf16(o[0]);
+            else if (ep.out_dtype == MMX_I8) reinterpret_cast<int8_t*>(row)[n + e] = to_s8_sat(o[0]);
+            else reinterpret_cast<float*>(row)[n + e] = o[0];
+            o[0] = o[1], o[1] = o[2], o[2] = o[3];
+        }
     }
 }
 
-static int row_blocks(int M) { return M <= 16 ? 1 : (M <= 32 ? 2 : 4); }
-static int row_tiles(int M) { return (M + 16 * row_blocks(M) - 1) / (16 * row_blocks(M)); }
-static int tile_count(int M, int N) { return (N + STRIP - 1) / STRIP * row_tiles(M); }
-static size_t workspace_for_slices(int M, int N, int S) { return COUNTER_BYTES + (size_t)tile_count(M, N) * S * row_blocks(M) * 16 * STRIP * 4; }
+// How a call is shared out: blocks of 16 rows of A per workgroup, and K slices.
+struct Share {
+    int row_blocks, slices;
+};
+static int row_tiles(int M, int row_blocks) { return (M + 16 * row_blocks - 1) / (16 * row_blocks); }
+static int tile_count(int M, int N, int row_blocks) { return (N + STRIP - 1) / STRIP * row_tiles(M, row_blocks); }
+static size_t slice_sums(int tiles, int row_blocks) { return (size_t)tiles * row_blocks * 16 * STRIP * 4; }
+static size_t workspace_of(int M, int N, Share h) {
+    return h.slices > 1 ? COUNTER_BYTES + slice_sums(tile_count(M, N, h.row_blocks), h.row_blocks) * h.slices : 0;
+}
 
-// K slices: the least of an estimate in us, fitted to sweeps of S over K x N from 256 x 8192 to 10240 x 10240 at 1 to 256 rows.
-// A workgroup takes 1.2 us (4 wavefronts) to 2.2 us (8) for a step of each wavefront, 2.4 times that from [N, K], whose
-// step is twice as long and comes in pieces of 64 bytes; the chip as a whole
-// does not take B in faster than 5.5 TB/s; each slice adds to the combination.
-static int choose_slices(int M, int K, int N, int transpose, size_t ws_bytes) {
+// The least of an estimate in us, fitted to 20 000 timings (K 32 ... 11008, N 64 ... 65536, M 1 ... 256, both orders of B, every
+// number of blocks, ten numbers of slices); over those its choice takes 2.3 % longer than the best one on average, 18 % at the
+// 99th percentile.
+//   busy: a workgroup alone on its CU takes `first` (start, sums over the wavefronts, post-op) and `step` for a step of each
+//   wavefront (from [N, K] a step is twice as long and comes in pieces of 64 bytes); each further one of the CU adds `next`.
+//   stream: the chip takes B in at 5 TB/s, and the row tiles behind the first read it again, mostly from the L2.
+//   The two hide behind each other in part; each slice adds to the combination.
+// Fewer rows per workgroup mean more of them and less for each to do one after another, more rows fewer passes over B:
+// 64 x 512 x 512 from [K, N] 10.3 us in workgroups of 64 rows, 5.8 of 16; 64 x 512 x 65536 22 and 38.
+static Share choose_share(int M, int K, int N, int transpose, size_t ws_bytes) {
     if (ws_bytes > STANDARD_WORKSPACE_BYTES) ws_bytes = STANDARD_WORKSPACE_BYTES;
-    const int mb = row_blocks(M), nw = mb == 4 ? 4 : 8;
-    const int tiles = tile_count(M, N);
+    static const struct { int row_blocks; float first, step, next; } forms[2][3] = {
+        {{1, 0.6f, 1.85f, 1.35f}, {2, 4.9f, 1.55f, 4.6f}, {4, 7.9f, 1.05f, 6.1f}}, {{1, 0.2f, 3.8f, 0.9f}, {2, 0.8f, 5.2f, 3.0f}, {4, 7.2f, 2.45f, 10.6f}}};
     const int steps = transpose ? (K + 63) / 64 : K / 32, cus = num_cus();
-    const float step_us = (transpose ? 2.4f : 1.0f) * (nw == 4 ? 1.2f : 1.6f + 0.3f * mb), stream_us = (float)K * N * 2 / 5.5e6f;
-    int best = 1;
-    float best_cost = 0.0f;
-    for (int S = 1; S <= MAX_SLICES; S++) {
-        const int per_slice = (steps + S - 1) / S;
-        if (S > 1 && ((S - 1) * per_slice >= steps || per_slice < nw || tiles > MAX_TILES || workspace_for_slices(M, N, S) > ws_bytes)) continue;
-        const int rounds = (tiles * S + cus - 1) / cus;
-        const float busy_us = rounds * (2.0f + step_us * ((per_slice + nw - 1) / nw));
-        const float cost = (busy_us > stream_us ? busy_us : stream_us) + (S > 1 ? 1.5f + 0.6f * S : 0.0f);
-        if (S == 1 || cost < best_cost) best = S, best_cost = cost;
+    Share best = {4, 1};
+    float best_us = 0.0f;
+    for (const auto& f : forms[transpose ? 1 : 0]) {
+        if ((f.row_blocks == 1 && M > 64) || (f.row_blocks > 1 && M <= 8 * f.row_blocks)) continue;
+        const int nw_log2 = f.row_blocks == 4 ? 2 : 3, nw = 1 << nw_log2, tiles = tile_count(M, N, f.row_blocks);
+        const size_t slice_bytes = slice_sums(tiles, f.row_blocks);
+        if (f.row_blocks == 1 && M > 32 && tiles > 2 * cus) continue;  // (33 x 512 x 131072 from [N, K] 74 us against 54 with 64 rows)
+        const float stream_us = 0.8f + (float)K * N * 2e-6f * (1 / 4.35f + (row_tiles(M, f.row_blocks) - 1) / 57.0f);
+        int steps_before = 0;
+        for (int S = 1; S <= MAX_SLICES; S++) {
+            const int per_slice = (steps + S - 1) / S, wave_steps = (per_slice + nw - 1) >> nw_log2;
+            if (S > 1 && (2 * per_slice < nw || tiles > MAX_TILES || 2 * tiles * S > 5 * cus || COUNTER_BYTES + slice_bytes * S > ws_bytes)) break;
+            if (wave_steps == steps_before || (S - 1) * per_slice >= steps) continue;  // (nothing gained by the slice, or nothing in it)
+            steps_before = wave_steps;
+            const float work_us = f.step * wave_steps;
+            const float busy_us = f.first + work_us + ((tiles * S + cus - 1) / cus - 1) * (f.next + work_us);
+            const float us = sqrtf(busy_us * busy_us + stream_us * stream_us) + (S > 1 ? 0.9f + 0.26f * S : 0.0f);
+            if (best_us == 0.0f || us < best_us) best = {f.row_blocks, S}, best_us = us;
+        }
     }
     return best;
 }
@@ -327,48 +356,54 @@ bool unpacked_can(int M, int K, int N, int64_t lda, int64_t ldb, int transpose) 
 }
 
 // Whether a call is better off with it than with packing B first.  Device time, pack + GEMM -> this kernel, B new at every
-// call: from [K, N] 10240 x 10240 at M = 1 / 32 / 128 112 / 135 / 135 -> 38 / 44 / 90 us, 8192 x 8192 at M = 1 / 64 / 256
-// 77 / 90 / 111 -> 27 / 36 / 85, 4096 x 4096 at M = 16 / 128 24 / 31 -> 11 / 20, 512 x 512 at M = 1 / 64 8 / 9.7 -> 4.8 / 9.3;
-// from [N, K] 8192 x 8192 at M = 1 / 64 / 128 68 / 84 / 92 -> 32 / 39 / 57, 4096 x 4096 at M = 16 / 128 23 / 30 -> 14 / 24.
-// Every 64 rows of A read B once more (from the L2), so from some M on packing wins: 10240 x 10240 at M = 256 162 against
-// 169, 3072 x 5120 34 against 36 (160 tiles: one round leaves CUs idle, a K split takes two), from [N, K] 35 against 42.
-// From [N, K] packing also stays ahead where few strips are deep (8192 x 256 at M = 1 / 32 12.5 / 14 against 16 / 20 us) and
-// with more than 32 rows of a small B (512 x 512 at M = 64 9.6 against 12.9).
+// call: from [K, N] 8192 x 8192 at M = 1 / 64 / 256 73 / 73 / 90 -> 27 / 37 / 84 us, 4096 x 4096 at M = 16 / 128 24 / 28 -> 13 / 20,
+// 512 x 640 at M = 64 / 128 9.7 / 9.6 -> 5.9 / 7.4; from [N, K] 8192 x 8192 at M = 1 / 64 / 128 69 / 69 / 74 -> 32 / 37 / 54,
+// 4096 x 4096 at M = 16 / 128 24 / 28 -> 12 / 23, 512 x 640 at M = 64 / 128 9.1 / 9.4 -> 7.1 / 8.7.
+// Over 4032 shapes (K 32 ... 11008, N 64 ... 131072, M 1 ... 256) the way taken is on average 0.70 of packing, at most 1.15 of it
+// (a microsecond, 1 x 4096 x 256 from [N, K] 8.4 and 9.5).  Packing is the faster way
+//   where many workgroups of 64 rows have little to multiply (96 x 64 x 65536 15.7 against 16.2 us, from [N, K], whose form takes
+//   a CU alone, 17.4 against 24.8), or come one and a half to a CU over a deep K (128 x 2560 x 24576 from [N, K] 62 against 73);
+//   for more than 192 rows of a deep K if its slices leave CUs idle (256 x 11008 x 6144 99 against 113);
+//   from [N, K] for more than 128 rows, and for a few strips deeper than 8192 (16 x 11008 x 256 14 against 17).
 bool unpacked_takes(int M, int K, int N, int64_t lda, int64_t ldb, int transpose) {
     if (!unpacked_can(M, K, N, lda, ldb, transpose) || M > 256) return false;
-    const int tiles = tile_count(M, N), cus = num_cus();
-    if (transpose) return M <= 128 && (N > 3 * STRIP || K <= 4096) && (M <= 32 || (int64_t)K * N >= 1 << 20);
-    return M <= 128 || 2 * tiles <= cus || (4 * tiles >= 3 * cus && tiles <= cus);
+    const int tiles = tile_count(M, N, 4), cus = num_cus();
+    if (transpose) {
+        if (M <= 32) return N > 3 * STRIP || K <= 8192;
+        return M <= 64 || (M <= 128 && (tiles <= cus || (K >= 2048 && tiles >= 2 * cus)));
+    }
+    if (M <= 128) return M <= 64 || tiles <= 2 * cus || K >= 128;
+    if (tiles > cus) return false;
+    return M <= 192 || K <= 4096 || 4 * tiles <= cus || 10 * (cus / tiles * tiles) >= 9 * cus;
 }
 
 size_t unpacked_workspace_bytes(int M, int K, int N, int transpose) {
-    const int S = choose_slices(M, K, N, transpose, STANDARD_WORKSPACE_BYTES);
-    return S > 1 ? workspace_for_slices(M, N, S) : 0;
+    return workspace_of(M, N, choose_share(M, K, N, transpose, STANDARD_WORKSPACE_BYTES));
 }
 
 int launch_unpacked(const void* A, int64_t lda, const void* B, int64_t ldb, int transpose, int M, int K, int N, const Epilogue& ep, char* ws,
                     size_t ws_bytes, hipStream_t st) {
-    const int mb = row_blocks(M);
+    const Share h = choose_share(M, K, N, transpose, ws ? ws_bytes : 0);
     UnpackedArgs s;
     s.A = static_cast<const char*>(A);
     s.lda = M == 1 ? 0 : lda;
     s.B = static_cast<const char*>(B);
     s.ldb = ldb;
     s.M = M, s.K = K, s.N = N;
-    s.mtiles = row_tiles(M);
-    s.S = ws ? choose_slices(M, K, N, transpose, ws_bytes) : 1;
-    s.units = tile_count(M, N) * s.S;
+    s.mtiles = row_tiles(M, h.row_blocks);
+    s.S = h.slices;
+    s.units = tile_count(M, N, h.row_blocks) * s.S;
     s.cnt = reinterpret_cast<uint32_t*>(ws);
     s.parts = ws ? ws + COUNTER_BYTES : nullptr;
     s.ep = ep;
     const dim3 grid((s.units + 7) / 8 * 8);
     char name[64];
-    snprintf(name, sizeof name, "unpacked_%s_rows%d_ksplit%d", transpose ? "nk" : "kn", 16 * mb, s.S);
+    snprintf(name, sizeof name, "unpacked_%s_rows%d_ksplit%d", transpose ? "nk" : "kn", 16 * h.row_blocks, s.S);
     note_kernel(name);
-    if (mb == 1) {
+    if (h.row_blocks == 1) {
         if (transpose) unpacked_kernel<true, 1, 8><<<grid, 512, 0, st>>>(s);
         else unpacked_kernel<false, 1, 8><<<grid, 512, 0, st>>>(s);
-    } else if (mb == 2) {
+    } else if (h.row_blocks == 2) {
         if (transpose) unpacked_kernel<true, 2, 8><<<grid, 512, 0, st>>>(s);
         else unpacked_kernel<false, 2, 8><<<grid, 512, 0, st>>>(s);
     } else {

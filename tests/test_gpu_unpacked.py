@@ -7,6 +7,7 @@ import pytest
 import torch
 
 import mm_amx_amd as mx
+from gpu_util import call_us
 from mm_amx_amd import _lib as L
 
 pytestmark = pytest.mark.gpu
@@ -54,6 +55,8 @@ def test_exact_sums(M, K, N, trans, pad):
     wide = torch.full((M + 1, N + 3), -7.0, device="cuda")
     _entry(trans, A, B, wide[:M, :N])
     assert mx.last_kernel().startswith("unpacked_" + ("nk" if trans else "kn")), mx.last_kernel()
+    if K >= 4096 and M <= 32:  # (few strips and a long K)
+        assert not mx.last_kernel().endswith("ksplit1"), mx.last_kernel()
     ref = A.double() @ (B.double().t() if trans else B.double())
     assert torch.equal(wide[:M, :N].double(), ref)
     assert (wide[M] == -7.0).all() and (wide[:, N:] == -7.0).all()  # nothing beyond the result is written
@@ -62,6 +65,25 @@ def test_exact_sums(M, K, N, trans, pad):
         _entry(trans, A, B, again)
     assert torch.equal(again.double(), ref)
     assert torch.equal(_run(False, trans, A, B, again.zero_()).double(), ref)  # whichever way the rule takes
+
+
+@pytest.mark.parametrize("trans", [False, True])
+def test_a_smaller_workspace_means_fewer_slices(trans):
+    """All of the workspace it asks for, half of it, and none; another call's workspace is left as it is behind the limit."""
+    M, K, N = 16, 8192, 520
+    A, B = _ints((M, K), 30), _ints((N, K) if trans else (K, N), 31)
+    ref = A.double() @ (B.double().t() if trans else B.double())
+    need = L.lib().mmx_gemm_unpacked_workspace_bytes(L.BF16, M, K, N, K * 2, B.shape[1] * 2, int(trans))
+    ws, slices = torch.zeros(need, dtype=torch.uint8, device="cuda"), []
+    for limit in (need, need // 2, 1 << 14, 0):
+        C = torch.empty((M, N), device="cuda")
+        s = L.Epilogue(C).struct()
+        ws[limit:] = 0xA5
+        L._check(L.lib().mmx_gemm_unpacked(L.BF16, A.data_ptr(), K * 2, B.data_ptr(), B.shape[1] * 2, int(trans), M, K, N, ctypes.byref(s),
+                                           ws.data_ptr() if limit else None, limit, L._stream()))
+        assert torch.equal(C.double(), ref) and (ws[limit:] == 0xA5).all()
+        slices.append(int(mx.last_kernel().split("ksplit")[1]))
+    assert slices[0] > slices[1] > 1 and slices[2:] == [1, 1], slices
 
 
 @pytest.mark.parametrize("trans", [False, True])
@@ -76,6 +98,49 @@ def test_b_at_an_odd_address(trans):
     L._check(L.lib().mmx_gemm_unpacked(L.BF16, A.data_ptr(), K * 2, room.data_ptr() + 1, B.shape[1] * 2, int(trans), M, K, N, ctypes.byref(s),
                                        None, 0, L._stream()))
     assert torch.equal(C.double(), A.double() @ (B.double().t() if trans else B.double()))
+
+
+# 16, 32 and 64 rows to a workgroup, with K slices and without, the last workgroup with a few rows; one step of k and a
+# column of C's last four that stands alone
+@pytest.mark.parametrize("trans", [False, True])
+@pytest.mark.parametrize("M,K,N,rows", [(50, 512, 520, 16), (100, 512, 520, 32), (129, 2080, 2056, 32), (250, 1024, 4104, 64),
+                                        (64, 4096, 8200, 64), (49, 32, 72, 16)])
+@pytest.mark.parametrize("out", [torch.float32, torch.bfloat16, torch.int8])
+def test_every_row_block_and_store(out, M, K, N, rows, trans):
+    A, B = _ints((M, K), 32), _ints((N, K) if trans else (K, N), 33)
+    N -= 3 if trans else 0  # (from [N, K] any column count)
+    B = B[:N] if trans else B
+    wide = torch.full((M + 1, N + 5), -7, dtype=out, device="cuda")
+    _entry(trans, A, B, wide[:M, 1:N + 1])  # rows of C at any multiple of an element
+    assert f"_rows{rows}_" in mx.last_kernel(), mx.last_kernel()
+    ref = A.double() @ (B.double().t() if trans else B.double())
+    assert torch.equal(wide[:M, 1:N + 1], ref.clamp(-128, 127).to(out) if out == torch.int8 else ref.to(out))
+    assert (wide[M] == -7).all() and (wide[:, N + 1:] == -7).all() and (wide[:, 0] == -7).all()
+
+
+@pytest.mark.parametrize("trans", [False, True])
+@pytest.mark.parametrize("M,K,N", [(96, 64, 65536), (128, 128, 32768), (96, 256, 65536), (64, 512, 512), (64, 1024, 256), (128, 512, 1024),
+                                   (96, 1024, 2048), (1, 8192, 640)])
+def test_the_faster_way_is_taken(M, K, N, trans):
+    """Device time of the way the query names against packing first.  In workgroups of 64 rows throughout, with two-byte
+    stores, these took up to 2.1 times as long as packing first; now 0.5 to 1.0 times."""
+    lib, C = L.lib(), torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
+    A, B = (torch.randn(shape, device="cuda").to(torch.bfloat16) for shape in ((M, K), (N, K) if trans else (K, N)))
+    s, ws, ldb = L.Epilogue(C).struct(), L.workspace(), B.shape[1] * 2
+    packed = torch.empty(mx.packed_b_bytes(mx.BF16, K, N), dtype=torch.uint8, device="cuda")
+    if lib.mmx_gemm_unpacked_workspace_bytes(L.BF16, M, K, N, K * 2, ldb, int(trans)) < 0:
+        return  # packed first
+
+    def unpacked():
+        L._check(lib.mmx_gemm_unpacked(L.BF16, A.data_ptr(), K * 2, B.data_ptr(), ldb, int(trans), M, K, N, ctypes.byref(s), ws.data_ptr(),
+                                       ws.numel(), L._stream()))
+
+    def pack_first():
+        L._check(lib.mmx_repack_b(L.BF16, B.data_ptr(), ldb, K, N, int(trans), packed.data_ptr(), L._stream()))
+        L._check(lib.mmx_gemm_splitk(L.BF16, L.BF16, A.data_ptr(), K * 2, packed.data_ptr(), M, K, N, 0, N, ctypes.byref(s), 0, ws.data_ptr(),
+                                     ws.numel(), L._stream()))
+    took = [call_us(f, n=30) for f in (unpacked, pack_first)]
+    assert took[0] <= 1.25 * took[1], took
 
 
 @pytest.mark.parametrize("N", [8, 131, 250])
@@ -100,12 +165,16 @@ def test_post_ops_equal_the_packed_form(out, steps):
     assert torch.equal(got, want)
 
 
-def test_infinities_stay_in_their_column_and_row():
+@pytest.mark.parametrize("trans", [False, True])
+def test_infinities_stay_in_their_column_and_row(trans):
     M, K, N = 20, 320, 200
-    A, B = _ints((M, K), 7), _ints((N, K), 8)
-    B[5, 0], A[3, 1] = float("inf"), float("nan")
-    got = _run(False, True, A, B, torch.empty((M, N), device="cuda"))
-    want = _run(True, True, A, B, torch.empty((M, N), device="cuda"))
+    A, B = _ints((M, K), 7), _ints((N, K) if trans else (K, N), 8)
+    A[3, 1] = float("nan")
+    (B if trans else B.t())[5, 0], (B if trans else B.t())[199, 319] = float("inf"), float("-inf")
+    got = _run(False, trans, A, B, torch.empty((M, N), device="cuda"))
+    assert mx.last_kernel().startswith("unpacked"), mx.last_kernel()
+    want = _run(True, trans, A, B, torch.empty((M, N), device="cuda"))
+    assert not torch.isfinite(want[:, [5, 199]]).any() and torch.isfinite(want[0, :5]).all()
     assert torch.equal(torch.isfinite(got), torch.isfinite(want))
     ok = torch.isfinite(want)
     assert torch.equal(got[ok], want[ok])
@@ -153,6 +222,7 @@ def test_replays_from_a_hip_graph():
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph, stream=side):
             op(A, B, ppkernel=pp)
+        assert mx.last_kernel().startswith("unpacked") and not mx.last_kernel().endswith("ksplit1"), mx.last_kernel()
     for seed in range(15, 19):
         A.copy_(_ints((M, K), seed))
         C.zero_()
