@@ -24,8 +24,8 @@
 //           offsets MODE 2 addresses with, and a tested alternative;
 //   MODE 3  MODE 0 for A rows of any alignment and any K: 16-byte loads from wherever the row starts,
 //           masked in the last k-iteration only (elements past K are read as zero, never touched in memory).
-//           (Masked element by element it was 4-10 times slower: 391 x 1001 x 3001 bf16 108 -> 25 us,
-//           2000 x 8001 x 8000 4322 -> 452.)
+//           (Masked element by element it was 5-10 times slower: a call of 391 x 1001 x 3001 bf16 108 -> 19 us,
+//           of 2000 x 8001 x 8000 4315 -> 457.)
 #pragma once
 #include <atomic>
 #include <type_traits>
@@ -635,7 +635,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
         // MODE 4: the part of K behind the last whole k-iteration, once: A through registers (its rows end inside the 128
         // bytes) and the weights, whose padding is there, into the first slots of the rings; then four k-steps.  The trip to
         // memory is not hidden behind anything, but it is one: the masked pipeline, which this replaces for aligned rows,
-        // waits for one per k-iteration (bf16 1064 x 3544 x 786 62 -> 31 us, 64 x 4104 x 4096 52 -> 14).  (A mode of its own:
+        // waits for one per k-iteration (bf16 1064 x 3544 x 786 62 -> 27 us, 64 x 4104 x 4096 52 -> 14).  (A mode of its own:
         // behind this branch the compiler keeps the accumulators twice, which the largest tiles have no registers for.)
         if constexpr (MODE == 4) {
             if (SMAX == 1 || kt0 + nk == g.nk) {
