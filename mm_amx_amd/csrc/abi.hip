@@ -70,7 +70,7 @@ int launch_gemm_tiles_i8(const void* A, int64_t lda, const void* Bp, int M, int 
 int launch_gemm_tiles_w8(const void* A, int64_t lda, const void* Bp, int M, int K, int N, int n0, int n1,
                          const Epilogue& ep, const SplitRequest& rq, hipStream_t st);
 size_t plan_workspace_bytes(int elesz, bool w8, int M, int K, int Ncols, uint32_t steps, int k_splits);
-bool skinny_i8_eligible(const void* x, int64_t ldx, int M, int K);
+bool skinny_i8_eligible(const void* x, int64_t ldx, int M, int K, int k_splits);
 int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int K, int N, int n0, int n1,
                   const Epilogue& ep, hipStream_t st, const SplitRequest* rq);
 bool unpacked_can(int M, int K, int N, int64_t lda, int64_t ldb, int transpose);
@@ -188,11 +188,11 @@ static int gemm_dispatch(int a_dtype, int b_dtype, const void* A, int64_t lda_by
     if (rq.k_splits < 0) return set_error(MMX_E_INVALID, "mmx_gemm: k_splits = %d", rq.k_splits);
     if (rq.ws && (reinterpret_cast<uintptr_t>(rq.ws) & 255)) return set_error(MMX_E_INVALID, "mmx_gemm: the workspace must be 256-byte aligned");
     // the decode kernels choose their own K split (the chunked form, given a workspace); they take no count of slices
-    const bool decode = (M <= 32 && !i8) || (i8 && skinny_i8_eligible(A, lda_bytes, M, K) && forced_tile().bm == 0);
+    const bool decode = (M <= 32 && !i8) || (i8 && skinny_i8_eligible(A, lda_bytes, M, K, rq.k_splits) && forced_tile().bm == 0);
     if (decode && rq.k_splits > 1) return set_error(MMX_E_UNSUPPORTED, "mmx_gemm: the decode kernels (M <= 32) take k_splits = 0 or 1, not a count of slices");
     if ((ep.steps & MMX_PP_SILU_GATE) && ((n1 - n0) % 64)) return set_error(MMX_E_INVALID, "mmx_gemm: SILU_GATE needs (n1 - n0) %% 64 == 0");
     if (M <= 32 && !i8) return launch_skinny(w4 ? 2 : (w8 ? 1 : 0), A, lda_bytes, Bpacked, M, K, N, n0, n1, ep, st, &rq);
-    if (i8 && skinny_i8_eligible(A, lda_bytes, M, K) && forced_tile().bm == 0)
+    if (i8 && skinny_i8_eligible(A, lda_bytes, M, K, rq.k_splits) && forced_tile().bm == 0)
         return launch_skinny(3, A, lda_bytes, Bpacked, M, K, N, n0, n1, ep, st, &rq);
     if (w4) return set_error(MMX_E_UNSUPPORTED, "mmx_gemm: bf16 x int4-weight is a decode path (M <= 32)");
     if (w8) return launch_gemm_tiles_w8(A, lda_bytes, Bpacked, M, K, N, n0, n1, ep, rq, st);
@@ -349,7 +349,7 @@ size_t mmx_gemm_workspace_bytes(int a_dtype, int b_dtype, int M, int K, int N, i
     const bool w8 = a_dtype == MMX_BF16 && b_dtype == MMX_I8;
     const bool w4 = a_dtype == MMX_BF16 && b_dtype == MMX_I4;
     // int8 activations that the decode kernels do not take, by K or by a forced tile, go to the tile kernels at any M
-    const bool i8_tiles = i8 && M > 0 && K > 0 && (forced_tile().bm != 0 || !skinny_i8_eligible(nullptr, 0, M, K));
+    const bool i8_tiles = i8 && M > 0 && K > 0 && (forced_tile().bm != 0 || !skinny_i8_eligible(nullptr, 0, M, K, k_splits));
     if (M > 0 && M <= 32 && !i8_tiles && (bf || w8 || i8 || w4) && K > 0 && N > 0 && n0 >= 0 && n1 <= N && n0 < n1)
         return k_splits == 0 && !(steps & MMX_PP_SILU_GATE) ? skinny_workspace_bytes(i8 ? 3 : (w4 ? 2 : (w8 ? 1 : 0)), M, K, n0, n1) : 0;
     if ((!bf && !i8 && !w8) || (M <= 32 && !i8_tiles) || K <= 0 || N <= 0 || n0 < 0 || n1 > N || n0 >= n1 || k_splits < 0) return 0;

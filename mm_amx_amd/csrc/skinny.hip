@@ -33,10 +33,12 @@ struct SkinnyArgs {
     const char* Wp;
     int64_t panel_stride;  // bytes
     int M, K;
-    int nfrag;    // 1 KiB fragments per panel
+    int nfrag;    // 1 KiB fragments per panel that hold weights (what the panel is padded with behind them is zero and not read)
     int npanels;  // panels in Wp
     int n0, n1;
-    int x_vec_ok;
+    int x_vec_ok;  // rows of x start on 16 bytes
+    int x_direct;  // ... and are whole pieces of 16 bytes: they can go to LDS without passing through registers
+    int xpitch;    // bytes of a row of x in LDS: nfrag fragments' worth, zero behind its end
     Epilogue ep;
     // K split of the chunked kernel (kslices > 1): slice blockIdx.y walks its share of the chunks, parks its sums in
     // ws_part and counts itself in at ws_cnt[blockIdx.x]; the slice that arrives last adds them up and stores
@@ -264,6 +266,61 @@ __device__ __forceinline__ void skinny_finish(const SkinnyArgs& s, const float (
     }
 }
 
+// All of x -> LDS: M rows of `pitch` bytes, zero behind the row_bytes (16 or more) of each, and a row of zeros at zero_off.
+// Whole 16-byte pieces go there directly (global_load_lds, 1 KiB per wavefront and instruction; the lanes past the last row
+// re-read its last 16 bytes into the gap in front of the zero row, zero_off being the next multiple of 1 KiB); other rows
+// pass through registers, four loads in flight.  The caller waits for the loads and the writes, and then has the barrier.
+// WHOLE: aligned rows that fill their last fragment.  A form of its own: with the tests of the others beside it the staging of
+// such rows took 0.1 to 0.3 us longer (half panels, bf16 4 x 7680 x 384 7.8 -> 8.4 us).
+// What bounds these calls is the weight stream.  With a K that ends inside the last fragments, or unaligned rows, they went to
+// skinny_kernel, whose lanes read their x from memory beside the weights, 32 rows to an instruction, before -> now: int4
+// weights 1 x 10688 x 3072 16.0 -> 9.9 us, 29 x 6976 x 11232 (in chunks) 37.8 -> 23.3; int8 6 x 4544 x 11200 15.2 -> 11.6;
+// bf16 4 x 1135 x 5337 12.1 -> 4.6, 21 x 7476 x 1007 (in chunks, four K slices) 77 -> 10; int8 x int8 7 x 1728 x 672, a tile
+// kernel before, 8.1 -> 3.3.
+template <int NW, bool WHOLE>
+__device__ __forceinline__ void stage_x(const SkinnyArgs& s, char* xs, int row_bytes, int pitch, int zero_off, int tid, int wave) {
+    const int lane = tid & 63, real_bytes = s.M * pitch;
+    const uint32_t lds_base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)xs);
+    if (WHOLE || s.x_direct) {
+        for (int off = wave * 1024; off < real_bytes; off += NW * 1024) {
+            int bo = off + lane * 16;
+            bo = bo < real_bytes ? bo : real_bytes - 16;
+            const int m = bo / pitch, at = bo - m * pitch;
+            const char* src = s.x + (int64_t)m * s.ldx + at;
+            const uint32_t m0v = lds_base + off;
+            if (WHOLE || at < row_bytes)
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(m0v), "v"(src) : "memory");
+        }
+        if constexpr (!WHOLE) {
+            const int pad = (pitch - row_bytes) >> 4;  // pieces behind the end of a row
+            for (int i = tid; i < s.M * pad; i += NW * 64) {
+                const int m = i / pad;
+                *reinterpret_cast<u32x4*>(xs + m * pitch + row_bytes + (i - m * pad) * 16) = u32x4{0u, 0u, 0u, 0u};
+            }
+        }
+    } else {
+        constexpr int UNR = 4;
+        const int pieces = real_bytes >> 4, per_row = pitch >> 4;
+        for (int i0 = tid; i0 < pieces; i0 += UNR * NW * 64) {
+            u32x4 v[UNR];
+            int at[UNR];
+#pragma unroll
+            for (int u = 0; u < UNR; u++) {
+                const int i = i0 + u * NW * 64 < pieces ? i0 + u * NW * 64 : pieces - 1, m = i / per_row;
+                at[u] = (i - m * per_row) * 16;
+                v[u] = fetch16_in_row(s.x + (int64_t)m * s.ldx, at[u], row_bytes);
+            }
+#pragma unroll
+            for (int u = 0; u < UNR; u++)
+                if (i0 + u * NW * 64 < pieces)
+                    *reinterpret_cast<u32x4*>(xs + (i0 + u * NW * 64) * 16) = settle16_in_row(v[u], at[u], row_bytes);
+        }
+    }
+    for (int c = tid * 16; c < pitch; c += NW * 64 * 16) *reinterpret_cast<u32x4*>(xs + zero_off + c) = u32x4{0u, 0u, 0u, 0u};
+}
+
+// The fully general form: what the kernels below leave - rows of x shorter than 16 bytes, and gate/up pairs over compressed
+// weights whose x does not fit in LDS.
 // WK: weights are bf16 (0), int8 (1) or int4 (2); a 1 KiB fragment is 32 columns x 16, 32 or 64 of k
 template <int WK, int NP>
 __global__ __launch_bounds__(512) void skinny_kernel(const SkinnyArgs s) {
@@ -450,18 +507,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 // c+1 is what allows chunk c+2 to overwrite chunk c.  16-byte pieces of a row are XOR-swizzled with
 // the row so that the 32 rows an operand reads spread over the banks.
 // Lanes of rows >= M read row 0 (their output columns are never stored); fragments past the end of K
-// get zero weights and a clamped (finite) x.
+// get zero weights and a clamped (finite) x.  TAIL: rows of x of any alignment, 16 bytes and longer, zero past the end of K.
 // WK: weights are bf16 (0), int8 (1) or int4 (2), 3: int8 weights and int8 activations (int32 sums);
 // XD: 16-byte x loads per thread per chunk (8 KiB of x each)
-template <int WK, int NP, int FPW, int XD, int WIN = 0>  // WIN: chunks in flight (0: what the case's registers hold)
+// TAIL: the rows of x end inside a group of four fragments, or do not start on 16 bytes
+constexpr int chunk_row_bytes(int wk, int fpw) { return 8 * fpw * (wk == 2 ? 128 : (wk == 1 ? 64 : 32)); }
+template <int WK, int NP, int FPW, int XD, int WIN, bool TAIL>  // WIN: chunks in flight (0: what the case's registers hold)
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void skinny_chunk_kernel(const SkinnyArgs s) {
     constexpr bool W8 = WK == 1, W4 = WK == 2, I8A = WK == 3;
     using accv = std::conditional_t<I8A, i32x16, f32x16>;
     // chunks in flight (what 128 registers hold)
     constexpr int W = WIN ? WIN : (W4 ? (XD >= 4 ? 2 : 3) : ((FPW == 2 && (W8 || NP == 2)) ? 2 : 3));
-    constexpr int XB = W4 ? 128 : (W8 ? 64 : 32);  // bytes of a row of x one fragment covers (int8 x int8: 32)
     constexpr int FC = 8 * FPW;          // fragments per chunk
-    constexpr int RB = FC * XB;          // bytes of a row of x per chunk
+    constexpr int RB = chunk_row_bytes(WK, FPW);  // bytes of a row of x per chunk
     constexpr int BUF = 8 * XD * 1024;   // one LDS buffer: BUF / RB rows of x (the launcher checks M against it)
     static_assert(RB >= 256 && BUF / RB >= 16, "chunk geometry");
     extern __shared__ __attribute__((aligned(1024))) char smem[];  // 2 x BUF, later the cross-wave reduction
@@ -515,13 +573,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     const int xswz = mrow & 15;
 
     u32x4 w[W][FPW][NP];
-    bf16x8 xr[W][XD];
+    u32x4 xr[W][XD];
 #define MMX_LOAD(C, J)                                                                                         \
     do {                                                                                                       \
         _Pragma("unroll") for (int t = 0; t < XD; t++) {                                                       \
-            int kb_ = (C) * RB + xcol[t];                                                                      \
-            kb_ = kb_ < row_bytes - 16 ? kb_ : row_bytes - 16;                                                 \
-            xr[J][t] = *reinterpret_cast<const bf16x8*>(xsrc[t] + kb_);                                        \
+            xr[J][t] = fetch16_in_row(xsrc[t], (C) * RB + xcol[t], row_bytes);                                 \
         }                                                                                                      \
         _Pragma("unroll") for (int u = 0; u < FPW; u++) {                                                      \
             int f_ = (C) * FC + wave * FPW + u;                                                                \
@@ -533,7 +589,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 #define MMX_CHUNK(C, J)                                                                                        \
     do {                                                                                                       \
         char* buf_ = smem + ((C) & 1) * BUF;                                                                   \
-        _Pragma("unroll") for (int t = 0; t < XD; t++) *reinterpret_cast<bf16x8*>(buf_ + xdst[t]) = xr[J][t];  \
+        if (TAIL && ((C) + 1) * RB > row_bytes) { /* scalar: the rows of x end in this chunk */                 \
+            _Pragma("unroll") for (int t = 0; t < XD; t++)                                                     \
+                xr[J][t] = settle16_in_row(xr[J][t], (C) * RB + xcol[t], row_bytes);                           \
+        }                                                                                                      \
+        _Pragma("unroll") for (int t = 0; t < XD; t++) *reinterpret_cast<u32x4*>(buf_ + xdst[t]) = xr[J][t];   \
         __syncthreads();                                                                                       \
         _Pragma("unroll") for (int u = 0; u < FPW; u++) {                                                      \
             const int fl_ = wave * FPW + u;                                                                    \
@@ -604,6 +664,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     else skinny_finish<NP, I8A>(s, red, panel_first, tid, fin);
 }
 
+template <int WK, int NP, int FPW, int XD, int WIN = 0>
+static int launch_chunk(dim3 grid, const SkinnyArgs& s, hipStream_t st) {
+    constexpr int lds = (2 * 8 * XD * 1024) > (8 * NP * 16 * 64 * 4) ? (2 * 8 * XD * 1024) : (8 * NP * 16 * 64 * 4);  // two buffers of x, later the reduction scratch
+    // (a K that fills the panels' last group of fragments ends between two fragments: the test per chunk is not needed there,
+    // and cost int4 30 x 2304 x 16192 4 %)
+    const bool tail = !s.x_vec_ok || s.K % (WK == 2 ? 256 : (WK == 0 ? 64 : 128)) != 0;
+    hipLaunchKernelGGL((tail ? skinny_chunk_kernel<WK, NP, FPW, XD, WIN, true> : skinny_chunk_kernel<WK, NP, FPW, XD, WIN, false>), grid, dim3(512), lds, st, s);
+    return check_hip(hipGetLastError(), "skinny_chunk_kernel launch");
+}
+
 // ---- streaming variant for the smallest M -----------------------------------------------------------
 // When the activations fit in LDS the kernel is organised around one goal: have every byte of the
 // weights requested from HBM as early as possible.  x goes from global memory straight into LDS
@@ -612,13 +682,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 // means x has landed: one barrier, and the weights are consumed in arrival order.  x fragments are
 // read from LDS (their own counter: they never queue behind the weight stream).  Lanes of rows >= M
 // and fragments past the end of K read a row of zeros instead, so the loop has no branches.
-// Requires K to fill whole 128-byte groups of the packed weights (no zero padding of x needed).
 // 128 VGPRs at most: two workgroups per CU, so that every panel of an 11008-column matrix is resident at once.
 // ONE: every wave's share of K is a single batch (the common decode shapes); a variant of its own so that
 // each kernel holds one code path and stays within its registers.
 // UW: batch of the rolling window if not the full register set (the last batch of a wave's share of K is filled up with
 // repeats of the last load, which cost what they are a share of the loads: the launcher picks the batch with the fewest)
-template <int WK, int NP, bool ONE, int UW = 0>
+template <int WK, int NP, bool ONE, bool WHOLE, int UW = 0>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void skinny_stream_kernel(const SkinnyArgs s, int zero_off) {
     constexpr bool W8 = WK == 1, W4 = WK == 2, I8A = WK == 3;  // 3: int8 weights AND int8 activations, int32 sums
     // 4: int8 weights and ONE row of x without the matrix cores: every lane owns one column and half of a fragment's
@@ -630,7 +699,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     // fragments per panel per wave in flight at once (16 KiB of weights; int4: 8 KiB, a fragment holds 64 of k
     // and unpacking it costs more than streaming it)
     constexpr int U = UW ? UW : (W4 ? 8 : 16) / NP;
-    // [M][K] bf16, then at zero_off a row of zeros; once x has been used up, the cross-wave reduction scratch
+    // [M][xpitch], then at zero_off a row of zeros; once x has been used up, the cross-wave reduction scratch
     // (the launcher allocates the larger of the two: stream_lds_bytes)
     extern __shared__ __attribute__((aligned(1024))) char xs[];
     typedef float Red[8][NP][16][64];
@@ -641,25 +710,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     const int l32 = lane & 31, g32 = lane >> 5;
     const int panel_first = (s.n0 >> 5) + blockIdx.x * NP;
     const int panel_end = (s.n1 + 31) >> 5;
-    const int row_bytes = s.K * (I8A ? 1 : 2);
-    const int real_bytes = s.M * row_bytes;
     SKINNY_STAMP(0);
     SKINNY_STAMP(1);
-
-    // x -> LDS, 1 KiB per wave per instruction; the lanes past the end of x re-read its last 16 bytes
-    // into the gap in front of the zero row (zero_off is the next multiple of 1 KiB)
-    {
-        const uint32_t lds_base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)xs);
-        for (int off = wave * 1024; off < real_bytes; off += 8 * 1024) {
-            int bo = off + lane * 16;
-            bo = bo < real_bytes ? bo : real_bytes - 16;
-            const int m = bo / row_bytes;
-            const char* src = s.x + (int64_t)m * s.ldx + (bo - m * row_bytes);
-            const uint32_t m0v = lds_base + off;
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(m0v), "v"(src) : "memory");
-        }
-        for (int c = tid * 16; c < row_bytes; c += 512 * 16) *reinterpret_cast<u32x4*>(xs + zero_off + c) = u32x4{0u, 0u, 0u, 0u};
-    }
+    const int row_bytes = s.K * (I8A ? 1 : 2), pitch = WHOLE ? row_bytes : s.xpitch;
+    stage_x<8, WHOLE>(s, xs, row_bytes, pitch, zero_off, tid, wave);
     // the few per-column operands of the post-op travel ahead of the weights as well
     FinishOperands<NP> fin;
     skinny_prefetch<NP>(s, panel_first, tid, fin);
@@ -685,7 +739,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
         wbase[p] = s.Wp + (int64_t)panel * s.panel_stride + lane * 16;
     }
     const char* zrow = xs + zero_off;
-    const char* xrow = (VALU || l32 < s.M) ? xs + (VALU ? 0 : l32) * row_bytes : zrow;
+    const char* xrow = (VALU || l32 < s.M) ? xs + (VALU ? 0 : l32) * pitch : zrow;
     const int nbatch = (per_wave + U - 1) / U;  // same for every wave
     // U fragments per panel are in flight per wave at all times: register set u holds fragment u of a
     // batch and is re-requested for the next batch as soon as it has been multiplied
@@ -1115,13 +1169,12 @@ __global__ __launch_bounds__(1024) void skinny_resident_pair_kernel(const Skinny
 // 16-31/48-63: fragment 2u+1), so every lane still fetches its own 16 bytes.  As an MFMA operand that is 16
 // columns x two different k-ranges, so each load is multiplied twice, once with the x of either fragment,
 // into two accumulators: rows 0-15 of the first and rows 16-31 of the second are the two partial sums of
-// the 16 columns (the other rows are never looked at).  K * sizeof(T) is a multiple of 128 on this path,
-// so a panel has an even number of fragments.
-template <bool W8, int NP, bool ONE, int U>  // U: loads per panel per wave in flight at once (1 KiB each)
+// the 16 columns (the other rows are never looked at).  (The launcher makes nfrag even; panels hold a multiple of four.)
+template <bool W8, int NP, bool ONE, bool WHOLE, int U>  // U: loads per panel per wave in flight at once (1 KiB each)
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void skinny_half_kernel(const SkinnyArgs s, int zero_off) {
     constexpr int NW = 4;
     __shared__ float red[NW][NP][16][64];
-    extern __shared__ __attribute__((aligned(1024))) char xs[];  // [M][K] bf16, then at zero_off a row of zeros
+    extern __shared__ __attribute__((aligned(1024))) char xs[];  // [M][xpitch], then at zero_off a row of zeros
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1129,22 +1182,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     const int half = blockIdx.x & 1;
     const int panel_first = (s.n0 >> 5) + (int)(blockIdx.x >> 1) * NP;
     const int panel_end = (s.n1 + 31) >> 5;
-    const int row_bytes = s.K * 2;
-    const int real_bytes = s.M * row_bytes;
     const Epilogue& ep = s.ep;
-
-    {   // x -> LDS as in skinny_stream_kernel
-        const uint32_t lds_base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)xs);
-        for (int off = wave * 1024; off < real_bytes; off += NW * 1024) {
-            int bo = off + lane * 16;
-            bo = bo < real_bytes ? bo : real_bytes - 16;
-            const int m = bo / row_bytes;
-            const char* src = s.x + (int64_t)m * s.ldx + (bo - m * row_bytes);
-            const uint32_t m0v = lds_base + off;
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(m0v), "v"(src) : "memory");
-        }
-        for (int c = tid * 16; c < row_bytes; c += NW * 64 * 16) *reinterpret_cast<u32x4*>(xs + zero_off + c) = u32x4{0u, 0u, 0u, 0u};
-    }
+    const int row_bytes = s.K * 2, pitch = WHOLE ? row_bytes : s.xpitch;
+    stage_x<NW, WHOLE>(s, xs, row_bytes, pitch, zero_off, tid, wave);
     // per-column operands of the post-op: thread -> (accumulator register v < 8, lane) -> column of the half-panel
     float o_deq[2][NP], o_bias[2][NP], o_q[2][NP];
 #pragma unroll
@@ -1185,7 +1225,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
         wbase[p] = s.Wp + (int64_t)panel * s.panel_stride + (l32 >> 4) * 1024 + (g32 * 32 + 16 * half + (l32 & 15)) * 16;
     }
     const char* zrow = xs + zero_off;
-    const char* xrow = l32 < s.M ? xs + l32 * row_bytes : zrow;
+    const char* xrow = l32 < s.M ? xs + l32 * pitch : zrow;
     const int nbatch = (per_wave + U - 1) / U;  // same for every wave
     u32x4 w[NP][U];
 #define MMX_REQUEST(BT, UU)                                                                                     \
@@ -1302,8 +1342,6 @@ int decode_valu();
 int decode_resident();
 int decode_pair();
 
-// int8 x int8 at M <= 32 can use the decode kernels if x is 16-byte aligned and K fills whole 128-byte groups of
-// the packed weights: the streaming form if x fits in LDS, else the chunked one, which walks K in chunks of 256
 // dynamic LDS of skinny_stream_kernel: x + the zero row, reused afterwards as the reduction scratch (32 KiB per panel)
 // Workspace of a K split: arrival counters first (one per workgroup column, zero between launches), the slices' sums after
 // them - the layout the tile kernels use, so one workspace serves both.
@@ -1330,21 +1368,30 @@ static int chunk_slices(bool w8, int M, int nfrag, int panels, size_t ws_bytes) 
     return S;
 }
 
+// Fragments of a panel that hold weights, and the bytes of a row of x that one covers.  wk as for launch_skinny.
+static int fragments(int wk, int K) {
+    const int k = wk == 2 ? 64 : (wk == 0 ? 16 : 32);
+    return (K + k - 1) / k;
+}
+static int fragment_x_bytes(int wk) { return wk == 2 ? 128 : (wk == 1 ? 64 : 32); }
+
 // Bytes of workspace a decode launch of this shape can use (0: it takes no K split)
 size_t skinny_workspace_bytes(int wk, int M, int K, int n0, int n1) {
-    const int nfrag = wk == 2 ? (K + 255) / 256 * 4 : (K * ((wk == 1 || wk == 3) ? 1 : 2) + 127) / 128 * 128 / 32;
     const int panels = ((n1 + 31) >> 5) - (n0 >> 5);
-    const int S = chunk_slices(wk != 0, M, nfrag, panels, ~(size_t)0);
+    const int S = chunk_slices(wk != 0, M, fragments(wk, K), panels, ~(size_t)0);
     return S > 1 ? SPLIT_COUNTER_BYTES + (size_t)panels * S * 4096 : 0;
 }
 
 static inline int stream_lds_bytes(int xbytes, int np) { return xbytes > 32768 * np ? xbytes : 32768 * np; }
 
-bool skinny_i8_eligible(const void* x, int64_t ldx, int M, int K) {
+// int8 x int8 at M <= 32 can use the decode kernels if x is 16-byte aligned: the streaming form if its rows are whole 16-byte
+// pieces and fit in LDS, else the chunked one if K fills its chunks of 256.  A forced count of K slices is something only the
+// tile kernels take, so it leaves them every K that is not one of 128-byte groups.
+bool skinny_i8_eligible(const void* x, int64_t ldx, int M, int K, int k_splits) {
     if (M > 32 || K > (1 << 24)) return false;
-    const int zoff = (M * K + 1023) & ~1023;
-    return K % 128 == 0 && (zoff + K <= 46 * 1024 || K % 256 == 0) && ((reinterpret_cast<uintptr_t>(x) & 15) == 0) &&
-           ((ldx & 15) == 0);
+    if (K % 16 || (K % 128 && k_splits > 1)) return false;
+    const int pitch = fragments(3, K) * 32, zoff = (M * pitch + 1023) & ~1023;
+    return (zoff + pitch <= 46 * 1024 || K % 256 == 0) && ((reinterpret_cast<uintptr_t>(x) & 15) == 0) && ((ldx & 15) == 0);
 }
 
 // The rolling-window form of the half-panel kernel re-requests its loads in batches of U; the last batch is filled up
@@ -1354,22 +1401,22 @@ bool skinny_i8_eligible(const void* x, int64_t ldx, int M, int K) {
 // 16.8 / 17.7 us at M = 1 / 4 with 16, 16.7 / 18.3 with 8), over int8 weights the smaller (11008 x 4096: 11.2 with 8, 11.8
 // with 12).  Gate/up pairs: batches of 4 per panel (3: +3 %, 2: +5 %, 6: +38 %).
 typedef void (*HalfKernel)(const SkinnyArgs, int);
-template <bool W8, int NP>
+template <bool W8, int NP, bool WHOLE>
 static HalfKernel half_window_kernel(int nfrag) {
     if constexpr (NP == 2) {
-        return skinny_half_kernel<W8, 2, false, 4>;
+        return skinny_half_kernel<W8, 2, false, WHOLE, 4>;
     } else {
         const int n = ((nfrag >> 1) + 3) / 4;  // loads per wave
         auto repeats = [n](int u) { return (n + u - 1) / u * u - n; };
         if constexpr (W8) {
-            return repeats(12) < repeats(8) ? skinny_half_kernel<true, 1, false, 12> : skinny_half_kernel<true, 1, false, 8>;
+            return repeats(12) < repeats(8) ? skinny_half_kernel<true, 1, false, WHOLE, 12> : skinny_half_kernel<true, 1, false, WHOLE, 8>;
         } else {
             int best = 16;
             for (int u : {10, 8, 6})
                 if (repeats(u) < repeats(best)) best = u;
-            return best == 16 ? skinny_half_kernel<false, 1, false, 16>
-                              : (best == 10 ? skinny_half_kernel<false, 1, false, 10>
-                                            : (best == 8 ? skinny_half_kernel<false, 1, false, 8> : skinny_half_kernel<false, 1, false, 6>));
+            return best == 16 ? skinny_half_kernel<false, 1, false, WHOLE, 16>
+                              : (best == 10 ? skinny_half_kernel<false, 1, false, WHOLE, 10>
+                                            : (best == 8 ? skinny_half_kernel<false, 1, false, WHOLE, 8> : skinny_half_kernel<false, 1, false, WHOLE, 6>));
         }
     }
 }
@@ -1379,15 +1426,19 @@ static HalfKernel half_window_kernel(int nfrag) {
 // 2560 x 10240 at M = 1 10.0 us against 7.6 for its bytes).  Beyond: the rolling window in batches of 16, 10 or 8,
 // whichever repeats the fewest loads, the larger at equal repeats (a share of 20 fragments in batches of 16 is 12 repeats
 // in 32 loads: int8 5120 x 13824 at M = 1 20.0 us, 14.3 in batches of 10; bf16 2560 x 10752 16.2 -> 12.0).
-// *index: the kernel's place in a list of STREAM_KERNELS per weight type (for per-kernel set-up).
+// *index: the kernel's place in a list of 2 STREAM_KERNELS per weight type (for per-kernel set-up).
 typedef void (*StreamKernel)(const SkinnyArgs, int);
 constexpr int STREAM_KERNELS = 9;
-template <int WK>
-static StreamKernel stream_kernel_for(int per_wave, int* index) {
+template <int WK, bool WHOLE>
+static StreamKernel stream_kernel_at(int i) {
     static const StreamKernel list[STREAM_KERNELS] = {
-        skinny_stream_kernel<WK, 1, true, 4>,  skinny_stream_kernel<WK, 1, true, 6>,  skinny_stream_kernel<WK, 1, true, 8>,
-        skinny_stream_kernel<WK, 1, true, 10>, skinny_stream_kernel<WK, 1, true, 12>, skinny_stream_kernel<WK, 1, true>,
-        skinny_stream_kernel<WK, 1, false>,    skinny_stream_kernel<WK, 1, false, 10>, skinny_stream_kernel<WK, 1, false, 8>};
+        skinny_stream_kernel<WK, 1, true, WHOLE, 4>,  skinny_stream_kernel<WK, 1, true, WHOLE, 6>,  skinny_stream_kernel<WK, 1, true, WHOLE, 8>,
+        skinny_stream_kernel<WK, 1, true, WHOLE, 10>, skinny_stream_kernel<WK, 1, true, WHOLE, 12>, skinny_stream_kernel<WK, 1, true, WHOLE>,
+        skinny_stream_kernel<WK, 1, false, WHOLE>,    skinny_stream_kernel<WK, 1, false, WHOLE, 10>, skinny_stream_kernel<WK, 1, false, WHOLE, 8>};
+    return list[i];
+}
+template <int WK>
+static StreamKernel stream_kernel_for(int per_wave, bool whole, int* index) {
     int i;
     if (per_wave <= 16) {
         i = per_wave <= 4 ? 0 : (per_wave <= 6 ? 1 : (per_wave <= 8 ? 2 : (per_wave <= 10 ? 3 : (per_wave <= 12 ? 4 : 5))));
@@ -1397,8 +1448,8 @@ static StreamKernel stream_kernel_for(int per_wave, int* index) {
         if (repeats(10) < repeats(16)) i = 7;
         if (repeats(8) < repeats(i == 7 ? 10 : 16)) i = 8;
     }
-    *index = i;
-    return list[i];
+    *index = i + (whole ? 0 : STREAM_KERNELS);
+    return whole ? stream_kernel_at<WK, true>(i) : stream_kernel_at<WK, false>(i);
 }
 
 // wk: weights are bf16 (0), int8 (1) or int4 (2); 3: int8 weights and int8 activations
@@ -1413,13 +1464,15 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
     s.Wp = static_cast<const char*>(Wp);
     s.M = M;
     s.K = K;
-    const int kbytes_pad = ((K * ((wk == 1 || wk == 3) ? 1 : 2)) + 127) / 128 * 128;
-    s.nfrag = wk == 2 ? (K + 255) / 256 * 4 : kbytes_pad / 32;  // 32 bytes of K per column per fragment
-    s.panel_stride = (int64_t)s.nfrag * 1024;
+    const int row_bytes = K * (wk == 3 ? 1 : 2);
+    s.nfrag = fragments(wk, K);
+    s.panel_stride = wk == 2 ? (int64_t)((K + 255) / 256) * 4096 : (int64_t)((K * (wk == 0 ? 2 : 1) + 127) / 128) * 4096;
     s.npanels = (N + 31) / 32;
     s.n0 = n0;
     s.n1 = n1;
     s.x_vec_ok = ((reinterpret_cast<uintptr_t>(x) & 15) == 0) && ((ldx & 15) == 0);
+    s.x_direct = s.x_vec_ok && row_bytes % 16 == 0;
+    s.xpitch = s.nfrag * fragment_x_bytes(wk);
     s.ep = ep;
     s.ws_part = nullptr;
     s.ws_cnt = nullptr;
@@ -1434,8 +1487,8 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
     if (wk == 3) {
         // int8 activations x int8 weights (int32 sums): the caller has checked skinny_i8_eligible and uses the tile
         // kernel otherwise
-        const int zoff = (M * K + 1023) & ~1023;
-        if (zoff + K > 46 * 1024) {  // x does not fit in LDS: through LDS chunk by chunk (32 rows x 256 bytes per buffer)
+        const int zoff = (M * s.xpitch + 1023) & ~1023;
+        if (zoff + s.xpitch > 46 * 1024) {  // x does not fit in LDS: through LDS chunk by chunk (32 rows x 256 bytes per buffer)
             // (few panels, a workspace at hand: K in slices as for bf16 activations; int32 sums, the same bits in any order)
             const int ksl3 = (rq && rq->ws && rq->k_splits == 0) ? chunk_slices(true, M, s.nfrag, panels, rq->ws_bytes) : 1;
             if (ksl3 > 1) {
@@ -1445,46 +1498,44 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
                 char name_[40];
                 snprintf(name_, sizeof name_, "skinny_chunk_i8_ksplit%d", ksl3);
                 note_kernel(name_);
-                hipLaunchKernelGGL((skinny_chunk_kernel<3, 1, 1, 1, 6>), dim3(panels, ksl3), dim3(512), 8 * 1 * 16 * 64 * 4, st, s);
-                return check_hip(hipGetLastError(), "skinny_chunk_kernel launch");
+                return launch_chunk<3, 1, 1, 1, 6>(dim3(panels, ksl3), s, st);
             }
             note_kernel("skinny_chunk_i8");
-            hipLaunchKernelGGL((skinny_chunk_kernel<3, 1, 1, 1>), dim3(panels), dim3(512), 8 * 1 * 16 * 64 * 4, st, s);
-            return check_hip(hipGetLastError(), "skinny_chunk_kernel launch");
+            return launch_chunk<3, 1, 1, 1>(dim3(panels), s, st);
         }
         note_kernel("skinny_stream_i8");
         int unused;
-        hipLaunchKernelGGL(stream_kernel_for<3>((s.nfrag + 7) / 8, &unused), dim3(panels), dim3(512), stream_lds_bytes(zoff + K, 1), st, s, zoff);
+        hipLaunchKernelGGL(stream_kernel_for<3>((s.nfrag + 7) / 8, s.xpitch == row_bytes, &unused), dim3(panels), dim3(512), stream_lds_bytes(zoff + s.xpitch, 1), st, s, zoff);
         return check_hip(hipGetLastError(), "skinny_stream_kernel launch");
     }
     if (wk == 2) {
-        // int4 weights: the streaming kernel if x fits in LDS and K fills whole fragments, else the general one
+        // int4 weights: the streaming kernel if x fits in LDS, else the chunked one
         if (pairs && (panels & 1)) return set_error(MMX_E_INVALID, "SILU_GATE needs an even number of 32-column panels");
-        const int zoff = (M * K * 2 + 1023) & ~1023;
-        const int xb = zoff + K * 2;
-        if (s.nfrag * 64 == K && xb <= 46 * 1024 && s.x_vec_ok) {
-            note_kernel(pairs ? "skinny_stream_w4_gateup" : "skinny_stream_w4");
-            if (pairs) {  // gate and up panels side by side: four fragments of each in flight per wave
-                if ((s.nfrag + 7) / 8 <= 4)
-                    hipLaunchKernelGGL((skinny_stream_kernel<2, 2, true>), dim3(panels / 2), dim3(512), stream_lds_bytes(xb, 2), st, s, zoff);
-                else
-                    hipLaunchKernelGGL((skinny_stream_kernel<2, 2, false>), dim3(panels / 2), dim3(512), stream_lds_bytes(xb, 2), st, s, zoff);
-            } else if ((s.nfrag + 7) / 8 <= 4)  // (register sets sized to the share of K, as for the other weight types)
-                hipLaunchKernelGGL((skinny_stream_kernel<2, 1, true, 4>), dim3(panels), dim3(512), stream_lds_bytes(xb, 1), st, s, zoff);
-            else if ((s.nfrag + 7) / 8 <= 6)
-                hipLaunchKernelGGL((skinny_stream_kernel<2, 1, true, 6>), dim3(panels), dim3(512), stream_lds_bytes(xb, 1), st, s, zoff);
-            else if ((s.nfrag + 7) / 8 <= 8)
-                hipLaunchKernelGGL((skinny_stream_kernel<2, 1, true>), dim3(panels), dim3(512), stream_lds_bytes(xb, 1), st, s, zoff);
-            else
-                hipLaunchKernelGGL((skinny_stream_kernel<2, 1, false>), dim3(panels), dim3(512), stream_lds_bytes(xb, 1), st, s, zoff);
+        const int zoff = (M * s.xpitch + 1023) & ~1023;
+        const int xb = zoff + s.xpitch;
+        if (row_bytes >= 16 && xb <= 46 * 1024) {
+            // (a K that ends inside the panel's last four fragments has names of its own)
+            note_kernel(K % 256 ? (pairs ? "skinny_w4_k_tail_gateup" : "skinny_w4_k_tail") : (pairs ? "skinny_stream_w4_gateup" : "skinny_stream_w4"));
+            const int per_wave = (s.nfrag + 7) / 8;
+            const bool fills = s.x_direct && s.xpitch == row_bytes;
+            StreamKernel kern;  // (register sets sized to the share of K, as for the other weight types)
+            if (pairs)          // gate and up panels side by side: four fragments of each in flight per wave
+                kern = per_wave <= 4 ? (fills ? skinny_stream_kernel<2, 2, true, true> : skinny_stream_kernel<2, 2, true, false>)
+                                     : (fills ? skinny_stream_kernel<2, 2, false, true> : skinny_stream_kernel<2, 2, false, false>);
+            else if (per_wave <= 4) kern = fills ? skinny_stream_kernel<2, 1, true, true, 4> : skinny_stream_kernel<2, 1, true, false, 4>;
+            else if (per_wave <= 6) kern = fills ? skinny_stream_kernel<2, 1, true, true, 6> : skinny_stream_kernel<2, 1, true, false, 6>;
+            else if (per_wave <= 8) kern = fills ? skinny_stream_kernel<2, 1, true, true> : skinny_stream_kernel<2, 1, true, false>;
+            else kern = fills ? skinny_stream_kernel<2, 1, false, true> : skinny_stream_kernel<2, 1, false, false>;
+            const int np = pairs ? 2 : 1;
+            hipLaunchKernelGGL(kern, dim3(panels / np), dim3(512), stream_lds_bytes(xb, np), st, s, zoff);
             return check_hip(hipGetLastError(), "skinny_stream_kernel launch");
         }
-        if (pairs) {  // x too large for LDS or a ragged K: the general kernel
+        if (pairs) {  // x too large for LDS: the general kernel
             note_kernel("skinny_w4_gateup");
             hipLaunchKernelGGL((skinny_kernel<2, 2>), dim3(panels / 2), dim3(512), 0, st, s);
             return check_hip(hipGetLastError(), "skinny_kernel launch");
         }
-        if (s.nfrag * 64 == K && s.x_vec_ok) {
+        if (row_bytes >= 16) {
             // x too large for LDS: through LDS chunk by chunk (two buffers of 16 or 32 rows x 1 KiB)
             const int ksl4 = (rq && rq->ws && rq->k_splits == 0) ? chunk_slices(true, M, s.nfrag, panels, rq->ws_bytes) : 1;
             if (ksl4 > 1) {  // few panels, a workspace at hand: K in slices as for the other weight types
@@ -1492,41 +1543,39 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
                 s.ws_part = rq->ws + SPLIT_COUNTER_BYTES;
                 s.kslices = ksl4;
                 char name_[40];
-                snprintf(name_, sizeof name_, "skinny_chunk_w4_ksplit%d", ksl4);
+                snprintf(name_, sizeof name_, K % 256 ? "skinny_w4_k_tail_ksplit%d" : "skinny_chunk_w4_ksplit%d", ksl4);
                 note_kernel(name_);
-                if (M <= 16) hipLaunchKernelGGL((skinny_chunk_kernel<2, 1, 1, 2, 3>), dim3(panels, ksl4), dim3(512), 2 * 8 * 2 * 1024, st, s);
-                else hipLaunchKernelGGL((skinny_chunk_kernel<2, 1, 1, 4, 2>), dim3(panels, ksl4), dim3(512), 2 * 8 * 4 * 1024, st, s);
-                return check_hip(hipGetLastError(), "skinny_chunk_kernel launch");
+                if (M <= 16) return launch_chunk<2, 1, 1, 2, 3>(dim3(panels, ksl4), s, st);
+                return launch_chunk<2, 1, 1, 4, 2>(dim3(panels, ksl4), s, st);
             }
-            note_kernel("skinny_chunk_w4");
-            if (M <= 16) hipLaunchKernelGGL((skinny_chunk_kernel<2, 1, 1, 2>), dim3(panels), dim3(512), 2 * 8 * 2 * 1024, st, s);
-            else hipLaunchKernelGGL((skinny_chunk_kernel<2, 1, 1, 4>), dim3(panels), dim3(512), 2 * 8 * 4 * 1024, st, s);
-            return check_hip(hipGetLastError(), "skinny_chunk_kernel launch");
+            note_kernel(K % 256 ? "skinny_w4_k_tail_long" : "skinny_chunk_w4");
+            if (M <= 16) return launch_chunk<2, 1, 1, 2>(dim3(panels), s, st);
+            return launch_chunk<2, 1, 1, 4>(dim3(panels), s, st);
         }
         note_kernel("skinny_w4");
         hipLaunchKernelGGL((skinny_kernel<2, 1>), dim3(panels), dim3(512), 0, st, s);
         return check_hip(hipGetLastError(), "skinny_kernel launch");
     }
-    const int kpad = kbytes_pad / (w8 ? 1 : 2);  // elements of K the packed weights cover
-    const int zero_off = (M * K * 2 + 1023) & ~1023;
-    const int xbytes = zero_off + K * 2;  // x, a gap up to the next KiB, one row of zeros
-    if (kpad == K && s.x_vec_ok && !w8 && !pairs && M >= 2 && M <= 4 && xbytes > 46 * 1024 && xbytes <= 128 * 1024 &&
+    const bool whole = K % (w8 ? 128 : 64) == 0 && s.x_vec_ok;  // K fills 128-byte groups of the weights, aligned rows of x
+    int zero_off = (M * s.xpitch + 1023) & ~1023;
+    int xbytes = zero_off + s.xpitch;  // x, a gap up to the next KiB, one row of zeros
+    if (whole && !w8 && !pairs && M >= 2 && M <= 4 && xbytes > 46 * 1024 && xbytes <= 128 * 1024 &&
         decode_halves() != 0 && panels <= num_cus() && (int64_t)s.nfrag * 512 >= 128 * 1024) {
         // A few rows of a long x (the MLP's down projection at M = 2-4: 66-110 KiB with the zero row) and at
         // most one half-panel per CU: the half-panel form with one workgroup per CU still has all of x in LDS.
         static std::atomic<uint64_t> attr_done[5];
-        const HalfKernel kernels[5] = {skinny_half_kernel<false, 1, true, 16>, skinny_half_kernel<false, 1, false, 16>,
-                                       skinny_half_kernel<false, 1, false, 10>, skinny_half_kernel<false, 1, false, 8>,
-                                       skinny_half_kernel<false, 1, false, 6>};
+        const HalfKernel kernels[5] = {skinny_half_kernel<false, 1, true, true, 16>, skinny_half_kernel<false, 1, false, true, 16>,
+                                       skinny_half_kernel<false, 1, false, true, 10>, skinny_half_kernel<false, 1, false, true, 8>,
+                                       skinny_half_kernel<false, 1, false, true, 6>};
         for (int i = 0; i < 5; i++) {
             const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernels[i]), 128 * 1024, attr_done[i]);
             if (rc) return rc;
         }
         note_kernel("skinny_half_bf16");
         if (((s.nfrag >> 1) + 3) / 4 <= 16)
-            hipLaunchKernelGGL((skinny_half_kernel<false, 1, true, 16>), dim3(2 * panels), dim3(256), xbytes, st, s, zero_off);
+            hipLaunchKernelGGL((skinny_half_kernel<false, 1, true, true, 16>), dim3(2 * panels), dim3(256), xbytes, st, s, zero_off);
         else
-            hipLaunchKernelGGL((half_window_kernel<false, 1>(s.nfrag)), dim3(2 * panels), dim3(256), xbytes, st, s, zero_off);
+            hipLaunchKernelGGL((half_window_kernel<false, 1, true>(s.nfrag)), dim3(2 * panels), dim3(256), xbytes, st, s, zero_off);
         return check_hip(hipGetLastError(), "skinny_half_kernel launch");
     }
     {
@@ -1550,7 +1599,7 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
         // K = 8 waves x U fragments for the U that exist: 16, 32 (K = 2048, 4096 of bf16 weights; 4096, 8192 of int8 weights) and,
         // for int8 weights, 20 and 43 (K = 5120, 11008)
         const bool k_ok = s.nfrag == 128 || s.nfrag == 256 || (w8 && (s.nfrag == 160 || s.nfrag == 344));
-        const bool shape_ok = kpad == K && s.x_vec_ok && !pairs && k_ok && panels > 0 &&
+        const bool shape_ok = whole && !pairs && k_ok && panels > 0 &&
                               panels <= 2 * num_cus() && lds <= 160 * 1024;
         const bool one_each = panels <= num_cus();
         // (two panels on some CUs: ahead of the chunked form while a good part of the CUs has one, 344 or 432 panels on 256
@@ -1603,14 +1652,15 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
     // form; with one workgroup per CU, M = 12-16, it loses: 16.6-17.7 against 13.7-14.5 us).
     const bool bigx = !pairs && xbytes > 46 * 1024 && xbytes <= 80 * 1024;
     const int per_wave = (s.nfrag + 7) / 8;
+    const bool fills = s.x_direct && s.xpitch == row_bytes;  // (the WHOLE forms)
     int stream_index = 0;
-    const StreamKernel stream_kernel = w8 ? stream_kernel_for<1>(per_wave, &stream_index) : stream_kernel_for<0>(per_wave, &stream_index);
+    const StreamKernel stream_kernel = w8 ? stream_kernel_for<1>(per_wave, fills, &stream_index) : stream_kernel_for<0>(per_wave, fills, &stream_index);
     if (bigx) {
-        static std::atomic<uint64_t> attr_done[2][STREAM_KERNELS];
+        static std::atomic<uint64_t> attr_done[2][2 * STREAM_KERNELS];
         const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(stream_kernel), 80 * 1024, attr_done[w8 ? 1 : 0][stream_index]);
         if (rc) return rc;
     }
-    if (kpad == K && (xbytes <= 46 * 1024 || bigx) && s.x_vec_ok) {
+    if (row_bytes >= 16 && (xbytes <= 46 * 1024 || bigx)) {
         // the activations fit in LDS: streaming variant
         if (pairs && (panels & 1)) return set_error(MMX_E_INVALID, "SILU_GATE needs an even number of 32-column panels");
         note_kernel(pairs ? (w8 ? "skinny_stream_w8_gateup" : "skinny_stream_bf16_gateup") : (w8 ? "skinny_stream_w8" : "skinny_stream_bf16"));
@@ -1625,20 +1675,33 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
         const int force = decode_halves();  // -1: by the rule above, 0: never, 1: for every M <= 4 (tests pin the path with it)
         const bool halves = M <= 4 && !bigx && !(pairs && w8) && force != 0 &&
                             (force == 1 || (2 * units <= 2 * num_cus() * wg_per_cu && unit_bytes >= (pairs ? 128 : (w8 ? 160 : 80)) * 1024));
+        if (halves) {  // (fragments in pairs)
+            s.nfrag = (s.nfrag + 1) & ~1;
+            s.xpitch = s.nfrag * fragment_x_bytes(wk);
+            zero_off = (M * s.xpitch + 1023) & ~1023;
+            xbytes = zero_off + s.xpitch;
+        }
         const int per_wave_h = ((s.nfrag >> 1) + 3) / 4;
-#define MMX_STREAM(W8, NP, GRID)                                                                                     \
-    do {                                                                                                             \
-        if (halves && per_wave_h <= 16 / NP)                                                                         \
-            hipLaunchKernelGGL((skinny_half_kernel<W8, NP, true, 16 / NP>), dim3(2 * (GRID)), dim3(256), xbytes, st, s, zero_off); \
-        else if (halves) /* the rolling window holds fewer registers where two accumulator pairs need them */      \
-            hipLaunchKernelGGL((half_window_kernel<W8, NP>(s.nfrag)), dim3(2 * (GRID)), dim3(256), xbytes, st, s, zero_off); \
-        else if (NP == 1)                                                                                            \
-            hipLaunchKernelGGL(stream_kernel, dim3(GRID), dim3(512), stream_lds_bytes(xbytes, 1), st, s, zero_off);       \
-        else if (per_wave <= 16 / NP)                                                                                \
-            hipLaunchKernelGGL((skinny_stream_kernel<W8, NP, true>), dim3(GRID), dim3(512), stream_lds_bytes(xbytes, NP), st, s, zero_off); \
-        else                                                                                                         \
-            hipLaunchKernelGGL((skinny_stream_kernel<W8, NP, false>), dim3(GRID), dim3(512), stream_lds_bytes(xbytes, NP), st, s, zero_off); \
-    } while (0)
+        auto stream = [&](auto w8_c, auto np_c, int grid) {
+            constexpr bool W8 = decltype(w8_c)::value;
+            constexpr int NP = decltype(np_c)::value;
+            if constexpr (!(W8 && NP == 2)) {
+                if (halves) {  // (the rolling window holds fewer registers where two accumulator pairs need them)
+                    const bool fill = s.xpitch == row_bytes && s.x_direct;
+                    HalfKernel kern;
+                    if (per_wave_h <= 16 / NP) kern = fill ? skinny_half_kernel<W8, NP, true, true, 16 / NP> : skinny_half_kernel<W8, NP, true, false, 16 / NP>;
+                    else kern = fill ? half_window_kernel<W8, NP, true>(s.nfrag) : half_window_kernel<W8, NP, false>(s.nfrag);
+                    hipLaunchKernelGGL(kern, dim3(2 * grid), dim3(256), xbytes, st, s, zero_off);
+                    return;
+                }
+            }
+            StreamKernel kern = stream_kernel;
+            if constexpr (NP == 2) {
+                if (per_wave <= 8) kern = fills ? skinny_stream_kernel<W8, 2, true, true> : skinny_stream_kernel<W8, 2, true, false>;
+                else kern = fills ? skinny_stream_kernel<W8, 2, false, true> : skinny_stream_kernel<W8, 2, false, false>;
+            }
+            hipLaunchKernelGGL(kern, dim3(grid), dim3(512), stream_lds_bytes(xbytes, NP), st, s, zero_off);
+        };
         if (halves) note_kernel(pairs ? "skinny_half_bf16_gateup" : (w8 ? "skinny_half_w8" : "skinny_half_bf16"));
         // One row of x over int8 weights: a lane can own a column and half of a fragment's k (v_dot2_f32_bf16, one
         // cross-lane add), which costs half the issue cycles of a 32x32 MFMA that fills 31 unused rows.  It wins while a
@@ -1651,36 +1714,30 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
         if (valu) {
             note_kernel("skinny_stream_w8_valu");
             int unused;
-            hipLaunchKernelGGL(stream_kernel_for<4>(per_wave, &unused), dim3(panels), dim3(512), stream_lds_bytes(xbytes, 1), st, s, zero_off);
-        } else if (pairs && w8) {
-            if (per_wave <= 8) hipLaunchKernelGGL((skinny_stream_kernel<1, 2, true>), dim3(panels / 2), dim3(512), stream_lds_bytes(xbytes, 2), st, s, zero_off);
-            else hipLaunchKernelGGL((skinny_stream_kernel<1, 2, false>), dim3(panels / 2), dim3(512), stream_lds_bytes(xbytes, 2), st, s, zero_off);
-        } else if (pairs) MMX_STREAM(false, 2, panels / 2);
-        else if (w8) MMX_STREAM(true, 1, panels);
-        else MMX_STREAM(false, 1, panels);
-#undef MMX_STREAM
+            hipLaunchKernelGGL(stream_kernel_for<4>(per_wave, fills, &unused), dim3(panels), dim3(512), stream_lds_bytes(xbytes, 1), st, s, zero_off);
+        } else {
+            using std::integral_constant;
+            if (pairs && w8) stream(integral_constant<bool, true>{}, integral_constant<int, 2>{}, panels / 2);
+            else if (pairs) stream(integral_constant<bool, false>{}, integral_constant<int, 2>{}, panels / 2);
+            else if (w8) stream(integral_constant<bool, true>{}, integral_constant<int, 1>{}, panels);
+            else stream(integral_constant<bool, false>{}, integral_constant<int, 1>{}, panels);
+        }
         return check_hip(hipGetLastError(), "skinny_stream_kernel launch");
     }
     // K split of the chunked kernel (a workspace at hand, the library left to choose)
-    const int ksl = (kpad == K && s.x_vec_ok && !pairs && wk <= 1 && rq && rq->ws && rq->k_splits == 0)
+    const int ksl = (row_bytes >= 16 && !pairs && wk <= 1 && rq && rq->ws && rq->k_splits == 0)
                         ? chunk_slices(w8, M, s.nfrag, panels, rq->ws_bytes) : 1;
-    if (kpad == K && s.x_vec_ok && !w8 && !pairs && M <= 8 && ksl == 1) {
+    if (whole && !w8 && !pairs && M <= 8 && ksl == 1) {
         // aligned, x too large for LDS, few rows, plain bf16 weights: every lane reads its own part of x
         // (measured: for int8 weights and for gate/up pairs the chunked kernel below is faster at these M too)
         note_kernel("skinny_direct_bf16");
         hipLaunchKernelGGL((skinny_direct_kernel<false, 1>), dim3(panels), dim3(512), 0, st, s);
         return check_hip(hipGetLastError(), "skinny_direct_kernel launch");
     }
-    if (kpad == K && s.x_vec_ok && !(pairs && w8)) {
-        // aligned, x too large for LDS, many rows: x goes through LDS chunk by chunk
+    if (row_bytes >= 16 && !(pairs && w8)) {
+        // x too large for LDS, many rows: x goes through LDS chunk by chunk
         if (pairs && (panels & 1)) return set_error(MMX_E_INVALID, "SILU_GATE needs an even number of 32-column panels");
         note_kernel(pairs ? "skinny_chunk_bf16_gateup" : (w8 ? "skinny_chunk_w8" : "skinny_chunk_bf16"));
-        // LDS: two x buffers of 8 or 16 KiB, later the reduction scratch (32 KiB per panel)
-#define MMX_CHUNKED(W8, NP, FPW, XD, GRID)                                                                          \
-    do {                                                                                                            \
-        constexpr int lds_ = (2 * 8 * XD * 1024) > (8 * NP * 16 * 64 * 4) ? (2 * 8 * XD * 1024) : (8 * NP * 16 * 64 * 4); \
-        hipLaunchKernelGGL((skinny_chunk_kernel<W8, NP, FPW, XD>), dim3(GRID), dim3(512), lds_, st, s);            \
-    } while (0)
         dim3 grid(panels);
         if (ksl > 1) {
             s.ws_cnt = reinterpret_cast<uint32_t*>(rq->ws);
@@ -1702,32 +1759,29 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
             const dim3 g2((panels + 1) / 2);  // (an odd last panel: the second one of the last workgroup stores nothing)
             // (bf16 weights: four chunks in flight, 2-4 % ahead of three - 4096 x 11008 at M = 32 23.0 -> 22.4 us; six spill.
             // int8 weights: three, four already spill - 17.6 -> 23.1)
-            if (w8) hipLaunchKernelGGL((skinny_chunk_kernel<true, 2, 1, 2>), g2, dim3(512), 65536, st, s);
-            else hipLaunchKernelGGL((skinny_chunk_kernel<false, 2, 1, 1, 4>), g2, dim3(512), 65536, st, s);
-            return check_hip(hipGetLastError(), "skinny_chunk_kernel launch");
+            if (w8) return launch_chunk<true, 2, 1, 2>(g2, s, st);
+            return launch_chunk<false, 2, 1, 1, 4>(g2, s, st);
         }
         // rows of x per buffer = 8 KiB * XD / (8 * FPW fragments * 64 or 32 bytes)
         if (pairs) {
-            if (M <= 16) MMX_CHUNKED(false, 2, 2, 1, panels / 2);
-            else MMX_CHUNKED(false, 2, 1, 1, panels / 2);
+            if (M <= 16) return launch_chunk<false, 2, 2, 1>(dim3(panels / 2), s, st);
+            else return launch_chunk<false, 2, 1, 1>(dim3(panels / 2), s, st);
         } else if (w8) {
             // With at most one workgroup per CU, six chunks in flight instead of three (11008 x 4096 at M = 8 / 32: 22.0 / 27.4
             // -> 19.1 / 24.7 us; 4096 x 4096 at M = 16: 10.4 -> 9.5); with two per CU three are better (4096 x 11008 at
             // M = 16: 14.6 against 15.0), and nine no longer fit the registers.
-            if (panels <= num_cus() && M <= 16) hipLaunchKernelGGL((skinny_chunk_kernel<true, 1, 1, 1, 6>), grid, dim3(512), 32768, st, s);
-            else if (panels <= num_cus()) hipLaunchKernelGGL((skinny_chunk_kernel<true, 1, 1, 2, 6>), grid, dim3(512), 32768, st, s);
-            else if (M <= 16) MMX_CHUNKED(true, 1, 1, 1, panels);
-            else MMX_CHUNKED(true, 1, 1, 2, panels);
+            if (panels <= num_cus() && M <= 16) return launch_chunk<true, 1, 1, 1, 6>(grid, s, st);
+            else if (panels <= num_cus()) return launch_chunk<true, 1, 1, 2, 6>(grid, s, st);
+            else if (M <= 16) return launch_chunk<true, 1, 1, 1>(grid, s, st);
+            else return launch_chunk<true, 1, 1, 2>(grid, s, st);
         } else {
             // (six chunks in flight with at most one workgroup per CU, as above: 11008 x 4096 at M = 16 / 32 28.9 / 39.3 ->
             // 26.2 / 34.1 us, 4096 x 4096 at M = 32 16.4 -> 14.6)
-            if (panels <= num_cus() && M <= 16) hipLaunchKernelGGL((skinny_chunk_kernel<false, 1, 2, 1, 6>), grid, dim3(512), 32768, st, s);
-            else if (panels <= num_cus()) hipLaunchKernelGGL((skinny_chunk_kernel<false, 1, 1, 1, 6>), grid, dim3(512), 32768, st, s);
-            else if (M <= 16) MMX_CHUNKED(false, 1, 2, 1, panels);
-            else MMX_CHUNKED(false, 1, 1, 1, panels);
+            if (panels <= num_cus() && M <= 16) return launch_chunk<false, 1, 2, 1, 6>(grid, s, st);
+            else if (panels <= num_cus()) return launch_chunk<false, 1, 1, 1, 6>(grid, s, st);
+            else if (M <= 16) return launch_chunk<false, 1, 2, 1>(grid, s, st);
+            else return launch_chunk<false, 1, 1, 1>(grid, s, st);
         }
-#undef MMX_CHUNKED
-        return check_hip(hipGetLastError(), "skinny_chunk_kernel launch");
     }
     if (pairs) {
         if (panels & 1) return set_error(MMX_E_INVALID, "SILU_GATE needs an even number of 32-column panels");

@@ -1,0 +1,132 @@
+"""The decode kernels (M <= 32) at a K that ends inside the last fragments of the packed weights, and with rows of x of any
+length and alignment, against the oracle: every form that stages x (streaming, half panels, chunks with and without a K
+split, two panels at a time, gate/up pairs), remainders of 1 element to one less than a fragment; and that the general
+kernel is not what ran."""
+import numpy as np
+import pytest
+import torch
+
+import mm_amx_amd as mx
+from gpu_util import check_float_parity, dev, dev_bf16, host_bits
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _init():
+    mx.init(0)
+
+
+def _in_nan(t, pad):
+    """t inside a wider matrix of NaN (bf16) or 77 (int8): what lies behind a row must not enter the result."""
+    wide = torch.full((t.shape[0], t.shape[1] + pad), float("nan") if t.dtype == torch.bfloat16 else 77, dtype=t.dtype, device="cuda")
+    wide[:, :t.shape[1]] = t
+    return wide[:, :t.shape[1]]
+
+
+def _operands(po, kind, M, K, N, seed):
+    """x, the packed weights and the exact product's oracle (int4: of the quantised values, before the scales)."""
+    rng = np.random.default_rng(seed)
+    x = rng.integers(-127, 128, (M, K)).astype(np.int8) if kind == "i8" else po.f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32))
+    if kind in ("w8", "i8"):
+        W = rng.integers(-127, 128, (K, N)).astype(np.int8)
+        return x, mx.repack_b(dev(W)), (po.gemm_i8(x, W) if kind == "i8" else po.gemm_bf16(x, po.f32_to_bf16(W.astype(np.float32))))
+    W = po.f32_to_bf16((rng.standard_normal((K, N)) * 0.05).astype(np.float32))
+    if kind == "bf16":
+        return x, mx.repack_b(dev_bf16(W)), po.gemm_bf16(x, W)
+    q, deq = po.quantize_int4(W)
+    return x, mx.quantize_pack_int4(dev_bf16(W))[0], po.gemv_w8(x, q, deq, want_acc=True)[1]
+
+
+KW = {"bf16": {}, "w8": {"b_dtype": mx.I8}, "w4": {"b_dtype": mx.I4}, "i8": {}}
+
+
+@pytest.mark.parametrize("M", [1, 4, 7, 32])
+@pytest.mark.parametrize("K", [8, 9, 15, 17, 63, 65, 96, 190, 1000, 1088, 1337])
+@pytest.mark.parametrize("kind", ["bf16", "w8", "w4", "i8"])
+def test_x_in_lds(po, kind, K, M):
+    """Short x: the streaming kernel, with every alignment of the rows."""
+    if kind == "i8":
+        K = (K + 15) // 16 * 16   # (rows that are not whole 16-byte pieces go to the tile kernels)
+    N = 100
+    x, packed, ref = _operands(po, kind, M, K, N, K + M)
+    es = 1 if kind == "i8" else 2
+    for pad in ((-K * es % 16) // es + 16 // es, 0, 3):
+        C = torch.zeros((M, N), dtype=torch.int32 if kind == "i8" else torch.float32, device="cuda")
+        mx.gemm(_in_nan((dev if kind == "i8" else dev_bf16)(x), pad), packed, N, mx.Epilogue(C), **KW[kind])
+        if kind != "i8" or pad != 3 or M == 1:
+            if (M + 1) * K * es <= 40000:
+                assert ("skinny_w4_k_tail" if kind == "w4" else "skinny_stream") in mx.last_kernel(), mx.last_kernel()
+            assert mx.last_kernel() not in ("skinny_bf16", "skinny_w8", "skinny_w4")
+        if kind == "i8":
+            assert np.array_equal(host_bits(C), ref), mx.last_kernel()
+        else:
+            check_float_parity(host_bits(C), ref, f"{kind} {M}x{K} pad={pad} {mx.last_kernel()}")
+
+
+@pytest.mark.parametrize("kind,M,K,N,splits,want", [
+    ("bf16", 3, 2600, 1000, 0, "skinny_half_bf16"),       # half panels: an odd number of fragments (163)
+    ("w8", 1, 10450, 1000, 1, "skinny_half_w8"),          # (327)
+    ("bf16", 12, 3680, 160, 1, "skinny_chunk_bf16"),      # chunks, two fragments per wavefront
+    ("bf16", 30, 3681, 160, 1, "skinny_chunk_bf16"),
+    ("bf16", 20, 7476, 1007, 0, "skinny_chunk_bf16_ksplit"),
+    ("bf16", 21, 2500, 8300, 0, "skinny_chunk_bf16_2p"),
+    ("w8", 16, 4160, 8300, 0, "skinny_chunk_w8"),
+    ("w8", 32, 4190, 700, 0, "skinny_chunk_w8_ksplit"),
+    ("w8", 24, 2611, 8300, 0, "skinny_chunk_w8_2p"),
+    ("w4", 11, 5313, 300, 0, "skinny_w4_k_tail_ksplit"),
+    ("w4", 29, 1800, 300, 1, "skinny_w4_k_tail_long"),
+    ("w4", 9, 6850, 8300, 1, "skinny_w4_k_tail_long"),
+])
+def test_x_through_lds_in_chunks_and_half_panels(po, kind, M, K, N, splits, want):
+    x, packed, ref = _operands(po, kind, M, K, N, K)
+    for pad in ((-K % 8) + 8, 1):
+        C = torch.zeros((M, N), dtype=torch.float32, device="cuda")
+        mx.gemm(_in_nan(dev_bf16(x), pad), packed, N, mx.Epilogue(C), k_splits=splits, **KW[kind])
+        assert mx.last_kernel().startswith(want), mx.last_kernel()
+        check_float_parity(host_bits(C), ref, f"{kind} {M}x{K}x{N} pad={pad} {mx.last_kernel()}")
+
+
+@pytest.mark.parametrize("M,K", [(3, 200), (2, 2104), (16, 2104), (32, 1001)])
+@pytest.mark.parametrize("kind", ["bf16", "w8", "w4"])
+def test_gate_up(po, kind, M, K):
+    N = 96
+    rng = np.random.default_rng(K)
+    x = po.f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32))
+    w = rng.integers(-7, 8, (2, N, K)).astype(np.float32)  # whole numbers: exact in all three weight types, int4's scale is 1
+    w[:, :, 0] = 7.0
+    g, u = (po.gemm_bf16(x, np.ascontiguousarray(po.f32_to_bf16(v).T)).astype(np.float64) * 2.0 ** -6 for v in w)
+    both = np.concatenate([v[n:n + 32] for n in range(0, N, 32) for v in w])  # gate and up in turn, 32 columns each
+    packed = {"bf16": lambda: mx.repack_b(dev_bf16(po.f32_to_bf16(both)), transpose=True), "w8": lambda: mx.repack_b(dev(both.astype(np.int8)), transpose=True),
+              "w4": lambda: mx.quantize_pack_int4(dev_bf16(po.f32_to_bf16(both)), transpose=True)[0]}[kind]()
+    h = torch.zeros((M, N), dtype=torch.float32, device="cuda")
+    mx.gemm(_in_nan(dev_bf16(x), 5), packed, 2 * N, mx.Epilogue(h, mx.PP_SILU_GATE | mx.PP_DEQUANT, deq_scale=2.0 ** -6), **KW[kind])
+    assert "gateup" in mx.last_kernel(), mx.last_kernel()
+    # silu is a 2^-14 approximation of g / (1 + exp(-g)); twice that for the roundings around it
+    want, got = g / (1.0 + np.exp(-g)) * u, host_bits(h).astype(np.float64)
+    assert np.linalg.norm(got - want) <= 2.0 ** -13 * np.linalg.norm(want), mx.last_kernel()
+
+
+@pytest.mark.parametrize("kind", ["bf16", "w8", "w4"])
+def test_infinite_x_at_the_end_of_k(po, kind):
+    """Nothing of a row is multiplied twice, by zero weights or otherwise: an infinite last element gives infinities, no NaN."""
+    M, K, N = 12, 2600, 64
+    x = torch.ones((M, K), dtype=torch.bfloat16, device="cuda")
+    x[:, K - 1] = float("inf")
+    W = torch.ones((K, N), dtype=torch.bfloat16, device="cuda")
+    packed = {"bf16": lambda: mx.repack_b(W), "w8": lambda: mx.repack_b(W.to(torch.int8)), "w4": lambda: mx.quantize_pack_int4(W)[0]}[kind]()
+    C = torch.zeros((M, N), dtype=torch.float32, device="cuda")
+    mx.gemm(x, packed, N, mx.Epilogue(C), **KW[kind])
+    assert torch.isinf(C).all(), mx.last_kernel()
+
+
+def test_int8_with_a_count_of_slices_is_refused_as_ever(po):
+    """A forced K split belongs to the tile kernels, which refuse it at such a K; the call without one takes the decode kernels."""
+    M, K, N = 8, 2112, 256
+    x, packed, ref = _operands(po, "i8", M, K, N, 1)
+    C = torch.zeros((M, N), dtype=torch.int32, device="cuda")
+    with pytest.raises(mx.MmxError, match="K a multiple of 128 bytes"):
+        mx.gemm(dev(x), packed, N, mx.Epilogue(C), k_splits=2)
+    mx.gemm(dev(x), packed, N, mx.Epilogue(C))
+    assert mx.last_kernel() == "skinny_stream_i8", mx.last_kernel()
+    assert np.array_equal(host_bits(C), ref)
