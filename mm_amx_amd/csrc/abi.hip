@@ -73,6 +73,10 @@ size_t plan_workspace_bytes(int elesz, bool w8, int M, int K, int Ncols, uint32_
 bool skinny_i8_eligible(const void* x, int64_t ldx, int M, int K, int k_splits);
 int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int K, int N, int n0, int n1,
                   const Epilogue& ep, hipStream_t st, const SplitRequest* rq);
+int launch_wave_ring(int type, const void* A, int64_t lda, const void* Bp, int M, int K, int N, int n0, int n1, const Epilogue& ep,
+                     const SplitRequest& rq, float tiles_us, hipStream_t st);
+int64_t wave_ring_workspace_bytes(int type, int M, int K, int Ncols, bool pairs, int k_splits, float tiles_us);
+float plan_us(int elesz, bool w8, int M, int K, int Ncols, uint32_t steps, const SplitRequest& rq);
 bool unpacked_can(int M, int K, int N, int64_t lda, int64_t ldb, int transpose);
 bool unpacked_takes(int M, int K, int N, int64_t lda, int64_t ldb, int transpose);
 size_t unpacked_workspace_bytes(int M, int K, int N, int transpose);
@@ -195,6 +199,11 @@ static int gemm_dispatch(int a_dtype, int b_dtype, const void* A, int64_t lda_by
     if (i8 && skinny_i8_eligible(A, lda_bytes, M, K, rq.k_splits) && forced_tile().bm == 0)
         return launch_skinny(3, A, lda_bytes, Bpacked, M, K, N, n0, n1, ep, st, &rq);
     if (w4) return set_error(MMX_E_UNSUPPORTED, "mmx_gemm: bf16 x int4-weight is a decode path (M <= 32)");
+    if (rq.k_splits <= 1 && forced_tile().bm == 0 && load_mode() == 2) {  // small tiles, where they promise to be faster
+        SplitRequest any = {rq.ws ? rq.k_splits : 1, rq.ws, rq.ws_bytes};
+        rc = launch_wave_ring(i8 ? 3 : (w8 ? 1 : 0), A, lda_bytes, Bpacked, M, K, N, n0, n1, ep, rq, plan_us(esa, w8, M, K, n1 - n0, ep.steps, any), st);
+        if (rc <= 0) return rc;
+    }
     if (w8) return launch_gemm_tiles_w8(A, lda_bytes, Bpacked, M, K, N, n0, n1, ep, rq, st);
     return i8 ? launch_gemm_tiles_i8(A, lda_bytes, Bpacked, M, K, N, n0, n1, ep, rq, st)
               : launch_gemm_tiles_bf16(A, lda_bytes, Bpacked, M, K, N, n0, n1, ep, rq, st);
@@ -353,6 +362,12 @@ size_t mmx_gemm_workspace_bytes(int a_dtype, int b_dtype, int M, int K, int N, i
     if (M > 0 && M <= 32 && !i8_tiles && (bf || w8 || i8 || w4) && K > 0 && N > 0 && n0 >= 0 && n1 <= N && n0 < n1)
         return k_splits == 0 && !(steps & MMX_PP_SILU_GATE) ? skinny_workspace_bytes(i8 ? 3 : (w4 ? 2 : (w8 ? 1 : 0)), M, K, n0, n1) : 0;
     if ((!bf && !i8 && !w8) || (M <= 32 && !i8_tiles) || K <= 0 || N <= 0 || n0 < 0 || n1 > N || n0 >= n1 || k_splits < 0) return 0;
+    if (k_splits <= 1 && forced_tile().bm == 0 && load_mode() == 2) {
+        const SplitRequest any = {k_splits, reinterpret_cast<char*>(256), ~(size_t)0};
+        const int64_t need = wave_ring_workspace_bytes(i8 ? 3 : (w8 ? 1 : 0), M, K, n1 - n0, (steps & MMX_PP_SILU_GATE) != 0, k_splits,
+                                                       plan_us(i8 ? 1 : 2, w8, M, K, n1 - n0, steps, any));
+        if (need >= 0) return (size_t)need;
+    }
     return plan_workspace_bytes(i8 ? 1 : 2, w8, M, K, n1 - n0, steps, k_splits);
 }
 

@@ -22,6 +22,16 @@ int launch_gemm_tiles_bf16(const void* A, int64_t lda, const void* Bp, int M, in
     }
 }
 
+// What the plan for this shape is estimated to take, in us, for operands the ring pipeline takes (fitted to the 840 shapes of the
+// small tiles' rule: 15 % rms; gate/up pairs take 1.19 times as long as the products of their size).
+float plan_us(int elesz, bool w8, int M, int K, int Ncols, uint32_t steps, const SplitRequest& rq_in) {
+    const int64_t kbytes = (int64_t)K * elesz;
+    const bool pairs = (steps & MMX_PP_SILU_GATE) != 0;
+    SplitRequest rq = rq_in;
+    if (pairs) rq.k_splits = 1;
+    return (pairs ? 1.2f : 1.0f) * (1.3f + 0.0004f * choose_plan(M, Ncols, (int)((kbytes + 127) / 128), pairs, w8, kbytes % 128 ? 4 : 2, rq, elesz == 1).cycles);
+}
+
 // Bytes of workspace the plan for this shape would use (0: no K split), assuming operands the ring pipeline takes: rows of
 // any K can be aligned through their stride, so this is an upper bound for those that are not.
 size_t plan_workspace_bytes(int elesz, bool w8, int M, int K, int Ncols, uint32_t steps, int k_splits) {

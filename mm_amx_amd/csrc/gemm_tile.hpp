@@ -1060,6 +1060,7 @@ static inline int slice_kiters(int nk, int S) { return 4 * (((nk + 3) / 4 + S - 
 struct Plan {
     TileCfg t;
     int S;
+    float cycles;  // the model's estimate
 };
 
 // Pick the tile shape and the number of K slices that minimise a model of the launch's duration, in
@@ -1078,7 +1079,7 @@ static inline Plan choose_plan(int M, int Ncols, int nk, bool need_pairs, bool w
     // takes 5.5k cycles, adding one in 2.9k
     const float l1_bytes_per_clk = 36.6f, ws_bytes_per_clk = 22.5f;
     float best = 1e30f;
-    Plan pick = {{128, 128}, 1};
+    Plan pick = {{128, 128}, 1, best};
     for (const auto& c : cand) {
         if (f.bm && (f.bm != c.bm || f.bn != c.bn)) continue;
         if (need_pairs && (c.bn % 128) != 0) continue;
@@ -1116,7 +1117,7 @@ static inline Plan choose_plan(int M, int Ncols, int nk, bool need_pairs, bool w
             // (not for int8 x int8: on a sweep of forced tiles the plan without the margin is within 4 % of the best tile on
             // all 24 shapes, with it 9-16 % behind on 4096 x 4096 at M = 192-256 and 11008 x 4096 at M = 384-512)
             const float t = (float)per_cu * (3700.0f + loop + epi + split) * (S > 1 && !int8_a ? 1.15f : 1.0f);
-            if (t < best) { best = t; pick = {{c.bm, c.bn}, S}; }
+            if (t < best) { best = t; pick = {{c.bm, c.bn}, S, t}; }
         }
     }
     return pick;
