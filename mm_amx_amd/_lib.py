@@ -38,6 +38,7 @@ class _Epilogue(C.Structure):
 
 
 _lib = None
+_native = None  # the host side of a call in native code (module _host_call), once the library is loaded
 _initialised = set()
 
 
@@ -97,6 +98,11 @@ def lib():
         l.mmx_probe_mfma.argtypes = [C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.POINTER(C.c_float),
                                      C.POINTER(C.c_float)]
         l.mmx_probe_read.argtypes = [C.c_void_p, C.c_size_t, C.c_int, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p]
+        from . import _host_call  # (built with the library; see csrc/host_call.cpp)
+        _host_call.bind(*(C.cast(f, C.c_void_p).value for f in (l.mmx_gemm_splitk, l.mmx_gemm_workspace_bytes, l.mmx_gemm_unpacked,
+                                                                l.mmx_gemm_unpacked_workspace_bytes, l.mmx_matvec)))
+        global _native
+        _native = _host_call
         _lib = l
     return _lib
 
@@ -371,6 +377,15 @@ def gemm(A, Bpacked, N, ep, b_dtype=None, n0=0, n1=None, k_splits=0, ws=None):
     the first call that can use one).  A first call of a shape made while the stream is being captured into a graph
     finds no workspace and runs unsplit: its sums can differ in the last bits from an eager call of the same shape,
     which splits.  Call the shape once eagerly before capturing (or pass ws) to have both take the same form."""
+    if _native is not None and type(ep) is Epilogue:
+        # Regular calls on the current GPU go through native code, with the workspace that the stream already has: the lines
+        # below it cost 5 us of host time, as much as a small product takes on the device.  None: not a regular call, nothing was done.
+        device = _current_device()
+        stream = _raw_stream(device)
+        rc = _native.gemm(A, Bpacked, N, b_dtype, n0, n1, k_splits, _workspaces.get((device, stream)) if ws is None and k_splits == 0 else ws,
+                          device, stream, ep.C, ep.steps, ep.bias, ep.deq, ep.deq_oc, ep.q, ep.q_oc)
+        if rc is not None:
+            return _check(rc)
     n1 = N if n1 is None else n1
     b_dt = (dtype_code(A) if isinstance(A, torch.Tensor) else None) if b_dtype is None else b_dtype
     M, K, a_dt = _check_gemm_args(A, Bpacked, N, ep, b_dt, n0, n1)
@@ -397,6 +412,14 @@ def gemm_unpacked(A, B, transpose, ep):
     and does nothing, where packing B first is faster or the only way (repack_b, gemm): also for a call that wants K slices
     while the stream is being captured into a graph and has no workspace.  Such a first call is packed and not split, so its
     sums can differ in the last bits from an eager call's; call the shape once eagerly before capturing to have the same."""
+    if _native is not None and type(ep) is Epilogue:  # as in gemm()
+        device = _current_device()
+        stream = _raw_stream(device)
+        rc = _native.gemm_unpacked(A, B, transpose, _workspaces.get((device, stream)), device, stream,
+                                   ep.C, ep.steps, ep.bias, ep.deq, ep.deq_oc, ep.q, ep.q_oc)
+        if rc is not None:
+            _check(rc)
+            return True
     _is_2d(A, "A"), _is_2d(B, "B")
     if A.dtype != torch.bfloat16 or B.dtype != torch.bfloat16 or ep.steps & PP_SILU_GATE:
         return False
@@ -511,6 +534,12 @@ def probe_read(buf, workgroups, kib_in_flight, sink, waves=8, blocked=False):
 
 def matvec(A, b, out=None):
     """c[M] = A[M,K] · b[K]; bf16 (c fp32) or int8 (c int32)."""
+    if _native is not None and type(out) is torch.Tensor and out.is_cuda:  # as in gemm()
+        device = _current_device()
+        rc = _native.matvec(A, b, out, device, _raw_stream(device))
+        if rc is not None:
+            _check(rc)
+            return out
     _is_2d(A, "A")
     M, K = A.shape
     dt = dtype_code(A)

@@ -1,4 +1,4 @@
-"""Builds libmm_amx_amd.so (HIP kernels + C ABI) in-tree for gfx950 with hipcc.
+"""Builds libmm_amx_amd.so (HIP kernels + C ABI) in-tree for gfx950 with hipcc, and _host_call.so (a CPython module) with g++.
 
     python -m mm_amx_amd.build [--incremental] [--stamps]
 
@@ -14,6 +14,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libmm_amx_amd.so")
+HOST_CALL = os.path.join(HERE, "_host_call.so")
 # the MFMA tile GEMM is instantiated per (input type, output type) pair in a file of its own, so that the
 # pairs compile side by side
 SOURCES = ["abi.hip", "gemm_bf16.hip", "gemm_i8.hip", "gemm_w8.hip",
@@ -38,6 +39,18 @@ def _stale(obj, src):
     return any(os.path.getmtime(d) > t for d in deps)
 
 
+def host_call_command():
+    """The CPython module with the host side of a GEMM call: host code, compiled against this Python and this torch."""
+    import sysconfig
+
+    import torch
+    at = os.path.dirname(torch.__file__)
+    include = [os.path.join(at, "include"), os.path.join(at, "include", "torch", "csrc", "api", "include"), sysconfig.get_paths()["include"]]
+    return (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"] +
+            ["-isystem" + d for d in include] + [os.path.join(CSRC, "host_call.cpp"), "-o", HOST_CALL, "-L" + os.path.join(at, "lib"),
+                                                 "-ltorch_python", "-ltorch_cpu", "-lc10"])
+
+
 def build(verbose=False, incremental=False, stamps=False):
     lib = LIB.replace(".so", "_stamps.so") if stamps else LIB
     flags = FLAGS + (["-DMMX_STAMPS"] if stamps else [])
@@ -46,6 +59,7 @@ def build(verbose=False, incremental=False, stamps=False):
             if not incremental or _stale(obj, os.path.join(CSRC, src))]
     failed = False
     running = []
+    host = subprocess.Popen(host_call_command())
 
     def reap(p_src, p):
         nonlocal failed
@@ -69,6 +83,8 @@ def build(verbose=False, incremental=False, stamps=False):
     if failed:
         raise RuntimeError("hipcc failed")
     subprocess.check_call(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-o", lib] + objs)
+    if host.wait() != 0:
+        raise RuntimeError("g++ failed on host_call.cpp")
     if not incremental:
         for obj in objs:
             os.remove(obj)

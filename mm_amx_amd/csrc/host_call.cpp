@@ -1,0 +1,234 @@
+// The host side of one call, from tensors to mmx_gemm_splitk, mmx_gemm_unpacked or mmx_matvec, as CPython functions (module
+// mm_amx_amd._host_call).
+//
+// What bounds a small product is the host: the same checks as Python statements, the descriptor as a ctypes structure, the query
+// of the workspace and the call through ctypes took 9.7 us for 256 x 256 x 256, under 4 us of which are on the device; 4.6 now.
+// (One decode row over 512 x 512 int4 weights 9.2 -> 4.2, a 64 x 512 x 512 layer with a bias 10.2 -> 5.2.)  The functions below
+// take the calls that are regular in every respect - tensors of exactly torch's own type on one GPU, the current one, everything
+// large enough - and leave all others to the Python form (they return None, and have done nothing), which accepts them or says
+// what is wrong.  They keep nothing from one call for the next.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <torch/csrc/autograd/python_variable.h>
+
+#include "../../include/mm_amx_amd.h"
+
+namespace {
+
+using gemm_fn = decltype(&mmx_gemm_splitk);
+using need_fn = decltype(&mmx_gemm_workspace_bytes);
+using unpacked_fn = decltype(&mmx_gemm_unpacked);
+using unpacked_need_fn = decltype(&mmx_gemm_unpacked_workspace_bytes);
+using matvec_fn = decltype(&mmx_matvec);
+gemm_fn call_gemm = nullptr;  // of the library that the package has loaded, set once
+need_fn call_need = nullptr;
+unpacked_fn call_unpacked = nullptr;
+unpacked_need_fn call_unpacked_need = nullptr;
+matvec_fn call_matvec = nullptr;
+
+struct Leave {};  // not a regular call
+
+bool whole_number(PyObject* o, long long lo, long long hi, int& v) {
+    if (!PyLong_CheckExact(o)) return false;
+    int over = 0;
+    const long long x = PyLong_AsLongLongAndOverflow(o, &over);
+    if (over || x < lo || x > hi) return false;
+    v = (int)x;
+    return true;
+}
+
+int code_of(at::ScalarType t) {
+    switch (t) {
+    case at::kFloat: return MMX_F32;
+    case at::kBFloat16: return MMX_BF16;
+    case at::kChar: return MMX_I8;
+    case at::kInt: return MMX_I32;
+    case at::kByte: return MMX_U8;
+    default: return -1;
+    }
+}
+
+const at::Tensor& tensor_on(PyObject* o, int device) {
+    if (!THPVariable_CheckExact(o)) throw Leave();
+    const at::Tensor& t = THPVariable_Unpack(o);
+    if (!t.is_cuda() || t.get_device() != device || t.layout() != at::kStrided) throw Leave();
+    return t;
+}
+
+// a matrix whose elements of a row follow each other; of a single row or column torch leaves the other stride arbitrary
+int64_t row_stride_bytes(const at::Tensor& t) {
+    if (t.dim() != 2 || (t.stride(1) != 1 && t.size(1) != 1)) throw Leave();
+    return (t.size(0) == 1 ? t.size(1) : t.stride(0)) * (int64_t)t.element_size();
+}
+
+const float* column_operand(PyObject* o, int device, int n1) {
+    if (o == Py_None) return nullptr;
+    const at::Tensor& t = tensor_on(o, device);
+    if (t.scalar_type() != at::kFloat || !t.is_contiguous() || t.numel() < n1) throw Leave();
+    return static_cast<const float*>(t.mutable_data_ptr());
+}
+
+void* stream_of(PyObject* o) {
+    void* const stream = PyLong_AsVoidPtr(o);
+    if (!stream && PyErr_Occurred()) {
+        PyErr_Clear();
+        throw Leave();
+    }
+    return stream;
+}
+
+// a: C, steps, bias, deq, deq_per_oc, q, q_per_oc; C holds the M x n1 result (half the columns with SILU_GATE)
+mmx_epilogue epilogue_of(PyObject* const* a, int device, int64_t M, int n1) {
+    const at::Tensor& C = tensor_on(a[0], device);
+    int steps;
+    if (!whole_number(a[1], 0, INT32_MAX, steps) || !PyFloat_CheckExact(a[3]) || !PyFloat_CheckExact(a[5])) throw Leave();
+    mmx_epilogue e = {};
+    e.steps = (uint32_t)steps;
+    e.out_dtype = code_of(C.scalar_type());
+    e.ldc_bytes = row_stride_bytes(C);
+    if (e.out_dtype < 0 || C.size(0) < M || C.size(1) < ((steps & MMX_PP_SILU_GATE) ? n1 / 2 : n1)) throw Leave();
+    e.C = C.mutable_data_ptr();
+    e.bias = column_operand(a[2], device, n1);
+    e.deq_scale = (float)PyFloat_AS_DOUBLE(a[3]);
+    e.deq_scale_per_oc = column_operand(a[4], device, n1);
+    e.q_scale = (float)PyFloat_AS_DOUBLE(a[5]);
+    e.q_scale_per_oc = column_operand(a[6], device, n1);
+    return e;
+}
+
+// gemm(A, Bpacked, N, b_dtype, n0, n1, k_splits, ws, device, stream, C, steps, bias, deq, deq_per_oc, q, q_per_oc)
+//   b_dtype: None = that of A; n1: None = N; ws: None = unsplit if the call has no use for one
+PyObject* gemm(PyObject*, PyObject* const* a, Py_ssize_t count) {
+    if (count != 17 || !call_gemm) Py_RETURN_NONE;
+    int rc;
+    try {
+        int N, n0, n1, ks, device, b_dt;
+        if (!whole_number(a[8], 0, 1 << 20, device) || !whole_number(a[2], 1, INT32_MAX, N)) throw Leave();
+        n1 = N;
+        if (a[5] != Py_None && !whole_number(a[5], 1, N, n1)) throw Leave();
+        if (!whole_number(a[4], 0, n1 - 1, n0) || !whole_number(a[6], 0, 1 << 20, ks)) throw Leave();
+        const at::Tensor &A = tensor_on(a[0], device), &B = tensor_on(a[1], device);
+        const int64_t lda = row_stride_bytes(A), M = A.size(0), K = A.size(1);
+        const int a_dt = code_of(A.scalar_type());
+        if (M < 1 || M > INT32_MAX || K < 1 || K > INT32_MAX || (a_dt != MMX_BF16 && a_dt != MMX_I8)) throw Leave();
+        b_dt = a_dt;
+        if (a[3] != Py_None && !whole_number(a[3], 0, 255, b_dt)) throw Leave();
+        if (b_dt != MMX_BF16 && b_dt != MMX_I8 && b_dt != MMX_I4) throw Leave();
+        // everything that the kernels take on trust: what is too small is an error, and the Python form says which
+        const int64_t panels = ((int64_t)N + 31) / 32;
+        const int64_t need = b_dt == MMX_I4 ? panels * ((K + 255) / 256 * 4) * 1024 : panels * 32 * ((K * (b_dt == MMX_BF16 ? 2 : 1) + 127) / 128 * 128);
+        if (B.scalar_type() != at::kByte || !B.is_contiguous() || B.numel() < need) throw Leave();
+        const mmx_epilogue e = epilogue_of(a + 10, device, M, n1);
+        void* ws = nullptr;
+        size_t ws_bytes = 0;
+        if (a[7] != Py_None) {
+            const at::Tensor& w = tensor_on(a[7], device);
+            if (w.scalar_type() != at::kByte || !w.is_contiguous()) throw Leave();
+            ws = w.mutable_data_ptr();
+            ws_bytes = (size_t)w.numel();
+        } else if (ks != 1) {
+            // an explicit count of slices, or a first call that has a use for a workspace: it is made outside
+            if (ks || call_need(a_dt, b_dt, (int)M, (int)K, N, n0, n1, e.steps, 0)) throw Leave();
+            ks = 1;
+        }
+        void* const stream = stream_of(a[9]);
+        const void *pa = A.mutable_data_ptr(), *pb = B.mutable_data_ptr();
+        Py_BEGIN_ALLOW_THREADS
+        rc = call_gemm(a_dt, b_dt, pa, lda, pb, (int)M, (int)K, N, n0, n1, &e, ks, ws, ws_bytes, stream);
+        Py_END_ALLOW_THREADS
+    } catch (...) {  // (tensors without memory of their own throw when asked for it)
+        Py_RETURN_NONE;
+    }
+    return PyLong_FromLong(rc);
+}
+
+// gemm_unpacked(A, B, transpose, ws, device, stream, C, steps, bias, deq, deq_per_oc, q, q_per_oc): a B that is used once, where
+// the library reads it in place
+PyObject* gemm_unpacked(PyObject*, PyObject* const* a, Py_ssize_t count) {
+    if (count != 13 || !call_unpacked) Py_RETURN_NONE;
+    int rc;
+    try {
+        int device;
+        if (!whole_number(a[4], 0, 1 << 20, device) || !PyBool_Check(a[2])) throw Leave();
+        const int transpose = a[2] == Py_True;
+        const at::Tensor &A = tensor_on(a[0], device), &B = tensor_on(a[1], device);
+        const int64_t lda = row_stride_bytes(A), ldb = row_stride_bytes(B), M = A.size(0), K = A.size(1), N = B.size(transpose ? 0 : 1);
+        if (A.scalar_type() != at::kBFloat16 || B.scalar_type() != at::kBFloat16 || B.size(transpose ? 1 : 0) != K) throw Leave();
+        if (M < 1 || M > INT32_MAX || K < 1 || K > INT32_MAX || N < 1 || N > INT32_MAX) throw Leave();
+        const int64_t need = call_unpacked_need(MMX_BF16, (int)M, (int)K, (int)N, lda, ldb, transpose);
+        if (need < 0) throw Leave();
+        const mmx_epilogue e = epilogue_of(a + 6, device, M, (int)N);
+        if (e.steps & MMX_PP_SILU_GATE) throw Leave();
+        const char *pa = static_cast<const char*>(A.mutable_data_ptr()), *pb = static_cast<const char*>(B.mutable_data_ptr()), *pc = static_cast<const char*>(e.C);
+        // (a result that is written over B is not computed from B in place)
+        if (pc < pb + (B.size(0) - 1) * ldb + 2 * B.size(1) && pb < pc + (M - 1) * e.ldc_bytes + N * (e.out_dtype == MMX_BF16 ? 2 : (e.out_dtype == MMX_I8 ? 1 : 4))) throw Leave();
+        void* ws = nullptr;
+        size_t ws_bytes = 0;
+        if (need) {
+            const at::Tensor& w = tensor_on(a[3], device);
+            if (w.numel() < need) throw Leave();  // (it is made outside)
+            ws = w.mutable_data_ptr();
+            ws_bytes = (size_t)w.numel();
+        }
+        void* const stream = stream_of(a[5]);
+        Py_BEGIN_ALLOW_THREADS
+        rc = call_unpacked(MMX_BF16, pa, lda, pb, ldb, transpose, (int)M, (int)K, (int)N, &e, ws, ws_bytes, stream);
+        Py_END_ALLOW_THREADS
+    } catch (...) {
+        Py_RETURN_NONE;
+    }
+    return PyLong_FromLong(rc);
+}
+
+// matvec(A, b, out, device, stream)
+PyObject* matvec(PyObject*, PyObject* const* a, Py_ssize_t count) {
+    if (count != 5 || !call_matvec) Py_RETURN_NONE;
+    int rc;
+    try {
+        int device;
+        if (!whole_number(a[3], 0, 1 << 20, device)) throw Leave();
+        const at::Tensor &A = tensor_on(a[0], device), &b = tensor_on(a[1], device), &c = tensor_on(a[2], device);
+        const int64_t lda = row_stride_bytes(A), M = A.size(0), K = A.size(1);
+        const int dt = code_of(A.scalar_type());
+        if (M < 1 || M > INT32_MAX || K < 1 || K > INT32_MAX || (dt != MMX_BF16 && dt != MMX_I8)) throw Leave();
+        if (b.scalar_type() != A.scalar_type() || b.numel() != K || !b.is_contiguous()) throw Leave();
+        if (c.scalar_type() != (dt == MMX_BF16 ? at::kFloat : at::kInt) || c.numel() < M || !c.is_contiguous()) throw Leave();
+        const void *pa = A.mutable_data_ptr(), *pb = b.mutable_data_ptr();
+        void *pc = c.mutable_data_ptr(), *stream = stream_of(a[4]);
+        Py_BEGIN_ALLOW_THREADS
+        rc = call_matvec(dt, pa, lda, pb, pc, (int)M, (int)K, stream);
+        Py_END_ALLOW_THREADS
+    } catch (...) {
+        Py_RETURN_NONE;
+    }
+    return PyLong_FromLong(rc);
+}
+
+// bind(addresses of mmx_gemm_splitk, mmx_gemm_workspace_bytes, mmx_gemm_unpacked, mmx_gemm_unpacked_workspace_bytes, mmx_matvec)
+PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t count) {
+    if (count != 5) {
+        PyErr_SetString(PyExc_TypeError, "bind takes five addresses");
+        return nullptr;
+    }
+    void* at[5];
+    for (int i = 0; i < 5; i++) at[i] = PyLong_AsVoidPtr(a[i]);
+    if (PyErr_Occurred()) return nullptr;
+    call_gemm = reinterpret_cast<gemm_fn>(at[0]);
+    call_need = reinterpret_cast<need_fn>(at[1]);
+    call_unpacked = reinterpret_cast<unpacked_fn>(at[2]);
+    call_unpacked_need = reinterpret_cast<unpacked_need_fn>(at[3]);
+    call_matvec = reinterpret_cast<matvec_fn>(at[4]);
+    Py_RETURN_NONE;
+}
+
+PyMethodDef methods[] = {{"gemm", (PyCFunction)(void (*)(void))gemm, METH_FASTCALL, nullptr},
+                         {"gemm_unpacked", (PyCFunction)(void (*)(void))gemm_unpacked, METH_FASTCALL, nullptr},
+                         {"matvec", (PyCFunction)(void (*)(void))matvec, METH_FASTCALL, nullptr},
+                         {"bind", (PyCFunction)(void (*)(void))bind, METH_FASTCALL, nullptr},
+                         {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_call", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host_call(void) { return PyModule_Create(&module); }
