@@ -99,8 +99,9 @@ def lib():
                                      C.POINTER(C.c_float)]
         l.mmx_probe_read.argtypes = [C.c_void_p, C.c_size_t, C.c_int, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p]
         from . import _host_call  # (built with the library; see csrc/host_call.cpp)
-        _host_call.bind(*(C.cast(f, C.c_void_p).value for f in (l.mmx_gemm_splitk, l.mmx_gemm_workspace_bytes, l.mmx_gemm_unpacked,
-                                                                l.mmx_gemm_unpacked_workspace_bytes, l.mmx_matvec)))
+        _host_call.bind(*(C.cast(f, C.c_void_p).value for f in (
+            l.mmx_gemm_splitk, l.mmx_gemm_workspace_bytes, l.mmx_gemm_unpacked, l.mmx_gemm_unpacked_workspace_bytes, l.mmx_matvec,
+            l.mmx_packed_b_bytes, l.mmx_repack_b, l.mmx_quantize_weights, l.mmx_quantize_weights_scaled, l.mmx_quantize_pack_int4)))
         global _native
         _native = _host_call
         _lib = l
@@ -192,6 +193,17 @@ def _column_operand(v, name):
         raise MmxError(f"{name} must be a contiguous fp32 tensor on the GPU")
 
 
+def _made(native, *args):
+    """What a native packing or quantising call on the current GPU has made; None: not a regular call, nothing was done."""
+    device = _current_device()
+    if device not in _initialised:
+        return None
+    made = native(*args, device, _raw_stream(device))
+    if type(made) is int:
+        _check(made)
+    return made
+
+
 def packed_b_bytes(dtype, K, N):
     return lib().mmx_packed_b_bytes(dtype, K, N)
 
@@ -199,6 +211,10 @@ def packed_b_bytes(dtype, K, N):
 def repack_b(B, transpose=False):
     """B [K,N] (or [N,K] with transpose) bf16/int8/uint8 on the GPU -> packed weights (uint8 tensor).  uint8 weights
     (for gemm_u8) are stored as u - 128 in the int8 layout."""
+    if _native is not None and _initialised:  # as in gemm()
+        made = _made(_native.repack, B, transpose)
+        if made is not None:
+            return made
     _dev(B, "B")
     dt = dtype_code(B)
     if dt not in (BF16, I8, U8):
@@ -225,6 +241,10 @@ def repack_gate_up(w_gate, w_up):
 
 def quantize_weights(W):
     """Per-tensor symmetric int8 compression of a bf16 matrix; returns (Wq, scales[2] = {q, dq})."""
+    if _native is not None and _initialised:
+        made = _made(_native.quantize, W)
+        if made is not None:
+            return made
     _dev(W, "W")
     if W.dtype != torch.bfloat16:
         raise MmxError("W must be bf16")
@@ -239,6 +259,10 @@ def quantize_weights(W):
 def quantize_weights_scaled(W, scale):
     """q = trunc(bf16_rne(w * scale)) per element, int8: how repackB_1xL<int8_t> (weight_compression/fc16m.cpp:80-81)
     makes fc16m's int8 weights; the matching per-tensor dequant scale is 1 / scale."""
+    if _native is not None and _initialised:
+        made = _made(_native.quantize_scaled, W, float(scale))
+        if made is not None:
+            return made
     _dev(W, "W")
     if W.dtype != torch.bfloat16 or W.dim() != 2:
         raise MmxError("W must be a 2-D bf16 tensor")
@@ -251,6 +275,10 @@ def quantize_weights_scaled(W, scale):
 def quantize_pack_int4(W, transpose=False):
     """Per-output-channel symmetric int4 compression of a bf16 matrix W [K,N] (or [N,K] with transpose), packed for
     gemm(..., b_dtype=I4) with M <= 32; returns (packed uint8, deq_scales fp32 [N])."""
+    if _native is not None and _initialised:
+        made = _made(_native.quantize_pack_int4, W, transpose)
+        if made is not None:
+            return made
     _dev(W, "W")
     if W.dtype != torch.bfloat16 or W.dim() != 2:
         raise MmxError("W must be a 2-D bf16 tensor with unit column stride")

@@ -1,5 +1,5 @@
-// The host side of one call, from tensors to mmx_gemm_splitk, mmx_gemm_unpacked or mmx_matvec, as CPython functions (module
-// mm_amx_amd._host_call).
+// The host side of one call, from tensors to mmx_gemm_splitk, mmx_gemm_unpacked, mmx_matvec or the packing and quantising
+// entry points, as CPython functions (module mm_amx_amd._host_call).
 //
 // What bounds a small product is the host: the same checks as Python statements, the descriptor as a ctypes structure, the query
 // of the workspace and the call through ctypes took 9.7 us for 256 x 256 x 256, under 4 us of which are on the device; 4.6 now.
@@ -10,6 +10,7 @@
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
+#include <ATen/ops/empty.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "../../include/mm_amx_amd.h"
@@ -26,6 +27,11 @@ need_fn call_need = nullptr;
 unpacked_fn call_unpacked = nullptr;
 unpacked_need_fn call_unpacked_need = nullptr;
 matvec_fn call_matvec = nullptr;
+decltype(&mmx_packed_b_bytes) call_packed_bytes = nullptr;
+decltype(&mmx_repack_b) call_repack = nullptr;
+decltype(&mmx_quantize_weights) call_quantize = nullptr;
+decltype(&mmx_quantize_weights_scaled) call_quantize_scaled = nullptr;
+decltype(&mmx_quantize_pack_int4) call_quantize_int4 = nullptr;
 
 struct Leave {};  // not a regular call
 
@@ -205,28 +211,154 @@ PyObject* matvec(PyObject*, PyObject* const* a, Py_ssize_t count) {
     return PyLong_FromLong(rc);
 }
 
-// bind(addresses of mmx_gemm_splitk, mmx_gemm_workspace_bytes, mmx_gemm_unpacked, mmx_gemm_unpacked_workspace_bytes, mmx_matvec)
+// ---- packing and quantising: results are made here; an error of the library comes back as its number -------------------
+// f() with the interpreter's lock released, as torch's own calls and ctypes have it; what it throws (no memory
+// left, say) is left to the Python form, which then says so
+template <typename F>
+bool unlocked(F&& f) {
+    bool ok = true;
+    PyThreadState* const state = PyEval_SaveThread();
+    try {
+        f();
+    } catch (...) {
+        ok = false;
+    }
+    PyEval_RestoreThread(state);
+    return ok;
+}
+
+at::Tensor make(at::IntArrayRef sizes, at::ScalarType type, const at::Tensor& like) {
+    return at::empty(sizes, at::TensorOptions().dtype(type).device(like.device()));
+}
+
+struct Matrix {
+    const at::Tensor* t;
+    int64_t ld;
+    int rows, cols;
+    const void* data;
+};
+Matrix matrix(PyObject* o, int device) {
+    const at::Tensor& t = tensor_on(o, device);
+    const int64_t ld = row_stride_bytes(t);
+    if (t.size(0) < 1 || t.size(0) > INT32_MAX || t.size(1) < 1 || t.size(1) > INT32_MAX) throw Leave();
+    return {&t, ld, (int)t.size(0), (int)t.size(1), t.mutable_data_ptr()};
+}
+
+// repack(B, transpose, device, stream) -> packed
+PyObject* repack(PyObject*, PyObject* const* a, Py_ssize_t count) {
+    if (count != 4 || !call_repack) Py_RETURN_NONE;
+    try {
+        int device, rc = 0;
+        if (!whole_number(a[2], 0, 1 << 20, device) || !PyBool_Check(a[1])) throw Leave();
+        const Matrix B = matrix(a[0], device);
+        const int dt = code_of(B.t->scalar_type()), transpose = a[1] == Py_True, K = transpose ? B.cols : B.rows, N = transpose ? B.rows : B.cols;
+        if (dt != MMX_BF16 && dt != MMX_I8 && dt != MMX_U8) throw Leave();
+        void* const stream = stream_of(a[3]);
+        at::Tensor out;
+        if (!unlocked([&] {
+                out = make({(int64_t)call_packed_bytes(dt, K, N)}, at::kByte, *B.t);
+                rc = call_repack(dt, B.data, B.ld, K, N, transpose, out.mutable_data_ptr(), stream);
+            })) throw Leave();
+        return rc ? PyLong_FromLong(rc) : THPVariable_Wrap(out);
+    } catch (...) {
+        Py_RETURN_NONE;
+    }
+}
+
+// quantize(W, device, stream) -> (Wq, scales)
+PyObject* quantize(PyObject*, PyObject* const* a, Py_ssize_t count) {
+    if (count != 3 || !call_quantize) Py_RETURN_NONE;
+    try {
+        int device, rc = 0;
+        if (!whole_number(a[1], 0, 1 << 20, device)) throw Leave();
+        const Matrix W = matrix(a[0], device);
+        if (W.t->scalar_type() != at::kBFloat16) throw Leave();
+        void* const stream = stream_of(a[2]);
+        at::Tensor Wq, scales, scratch;
+        if (!unlocked([&] {
+                Wq = make({W.rows, W.cols}, at::kChar, *W.t);
+                scales = make({2}, at::kFloat, *W.t);
+                scratch = make({1}, at::kInt, *W.t);
+                rc = call_quantize(W.data, W.ld, W.rows, W.cols, Wq.mutable_data_ptr(), W.cols, static_cast<float*>(scales.mutable_data_ptr()),
+                                   static_cast<uint32_t*>(scratch.mutable_data_ptr()), stream);
+            })) throw Leave();
+        return rc ? PyLong_FromLong(rc) : Py_BuildValue("(NN)", THPVariable_Wrap(Wq), THPVariable_Wrap(scales));
+    } catch (...) {
+        Py_RETURN_NONE;
+    }
+}
+
+// quantize_scaled(W, scale, device, stream) -> Wq
+PyObject* quantize_scaled(PyObject*, PyObject* const* a, Py_ssize_t count) {
+    if (count != 4 || !call_quantize_scaled) Py_RETURN_NONE;
+    try {
+        int device, rc = 0;
+        if (!whole_number(a[2], 0, 1 << 20, device) || !PyFloat_CheckExact(a[1])) throw Leave();
+        const Matrix W = matrix(a[0], device);
+        if (W.t->scalar_type() != at::kBFloat16) throw Leave();
+        const float scale = (float)PyFloat_AS_DOUBLE(a[1]);
+        void* const stream = stream_of(a[3]);
+        at::Tensor Wq;
+        if (!unlocked([&] {
+                Wq = make({W.rows, W.cols}, at::kChar, *W.t);
+                rc = call_quantize_scaled(W.data, W.ld, W.rows, W.cols, scale, Wq.mutable_data_ptr(), W.cols, stream);
+            })) throw Leave();
+        return rc ? PyLong_FromLong(rc) : THPVariable_Wrap(Wq);
+    } catch (...) {
+        Py_RETURN_NONE;
+    }
+}
+
+// quantize_pack_int4(W, transpose, device, stream) -> (packed, deq)
+PyObject* quantize_pack_int4(PyObject*, PyObject* const* a, Py_ssize_t count) {
+    if (count != 4 || !call_quantize_int4) Py_RETURN_NONE;
+    try {
+        int device, rc = 0;
+        if (!whole_number(a[2], 0, 1 << 20, device) || !PyBool_Check(a[1])) throw Leave();
+        const Matrix W = matrix(a[0], device);
+        if (W.t->scalar_type() != at::kBFloat16) throw Leave();
+        const int transpose = a[1] == Py_True, K = transpose ? W.cols : W.rows, N = transpose ? W.rows : W.cols;
+        void* const stream = stream_of(a[3]);
+        at::Tensor packed, deq;
+        if (!unlocked([&] {
+                packed = make({(int64_t)call_packed_bytes(MMX_I4, K, N)}, at::kByte, *W.t);
+                deq = make({N}, at::kFloat, *W.t);
+                rc = call_quantize_int4(W.data, W.ld, K, N, transpose, packed.mutable_data_ptr(), static_cast<float*>(deq.mutable_data_ptr()), stream);
+            })) throw Leave();
+        return rc ? PyLong_FromLong(rc) : Py_BuildValue("(NN)", THPVariable_Wrap(packed), THPVariable_Wrap(deq));
+    } catch (...) {
+        Py_RETURN_NONE;
+    }
+}
+
+// bind(addresses of the ten entry points, in the order below)
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t count) {
-    if (count != 5) {
-        PyErr_SetString(PyExc_TypeError, "bind takes five addresses");
+    constexpr int ENTRIES = 10;
+    if (count != ENTRIES) {
+        PyErr_SetString(PyExc_TypeError, "bind takes ten addresses");
         return nullptr;
     }
-    void* at[5];
-    for (int i = 0; i < 5; i++) at[i] = PyLong_AsVoidPtr(a[i]);
+    void* at[ENTRIES];
+    for (int i = 0; i < ENTRIES; i++) at[i] = PyLong_AsVoidPtr(a[i]);
     if (PyErr_Occurred()) return nullptr;
-    call_gemm = reinterpret_cast<gemm_fn>(at[0]);
-    call_need = reinterpret_cast<need_fn>(at[1]);
-    call_unpacked = reinterpret_cast<unpacked_fn>(at[2]);
-    call_unpacked_need = reinterpret_cast<unpacked_need_fn>(at[3]);
-    call_matvec = reinterpret_cast<matvec_fn>(at[4]);
+    int i = 0;
+    auto set = [&](auto& f) { f = reinterpret_cast<std::remove_reference_t<decltype(f)>>(at[i++]); };
+    set(call_gemm);
+    set(call_need);
+    set(call_unpacked);
+    set(call_unpacked_need);
+    set(call_matvec);
+    set(call_packed_bytes);
+    set(call_repack);
+    set(call_quantize);
+    set(call_quantize_scaled);
+    set(call_quantize_int4);
     Py_RETURN_NONE;
 }
 
-PyMethodDef methods[] = {{"gemm", (PyCFunction)(void (*)(void))gemm, METH_FASTCALL, nullptr},
-                         {"gemm_unpacked", (PyCFunction)(void (*)(void))gemm_unpacked, METH_FASTCALL, nullptr},
-                         {"matvec", (PyCFunction)(void (*)(void))matvec, METH_FASTCALL, nullptr},
-                         {"bind", (PyCFunction)(void (*)(void))bind, METH_FASTCALL, nullptr},
-                         {nullptr, nullptr, 0, nullptr}};
+#define METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {METHOD(gemm), METHOD(gemm_unpacked), METHOD(matvec), METHOD(repack), METHOD(quantize), METHOD(quantize_scaled),
+                         METHOD(quantize_pack_int4), METHOD(bind), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_call", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

@@ -170,3 +170,29 @@ def test_matvec(monkeypatch, kind):
             (native, python), answers = _both(m, lambda: mx.MatmulVector()(rows, vec, torch.zeros(size, dtype=out_dt, device="cuda")))
         assert native[1] == python[1] and np.array_equal(native[0], python[0])
         assert [a is not None for a in answers] == [taken], answers
+
+
+@pytest.mark.parametrize("K,N", [(1, 1), (96, 33), (257, 130)])
+def test_packing(monkeypatch, K, N):
+    """repack_b and the quantisers: the same bytes, types and shapes either way, and the same refusals."""
+    mx.init(0)
+    mx.lib()
+    whole, i8 = _bf(N + 1, K + 4), torch.randint(-127, 128, (N, K), device="cuda", dtype=torch.int8)
+    W = whole[1:, 3:K + 3]  # rows with gaps, at an odd address
+    calls = [(True, lambda: mx.repack_b(W, transpose=True)), (True, lambda: mx.repack_b(W)), (True, lambda: mx.repack_b(i8, transpose=True)),
+             (True, lambda: mx.repack_b(i8.view(torch.uint8))), (True, lambda: mx.quantize_weights(W)), (True, lambda: mx.quantize_weights(W.contiguous())),
+             (True, lambda: L.quantize_weights_scaled(W, 100.0)), (True, lambda: mx.quantize_pack_int4(W, transpose=True)), (True, lambda: mx.quantize_pack_int4(W)),
+             (False, lambda: mx.repack_b(W, transpose=1)), (False, lambda: mx.repack_b(W.float())), (False, lambda: mx.quantize_weights(W.float())),
+             (False, lambda: mx.quantize_weights(W.cpu())), (False, lambda: L.quantize_weights_scaled(W[0], 100.0)), (False, lambda: mx.quantize_pack_int4(i8)),
+             (False, lambda: mx.quantize_weights(whole[:, :0]))]
+    for n, (taken, call) in enumerate(calls):
+        watch, got = _Watch(_host_call), []
+        for native in (watch, None):
+            monkeypatch.setattr(L, "_native", native)
+            try:
+                r = call()
+                got.append([(t.dtype, tuple(t.shape), t.stride(), host_bits(t).tobytes()) for t in (r if isinstance(r, tuple) else (r,))])
+            except L.MmxError as e:
+                got.append(str(e))
+        assert got[0] == got[1], (n, got[0][:200], got[1][:200])
+        assert [a is not None for a in watch.answers] == [taken], n
