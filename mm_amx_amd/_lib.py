@@ -130,9 +130,9 @@ except ImportError:
         return torch.cuda.current_stream(device).cuda_stream
 
 
-# What a call costs before its launch is what bounds the small shapes (256 x 256 x 256: 12.4 us a call, 6 us of them on the
-# device), so the helpers that every call passes are kept to plain attribute reads: the raw stream handle instead of a
-# Stream object, one stride() instead of several, no query of the library whose answer the call does not need.
+# What a call costs before its launch is what bounds the small shapes, so the regular ones go through native code, and the helpers
+# that the others pass are kept to plain attribute reads: the raw stream handle instead of a Stream object, one stride() instead
+# of several, no query of the library whose answer the call does not need (256 x 256 x 256: 9.7 us this way, 4.7 natively).
 def _stream():
     return _raw_stream(_current_device())
 
