@@ -354,7 +354,9 @@ namespace {
 // busiest CU pulls and what all of them read from memory plus 0.3 of the smaller, another round of workgroups, the slices'
 // meeting, and the blocks a CU finishes.  On those shapes the choice, taken where it promises 10 % over the tile kernels' own
 // model, is 0.73 of the tile kernels' time on average; none of the 840 loses more than 3 %.  (A 64x32 tile, and four
-// wavefronts on a 32x64 one, gained 0.2 % more.)
+// wavefronts on a 32x64 one, gained 0.2 % more.  128x64 and 64x128 tiles, four wavefronts with the whole tile each, are behind the
+// tile kernels' 128x64 where those are used: 512 x 4096 x 4096 int8 19.8 / 19.0 us against 17.6 with a slot per wavefront,
+// 22.7 / 20.4 with one ring for the workgroup and half the LDS reads; what a CU pulls from L2 bounds both.)
 struct Form {
     int mb, np, nw, per_cu;  // per_cu: workgroups that a CU holds
     float us_per_kib;        // pulled by one CU
