@@ -674,6 +674,19 @@ static int launch_chunk(dim3 grid, const SkinnyArgs& s, hipStream_t st) {
     return check_hip(hipGetLastError(), "skinny_chunk_kernel launch");
 }
 
+// What is known of a launch of the two kernels that hold x in LDS, where it makes them faster.
+enum Rows {
+    ANY_ROWS,    // nothing
+    WHOLE_ROWS,  // rows of x are aligned and fill their last fragment
+    NO_REPEATS,  // and the wavefronts' batches of loads hold their shares of K exactly (over bf16 weights; see zero_fragment)
+};
+// What a load behind the end of a wavefront's share of K reads over bf16 weights: the repeat of an infinite weight, multiplied by
+// the zeros that stand for x there, would be NaN.  (Zeros put in place of the load's result took 1 to 8 % of the call, and this
+// address takes up to 5 % where nothing is repeated, so those launches have a form without it: 8 x 4096 x 11008 20.0 us, 20.5
+// with zeros behind the load, 20.7 with the address; 32 x 512 x 4096 4.3, 4.7 and 4.5.  Where loads are repeated: 8 x 320 x 4096
+// 3.5 -> 3.7, 6 x 2600 x 4096 7.7 -> 7.7, 4 x 9600 x 2048 13.8 -> 13.4.)
+static __device__ __align__(1024) char zero_fragment[2048];
+
 // ---- streaming variant for the smallest M -----------------------------------------------------------
 // When the activations fit in LDS the kernel is organised around one goal: have every byte of the
 // weights requested from HBM as early as possible.  x goes from global memory straight into LDS
@@ -687,9 +700,10 @@ static int launch_chunk(dim3 grid, const SkinnyArgs& s, hipStream_t st) {
 // each kernel holds one code path and stays within its registers.
 // UW: batch of the rolling window if not the full register set (the last batch of a wave's share of K is filled up with
 // repeats of the last load, which cost what they are a share of the loads: the launcher picks the batch with the fewest)
-template <int WK, int NP, bool ONE, bool WHOLE, int UW = 0>
+template <int WK, int NP, bool ONE, int ROWS, int UW = 0>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void skinny_stream_kernel(const SkinnyArgs s, int zero_off) {
     constexpr bool W8 = WK == 1, W4 = WK == 2, I8A = WK == 3;  // 3: int8 weights AND int8 activations, int32 sums
+    constexpr bool WHOLE = ROWS != ANY_ROWS, ZEROS = WK == 0 && ROWS != NO_REPEATS;
     // 4: int8 weights and ONE row of x without the matrix cores: every lane owns one column and half of a fragment's
     // k, v_dot2_f32_bf16 on the converted pairs, and one cross-lane add at the end.  Kept as the measured
     // counterpart of WK = 1 (option "decode_valu"); the post-op is the same code.
@@ -727,7 +741,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
         for (int v = 0; v < 16; v++) acc[p][v] = 0;
 
     // wave w multiplies fragments [w*per_wave, (w+1)*per_wave); indices past the end are clamped for the
-    // load and paired with the zero row of x
+    // load (over bf16 weights: to zeros) and paired with the zero row of x
     const int per_wave = (s.nfrag + 7) / 8;
     const int f_begin = wave * per_wave;
     const int f_last = s.nfrag - 1;
@@ -736,7 +750,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     for (int p = 0; p < NP; p++) {
         int panel = panel_first + p;
         panel = (panel < panel_end && panel < s.npanels) ? panel : s.npanels - 1;  // columns past n1 are never stored
-        wbase[p] = s.Wp + (int64_t)panel * s.panel_stride + lane * 16;
+        wbase[p] = s.Wp + (int64_t)panel * s.panel_stride + (ZEROS ? 0 : lane * 16);
     }
     const char* zrow = xs + zero_off;
     const char* xrow = (VALU || l32 < s.M) ? xs + (VALU ? 0 : l32) * pitch : zrow;
@@ -747,9 +761,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 #define MMX_REQUEST(BT, UU)                                                                                     \
     do {                                                                                                        \
         int f_ = f_begin + (BT) * U + (UU);                                                                     \
+        const bool valid_ = (f_ - f_begin) < per_wave && f_ <= f_last; /* scalar */                             \
         f_ = f_ < f_last ? f_ : f_last;                                                                         \
-        _Pragma("unroll") for (int p = 0; p < NP; p++)                                                          \
-            w[p][UU] = MMX_WLOAD(wbase[p] + (int64_t)f_ * 1024);                                             \
+        _Pragma("unroll") for (int p = 0; p < NP; p++) {                                                        \
+            const char* at_ = wbase[p] + (int64_t)f_ * 1024;                                                    \
+            if constexpr (ZEROS) at_ = (valid_ ? at_ : zero_fragment) + lane * 16;                              \
+            w[p][UU] = MMX_WLOAD(at_);                                                                          \
+        }                                                                                                       \
     } while (0)
 #define MMX_MULTIPLY(BT, UU)                                                                                    \
     do {                                                                                                        \
@@ -1170,9 +1188,10 @@ __global__ __launch_bounds__(1024) void skinny_resident_pair_kernel(const Skinny
 // columns x two different k-ranges, so each load is multiplied twice, once with the x of either fragment,
 // into two accumulators: rows 0-15 of the first and rows 16-31 of the second are the two partial sums of
 // the 16 columns (the other rows are never looked at).  (The launcher makes nfrag even; panels hold a multiple of four.)
-template <bool W8, int NP, bool ONE, bool WHOLE, int U>  // U: loads per panel per wave in flight at once (1 KiB each)
+template <bool W8, int NP, bool ONE, int ROWS, int U>  // U: loads per panel per wave in flight at once (1 KiB each)
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void skinny_half_kernel(const SkinnyArgs s, int zero_off) {
     constexpr int NW = 4;
+    constexpr bool WHOLE = ROWS != ANY_ROWS, ZEROS = !W8 && ROWS != NO_REPEATS;
     __shared__ float red[NW][NP][16][64];
     extern __shared__ __attribute__((aligned(1024))) char xs[];  // [M][xpitch], then at zero_off a row of zeros
 
@@ -1212,17 +1231,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
         for (int v = 0; v < 16; v++) acc[p][0][v] = acc[p][1][v] = 0.0f;
 
     // wave w multiplies the fragment pairs [w*per_wave, (w+1)*per_wave); indices past the end are clamped
-    // for the load and paired with the zero row of x
+    // for the load (over bf16 weights: to zeros) and paired with the zero row of x
     const int npairs = s.nfrag >> 1;
     const int per_wave = (npairs + NW - 1) / NW;
     const int u_begin = wave * per_wave;
     const int u_last = npairs - 1;
     const char* wbase[NP];
+    const int wlane = (l32 >> 4) * 1024 + (g32 * 32 + 16 * half + (l32 & 15)) * 16;
 #pragma unroll
     for (int p = 0; p < NP; p++) {
         int panel = panel_first + p;
         panel = (panel < panel_end && panel < s.npanels) ? panel : s.npanels - 1;  // columns past n1 are never stored
-        wbase[p] = s.Wp + (int64_t)panel * s.panel_stride + (l32 >> 4) * 1024 + (g32 * 32 + 16 * half + (l32 & 15)) * 16;
+        wbase[p] = s.Wp + (int64_t)panel * s.panel_stride + (ZEROS ? 0 : wlane);
     }
     const char* zrow = xs + zero_off;
     const char* xrow = l32 < s.M ? xs + l32 * pitch : zrow;
@@ -1231,9 +1251,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 #define MMX_REQUEST(BT, UU)                                                                                     \
     do {                                                                                                        \
         int u_ = u_begin + (BT) * U + (UU);                                                                     \
+        const bool valid_ = (u_ - u_begin) < per_wave && u_ <= u_last; /* scalar */                             \
         u_ = u_ < u_last ? u_ : u_last;                                                                         \
-        _Pragma("unroll") for (int p = 0; p < NP; p++)                                                          \
-            w[p][UU] = MMX_WLOAD(wbase[p] + (int64_t)u_ * 2048);                                             \
+        _Pragma("unroll") for (int p = 0; p < NP; p++) {                                                        \
+            const char* at_ = wbase[p] + (int64_t)u_ * 2048;                                                    \
+            if constexpr (ZEROS) at_ = (valid_ ? at_ : zero_fragment) + wlane;                                  \
+            w[p][UU] = MMX_WLOAD(at_);                                                                          \
+        }                                                                                                       \
     } while (0)
 #define MMX_MULTIPLY(BT, UU)                                                                                    \
     do {                                                                                                        \
@@ -1401,24 +1425,47 @@ bool skinny_i8_eligible(const void* x, int64_t ldx, int M, int K, int k_splits) 
 // 16.8 / 17.7 us at M = 1 / 4 with 16, 16.7 / 18.3 with 8), over int8 weights the smaller (11008 x 4096: 11.2 with 8, 11.8
 // with 12).  Gate/up pairs: batches of 4 per panel (3: +3 %, 2: +5 %, 6: +38 %).
 typedef void (*HalfKernel)(const SkinnyArgs, int);
-template <bool W8, int NP, bool WHOLE>
-static HalfKernel half_window_kernel(int nfrag) {
-    if constexpr (NP == 2) {
-        return skinny_half_kernel<W8, 2, false, WHOLE, 4>;
-    } else {
-        const int n = ((nfrag >> 1) + 3) / 4;  // loads per wave
-        auto repeats = [n](int u) { return (n + u - 1) / u * u - n; };
-        if constexpr (W8) {
-            return repeats(12) < repeats(8) ? skinny_half_kernel<true, 1, false, WHOLE, 12> : skinny_half_kernel<true, 1, false, WHOLE, 8>;
+constexpr int HALF_KERNELS = 5;
+template <bool W8, int NP, int ROWS>
+static HalfKernel half_kernel_at(int i) {  // 0: a wave's share of K in one batch
+    if constexpr (NP == 2) return i == 0 ? skinny_half_kernel<W8, 2, true, ROWS, 8> : skinny_half_kernel<W8, 2, false, ROWS, 4>;
+    else if constexpr (W8)
+        return i == 0 ? skinny_half_kernel<true, 1, true, ROWS, 16>
+                      : (i == 1 ? skinny_half_kernel<true, 1, false, ROWS, 12> : skinny_half_kernel<true, 1, false, ROWS, 8>);
+    else {
+        static const HalfKernel list[HALF_KERNELS] = {skinny_half_kernel<false, 1, true, ROWS, 16>, skinny_half_kernel<false, 1, false, ROWS, 16>,
+                                                      skinny_half_kernel<false, 1, false, ROWS, 10>, skinny_half_kernel<false, 1, false, ROWS, 8>,
+                                                      skinny_half_kernel<false, 1, false, ROWS, 6>};
+        return list[i];
+    }
+}
+// *index: the kernel's place among the 2 HALF_KERNELS of whole rows (for per-kernel set-up).
+template <bool W8, int NP>
+static HalfKernel half_kernel_for(int nfrag, bool whole, int* index) {
+    const int pairs = nfrag >> 1, n = (pairs + 3) / 4;  // loads, and those of a wave
+    auto repeats = [n](int u) { return (n + u - 1) / u * u - n; };
+    int i = 0, u = 16 / NP;
+    if (n > u) {
+        i = 1;
+        if constexpr (NP == 2) u = 4;
+        else if constexpr (W8) {
+            i = repeats(12) < repeats(8) ? 1 : 2;
+            u = i == 1 ? 12 : 8;
         } else {
-            int best = 16;
-            for (int u : {10, 8, 6})
-                if (repeats(u) < repeats(best)) best = u;
-            return best == 16 ? skinny_half_kernel<false, 1, false, WHOLE, 16>
-                              : (best == 10 ? skinny_half_kernel<false, 1, false, WHOLE, 10>
-                                            : (best == 8 ? skinny_half_kernel<false, 1, false, WHOLE, 8> : skinny_half_kernel<false, 1, false, WHOLE, 6>));
+            const int batch[HALF_KERNELS] = {16, 16, 10, 8, 6};
+            for (int t = 2; t < HALF_KERNELS; t++)
+                if (repeats(batch[t]) < repeats(batch[i])) i = t;
+            u = batch[i];
         }
     }
+    if constexpr (!W8) {
+        if (whole && pairs == 4 * n && n % u == 0) {
+            *index = i + HALF_KERNELS;
+            return half_kernel_at<W8, NP, NO_REPEATS>(i);
+        }
+    }
+    *index = i;
+    return whole ? half_kernel_at<W8, NP, WHOLE_ROWS>(i) : half_kernel_at<W8, NP, ANY_ROWS>(i);
 }
 
 // The streaming kernel for single panels and a wave's share of per_wave fragments.  Up to 16: one batch, of the smallest
@@ -1426,19 +1473,21 @@ static HalfKernel half_window_kernel(int nfrag) {
 // 2560 x 10240 at M = 1 10.0 us against 7.6 for its bytes).  Beyond: the rolling window in batches of 16, 10 or 8,
 // whichever repeats the fewest loads, the larger at equal repeats (a share of 20 fragments in batches of 16 is 12 repeats
 // in 32 loads: int8 5120 x 13824 at M = 1 20.0 us, 14.3 in batches of 10; bf16 2560 x 10752 16.2 -> 12.0).
-// *index: the kernel's place in a list of 2 STREAM_KERNELS per weight type (for per-kernel set-up).
+// *index: the kernel's place in a list of 3 STREAM_KERNELS per weight type (for per-kernel set-up).
 typedef void (*StreamKernel)(const SkinnyArgs, int);
 constexpr int STREAM_KERNELS = 9;
-template <int WK, bool WHOLE>
+template <int WK, int ROWS>
 static StreamKernel stream_kernel_at(int i) {
     static const StreamKernel list[STREAM_KERNELS] = {
-        skinny_stream_kernel<WK, 1, true, WHOLE, 4>,  skinny_stream_kernel<WK, 1, true, WHOLE, 6>,  skinny_stream_kernel<WK, 1, true, WHOLE, 8>,
-        skinny_stream_kernel<WK, 1, true, WHOLE, 10>, skinny_stream_kernel<WK, 1, true, WHOLE, 12>, skinny_stream_kernel<WK, 1, true, WHOLE>,
-        skinny_stream_kernel<WK, 1, false, WHOLE>,    skinny_stream_kernel<WK, 1, false, WHOLE, 10>, skinny_stream_kernel<WK, 1, false, WHOLE, 8>};
+        skinny_stream_kernel<WK, 1, true, ROWS, 4>,  skinny_stream_kernel<WK, 1, true, ROWS, 6>,  skinny_stream_kernel<WK, 1, true, ROWS, 8>,
+        skinny_stream_kernel<WK, 1, true, ROWS, 10>, skinny_stream_kernel<WK, 1, true, ROWS, 12>, skinny_stream_kernel<WK, 1, true, ROWS>,
+        skinny_stream_kernel<WK, 1, false, ROWS>,    skinny_stream_kernel<WK, 1, false, ROWS, 10>, skinny_stream_kernel<WK, 1, false, ROWS, 8>};
     return list[i];
 }
 template <int WK>
-static StreamKernel stream_kernel_for(int per_wave, bool whole, int* index) {
+static StreamKernel stream_kernel_for(int nfrag, bool whole, int* index) {
+    const int per_wave = (nfrag + 7) / 8;
+    const int batch[STREAM_KERNELS] = {4, 6, 8, 10, 12, 16, 16, 10, 8};
     int i;
     if (per_wave <= 16) {
         i = per_wave <= 4 ? 0 : (per_wave <= 6 ? 1 : (per_wave <= 8 ? 2 : (per_wave <= 10 ? 3 : (per_wave <= 12 ? 4 : 5))));
@@ -1448,8 +1497,27 @@ static StreamKernel stream_kernel_for(int per_wave, bool whole, int* index) {
         if (repeats(10) < repeats(16)) i = 7;
         if (repeats(8) < repeats(i == 7 ? 10 : 16)) i = 8;
     }
+    if constexpr (WK == 0) {
+        if (whole && nfrag == 8 * per_wave && per_wave % batch[i] == 0) {
+            *index = i + 2 * STREAM_KERNELS;
+            return stream_kernel_at<WK, NO_REPEATS>(i);
+        }
+    }
     *index = i + (whole ? 0 : STREAM_KERNELS);
-    return whole ? stream_kernel_at<WK, true>(i) : stream_kernel_at<WK, false>(i);
+    return whole ? stream_kernel_at<WK, WHOLE_ROWS>(i) : stream_kernel_at<WK, ANY_ROWS>(i);
+}
+// Gate/up pairs: batches of 8 fragments per panel, 4 over int4 weights.
+template <int WK>
+static StreamKernel stream_pair_kernel_for(int nfrag, bool whole) {
+    constexpr int U = WK == 2 ? 4 : 8;
+    const int per_wave = (nfrag + 7) / 8;
+    const bool one = per_wave <= U;
+    if constexpr (WK == 0) {
+        if (whole && nfrag == 8 * per_wave && per_wave % U == 0)
+            return one ? skinny_stream_kernel<0, 2, true, NO_REPEATS> : skinny_stream_kernel<0, 2, false, NO_REPEATS>;
+    }
+    if (whole) return one ? skinny_stream_kernel<WK, 2, true, WHOLE_ROWS> : skinny_stream_kernel<WK, 2, false, WHOLE_ROWS>;
+    return one ? skinny_stream_kernel<WK, 2, true, ANY_ROWS> : skinny_stream_kernel<WK, 2, false, ANY_ROWS>;
 }
 
 // wk: weights are bf16 (0), int8 (1) or int4 (2); 3: int8 weights and int8 activations
@@ -1505,7 +1573,7 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
         }
         note_kernel("skinny_stream_i8");
         int unused;
-        hipLaunchKernelGGL(stream_kernel_for<3>((s.nfrag + 7) / 8, s.xpitch == row_bytes, &unused), dim3(panels), dim3(512), stream_lds_bytes(zoff + s.xpitch, 1), st, s, zoff);
+        hipLaunchKernelGGL(stream_kernel_for<3>(s.nfrag, s.xpitch == row_bytes, &unused), dim3(panels), dim3(512), stream_lds_bytes(zoff + s.xpitch, 1), st, s, zoff);
         return check_hip(hipGetLastError(), "skinny_stream_kernel launch");
     }
     if (wk == 2) {
@@ -1519,13 +1587,11 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
             const int per_wave = (s.nfrag + 7) / 8;
             const bool fills = s.x_direct && s.xpitch == row_bytes;
             StreamKernel kern;  // (register sets sized to the share of K, as for the other weight types)
-            if (pairs)          // gate and up panels side by side: four fragments of each in flight per wave
-                kern = per_wave <= 4 ? (fills ? skinny_stream_kernel<2, 2, true, true> : skinny_stream_kernel<2, 2, true, false>)
-                                     : (fills ? skinny_stream_kernel<2, 2, false, true> : skinny_stream_kernel<2, 2, false, false>);
-            else if (per_wave <= 4) kern = fills ? skinny_stream_kernel<2, 1, true, true, 4> : skinny_stream_kernel<2, 1, true, false, 4>;
-            else if (per_wave <= 6) kern = fills ? skinny_stream_kernel<2, 1, true, true, 6> : skinny_stream_kernel<2, 1, true, false, 6>;
-            else if (per_wave <= 8) kern = fills ? skinny_stream_kernel<2, 1, true, true> : skinny_stream_kernel<2, 1, true, false>;
-            else kern = fills ? skinny_stream_kernel<2, 1, false, true> : skinny_stream_kernel<2, 1, false, false>;
+            if (pairs) kern = stream_pair_kernel_for<2>(s.nfrag, fills);  // gate and up panels side by side
+            else if (per_wave <= 4) kern = fills ? skinny_stream_kernel<2, 1, true, WHOLE_ROWS, 4> : skinny_stream_kernel<2, 1, true, ANY_ROWS, 4>;
+            else if (per_wave <= 6) kern = fills ? skinny_stream_kernel<2, 1, true, WHOLE_ROWS, 6> : skinny_stream_kernel<2, 1, true, ANY_ROWS, 6>;
+            else if (per_wave <= 8) kern = fills ? skinny_stream_kernel<2, 1, true, WHOLE_ROWS> : skinny_stream_kernel<2, 1, true, ANY_ROWS>;
+            else kern = fills ? skinny_stream_kernel<2, 1, false, WHOLE_ROWS> : skinny_stream_kernel<2, 1, false, ANY_ROWS>;
             const int np = pairs ? 2 : 1;
             hipLaunchKernelGGL(kern, dim3(panels / np), dim3(512), stream_lds_bytes(xb, np), st, s, zoff);
             return check_hip(hipGetLastError(), "skinny_stream_kernel launch");
@@ -1563,19 +1629,13 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
         decode_halves() != 0 && panels <= num_cus() && (int64_t)s.nfrag * 512 >= 128 * 1024) {
         // A few rows of a long x (the MLP's down projection at M = 2-4: 66-110 KiB with the zero row) and at
         // most one half-panel per CU: the half-panel form with one workgroup per CU still has all of x in LDS.
-        static std::atomic<uint64_t> attr_done[5];
-        const HalfKernel kernels[5] = {skinny_half_kernel<false, 1, true, true, 16>, skinny_half_kernel<false, 1, false, true, 16>,
-                                       skinny_half_kernel<false, 1, false, true, 10>, skinny_half_kernel<false, 1, false, true, 8>,
-                                       skinny_half_kernel<false, 1, false, true, 6>};
-        for (int i = 0; i < 5; i++) {
-            const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kernels[i]), 128 * 1024, attr_done[i]);
-            if (rc) return rc;
-        }
+        static std::atomic<uint64_t> attr_done[2 * HALF_KERNELS];
+        int index;
+        const HalfKernel kern = half_kernel_for<false, 1>(s.nfrag, true, &index);
+        const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), 128 * 1024, attr_done[index]);
+        if (rc) return rc;
         note_kernel("skinny_half_bf16");
-        if (((s.nfrag >> 1) + 3) / 4 <= 16)
-            hipLaunchKernelGGL((skinny_half_kernel<false, 1, true, true, 16>), dim3(2 * panels), dim3(256), xbytes, st, s, zero_off);
-        else
-            hipLaunchKernelGGL((half_window_kernel<false, 1, true>(s.nfrag)), dim3(2 * panels), dim3(256), xbytes, st, s, zero_off);
+        hipLaunchKernelGGL(kern, dim3(2 * panels), dim3(256), xbytes, st, s, zero_off);
         return check_hip(hipGetLastError(), "skinny_half_kernel launch");
     }
     {
@@ -1651,12 +1711,11 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
     // be resident): 80 KiB of x each (4096 x 11008 int8 GEMV at M = 5-8: 13.0-13.4 -> 11.5-12.0 us against the chunked
     // form; with one workgroup per CU, M = 12-16, it loses: 16.6-17.7 against 13.7-14.5 us).
     const bool bigx = !pairs && xbytes > 46 * 1024 && xbytes <= 80 * 1024;
-    const int per_wave = (s.nfrag + 7) / 8;
-    const bool fills = s.x_direct && s.xpitch == row_bytes;  // (the WHOLE forms)
+    const bool fills = s.x_direct && s.xpitch == row_bytes;  // (WHOLE_ROWS)
     int stream_index = 0;
-    const StreamKernel stream_kernel = w8 ? stream_kernel_for<1>(per_wave, fills, &stream_index) : stream_kernel_for<0>(per_wave, fills, &stream_index);
+    const StreamKernel stream_kernel = w8 ? stream_kernel_for<1>(s.nfrag, fills, &stream_index) : stream_kernel_for<0>(s.nfrag, fills, &stream_index);
     if (bigx) {
-        static std::atomic<uint64_t> attr_done[2][2 * STREAM_KERNELS];
+        static std::atomic<uint64_t> attr_done[2][3 * STREAM_KERNELS];
         const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(stream_kernel), 80 * 1024, attr_done[w8 ? 1 : 0][stream_index]);
         if (rc) return rc;
     }
@@ -1681,25 +1740,18 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
             zero_off = (M * s.xpitch + 1023) & ~1023;
             xbytes = zero_off + s.xpitch;
         }
-        const int per_wave_h = ((s.nfrag >> 1) + 3) / 4;
         auto stream = [&](auto w8_c, auto np_c, int grid) {
             constexpr bool W8 = decltype(w8_c)::value;
             constexpr int NP = decltype(np_c)::value;
             if constexpr (!(W8 && NP == 2)) {
                 if (halves) {  // (the rolling window holds fewer registers where two accumulator pairs need them)
-                    const bool fill = s.xpitch == row_bytes && s.x_direct;
-                    HalfKernel kern;
-                    if (per_wave_h <= 16 / NP) kern = fill ? skinny_half_kernel<W8, NP, true, true, 16 / NP> : skinny_half_kernel<W8, NP, true, false, 16 / NP>;
-                    else kern = fill ? half_window_kernel<W8, NP, true>(s.nfrag) : half_window_kernel<W8, NP, false>(s.nfrag);
-                    hipLaunchKernelGGL(kern, dim3(2 * grid), dim3(256), xbytes, st, s, zero_off);
+                    int unused;
+                    hipLaunchKernelGGL((half_kernel_for<W8, NP>(s.nfrag, s.xpitch == row_bytes && s.x_direct, &unused)), dim3(2 * grid), dim3(256), xbytes, st, s, zero_off);
                     return;
                 }
             }
             StreamKernel kern = stream_kernel;
-            if constexpr (NP == 2) {
-                if (per_wave <= 8) kern = fills ? skinny_stream_kernel<W8, 2, true, true> : skinny_stream_kernel<W8, 2, true, false>;
-                else kern = fills ? skinny_stream_kernel<W8, 2, false, true> : skinny_stream_kernel<W8, 2, false, false>;
-            }
+            if constexpr (NP == 2) kern = stream_pair_kernel_for<W8 ? 1 : 0>(s.nfrag, fills);
             hipLaunchKernelGGL(kern, dim3(grid), dim3(512), stream_lds_bytes(xbytes, NP), st, s, zero_off);
         };
         if (halves) note_kernel(pairs ? "skinny_half_bf16_gateup" : (w8 ? "skinny_half_w8" : "skinny_half_bf16"));
@@ -1714,7 +1766,7 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
         if (valu) {
             note_kernel("skinny_stream_w8_valu");
             int unused;
-            hipLaunchKernelGGL(stream_kernel_for<4>(per_wave, fills, &unused), dim3(panels), dim3(512), stream_lds_bytes(xbytes, 1), st, s, zero_off);
+            hipLaunchKernelGGL(stream_kernel_for<4>(s.nfrag, fills, &unused), dim3(panels), dim3(512), stream_lds_bytes(xbytes, 1), st, s, zero_off);
         } else {
             using std::integral_constant;
             if (pairs && w8) stream(integral_constant<bool, true>{}, integral_constant<int, 2>{}, panels / 2);

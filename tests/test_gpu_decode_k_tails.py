@@ -120,6 +120,26 @@ def test_infinite_x_at_the_end_of_k(po, kind):
     assert torch.isinf(C).all(), mx.last_kernel()
 
 
+@pytest.mark.parametrize("M,K,N,splits,want", [
+    (12, 2600, 64, 0, "skinny_stream_bf16"),        # fragments that a wavefront's batch repeats behind the end of K
+    (12, 2624, 64, 0, "skinny_stream_bf16"),        # (whole 128-byte groups of K)
+    (2, 1000, 64, 1, "skinny_stream_bf16"),
+    (3, 2600, 1000, 0, "skinny_half_bf16"),
+    (3, 2624, 1000, 0, "skinny_half_bf16"),
+    (30, 3681, 160, 1, "skinny_chunk_bf16"),
+    (24, 2624, 160, 0, "skinny_chunk_bf16_ksplit"),
+    (6, 11072, 8300, 0, "skinny_direct_bf16"),
+])
+def test_infinite_weights_at_the_end_of_k(M, K, N, splits, want):
+    """What a load repeats behind the end of K is not multiplied: infinite weights in the last row of B give infinities, no NaN."""
+    W = torch.ones((K, N), dtype=torch.bfloat16, device="cuda")
+    W[K - 1] = float("inf")
+    C = torch.zeros((M, N), dtype=torch.float32, device="cuda")
+    mx.gemm(torch.ones((M, K), dtype=torch.bfloat16, device="cuda"), mx.repack_b(W), N, mx.Epilogue(C), k_splits=splits)
+    assert mx.last_kernel().startswith(want), mx.last_kernel()
+    assert torch.isinf(C).all(), mx.last_kernel()
+
+
 def test_int8_with_a_count_of_slices_is_refused_as_ever(po):
     """A forced K split belongs to the tile kernels, which refuse it at such a K; the call without one takes the decode kernels."""
     M, K, N = 8, 2112, 256
