@@ -456,18 +456,20 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
         xa[UU] = *reinterpret_cast<const bf16x8*>(xlane + (int64_t)f_ * XB);                \
         if constexpr (W8) xb[UU] = *reinterpret_cast<const bf16x8*>(xlane + (int64_t)f_ * XB + 16); \
     } while (0)
-    // a fragment index past this wave's share (or past the end of K) contributes nothing: its weights are zeroed
+    // a fragment index past this wave's share (or past the end of K) contributes nothing: its weights and its x are zeroed
 #define MMX_MULTIPLY(BT, UU)                                                                \
     do {                                                                                    \
         const int f_ = f_begin + (BT) * U + (UU);                                           \
         const bool valid_ = (f_ - f_begin) < per_wave && f_ <= f_last; /* scalar */         \
         _Pragma("unroll") for (int p = 0; p < NP; p++) {                                    \
             const u32x4 wv_ = valid_ ? w[p][UU] : u32x4{0u, 0u, 0u, 0u};                    \
+            const bf16x8 xa_ = valid_ ? xa[UU] : bf16x8{};                                  \
             if constexpr (W8) {                                                             \
-                acc[p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(s8x8_to_bf16(wv_.x, wv_.y), xa[UU], acc[p], 0, 0, 0); \
-                acc[p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(s8x8_to_bf16(wv_.z, wv_.w), xb[UU], acc[p], 0, 0, 0); \
+                const bf16x8 xb_ = valid_ ? xb[UU] : bf16x8{};                              \
+                acc[p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(s8x8_to_bf16(wv_.x, wv_.y), xa_, acc[p], 0, 0, 0); \
+                acc[p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(s8x8_to_bf16(wv_.z, wv_.w), xb_, acc[p], 0, 0, 0); \
             } else {                                                                        \
-                acc[p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, wv_), xa[UU], acc[p], 0, 0, 0); \
+                acc[p] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, wv_), xa_, acc[p], 0, 0, 0); \
             }                                                                               \
         }                                                                                   \
     } while (0)
@@ -493,6 +495,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     skinny_finish<NP>(s, red, panel_first, tid, fin);
 }
 
+// Read in place of what lies behind the end of K, where a repeat of its end would meet zeros on the other side of a product:
+// zero times an infinity is NaN.
+static __device__ __align__(1024) char zero_fragment[2048];
+
 // ---- chunked variant for aligned operands whose x does not fit in LDS, many rows (8 < M <= 32) ------
 // K is walked in chunks of 8*FPW fragments; in a chunk every wave multiplies FPW fragments of each
 // panel.  The x a chunk needs ([M][RB bytes], RB = 8*FPW fragments' worth of a row) is fetched by the
@@ -507,12 +513,19 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 // c+1 is what allows chunk c+2 to overwrite chunk c.  16-byte pieces of a row are XOR-swizzled with
 // the row so that the 32 rows an operand reads spread over the banks.
 // Lanes of rows >= M read row 0 (their output columns are never stored); fragments past the end of K
-// get zero weights and a clamped (finite) x.  TAIL: rows of x of any alignment, 16 bytes and longer, zero past the end of K.
+// get zero weights and a zero x (a repeat of the row's end might be infinite, and zero times that is NaN).
 // WK: weights are bf16 (0), int8 (1) or int4 (2), 3: int8 weights and int8 activations (int32 sums);
 // XD: 16-byte x loads per thread per chunk (8 KiB of x each)
-// TAIL: the rows of x end inside a group of four fragments, or do not start on 16 bytes
+// Where the rows of x end.  Behind the end of aligned rows the loads go to zeros: int4 11008 x 4096 at M = 16 / 32 12.7 / 14.9 us
+// -> 12.9 / 14.9, bf16 2624 x 8300 at M = 32 16.1 -> 16.3.  (Zeros put in place of what was loaded took up to 7 %, branches around
+// the products up to 15 %, the bytes moved as for unaligned rows 4 %: int4 30 x 2304 x 16192.)
+enum End {
+    ON_CHUNK,   // with a chunk
+    IN_CHUNK,   // between two fragments of a chunk
+    ANYWHERE,   // inside a group of four fragments, or they do not start on 16 bytes (rows of 16 bytes and longer)
+};
 constexpr int chunk_row_bytes(int wk, int fpw) { return 8 * fpw * (wk == 2 ? 128 : (wk == 1 ? 64 : 32)); }
-template <int WK, int NP, int FPW, int XD, int WIN, bool TAIL>  // WIN: chunks in flight (0: what the case's registers hold)
+template <int WK, int NP, int FPW, int XD, int WIN, int END>  // WIN: chunks in flight (0: what the case's registers hold)
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void skinny_chunk_kernel(const SkinnyArgs s) {
     constexpr bool W8 = WK == 1, W4 = WK == 2, I8A = WK == 3;
     using accv = std::conditional_t<I8A, i32x16, f32x16>;
@@ -577,7 +590,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 #define MMX_LOAD(C, J)                                                                                         \
     do {                                                                                                       \
         _Pragma("unroll") for (int t = 0; t < XD; t++) {                                                       \
-            xr[J][t] = fetch16_in_row(xsrc[t], (C) * RB + xcol[t], row_bytes);                                 \
+            if constexpr (END == IN_CHUNK)                                                                     \
+                xr[J][t] = *reinterpret_cast<const u32x4*>((C) * RB + xcol[t] < row_bytes ? xsrc[t] + (C) * RB + xcol[t] : zero_fragment); \
+            else                                                                                               \
+                xr[J][t] = fetch16_in_row(xsrc[t], (C) * RB + xcol[t], row_bytes);                             \
         }                                                                                                      \
         _Pragma("unroll") for (int u = 0; u < FPW; u++) {                                                      \
             int f_ = (C) * FC + wave * FPW + u;                                                                \
@@ -589,7 +605,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 #define MMX_CHUNK(C, J)                                                                                        \
     do {                                                                                                       \
         char* buf_ = smem + ((C) & 1) * BUF;                                                                   \
-        if (TAIL && ((C) + 1) * RB > row_bytes) { /* scalar: the rows of x end in this chunk */                 \
+        if (END == ANYWHERE && ((C) + 1) * RB > row_bytes) { /* scalar: the rows of x end in this chunk */                 \
             _Pragma("unroll") for (int t = 0; t < XD; t++)                                                     \
                 xr[J][t] = settle16_in_row(xr[J][t], (C) * RB + xcol[t], row_bytes);                           \
         }                                                                                                      \
@@ -667,10 +683,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 template <int WK, int NP, int FPW, int XD, int WIN = 0>
 static int launch_chunk(dim3 grid, const SkinnyArgs& s, hipStream_t st) {
     constexpr int lds = (2 * 8 * XD * 1024) > (8 * NP * 16 * 64 * 4) ? (2 * 8 * XD * 1024) : (8 * NP * 16 * 64 * 4);  // two buffers of x, later the reduction scratch
-    // (a K that fills the panels' last group of fragments ends between two fragments: the test per chunk is not needed there,
-    // and cost int4 30 x 2304 x 16192 4 %)
-    const bool tail = !s.x_vec_ok || s.K % (WK == 2 ? 256 : (WK == 0 ? 64 : 128)) != 0;
-    hipLaunchKernelGGL((tail ? skinny_chunk_kernel<WK, NP, FPW, XD, WIN, true> : skinny_chunk_kernel<WK, NP, FPW, XD, WIN, false>), grid, dim3(512), lds, st, s);
+    const int row_bytes = s.K * (WK == 3 ? 1 : 2);
+    void (*kern)(const SkinnyArgs);
+    if (!s.x_vec_ok || s.K % (WK == 2 ? 256 : (WK == 0 ? 64 : 128))) kern = skinny_chunk_kernel<WK, NP, FPW, XD, WIN, ANYWHERE>;
+    else if (row_bytes % chunk_row_bytes(WK, FPW)) kern = skinny_chunk_kernel<WK, NP, FPW, XD, WIN, IN_CHUNK>;
+    else kern = skinny_chunk_kernel<WK, NP, FPW, XD, WIN, ON_CHUNK>;
+    hipLaunchKernelGGL(kern, grid, dim3(512), lds, st, s);
     return check_hip(hipGetLastError(), "skinny_chunk_kernel launch");
 }
 
@@ -678,14 +696,12 @@ static int launch_chunk(dim3 grid, const SkinnyArgs& s, hipStream_t st) {
 enum Rows {
     ANY_ROWS,    // nothing
     WHOLE_ROWS,  // rows of x are aligned and fill their last fragment
-    NO_REPEATS,  // and the wavefronts' batches of loads hold their shares of K exactly (over bf16 weights; see zero_fragment)
+    NO_REPEATS,  // and the wavefronts' batches of loads hold their shares of K exactly (bf16 weights)
 };
-// What a load behind the end of a wavefront's share of K reads over bf16 weights: the repeat of an infinite weight, multiplied by
-// the zeros that stand for x there, would be NaN.  (Zeros put in place of the load's result took 1 to 8 % of the call, and this
-// address takes up to 5 % where nothing is repeated, so those launches have a form without it: 8 x 4096 x 11008 20.0 us, 20.5
-// with zeros behind the load, 20.7 with the address; 32 x 512 x 4096 4.3, 4.7 and 4.5.  Where loads are repeated: 8 x 320 x 4096
-// 3.5 -> 3.7, 6 x 2600 x 4096 7.7 -> 7.7, 4 x 9600 x 2048 13.8 -> 13.4.)
-static __device__ __align__(1024) char zero_fragment[2048];
+// Over bf16 weights a load behind the end of a wavefront's share of K reads zero_fragment, in the first two forms.  (Zeros put in
+// place of the load's result took 1 to 8 % of the call, and the choice of address takes up to 5 % where nothing is repeated, hence
+// the third: 8 x 4096 x 11008 20.0 us, 20.5 with zeros behind the load, 20.7 with the address; 32 x 512 x 4096 4.3, 4.7 and 4.5.
+// Where loads are repeated: 8 x 320 x 4096 3.5 -> 3.7, 6 x 2600 x 4096 7.7 -> 7.7, 4 x 9600 x 2048 13.8 -> 13.4.)
 
 // ---- streaming variant for the smallest M -----------------------------------------------------------
 // When the activations fit in LDS the kernel is organised around one goal: have every byte of the

@@ -107,16 +107,33 @@ def test_gate_up(po, kind, M, K):
     assert np.linalg.norm(got - want) <= 2.0 ** -13 * np.linalg.norm(want), mx.last_kernel()
 
 
-@pytest.mark.parametrize("kind", ["bf16", "w8", "w4"])
-def test_infinite_x_at_the_end_of_k(po, kind):
-    """Nothing of a row is multiplied twice, by zero weights or otherwise: an infinite last element gives infinities, no NaN."""
-    M, K, N = 12, 2600, 64
+@pytest.mark.parametrize("kind,M,K,N,splits,want", [
+    ("bf16", 12, 2600, 64, 0, "skinny_stream_bf16"),
+    ("w8", 12, 2600, 64, 0, "skinny_stream_w8"),
+    ("w4", 8, 2600, 64, 0, "skinny_w4_k_tail"),
+    ("bf16", 24, 2600, 64, 1, "skinny_chunk_bf16"),      # rows that end between two pieces of 16 bytes
+    ("w8", 20, 2612, 64, 1, "skinny_chunk_w8"),
+    ("w4", 12, 2600, 64, 1, "skinny_w4_k_tail_long"),
+    ("bf16", 24, 2624, 64, 1, "skinny_chunk_bf16"),      # rows that end between two fragments of a chunk
+    ("bf16", 12, 3712, 64, 1, "skinny_chunk_bf16"),      # (two fragments of a panel per wavefront)
+    ("bf16", 32, 4160, 1000, 0, "skinny_chunk_bf16_ksplit"),
+    ("bf16", 24, 2624, 8300, 0, "skinny_chunk_bf16_2p"),
+    ("w8", 32, 4224, 1000, 1, "skinny_chunk_w8"),
+    ("w8", 12, 4224, 1000, 0, "skinny_chunk_w8_ksplit"),
+    ("w8", 32, 4224, 8300, 0, "skinny_chunk_w8_2p"),
+    ("w4", 16, 2304, 64, 1, "skinny_chunk_w4"),
+    ("w4", 32, 2304, 64, 1, "skinny_chunk_w4"),
+    ("bf16", 6, 11072, 8300, 0, "skinny_direct_bf16"),
+])
+def test_infinite_x_at_the_end_of_k(kind, M, K, N, splits, want):
+    """The end of a row that a load repeats behind it is not multiplied again: an infinite last element gives infinities, no NaN."""
     x = torch.ones((M, K), dtype=torch.bfloat16, device="cuda")
     x[:, K - 1] = float("inf")
     W = torch.ones((K, N), dtype=torch.bfloat16, device="cuda")
     packed = {"bf16": lambda: mx.repack_b(W), "w8": lambda: mx.repack_b(W.to(torch.int8)), "w4": lambda: mx.quantize_pack_int4(W)[0]}[kind]()
     C = torch.zeros((M, N), dtype=torch.float32, device="cuda")
-    mx.gemm(x, packed, N, mx.Epilogue(C), **KW[kind])
+    mx.gemm(x, packed, N, mx.Epilogue(C), k_splits=splits, **KW[kind])
+    assert mx.last_kernel().startswith(want), mx.last_kernel()
     assert torch.isinf(C).all(), mx.last_kernel()
 
 
