@@ -5,6 +5,7 @@ current torch HIP stream cross the boundary.
 """
 import ctypes as C
 import os
+import warnings
 
 import torch
 
@@ -38,12 +39,30 @@ class _Epilogue(C.Structure):
 
 
 _lib = None
-_native = None  # the host side of a call in native code (module _host_call), once the library is loaded
+_native = None  # the host side of a call in native code (module _host_call), once the library is loaded, if it is there
 _initialised = set()
 
 
 def lib_path():
     return _LIB_PATH
+
+
+def _host_module(l):
+    """The module with the host side of a call in native code (csrc/host_call.cpp, built with the library), bound to the library
+    l; None if it is not there or was built for another Python or torch.  The Python form below takes every call then."""
+    try:
+        from . import _host_call
+        built_for = getattr(_host_call, "torch_version", None)
+        if built_for != str(torch.__version__):
+            raise ImportError(f"it was built for torch {built_for}, this is {torch.__version__}")
+    except ImportError as e:
+        warnings.warn(f"mm_amx_amd: the native host side of calls is not used ({e}): each call takes about 5 us longer. "
+                      "`python -m mm_amx_amd.build` builds it.", RuntimeWarning, stacklevel=4)
+        return None
+    _host_call.bind(*(C.cast(f, C.c_void_p).value for f in (
+        l.mmx_gemm_splitk, l.mmx_gemm_workspace_bytes, l.mmx_gemm_unpacked, l.mmx_gemm_unpacked_workspace_bytes, l.mmx_matvec,
+        l.mmx_packed_b_bytes, l.mmx_repack_b, l.mmx_quantize_weights, l.mmx_quantize_weights_scaled, l.mmx_quantize_pack_int4)))
+    return _host_call
 
 
 def lib():
@@ -98,12 +117,8 @@ def lib():
         l.mmx_probe_mfma.argtypes = [C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.POINTER(C.c_float),
                                      C.POINTER(C.c_float)]
         l.mmx_probe_read.argtypes = [C.c_void_p, C.c_size_t, C.c_int, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p]
-        from . import _host_call  # (built with the library; see csrc/host_call.cpp)
-        _host_call.bind(*(C.cast(f, C.c_void_p).value for f in (
-            l.mmx_gemm_splitk, l.mmx_gemm_workspace_bytes, l.mmx_gemm_unpacked, l.mmx_gemm_unpacked_workspace_bytes, l.mmx_matvec,
-            l.mmx_packed_b_bytes, l.mmx_repack_b, l.mmx_quantize_weights, l.mmx_quantize_weights_scaled, l.mmx_quantize_pack_int4)))
         global _native
-        _native = _host_call
+        _native = _host_module(l)
         _lib = l
     return _lib
 

@@ -1,4 +1,4 @@
-"""Builds libmm_amx_amd.so (HIP kernels + C ABI) in-tree for gfx950 with hipcc, and _host_call.so (a CPython module) with g++.
+"""Builds libmm_amx_amd.so (HIP kernels + C ABI) in-tree for gfx950 with hipcc, and the CPython module _host_call with g++.
 
     python -m mm_amx_amd.build [--incremental] [--stamps]
 
@@ -10,11 +10,12 @@ workgroup (-DMMX_STAMPS; read by mm_amx_amd.phase_stamps); the shipped library h
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libmm_amx_amd.so")
-HOST_CALL = os.path.join(HERE, "_host_call.so")
+HOST_CALL = os.path.join(HERE, "_host_call" + sysconfig.get_config_var("EXT_SUFFIX"))  # (of this Python only)
 # the MFMA tile GEMM is instantiated per (input type, output type) pair in a file of its own, so that the
 # pairs compile side by side
 SOURCES = ["abi.hip", "gemm_bf16.hip", "gemm_i8.hip", "gemm_w8.hip",
@@ -41,12 +42,11 @@ def _stale(obj, src):
 
 def host_call_command():
     """The CPython module with the host side of a GEMM call: host code, compiled against this Python and this torch."""
-    import sysconfig
-
     import torch
     at = os.path.dirname(torch.__file__)
     include = [os.path.join(at, "include"), os.path.join(at, "include", "torch", "csrc", "api", "include"), sysconfig.get_paths()["include"]]
-    return (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"] +
+    return (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+             f'-DMMX_TORCH_VERSION="{torch.__version__}"'] +
             ["-isystem" + d for d in include] + [os.path.join(CSRC, "host_call.cpp"), "-o", HOST_CALL, "-L" + os.path.join(at, "lib"),
                                                  "-ltorch_python", "-ltorch_cpu", "-lc10"])
 

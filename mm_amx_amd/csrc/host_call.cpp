@@ -363,4 +363,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_call", nullptr, -1, methods,
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host_call(void) { return PyModule_Create(&module); }
+// torch_version: of the torch that this was compiled against, whose classes may be laid out differently in another
+PyMODINIT_FUNC PyInit__host_call(void) {
+    PyObject* const m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "torch_version", MMX_TORCH_VERSION) < 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}
