@@ -2,12 +2,15 @@
 
     python -m mm_amx_amd.build [--incremental] [--stamps]
 
+The library needs hipcc alone.  The module is for the Python layer and is left out where torch, Python's headers or g++ are missing.
+
 By default every source is compiled again; --incremental keeps the object files of earlier runs and
 recompiles only what is older than its source or than a header.  --stamps builds a second library,
 libmm_amx_amd_stamps.so, whose tile kernels record the shader clock at the phase boundaries of every
 workgroup (-DMMX_STAMPS; read by mm_amx_amd.phase_stamps); the shipped library holds no such code.
 """
 import os
+import shutil
 import subprocess
 import sys
 import sysconfig
@@ -41,10 +44,17 @@ def _stale(obj, src):
 
 
 def host_call_command():
-    """The CPython module with the host side of a GEMM call: host code, compiled against this Python and this torch."""
-    import torch
+    """The CPython module with the host side of a call: host code, compiled against this Python and this torch.  None where
+    there is nothing to compile it with."""
+    python_include = sysconfig.get_paths()["include"]
+    try:
+        import torch
+    except ImportError:
+        return None
+    if not shutil.which("g++") or not os.path.isfile(os.path.join(python_include, "Python.h")):
+        return None
     at = os.path.dirname(torch.__file__)
-    include = [os.path.join(at, "include"), os.path.join(at, "include", "torch", "csrc", "api", "include"), sysconfig.get_paths()["include"]]
+    include = [os.path.join(at, "include"), os.path.join(at, "include", "torch", "csrc", "api", "include"), python_include]
     return (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
              f'-DMMX_TORCH_VERSION="{torch.__version__}"'] +
             ["-isystem" + d for d in include] + [os.path.join(CSRC, "host_call.cpp"), "-o", HOST_CALL, "-L" + os.path.join(at, "lib"),
@@ -59,7 +69,10 @@ def build(verbose=False, incremental=False, stamps=False):
             if not incremental or _stale(obj, os.path.join(CSRC, src))]
     failed = False
     running = []
-    host = subprocess.Popen(host_call_command())
+    command = host_call_command()
+    if command is None:
+        print("[build] no torch, Python.h or g++: without the module _host_call (calls from Python take 5 us longer)", file=sys.stderr)
+    host = subprocess.Popen(command) if command else None
 
     def reap(p_src, p):
         nonlocal failed
@@ -71,19 +84,22 @@ def build(verbose=False, incremental=False, stamps=False):
         elif out.strip() and verbose:
             print(out)
 
-    for src, obj in todo:
-        while len(running) >= JOBS:
-            reap(*running.pop(0))
-        cmd = ["hipcc"] + flags + ["-c", os.path.join(CSRC, src), "-o", obj]
-        if verbose:
-            print(" ".join(cmd), flush=True)
-        running.append((src, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
-    for item in running:
-        reap(*item)
-    if failed:
-        raise RuntimeError("hipcc failed")
-    subprocess.check_call(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-o", lib] + objs)
-    if host.wait() != 0:
+    try:
+        for src, obj in todo:
+            while len(running) >= JOBS:
+                reap(*running.pop(0))
+            cmd = ["hipcc"] + flags + ["-c", os.path.join(CSRC, src), "-o", obj]
+            if verbose:
+                print(" ".join(cmd), flush=True)
+            running.append((src, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
+        for item in running:
+            reap(*item)
+        if failed:
+            raise RuntimeError("hipcc failed")
+        subprocess.check_call(["hipcc", "--offload-arch=gfx950", "-shared", "-fPIC", "-o", lib] + objs)
+    finally:  # (whatever happened to the library, nothing is left running)
+        host_failed = host is not None and host.wait() != 0
+    if host_failed:
         raise RuntimeError("g++ failed on host_call.cpp")
     if not incremental:
         for obj in objs:
