@@ -579,7 +579,7 @@ def matvec(A, b, out=None):
     """c[M] = A[M,K] · b[K]; bf16 (c fp32) or int8 (c int32)."""
     if _native is not None and type(out) is torch.Tensor and out.is_cuda:  # as in gemm()
         device = _current_device()
-        rc = _native.matvec(A, b, out, device, _raw_stream(device))
+        rc = _native.matvec(A, b, out, device, _raw_stream(device)) if device in _initialised else None
         if rc is not None:
             _check(rc)
             return out

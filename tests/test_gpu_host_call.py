@@ -172,6 +172,19 @@ def test_matvec(monkeypatch, kind):
         assert [a is not None for a in answers] == [taken], answers
 
 
+def test_matvec_initialises_its_device(monkeypatch):
+    """The first call on a GPU asks the library whether it has code for it, before anything is launched there."""
+    A, b, out = _bf(64, 96), _bf(96), torch.zeros(64, device="cuda")
+    mx.lib()
+    watch = _Watch(L._native)
+    monkeypatch.setattr(L, "_native", watch)
+    monkeypatch.setattr(L, "_initialised", set())
+    mx.matvec(A, b, out)
+    assert L._initialised == {torch.cuda.current_device()} and not watch.answers
+    mx.matvec(A, b, out)
+    assert watch.answers == [0]
+
+
 @pytest.mark.parametrize("K,N", [(1, 1), (96, 33), (257, 130)])
 def test_packing(monkeypatch, K, N):
     """repack_b and the quantisers: the same bytes, types and shapes either way, and the same refusals."""
