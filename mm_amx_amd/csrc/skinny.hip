@@ -1598,8 +1598,7 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
         const int zoff = (M * s.xpitch + 1023) & ~1023;
         const int xb = zoff + s.xpitch;
         if (row_bytes >= 16 && xb <= 46 * 1024) {
-            // (a K that ends inside the panel's last four fragments has names of its own)
-            note_kernel(K % 256 ? (pairs ? "skinny_w4_k_tail_gateup" : "skinny_w4_k_tail") : (pairs ? "skinny_stream_w4_gateup" : "skinny_stream_w4"));
+            note_kernel(pairs ? "skinny_stream_w4_gateup" : "skinny_stream_w4");
             const int per_wave = (s.nfrag + 7) / 8;
             const bool fills = s.x_direct && s.xpitch == row_bytes;
             StreamKernel kern;  // (register sets sized to the share of K, as for the other weight types)
@@ -1625,12 +1624,12 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
                 s.ws_part = rq->ws + SPLIT_COUNTER_BYTES;
                 s.kslices = ksl4;
                 char name_[40];
-                snprintf(name_, sizeof name_, K % 256 ? "skinny_w4_k_tail_ksplit%d" : "skinny_chunk_w4_ksplit%d", ksl4);
+                snprintf(name_, sizeof name_, "skinny_chunk_w4_ksplit%d", ksl4);
                 note_kernel(name_);
                 if (M <= 16) return launch_chunk<2, 1, 1, 2, 3>(dim3(panels, ksl4), s, st);
                 return launch_chunk<2, 1, 1, 4, 2>(dim3(panels, ksl4), s, st);
             }
-            note_kernel(K % 256 ? "skinny_w4_k_tail_long" : "skinny_chunk_w4");
+            note_kernel("skinny_chunk_w4");
             if (M <= 16) return launch_chunk<2, 1, 1, 2>(dim3(panels), s, st);
             return launch_chunk<2, 1, 1, 4>(dim3(panels), s, st);
         }

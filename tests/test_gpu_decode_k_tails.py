@@ -56,7 +56,7 @@ def test_x_in_lds(po, kind, K, M):
         mx.gemm(_in_nan((dev if kind == "i8" else dev_bf16)(x), pad), packed, N, mx.Epilogue(C), **KW[kind])
         if kind != "i8" or pad != 3 or M == 1:
             if (M + 1) * K * es <= 40000:
-                assert ("skinny_w4_k_tail" if kind == "w4" else "skinny_stream") in mx.last_kernel(), mx.last_kernel()
+                assert mx.last_kernel().startswith(f"skinny_stream_{kind}"), mx.last_kernel()
             assert mx.last_kernel() not in ("skinny_bf16", "skinny_w8", "skinny_w4")
         if kind == "i8":
             assert np.array_equal(host_bits(C), ref), mx.last_kernel()
@@ -74,9 +74,9 @@ def test_x_in_lds(po, kind, K, M):
     ("w8", 16, 4160, 8300, 0, "skinny_chunk_w8"),
     ("w8", 32, 4190, 700, 0, "skinny_chunk_w8_ksplit"),
     ("w8", 24, 2611, 8300, 0, "skinny_chunk_w8_2p"),
-    ("w4", 11, 5313, 300, 0, "skinny_w4_k_tail_ksplit"),
-    ("w4", 29, 1800, 300, 1, "skinny_w4_k_tail_long"),
-    ("w4", 9, 6850, 8300, 1, "skinny_w4_k_tail_long"),
+    ("w4", 11, 5313, 300, 0, "skinny_chunk_w4_ksplit"),
+    ("w4", 29, 1800, 300, 1, "skinny_chunk_w4"),
+    ("w4", 9, 6850, 8300, 1, "skinny_chunk_w4"),
 ])
 def test_x_through_lds_in_chunks_and_half_panels(po, kind, M, K, N, splits, want):
     x, packed, ref = _operands(po, kind, M, K, N, K)
@@ -110,10 +110,10 @@ def test_gate_up(po, kind, M, K):
 @pytest.mark.parametrize("kind,M,K,N,splits,want", [
     ("bf16", 12, 2600, 64, 0, "skinny_stream_bf16"),
     ("w8", 12, 2600, 64, 0, "skinny_stream_w8"),
-    ("w4", 8, 2600, 64, 0, "skinny_w4_k_tail"),
+    ("w4", 8, 2600, 64, 0, "skinny_stream_w4"),
     ("bf16", 24, 2600, 64, 1, "skinny_chunk_bf16"),      # rows that end between two pieces of 16 bytes
     ("w8", 20, 2612, 64, 1, "skinny_chunk_w8"),
-    ("w4", 12, 2600, 64, 1, "skinny_w4_k_tail_long"),
+    ("w4", 12, 2600, 64, 1, "skinny_chunk_w4"),
     ("bf16", 24, 2624, 64, 1, "skinny_chunk_bf16"),      # rows that end between two fragments of a chunk
     ("bf16", 12, 3712, 64, 1, "skinny_chunk_bf16"),      # (two fragments of a panel per wavefront)
     ("bf16", 32, 4160, 1000, 0, "skinny_chunk_bf16_ksplit"),
