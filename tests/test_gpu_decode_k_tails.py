@@ -110,7 +110,7 @@ def test_gate_up(po, kind, M, K):
 @pytest.mark.parametrize("kind,M,K,N,splits,want", [
     ("bf16", 12, 2600, 64, 0, "skinny_stream_bf16"),
     ("w8", 12, 2600, 64, 0, "skinny_stream_w8"),
-    ("w4", 8, 2600, 64, 0, "skinny_stream_w4"),
+    ("w4", 7, 2600, 64, 0, "skinny_stream_w4"),
     ("bf16", 24, 2600, 64, 1, "skinny_chunk_bf16"),      # rows that end between two pieces of 16 bytes
     ("w8", 20, 2612, 64, 1, "skinny_chunk_w8"),
     ("w4", 12, 2600, 64, 1, "skinny_chunk_w4"),
