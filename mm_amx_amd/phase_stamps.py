@@ -4,7 +4,7 @@
 
 Each argument is  dtype,M,K,N,tile,k_splits[,waves]  (dtype bf16: the FC with BIAS+GELU and a bf16 store; i8: the int8 FC
 with DEQUANT+BIAS+QUANT and an int8 store; w8: bf16 activations on int8-compressed weights, DEQUANT, fp32 store; tile as for
-mmx_set_tile, empty = the library's choice; waves 4 or 8), or  gemv8,M,K,N / gemv4,M,K,N  (decode: bf16 activations on
+mmx_set_tile, empty = the library's choice, which for few tiles is a kernel without stamps; waves 4 or 8), or  gemv8,M,K,N / gemv4,M,K,N  (decode: bf16 activations on
 int8 / int4 weights through the streaming kernel, weights rotated over 540 MB).  The instrumented library is built on first use (several
 minutes) and whenever a kernel source is newer than it.
 The instrumented library (libmm_amx_amd_stamps.so, -DMMX_STAMPS) makes thread 0 of every workgroup write the shader
@@ -68,6 +68,10 @@ def run(ws, dt, M, K, N, tile, S, waves=8, out=sys.stdout):
         mx.set_option("waves", 8)
     st = ws[stamp_off:].view(torch.int64).cpu().numpy().reshape(-1, 8)
     st = st[st[:, 0] != 0]
+    if not len(st):
+        print(f"== {dt} {M}x{K}x{N} {kern}: {ms * 1e3:.2f} us/launch, no stamps (this kernel is not instrumented; a tile named in the "
+              "argument pins one that is)", file=out)
+        return
     fin = st[st[:, 7] != 0]               # workgroups that ran an epilogue (with a K split: the last to arrive at their tile)
     rt0 = st[:, 0].min()
     wall_us = (fin[:, 7] - fin[:, 0]) / 100.0   # 100 MHz wall-clock ticks
