@@ -60,9 +60,18 @@ def test_k_tail(po, kind, K, tile):
     mx.set_tile("")
 
 
+@pytest.fixture
+def tile(request):
+    """The tile of the case, forced (the small tiles, which have tests of their own, would take these shapes)."""
+    mx.set_tile(request.param)
+    yield request.param
+    mx.set_tile("")
+
+
+@pytest.mark.parametrize("tile", ["128x128", "64x128"], indirect=True)
 @pytest.mark.parametrize("K", [4104, 4400])
 @pytest.mark.parametrize("kind", ["bf16", "w8", "i8"])
-def test_k_tail_behind_a_k_split(po, kind, K):
+def test_k_tail_behind_a_k_split(po, kind, K, tile):
     """Few tiles and a long K: the last slice, and it alone, takes the tail (16 and 96 bytes of A)."""
     M, N = 64, 256
     rng = np.random.default_rng(K)
@@ -77,7 +86,7 @@ def test_k_tail_behind_a_k_split(po, kind, K):
         C, up = torch.zeros((M, N), dtype=torch.float32, device="cuda"), dev_bf16
         ref = po.gemm_bf16(A, B if kind == "bf16" else po.f32_to_bf16(B.astype(np.float32)))
     mx.gemm(up(A), mx.repack_b((dev_bf16 if kind == "bf16" else dev)(B)), N, mx.Epilogue(C), **({"b_dtype": mx.I8} if kind == "w8" else {}))
-    assert "ring" in mx.last_kernel() and "ksplit" in mx.last_kernel(), mx.last_kernel()
+    assert f"_{tile}_ring_" in mx.last_kernel() and "ksplit" in mx.last_kernel(), mx.last_kernel()
     if kind == "i8":
         assert np.array_equal(host_bits(C), ref), mx.last_kernel()
     else:
@@ -106,8 +115,9 @@ def test_the_plan_does_not_depend_on_earlier_calls(kind, M, K, pad):
     assert torch.equal(out[0], out[1])
 
 
+@pytest.mark.parametrize("tile", ["128x128"], indirect=True)  # (the only one with pairs and a tail)
 @pytest.mark.parametrize("kind", ["bf16", "w8"])
-def test_k_tail_gate_up(po, kind):
+def test_k_tail_gate_up(po, kind, tile):
     M, K, N = 70, 200, 96
     rng = np.random.default_rng(5)
     x = po.f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32))
@@ -120,7 +130,7 @@ def test_k_tail_gate_up(po, kind):
         both = np.concatenate([w[n:n + 32] for n in range(0, N, 32) for w in (wg, wu)])
         mx.gemm(dev_bf16(x), mx.repack_b(dev(both), transpose=True), 2 * N,
                 mx.Epilogue(h, mx.PP_SILU_GATE | mx.PP_DEQUANT, deq_scale=2.0 ** -10), b_dtype=mx.I8)
-    assert "ring" in mx.last_kernel(), mx.last_kernel()
+    assert f"_{tile}_ring_" in mx.last_kernel(), mx.last_kernel()
     g, u = (po.gemm_bf16(x, np.ascontiguousarray((w if kind == "bf16" else po.f32_to_bf16(w.astype(np.float32))).T)) for w in (wg, wu))
     if kind == "w8":
         g, u = g * 2.0 ** -10, u * 2.0 ** -10
