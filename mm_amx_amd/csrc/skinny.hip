@@ -683,11 +683,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 template <int WK, int NP, int FPW, int XD, int WIN = 0>
 static int launch_chunk(dim3 grid, const SkinnyArgs& s, hipStream_t st) {
     constexpr int lds = (2 * 8 * XD * 1024) > (8 * NP * 16 * 64 * 4) ? (2 * 8 * XD * 1024) : (8 * NP * 16 * 64 * 4);  // two buffers of x, later the reduction scratch
-    const int row_bytes = s.K * (WK == 3 ? 1 : 2);
-    void (*kern)(const SkinnyArgs);
-    if (!s.x_vec_ok || s.K % (WK == 2 ? 256 : (WK == 0 ? 64 : 128))) kern = skinny_chunk_kernel<WK, NP, FPW, XD, WIN, ANYWHERE>;
-    else if (row_bytes % chunk_row_bytes(WK, FPW)) kern = skinny_chunk_kernel<WK, NP, FPW, XD, WIN, IN_CHUNK>;
-    else kern = skinny_chunk_kernel<WK, NP, FPW, XD, WIN, ON_CHUNK>;
+    void (*kern)(const SkinnyArgs) = skinny_chunk_kernel<WK, NP, FPW, XD, WIN, ON_CHUNK>;
+    if constexpr (WK != 3) {  // (int8 x takes this kernel only if K fills its chunks: skinny_i8_eligible)
+        if (!s.x_vec_ok || s.K % (WK == 2 ? 256 : (WK == 0 ? 64 : 128))) kern = skinny_chunk_kernel<WK, NP, FPW, XD, WIN, ANYWHERE>;
+        else if (s.K * 2 % chunk_row_bytes(WK, FPW)) kern = skinny_chunk_kernel<WK, NP, FPW, XD, WIN, IN_CHUNK>;
+    }
     hipLaunchKernelGGL(kern, grid, dim3(512), lds, st, s);
     return check_hip(hipGetLastError(), "skinny_chunk_kernel launch");
 }

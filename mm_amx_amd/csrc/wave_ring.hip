@@ -6,8 +6,8 @@
 // (38 bytes per clock) even if it is alone on the chip, behind a barrier per half-stage, and 4 us with nothing to do.  So here
 //   - tiles are small (32x32, 32x64 or 64x64), hence many, and a CU pulls few bytes;
 //   - every wavefront holds the whole tile in its accumulators, and K goes round the wavefronts, 128 bytes at a time: each
-//     has a ring of LDS slots of its own, waits for its own loads only and meets the others once, when the sums are added;
-//   - a stage's operands are read into registers, its slot goes to the next load, and then come the products;
+//     has an LDS slot of its own, waits for its own loads only and meets the others once, when the sums are added;
+//   - a stage's operands are read into registers, the slot goes to the next stage's loads, and then come the products;
 //   - where tiles are few and K is long, K is also cut into 2 or 4 slices for as many workgroups (the protocol and workspace
 //     layout of the tile kernels' split).
 // bf16 40 x 1024 x 1024 8.4 -> 3.8 us, 900 x 1600 x 256 10.8 -> 4.6, 512 x 1024 x 1024 8.5 -> 5.0, 256 x 4096 x 4096 20.6 -> 17.1,
@@ -50,11 +50,10 @@ __device__ __forceinline__ void load_lds(uint32_t lds, uint32_t off, const char*
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(off), "s"(base) : "memory");
 }
 
-// MB x NP: 32x32 blocks of the tile; NW: wavefronts; D: stages in a wavefront's ring
-template <int T, int MB, int NP, int NW, int D>
+// MB x NP: 32x32 blocks of the tile; NW: wavefronts
+template <int T, int MB, int NP, int NW>
 __global__ __launch_bounds__(NW * 64, MB * NP == 1 ? 4 : 2) void wave_ring_kernel(const WaveRingArgs g) {
     constexpr int A_ST = MB * 4096, BP_ST = T == W8 ? 2048 : 4096, ST = A_ST + NP * BP_ST;
-    constexpr int NL = ST / 1024;  // loads per wavefront and stage
     using acc_t = typename std::conditional<T == I8, int, float>::type;
     using accv = typename std::conditional<T == I8, i32x16, f32x16>::type;
     typedef acc_t acc4 __attribute__((ext_vector_type(4)));
@@ -74,7 +73,7 @@ __global__ __launch_bounds__(NW * 64, MB * NP == 1 ? 4 : 2) void wave_ring_kerne
     const int s0 = slice * g.per_slice, s1 = s0 + g.per_slice < g.stages ? s0 + g.per_slice : g.stages;
     const Epilogue& ep = g.ep;
 
-    // ---- the wavefront's stages: s0 + wave, s0 + wave + NW, ... through its ring of D slots -------------------------
+    // ---- the wavefront's stages: s0 + wave, s0 + wave + NW, ... through its slot ------------------------------------
     // A: rows of 128 bytes, 16-byte chunk c of row r at position c ^ ((r >> 1) & 7) (an operand read of 32 rows then spreads
     // over the banks); a load covers 8 rows, whole lines.  B: fragments as they are packed.
     uint32_t aoff[MB * 4];
@@ -87,27 +86,26 @@ __global__ __launch_bounds__(NW * 64, MB * NP == 1 ? 4 : 2) void wave_ring_kerne
     const char* bbase[NP];
 #pragma unroll
     for (int p = 0; p < NP; p++) bbase[p] = g.Bp + (int64_t)(panel0 + p < g.npanels ? panel0 + p : g.npanels - 1) * g.panel_stride;
-    char* const ring = smem + wave * (D * ST);
-    const uint32_t ring_lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)ring);
+    char* const slot = smem + wave * ST;
+    const uint32_t slot_lds = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)slot);
     const int tail = g.kbytes & 127;  // bytes of the last stage, if it is not full: 16, 32, ... 112
-    auto issue = [&](int st, int slot) __attribute__((always_inline)) {
+    auto issue = [&](int st) __attribute__((always_inline)) {
         const char* const a = abase + (int64_t)st * 128;
-        const uint32_t lds = ring_lds + slot * ST;
         if (__builtin_expect(tail && st == g.stages - 1, 0)) {  // (scalar) chunks behind the end of the row are zero and not touched
 #pragma unroll
             for (int i = 0; i < MB * 4; i++) {
-                if (((lane & 7) ^ ((4 * i + (lane >> 4)) & 7)) * 16 < tail) load_lds(lds + i * 1024, aoff[i], a);
-                else *reinterpret_cast<u32x4*>(ring + slot * ST + i * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
+                if (((lane & 7) ^ ((4 * i + (lane >> 4)) & 7)) * 16 < tail) load_lds(slot_lds + i * 1024, aoff[i], a);
+                else *reinterpret_cast<u32x4*>(slot + i * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
             }
         } else {
 #pragma unroll
-            for (int i = 0; i < MB * 4; i++) load_lds(lds + i * 1024, aoff[i], a);
+            for (int i = 0; i < MB * 4; i++) load_lds(slot_lds + i * 1024, aoff[i], a);
         }
 #pragma unroll
         for (int p = 0; p < NP; p++)
 #pragma unroll
             for (int i = 0; i < BP_ST / 1024; i++)
-                load_lds(lds + A_ST + p * BP_ST + i * 1024, lane * 16, bbase[p] + (int64_t)st * BP_ST + i * 1024);
+                load_lds(slot_lds + A_ST + p * BP_ST + i * 1024, lane * 16, bbase[p] + (int64_t)st * BP_ST + i * 1024);
     };
     accv acc[MB][NP];
 #pragma unroll
@@ -116,13 +114,13 @@ __global__ __launch_bounds__(NW * 64, MB * NP == 1 ? 4 : 2) void wave_ring_kerne
         for (int p = 0; p < NP; p++)
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[b][p][v] = 0;
-    // A stage's operands are read from LDS into registers, its slot goes to the next load, and then come the products: with one
-    // slot per wavefront the next stage is on its way while this one is multiplied.
+    // A stage's operands are read from LDS into registers, the slot goes to the next stage's loads, and then come the products: the
+    // next stage is on its way while this one is multiplied.
     constexpr int BR = BP_ST / 1024;  // fragments of a panel in a stage
     u32x4 ra[4][MB], rb[BR][NP];
-    auto read = [&](int slot) __attribute__((always_inline)) {
-        const char* const sa = ring + slot * ST + l32 * 128;
-        const char* const sb = ring + slot * ST + A_ST + lane * 16;
+    auto read = [&]() __attribute__((always_inline)) {
+        const char* const sa = slot + l32 * 128;
+        const char* const sb = slot + A_ST + lane * 16;
         const int swz = (l32 >> 1) & 7;
 #pragma unroll
         for (int s = 0; s < 4; s++) {  // 32 bytes of K of a row of A at a time
@@ -160,12 +158,10 @@ __global__ __launch_bounds__(NW * 64, MB * NP == 1 ? 4 : 2) void wave_ring_kerne
     };
     const int first = s0 + wave;
     const int count = first < s1 ? (s1 - first + NW - 1) / NW : 0;
-#pragma unroll
-    for (int i = 0; i < D; i++)
-        if (i < count) issue(first + i * NW, i);
+    if (count > 0) issue(first);
 
     // the per-column operands of this thread's outputs (units of four columns of a row, the same columns in every unit of a
-    // thread) travel behind the first stages; gate/up pairs: column q of gate in deq, of up in bias
+    // thread) travel behind the first stage; gate/up pairs: column q of gate in deq, of up in bias
     const bool pairs = NP == 2 && (ep.steps & MMX_PP_SILU_GATE);
     constexpr int UNITS = MB * 32 * 8 * NP, UT = (UNITS + NW * 64 - 1) / (NW * 64);
     const int q0 = tid & (pairs ? 7 : 8 * NP - 1);  // unit of the row
@@ -180,22 +176,14 @@ __global__ __launch_bounds__(NW * 64, MB * NP == 1 ? 4 : 2) void wave_ring_kerne
         if (pairs) bias[e] = (ep.steps & MMX_PP_DEQUANT) && ep.deq_oc ? ep.deq_oc[c + 32 < g.n1 ? c + 32 : g.n1 - 1] : ep.deq;
     }
 
-    for (int i0 = 0; i0 < count; i0 += D) {
-#pragma unroll
-        for (int d = 0; d < D; d++) {
-            const int i = i0 + d;
-            if (i < count) {
-                // loads return in order: what is younger than this stage may still be on its way
-                if (D > 1 && i + D - 1 < count) asm volatile("s_waitcnt vmcnt(%0)" : : "n"((D - 1) * NL) : "memory");
-                else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                read(d);
-                if (i + D < count) {
-                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // every read of the slot is done
-                    issue(first + (i + D) * NW, d);
-                }
-                multiply();
-            }
+    for (int i = 0; i < count; i++) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        read();
+        if (i + 1 < count) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // every read of the slot is done
+            issue(first + (i + 1) * NW);
         }
+        multiply();
     }
 
     // ---- the wavefronts' sums meet in LDS, 4 registers (4 consecutive columns of a row) to a 16-byte piece ------------
@@ -329,12 +317,12 @@ __global__ __launch_bounds__(NW * 64, MB * NP == 1 ? 4 : 2) void wave_ring_kerne
 
 
 typedef void (*WaveRingKernel)(const WaveRingArgs);
-template <int T, int MB, int NP, int NW, int D>
+template <int T, int MB, int NP, int NW>
 int launch_cfg(const WaveRingArgs& g, hipStream_t st) {
-    constexpr int ring = NW * D * (MB * 4096 + NP * (T == W8 ? 2048 : 4096)), red = NW * MB * NP * 4096, lds = ring > red ? ring : red;
+    constexpr int slots = NW * (MB * 4096 + NP * (T == W8 ? 2048 : 4096)), red = NW * MB * NP * 4096, lds = slots > red ? slots : red;
     static_assert(lds <= 160 * 1024, "LDS of a CU");
     static std::atomic<uint64_t> attr_done{0};
-    const WaveRingKernel kern = wave_ring_kernel<T, MB, NP, NW, D>;
+    const WaveRingKernel kern = wave_ring_kernel<T, MB, NP, NW>;
     const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds, attr_done);
     if (rc) return rc;
     char name[96], split[16] = "";
@@ -396,14 +384,14 @@ WaveRingPlan choose_form(int type, int M, int K, int Ncols, bool pairs, int k_sp
 
 }  // namespace
 
-// Takes the call (returns MMX_OK or an error) or leaves it to the tile kernels (returns 1), whose own model says tiles_us.
-// type: 0 bf16, 1 bf16 over int8 weights, 3 int8.  The choice depends on the shape alone: a call without a workspace that would
-// have used one has k_splits = 1.
 static bool wave_ring_can(int type, int K, bool aligned) {
     const int64_t kbytes = (int64_t)K * (type == I8 ? 1 : 2);
     return aligned && kbytes % 16 == 0 && kbytes >= 128 && K <= (1 << 24);
 }
 
+// Takes the call (returns MMX_OK or an error) or leaves it to the tile kernels (returns 1), whose own model says tiles_us.
+// type: 0 bf16, 1 bf16 over int8 weights, 3 int8.  The choice depends on the shape and on the workspace: what it holds bounds the
+// slices, and a call without one has k_splits = 1.
 int launch_wave_ring(int type, const void* A, int64_t lda, const void* Bp, int M, int K, int N, int n0, int n1, const Epilogue& ep,
                      const SplitRequest& rq, float tiles_us, hipStream_t st) {
     const bool pairs = (ep.steps & MMX_PP_SILU_GATE) != 0;
@@ -437,26 +425,26 @@ int launch_wave_ring(int type, const void* A, int64_t lda, const void* Bp, int M
     auto launch = [&](auto type_c) {
         constexpr int T = decltype(type_c)::value;
         switch (p.form) {
-        case 0: return launch_cfg<T, 1, 1, 8, 1>(g, st);
-        case 1: return launch_cfg<T, 1, 2, 8, 1>(g, st);
-        case 2: return launch_cfg<T, 2, 2, 8, 1>(g, st);
+        case 0: return launch_cfg<T, 1, 1, 8>(g, st);
+        case 1: return launch_cfg<T, 1, 2, 8>(g, st);
+        case 2: return launch_cfg<T, 2, 2, 8>(g, st);
         }
-        if constexpr (T != I8) return launch_cfg<T, 2, 2, 4, 1>(g, st);
+        if constexpr (T != I8) return launch_cfg<T, 2, 2, 4>(g, st);
         return set_error(MMX_E_UNSUPPORTED, "no such form for int8");
     };
     using std::integral_constant;
     return type == I8 ? launch(integral_constant<int, I8>{}) : (type == W8 ? launch(integral_constant<int, W8>{}) : launch(integral_constant<int, BF16>{}));
 }
 
-// Bytes of workspace the call above would use (0: no slices), or -1 if it would leave the call to the tile kernels.  Rows of A
-// that are not aligned are the tile kernels' in any case.  (Sized for whole 64 rows: one answer for 1 to 64 of them.)
+// Bytes of workspace the call above would use (0: no slices), or -1 if it would leave the call to the tile kernels.  (Rows of A that
+// are not aligned go to the masked pipeline there, which takes no slices.)
 int64_t wave_ring_workspace_bytes(int type, int M, int K, int Ncols, bool pairs, int k_splits, float tiles_us) {
     if (!wave_ring_can(type, K, true)) return -1;
     const WaveRingPlan p = choose_form(type, M, K, Ncols, pairs, k_splits, ~(size_t)0);
     if (p.form < 0 || p.us >= 0.9f * tiles_us) return -1;
     const Form& c = FORMS[p.form];
     if (p.slices == 1) return 0;
-    return (int64_t)(COUNTER_BYTES + (size_t)((M + 63) / 64 * 2 / c.mb) * (((Ncols + 31) / 32 + c.np - 1) / c.np) * p.slices * c.mb * c.np * 4096);
+    return (int64_t)(COUNTER_BYTES + (size_t)((M + 32 * c.mb - 1) / (32 * c.mb)) * (((Ncols + 31) / 32 + c.np - 1) / c.np) * p.slices * c.mb * c.np * 4096);
 }
 
 }  // namespace mmx

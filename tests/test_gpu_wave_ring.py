@@ -7,6 +7,7 @@ import torch
 
 import mm_amx_amd as mx
 from gpu_util import check_float_parity, dev, dev_bf16, host_bits
+from mm_amx_amd._lib import WORKSPACE_BYTES
 
 pytestmark = pytest.mark.gpu
 
@@ -77,7 +78,7 @@ def test_slices(po, kind, M, K, N, slices):
     if kind == "i8":
         K *= 2
     A, packed, ref, kw, rng = _operands(po, kind, M, K, N)
-    ws = torch.zeros(mx.WORKSPACE_BYTES if hasattr(mx, "WORKSPACE_BYTES") else (64 << 20) + (16 << 10), dtype=torch.uint8, device="cuda")
+    ws = torch.zeros(WORKSPACE_BYTES, dtype=torch.uint8, device="cuda")
     outs = []
     for rep in range(3):
         acc = torch.zeros((M, N), dtype=torch.int32 if kind == "i8" else torch.float32, device="cuda")
@@ -97,6 +98,15 @@ def test_slices(po, kind, M, K, N, slices):
     deq = np.float32(2.0 ** -8)
     mx.gemm(A, packed, N, mx.Epilogue(y, 7, bias=dev(bias), deq_scale=float(deq)), ws=ws, **kw)
     assert np.array_equal(host_bits(y), po.pp(outs[0], 7, po.BF16, bias=bias, deq=deq))
+    # a workspace of the size that the query names holds the same slices, one of a byte less does not
+    need = mx.gemm_workspace_bytes(*{"bf16": (mx.BF16, mx.BF16), "w8": (mx.BF16, mx.I8), "i8": (mx.I8, mx.I8)}[kind], M, K, N)
+    split = mx.last_kernel().partition("_ksplit")[1:]
+    assert (need > 0) == (split[0] != ""), (need, split)
+    for size in (need, need - 1) if need else ():
+        acc = torch.zeros_like(acc)
+        mx.gemm(A, packed, N, mx.Epilogue(acc), ws=ws[:size], **kw)
+        assert (mx.last_kernel().partition("_ksplit")[1:] == split) == (size == need), (mx.last_kernel(), split)
+        assert size < need or np.array_equal(host_bits(acc), outs[0])
     # without the slices' memory the call is not split
     mx.gemm(A, packed, N, mx.Epilogue(acc), ws=ws[:(16 << 10) + 256], **kw)
     assert "ksplit" not in mx.last_kernel(), mx.last_kernel()
@@ -115,7 +125,7 @@ def test_slices_replay_from_a_hip_graph(po):
     M, K, N = 50, 8192, 320
     A, packed, ref, kw, rng = _operands(po, "bf16", M, K, N)
     A = A.clone()
-    ws = torch.zeros((64 << 20) + (16 << 10), dtype=torch.uint8, device="cuda")
+    ws = torch.zeros(WORKSPACE_BYTES, dtype=torch.uint8, device="cuda")
     y = torch.zeros((M, N), dtype=torch.float32, device="cuda")
     g, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
