@@ -19,8 +19,7 @@ static std::mutex g_attr_mutex;
 // tiles as in a caller's workspace, held by every GPU the library runs on until the process ends.  All zero when
 // the code object is loaded; every completed call leaves the counters zero.  `static_ws` is the host-side stand-in
 // of the array: its device address is taken once per device in mmx_init and only that address is ever used.
-constexpr size_t STATIC_WS_BYTES = ((size_t)64 << 20) + ((size_t)16 << 10);
-static __device__ __align__(256) unsigned char static_ws[STATIC_WS_BYTES];
+static __device__ __align__(256) unsigned char static_ws[WS_STANDARD_BYTES];
 constexpr int MAX_DEVICES = 64;
 static std::atomic<char*> g_static_ws[MAX_DEVICES];
 
@@ -345,11 +344,11 @@ int mmx_gemm_splitk_static(int a_dtype, int b_dtype, const void* A, int64_t lda_
     if (!ws) return set_error(MMX_E_INVALID, "mmx_gemm_splitk_static: call mmx_init(%d) first (it takes the address of this device's workspace)", dev);
     if (k_splits > 1 && M > 32) {
         const size_t need = mmx_gemm_workspace_bytes(a_dtype, b_dtype, M, K, N, n0, n1, ep ? ep->steps : 0, k_splits);
-        if (need > STATIC_WS_BYTES)
+        if (need > WS_STANDARD_BYTES)
             return set_error(MMX_E_INVALID, "mmx_gemm_splitk_static: %d K slices of this shape need %zu bytes of workspace, the built-in one holds %zu",
-                             k_splits, need, STATIC_WS_BYTES);
+                             k_splits, need, WS_STANDARD_BYTES);
     }
-    const SplitRequest rq = {k_splits, ws, STATIC_WS_BYTES};
+    const SplitRequest rq = {k_splits, ws, WS_STANDARD_BYTES};
     return gemm_dispatch(a_dtype, b_dtype, A, lda_bytes, Bpacked, M, K, N, n0, n1, ep, rq, static_cast<hipStream_t>(stream));
 }
 

@@ -86,6 +86,13 @@ struct SplitRequest {
     char* ws;         // workspace (NULL: no split possible)
     size_t ws_bytes;
 };
+// The layout that every kernel with a K split keeps to, since one workspace serves them all: one 32-bit arrival counter per output
+// tile (or panel), zero between launches, and the partial sums behind them.
+constexpr int WS_MAX_TILES = 4096;
+constexpr size_t WS_COUNTER_BYTES = (size_t)WS_MAX_TILES * 4;
+// The size that serves every split of the library's own choosing: what the front ends allocate once per stream, and the array of
+// mmx_gemm_splitk_static.
+constexpr size_t WS_STANDARD_BYTES = ((size_t)64 << 20) + WS_COUNTER_BYTES;
 
 // ---- element-wise epilogue arithmetic -----------------------------------------------------
 // All device code is compiled with -ffp-contract=off: a*b+c below never fuses unless written

@@ -1046,10 +1046,6 @@ int load_mode();
 int wave_count();
 int ensure_dynamic_lds(const void* kernel, int bytes, std::atomic<uint64_t>& done_on_device);
 
-// Where the partial sums of a K split live: the first WS_COUNTER_BYTES hold one arrival counter per tile
-// (zero between launches), the partial tiles follow.
-constexpr int WS_MAX_TILES = 4096;
-constexpr size_t WS_COUNTER_BYTES = (size_t)WS_MAX_TILES * 4;
 constexpr int KSPLIT_MAX = 4;  // slices a kernel instantiation can combine (its SMAX)
 
 // K slices are whole blocks of 512 bytes of K per row (256 bf16: the K block of AMX_MLP::Linear,

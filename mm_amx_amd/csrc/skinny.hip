@@ -1382,12 +1382,6 @@ int decode_valu();
 int decode_resident();
 int decode_pair();
 
-// dynamic LDS of skinny_stream_kernel: x + the zero row, reused afterwards as the reduction scratch (32 KiB per panel)
-// Workspace of a K split: arrival counters first (one per workgroup column, zero between launches), the slices' sums after
-// them - the layout the tile kernels use, so one workspace serves both.
-constexpr int SPLIT_MAX_PANELS = 4096;
-constexpr size_t SPLIT_COUNTER_BYTES = (size_t)SPLIT_MAX_PANELS * 4;
-
 // Slices of K for the chunked kernel: with a panel for at most every second CU the workgroups of a panel walk K in 2-4
 // slices (as many as give every CU one workgroup; more - 6, 8 - measured slower), none empty and each at least four
 // chunks long, and the last to arrive adds them up (int8 weights, weights rotated over 540 MB: 11008 x 4096 at
@@ -1396,14 +1390,14 @@ constexpr size_t SPLIT_COUNTER_BYTES = (size_t)SPLIT_MAX_PANELS * 4;
 // CUs, three slices of at least ten chunks fill the two workgroups a CU holds (11008 x 5120, int8 M = 16 / 32 20.9 / 25.8
 // -> 17.1 / 21.7, bf16 27.6 / 35.7 -> 24.2 / 26.7); shorter slices and more panels measured level or behind.
 static int chunk_slices(bool w8, int M, int nfrag, int panels, size_t ws_bytes) {
-    if (panels <= 0 || panels * 3 > 2 * num_cus() || panels > SPLIT_MAX_PANELS) return 1;
+    if (panels <= 0 || panels * 3 > 2 * num_cus() || panels > WS_MAX_TILES) return 1;
     const int fc = (!w8 && M <= 16) ? 16 : 8;  // fragments per chunk of the kernels launched for these shapes
     const int nchunk = (nfrag + fc - 1) / fc;
     const bool wide = panels * 2 > num_cus();
     int S = wide ? 3 : (num_cus() / panels < 4 ? num_cus() / panels : 4);
     const int shortest = wide ? 10 : 4;
     while (S > 1 && ((nchunk + S - 1) / S < shortest || (S - 1) * ((nchunk + S - 1) / S) >= nchunk ||
-                     SPLIT_COUNTER_BYTES + (size_t)panels * S * 4096 > ws_bytes))
+                     WS_COUNTER_BYTES + (size_t)panels * S * 4096 > ws_bytes))
         S = wide ? 1 : S - 1;
     return S;
 }
@@ -1419,9 +1413,10 @@ static int fragment_x_bytes(int wk) { return wk == 2 ? 128 : (wk == 1 ? 64 : 32)
 size_t skinny_workspace_bytes(int wk, int M, int K, int n0, int n1) {
     const int panels = ((n1 + 31) >> 5) - (n0 >> 5);
     const int S = chunk_slices(wk != 0, M, fragments(wk, K), panels, ~(size_t)0);
-    return S > 1 ? SPLIT_COUNTER_BYTES + (size_t)panels * S * 4096 : 0;
+    return S > 1 ? WS_COUNTER_BYTES + (size_t)panels * S * 4096 : 0;
 }
 
+// dynamic LDS of skinny_stream_kernel: x + the zero row, reused afterwards as the reduction scratch (32 KiB per panel)
 static inline int stream_lds_bytes(int xbytes, int np) { return xbytes > 32768 * np ? xbytes : 32768 * np; }
 
 // int8 x int8 at M <= 32 can use the decode kernels if x is 16-byte aligned: the streaming form if its rows are whole 16-byte
@@ -1564,8 +1559,8 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
     s.stamps = nullptr;
     const int panels = ((n1 + 31) >> 5) - (n0 >> 5);
 #ifdef MMX_STAMPS
-    if (rq && rq->ws && rq->ws_bytes >= SPLIT_COUNTER_BYTES + ((size_t)96 << 20) + (size_t)64 * 2 * panels)
-        s.stamps = reinterpret_cast<uint64_t*>(rq->ws + SPLIT_COUNTER_BYTES + ((size_t)96 << 20));
+    if (rq && rq->ws && rq->ws_bytes >= WS_COUNTER_BYTES + ((size_t)96 << 20) + (size_t)64 * 2 * panels)
+        s.stamps = reinterpret_cast<uint64_t*>(rq->ws + WS_COUNTER_BYTES + ((size_t)96 << 20));
 #endif
     const bool pairs = (ep.steps & MMX_PP_SILU_GATE) != 0;
     if (wk == 3) {
@@ -1577,7 +1572,7 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
             const int ksl3 = (rq && rq->ws && rq->k_splits == 0) ? chunk_slices(true, M, s.nfrag, panels, rq->ws_bytes) : 1;
             if (ksl3 > 1) {
                 s.ws_cnt = reinterpret_cast<uint32_t*>(rq->ws);
-                s.ws_part = rq->ws + SPLIT_COUNTER_BYTES;
+                s.ws_part = rq->ws + WS_COUNTER_BYTES;
                 s.kslices = ksl3;
                 char name_[40];
                 snprintf(name_, sizeof name_, "skinny_chunk_i8_ksplit%d", ksl3);
@@ -1621,7 +1616,7 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
             const int ksl4 = (rq && rq->ws && rq->k_splits == 0) ? chunk_slices(true, M, s.nfrag, panels, rq->ws_bytes) : 1;
             if (ksl4 > 1) {  // few panels, a workspace at hand: K in slices as for the other weight types
                 s.ws_cnt = reinterpret_cast<uint32_t*>(rq->ws);
-                s.ws_part = rq->ws + SPLIT_COUNTER_BYTES;
+                s.ws_part = rq->ws + WS_COUNTER_BYTES;
                 s.kslices = ksl4;
                 char name_[40];
                 snprintf(name_, sizeof name_, "skinny_chunk_w4_ksplit%d", ksl4);
@@ -1808,7 +1803,7 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
         dim3 grid(panels);
         if (ksl > 1) {
             s.ws_cnt = reinterpret_cast<uint32_t*>(rq->ws);
-            s.ws_part = rq->ws + SPLIT_COUNTER_BYTES;
+            s.ws_part = rq->ws + WS_COUNTER_BYTES;
             s.kslices = ksl;
             grid = dim3(panels, ksl);
             char name_[40];

@@ -31,12 +31,9 @@ struct UnpackedArgs {
 constexpr int STRIP = 128;           // columns of a workgroup
 constexpr int RED_ROW = STRIP + 4;   // floats; the pad spreads 16 rows over the banks
 constexpr int MAX_SLICES = 16;
-constexpr int MAX_TILES = 4096;      // counters at the head of a workspace
-constexpr size_t COUNTER_BYTES = (size_t)MAX_TILES * 4;
-// What the front ends allocate once per stream.  No launch asks for more or uses more: a larger answer would replace the
-// stream's buffer, which a graph captured earlier may still write to, and the slices of a call would depend on its history.
-// (It takes slices from wide results only, where the CUs have strips enough: 128 x 8192 x 50304 334 us unsplit, 338 in four.)
-constexpr size_t STANDARD_WORKSPACE_BYTES = ((size_t)64 << 20) + ((size_t)16 << 10);
+// No launch asks for more than WS_STANDARD_BYTES or uses more: a larger answer would replace the stream's buffer, which a graph
+// captured earlier may still write to, and the slices of a call would depend on its history.  (That takes slices from wide
+// results only, where the CUs have strips enough: 128 x 8192 x 50304 334 us unsplit, 338 in four.)
 
 // 16 bytes from any address (the hardware takes them at any)
 typedef u32x4 __attribute__((aligned(1))) u32x4_any;
@@ -310,7 +307,7 @@ static int row_tiles(int M, int row_blocks) { return (M + 16 * row_blocks - 1) /
 static int tile_count(int M, int N, int row_blocks) { return (N + STRIP - 1) / STRIP * row_tiles(M, row_blocks); }
 static size_t slice_sums(int tiles, int row_blocks) { return (size_t)tiles * row_blocks * 16 * STRIP * 4; }
 static size_t workspace_of(int M, int N, Share h) {
-    return h.slices > 1 ? COUNTER_BYTES + slice_sums(tile_count(M, N, h.row_blocks), h.row_blocks) * h.slices : 0;
+    return h.slices > 1 ? WS_COUNTER_BYTES + slice_sums(tile_count(M, N, h.row_blocks), h.row_blocks) * h.slices : 0;
 }
 
 // The least of an estimate in us, fitted to 20 000 timings (K 32 ... 11008, N 64 ... 65536, M 1 ... 256, both orders of B, every
@@ -323,7 +320,7 @@ static size_t workspace_of(int M, int N, Share h) {
 // Fewer rows per workgroup mean more of them and less for each to do one after another, more rows fewer passes over B:
 // 64 x 512 x 512 from [K, N] 10.3 us in workgroups of 64 rows, 5.8 of 16; 64 x 512 x 65536 22 and 38.
 static Share choose_share(int M, int K, int N, int transpose, size_t ws_bytes) {
-    if (ws_bytes > STANDARD_WORKSPACE_BYTES) ws_bytes = STANDARD_WORKSPACE_BYTES;
+    if (ws_bytes > WS_STANDARD_BYTES) ws_bytes = WS_STANDARD_BYTES;
     static const struct { int row_blocks; float first, step, next; } forms[2][3] = {
         {{1, 0.6f, 1.85f, 1.35f}, {2, 4.9f, 1.55f, 4.6f}, {4, 7.9f, 1.05f, 6.1f}}, {{1, 0.2f, 3.8f, 0.9f}, {2, 0.8f, 5.2f, 3.0f}, {4, 7.2f, 2.45f, 10.6f}}};
     const int steps = transpose ? (K + 63) / 64 : K / 32, cus = num_cus();
@@ -338,7 +335,7 @@ static Share choose_share(int M, int K, int N, int transpose, size_t ws_bytes) {
         int steps_before = 0;
         for (int S = 1; S <= MAX_SLICES; S++) {
             const int per_slice = (steps + S - 1) / S, wave_steps = (per_slice + nw - 1) >> nw_log2;
-            if (S > 1 && (2 * per_slice < nw || tiles > MAX_TILES || 2 * tiles * S > 5 * cus || COUNTER_BYTES + slice_bytes * S > ws_bytes)) break;
+            if (S > 1 && (2 * per_slice < nw || tiles > WS_MAX_TILES || 2 * tiles * S > 5 * cus || WS_COUNTER_BYTES + slice_bytes * S > ws_bytes)) break;
             if (wave_steps == steps_before || (S - 1) * per_slice >= steps) continue;  // (nothing gained by the slice, or nothing in it)
             steps_before = wave_steps;
             const float work_us = f.step * wave_steps;
@@ -378,7 +375,7 @@ bool unpacked_takes(int M, int K, int N, int64_t lda, int64_t ldb, int transpose
 }
 
 size_t unpacked_workspace_bytes(int M, int K, int N, int transpose) {
-    return workspace_of(M, N, choose_share(M, K, N, transpose, STANDARD_WORKSPACE_BYTES));
+    return workspace_of(M, N, choose_share(M, K, N, transpose, WS_STANDARD_BYTES));
 }
 
 int launch_unpacked(const void* A, int64_t lda, const void* B, int64_t ldb, int transpose, int M, int K, int N, const Epilogue& ep, char* ws,
@@ -394,7 +391,7 @@ int launch_unpacked(const void* A, int64_t lda, const void* B, int64_t ldb, int 
     s.S = h.slices;
     s.units = tile_count(M, N, h.row_blocks) * s.S;
     s.cnt = reinterpret_cast<uint32_t*>(ws);
-    s.parts = ws ? ws + COUNTER_BYTES : nullptr;
+    s.parts = ws ? ws + WS_COUNTER_BYTES : nullptr;
     s.ep = ep;
     const dim3 grid((s.units + 7) / 8 * 8);
     char name[64];

@@ -23,8 +23,6 @@ namespace {
 
 constexpr int AUX_SC1 = 16;  // cache policy operand of the buffer instructions: device scope
 constexpr int MAX_SLICES = 4;
-constexpr int MAX_TILES = 4096;  // of a launch with slices: one arrival counter each
-constexpr size_t COUNTER_BYTES = (size_t)MAX_TILES * 4;
 
 struct WaveRingArgs {
     const char* A;
@@ -369,8 +367,8 @@ WaveRingPlan choose_form(int type, int M, int K, int Ncols, bool pairs, int k_sp
         if (tiles > (1 << 24)) continue;
         for (int S = 1; S <= MAX_SLICES; S *= 2) {
             const int per_slice = (stages + S - 1) / S;
-            if (S > 1 && (pairs || k_splits == 1 || tiles * S > 2 * cus || tiles > MAX_TILES || (S - 1) * per_slice >= stages ||
-                          COUNTER_BYTES + (size_t)tiles * S * c.mb * c.np * 4096 > ws_bytes)) continue;
+            if (S > 1 && (pairs || k_splits == 1 || tiles * S > 2 * cus || tiles > WS_MAX_TILES || (S - 1) * per_slice >= stages ||
+                          WS_COUNTER_BYTES + (size_t)tiles * S * c.mb * c.np * 4096 > ws_bytes)) continue;
             const int on_cu = (int)((tiles * S + cus - 1) / cus), rounds = (int)((tiles * S + cus * c.per_cu - 1) / (cus * c.per_cu));
             const float kib = (float)per_slice * (c.mb * 4.0f + c.np * (type == W8 ? 2.0f : 4.0f));
             const float pull = on_cu * kib * c.us_per_kib, memory = 0.134f * mb_read;
@@ -420,7 +418,7 @@ int launch_wave_ring(int type, const void* A, int64_t lda, const void* Bp, int M
     g.units = tiles_m * tiles_n * p.slices;
     g.units_per_xcd = (g.units + 7) / 8;
     g.ws_cnt = reinterpret_cast<uint32_t*>(rq.ws);
-    g.ws_part = rq.ws ? rq.ws + COUNTER_BYTES : nullptr;
+    g.ws_part = rq.ws ? rq.ws + WS_COUNTER_BYTES : nullptr;
     g.ep = ep;
     auto launch = [&](auto type_c) {
         constexpr int T = decltype(type_c)::value;
@@ -444,7 +442,7 @@ int64_t wave_ring_workspace_bytes(int type, int M, int K, int Ncols, bool pairs,
     if (p.form < 0 || p.us >= 0.9f * tiles_us) return -1;
     const Form& c = FORMS[p.form];
     if (p.slices == 1) return 0;
-    return (int64_t)(COUNTER_BYTES + (size_t)((M + 32 * c.mb - 1) / (32 * c.mb)) * (((Ncols + 31) / 32 + c.np - 1) / c.np) * p.slices * c.mb * c.np * 4096);
+    return (int64_t)(WS_COUNTER_BYTES + (size_t)((M + 32 * c.mb - 1) / (32 * c.mb)) * (((Ncols + 31) / 32 + c.np - 1) / c.np) * p.slices * c.mb * c.np * 4096);
 }
 
 }  // namespace mmx
