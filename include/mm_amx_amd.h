@@ -147,18 +147,18 @@ int mmx_dequant_packed(const void* packed_i8, int K, int N, void* packed_bf16, v
  * A is [M, K] row-major with row stride lda_bytes; Bpacked comes from mmx_repack_b for the
  * FULL [K, N]; n0 % 32 == 0, 0 <= n0 < n1 <= N.  M <= 32 takes the bandwidth-bound decode
  * kernel (the M<=16 paths of the reference and weight_compression/fc16m.cpp:451-502), larger
- * M the MFMA tile kernel. */
+ * M the MFMA tile kernels. */
 int mmx_gemm(int a_dtype, int b_dtype, const void* A, int64_t lda_bytes, const void* Bpacked, int M, int K,
              int N, int n0, int n1, const mmx_epilogue* ep, void* stream);
 
 /* ---- the same product with K split over several workgroups per output tile ---------------------------------
  * AMX_MLP::Linear (tests/amx-mlp.cpp:560-593) gives each half of the K blocks of `down` to its own core and lets
  * the one that finishes last add the two fp32 partial results and round to bf16 (:648-682).  Here a tile's K range
- * is cut into k_splits slices of whole 512-byte blocks of K per row (256 bf16, the reference's K block; slice s
- * takes blocks [s*q, (s+1)*q), q = ceil(blocks / k_splits), so k_splits = 2 is the reference's partition), one
- * workgroup each; each parks its fp32 / int32 partial tile in `workspace`, and the workgroup that arrives last
- * adds them in slice order (so the result does not depend on the arrival order) and applies the post-op.  It
- * pays where a shape has fewer tiles than the GPU has CUs, or tiles bound by the bytes a CU can pull in.
+ * is cut into slices, one workgroup each; each parks its fp32 / int32 partial tile in `workspace`, and the workgroup
+ * that arrives last adds them in slice order (so the result does not depend on the arrival order) and applies the
+ * post-op.  A count of slices that is asked for cuts whole 512-byte blocks of K per row (256 bf16, the reference's K
+ * block; slice s takes blocks [s*q, (s+1)*q), q = ceil(blocks / k_splits), so k_splits = 2 is the reference's
+ * partition); with k_splits = 0 the library also chooses where to cut (its small tiles: 128-byte blocks).  It pays where a shape has fewer tiles than the GPU has CUs, or tiles bound by the bytes a CU can pull in.
  *   k_splits  0 = the library chooses (possibly no split), 1 = none, 2..4 = exactly that many slices
  *             (MMX_E_INVALID if K is too short or the workspace too small, MMX_E_UNSUPPORTED for M <= 32,
  *             SILU_GATE, unaligned A or K * sizeof(T) not a multiple of 128).  The decode kernels (M <= 32)
