@@ -434,7 +434,8 @@ int launch_wave_ring(int type, const void* A, int64_t lda, const void* Bp, int M
     return type == I8 ? launch(integral_constant<int, I8>{}) : (type == W8 ? launch(integral_constant<int, W8>{}) : launch(integral_constant<int, BF16>{}));
 }
 
-// Bytes of workspace the call above would use (0: no slices), or -1 if it would leave the call to the tile kernels.  (Rows of A that
+// Bytes of workspace the call above can use (0: no slices), or -1 if it would leave the call to the tile kernels.  Rows are counted in
+// whole 64s: an upper bound, and one answer for counts of rows in the same 64 that get the same form and slices.  (Rows of A that
 // are not aligned go to the masked pipeline there, which takes no slices.)
 int64_t wave_ring_workspace_bytes(int type, int M, int K, int Ncols, bool pairs, int k_splits, float tiles_us) {
     if (!wave_ring_can(type, K, true)) return -1;
@@ -442,7 +443,7 @@ int64_t wave_ring_workspace_bytes(int type, int M, int K, int Ncols, bool pairs,
     if (p.form < 0 || p.us >= 0.9f * tiles_us) return -1;
     const Form& c = FORMS[p.form];
     if (p.slices == 1) return 0;
-    return (int64_t)(WS_COUNTER_BYTES + (size_t)((M + 32 * c.mb - 1) / (32 * c.mb)) * (((Ncols + 31) / 32 + c.np - 1) / c.np) * p.slices * c.mb * c.np * 4096);
+    return (int64_t)(WS_COUNTER_BYTES + (size_t)((M + 63) / 64 * 2 / c.mb) * (((Ncols + 31) / 32 + c.np - 1) / c.np) * p.slices * c.mb * c.np * 4096);
 }
 
 }  // namespace mmx
