@@ -22,8 +22,9 @@ int launch_gemm_tiles_bf16(const void* A, int64_t lda, const void* Bp, int M, in
     }
 }
 
-// What the plan for this shape is estimated to take, in us, for operands the ring pipeline takes (fitted to the 840 shapes of the
-// small tiles' rule: 15 % rms; gate/up pairs take 1.19 times as long as the products of their size).
+// What the plan for this shape is estimated to take, in us, for operands the ring pipeline takes: a line fitted to the shapes of
+// the small tiles' rule (15 % rms; gate/up pairs take 1.19 times as long as the products of their size; a K tail, whose loads are
+// a trip to memory of their own, is not priced).
 float plan_us(int elesz, bool w8, int M, int K, int Ncols, uint32_t steps, const SplitRequest& rq_in) {
     const int64_t kbytes = (int64_t)K * elesz;
     const bool pairs = (steps & MMX_PP_SILU_GATE) != 0;

@@ -1056,7 +1056,7 @@ static inline int slice_kiters(int nk, int S) { return 4 * (((nk + 3) / 4 + S - 
 struct Plan {
     TileCfg t;
     int S;
-    float cycles;  // the model's estimate
+    float cycles;  // the model's estimate, without the margin that a K split has to win by
 };
 
 // Pick the tile shape and the number of K slices that minimise a model of the launch's duration, in
@@ -1112,8 +1112,8 @@ static inline Plan choose_plan(int M, int Ncols, int nk, bool need_pairs, bool w
             // at its power limit; 128x128 in two slices against 128x64: 2 % fewer cycles, 8 % lower clock)
             // (not for int8 x int8: on a sweep of forced tiles the plan without the margin is within 4 % of the best tile on
             // all 24 shapes, with it 9-16 % behind on 4096 x 4096 at M = 192-256 and 11008 x 4096 at M = 384-512)
-            const float t = (float)per_cu * (3700.0f + loop + epi + split) * (S > 1 && !int8_a ? 1.15f : 1.0f);
-            if (t < best) { best = t; pick = {{c.bm, c.bn}, S, t}; }
+            const float t = (float)per_cu * (3700.0f + loop + epi + split), margin = S > 1 && !int8_a ? 1.15f : 1.0f;
+            if (t * margin < best) { best = t * margin; pick = {{c.bm, c.bn}, S, t}; }
         }
     }
     return pick;

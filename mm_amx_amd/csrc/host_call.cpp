@@ -2,7 +2,7 @@
 // entry points, as CPython functions (module mm_amx_amd._host_call).
 //
 // What bounds a small product is the host: the same checks as Python statements, the descriptor as a ctypes structure, the query
-// of the workspace and the call through ctypes took 9.7 us for 256 x 256 x 256, under 4 us of which are on the device; 4.6 now.
+// of the workspace and the call through ctypes took 9.7 us for 256 x 256 x 256, under 4 us of which are on the device; 4.7 now.
 // (One decode row over 512 x 512 int4 weights 9.2 -> 4.2, a 64 x 512 x 512 layer with a bias 10.2 -> 5.2.)  The functions below
 // take the calls that are regular in every respect - tensors of exactly torch's own type on one GPU, the current one, everything
 // large enough - and leave all others to the Python form (they return None, and have done nothing), which accepts them or says

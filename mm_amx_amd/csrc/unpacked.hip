@@ -356,6 +356,9 @@ bool unpacked_can(int M, int K, int N, int64_t lda, int64_t ldb, int transpose) 
 // call: from [K, N] 8192 x 8192 at M = 1 / 64 / 256 73 / 73 / 90 -> 27 / 37 / 84 us, 4096 x 4096 at M = 16 / 128 24 / 28 -> 13 / 20,
 // 512 x 640 at M = 64 / 128 9.7 / 9.6 -> 5.9 / 7.4; from [N, K] 8192 x 8192 at M = 1 / 64 / 128 69 / 69 / 74 -> 32 / 37 / 54,
 // 4096 x 4096 at M = 16 / 128 24 / 28 -> 12 / 23, 512 x 640 at M = 64 / 128 9.1 / 9.4 -> 7.1 / 8.7.
+// (The product behind a packing ran on the tile kernels when this was measured.  With the small tiles behind it, over 260 shapes of
+// 33 to 256 rows the way taken is 1.03 of the better one on average: level from [K, N], 1.05 and 1.08 from [N, K] for 65 to 128
+// and 129 to 256 rows, at most 1.6, 140 x 608 x 4448 15.2 against 9.5 us: profiles/unpacked_against_packing.txt.)
 // Over 4032 shapes (K 32 ... 11008, N 64 ... 131072, M 1 ... 256) the way taken is on average 0.70 of packing, at most 1.15 of it
 // (a microsecond, 1 x 4096 x 256 from [N, K] 8.4 and 9.5).  Packing is the faster way
 //   where many workgroups of 64 rows have little to multiply (96 x 64 x 65536 15.7 against 16.2 us, from [N, K], whose form takes
