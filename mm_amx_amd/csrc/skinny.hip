@@ -9,6 +9,8 @@
 // (exact: |w| <= 128 has at most 8 significant bits, as in include/kernels_amx.hpp:490-506) or int4 -> bf16
 // (the reference has no int4 dequant, only a byte-copying stand-in: weight_compression/wcompress.hpp:90-134).
 // K is split across the wavefronts of a workgroup; partial 32x32 blocks are summed through LDS.
+#include <cstddef>
+
 #include "common.hpp"
 
 namespace mmx {
@@ -36,8 +38,9 @@ struct SkinnyArgs {
     int nfrag;    // 1 KiB fragments per panel that hold weights (what the panel is padded with behind them is zero and not read)
     int npanels;  // panels in Wp
     int n0, n1;
-    int x_vec_ok;  // rows of x start on 16 bytes
-    int x_direct;  // ... and are whole pieces of 16 bytes: they can go to LDS without passing through registers
+    // 1: rows of x start on 16 bytes; 2: and are whole pieces of 16 bytes, so that they can go to LDS without passing through
+    // registers.  (Eight numbers: with nine the post-op ends in a third cache line of arguments, 0.16 us of a launch of 2.8.)
+    int x_rows;
     int xpitch;    // bytes of a row of x in LDS: nfrag fragments' worth, zero behind its end
     Epilogue ep;
     // K split of the chunked kernel (kslices > 1): slice blockIdx.y walks its share of the chunks, parks its sums in
@@ -47,6 +50,7 @@ struct SkinnyArgs {
     int kslices;
     uint64_t* stamps;  // instrumented build only (-DMMX_STAMPS): 64 bytes per workgroup for its phase stamps, or null
 };
+static_assert(offsetof(SkinnyArgs, ws_part) <= 128, "what every launch reads of its arguments is two cache lines");
 
 // Development aid, compiled in with -DMMX_STAMPS only: thread 0 of workgroup blockIdx.x records the wall clock (100 MHz,
 // slots 0 and 7) or the shader clock (the others) at a few points of the workgroup's life.
@@ -281,7 +285,7 @@ template <int NW, bool WHOLE>
 __device__ __forceinline__ void stage_x(const SkinnyArgs& s, char* xs, int row_bytes, int pitch, int zero_off, int tid, int wave) {
     const int lane = tid & 63, real_bytes = s.M * pitch;
     const uint32_t lds_base = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)xs);
-    if (WHOLE || s.x_direct) {
+    if (WHOLE || s.x_rows == 2) {
         for (int off = wave * 1024; off < real_bytes; off += NW * 1024) {
             int bo = off + lane * 16;
             bo = bo < real_bytes ? bo : real_bytes - 16;
@@ -319,8 +323,8 @@ __device__ __forceinline__ void stage_x(const SkinnyArgs& s, char* xs, int row_b
     for (int c = tid * 16; c < pitch; c += NW * 64 * 16) *reinterpret_cast<u32x4*>(xs + zero_off + c) = u32x4{0u, 0u, 0u, 0u};
 }
 
-// The fully general form: what the kernels below leave - rows of x shorter than 16 bytes, and gate/up pairs over compressed
-// weights whose x does not fit in LDS.
+// The fully general form: rows of x shorter than 16 bytes, gate/up pairs over compressed weights whose x does not fit in LDS, and
+// aligned rows with a short K tail, for which staging x costs more than it saves (short_tail).
 // WK: weights are bf16 (0), int8 (1) or int4 (2); a 1 KiB fragment is 32 columns x 16, 32 or 64 of k
 template <int WK, int NP>
 __global__ __launch_bounds__(512) void skinny_kernel(const SkinnyArgs s) {
@@ -363,16 +367,16 @@ __global__ __launch_bounds__(512) void skinny_kernel(const SkinnyArgs s) {
             }
             if constexpr (W4) {
                 const int k0 = 64 * f + 32 * g32;
-                xa[u] = load_x8(xrow, k0, s.K, live && f < f_end, s.x_vec_ok);
-                xb[u] = load_x8(xrow, k0 + 8, s.K, live && f < f_end, s.x_vec_ok);
-                xc[u] = load_x8(xrow, k0 + 16, s.K, live && f < f_end, s.x_vec_ok);
-                xd[u] = load_x8(xrow, k0 + 24, s.K, live && f < f_end, s.x_vec_ok);
+                xa[u] = load_x8(xrow, k0, s.K, live && f < f_end, s.x_rows);
+                xb[u] = load_x8(xrow, k0 + 8, s.K, live && f < f_end, s.x_rows);
+                xc[u] = load_x8(xrow, k0 + 16, s.K, live && f < f_end, s.x_rows);
+                xd[u] = load_x8(xrow, k0 + 24, s.K, live && f < f_end, s.x_rows);
             } else if constexpr (W8) {
                 const int k0 = 32 * f + 16 * g32;
-                xa[u] = load_x8(xrow, k0, s.K, live && f < f_end, s.x_vec_ok);
-                xb[u] = load_x8(xrow, k0 + 8, s.K, live && f < f_end, s.x_vec_ok);
+                xa[u] = load_x8(xrow, k0, s.K, live && f < f_end, s.x_rows);
+                xb[u] = load_x8(xrow, k0 + 8, s.K, live && f < f_end, s.x_rows);
             } else {
-                xa[u] = load_x8(xrow, 16 * f + 8 * g32, s.K, live && f < f_end, s.x_vec_ok);
+                xa[u] = load_x8(xrow, 16 * f + 8 * g32, s.K, live && f < f_end, s.x_rows);
             }
         }
 #pragma unroll
@@ -496,8 +500,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 }
 
 // Read in place of what lies behind the end of K, where a repeat of its end would meet zeros on the other side of a product:
-// zero times an infinity is NaN.
-static __device__ __align__(1024) char zero_fragment[2048];
+// zero times an infinity is NaN.  (hidden: its address is computed then and not loaded from a table, 0.2 us of a small launch;
+// not const: the compiler would know what a load gives and choose behind it instead, see Rows.)
+__device__ __attribute__((visibility("hidden"))) __align__(1024) char zero_fragment[2048];
 
 // ---- chunked variant for aligned operands whose x does not fit in LDS, many rows (8 < M <= 32) ------
 // K is walked in chunks of 8*FPW fragments; in a chunk every wave multiplies FPW fragments of each
@@ -516,8 +521,8 @@ static __device__ __align__(1024) char zero_fragment[2048];
 // get zero weights and a zero x (a repeat of the row's end might be infinite, and zero times that is NaN).
 // WK: weights are bf16 (0), int8 (1) or int4 (2), 3: int8 weights and int8 activations (int32 sums);
 // XD: 16-byte x loads per thread per chunk (8 KiB of x each)
-// Where the rows of x end.  Behind the end of aligned rows the loads go to zeros: int4 11008 x 4096 at M = 16 / 32 12.7 / 14.9 us
-// -> 12.9 / 14.9, bf16 2624 x 8300 at M = 32 16.1 -> 16.3.  (Zeros put in place of what was loaded took up to 7 %, branches around
+// Where the rows of x end.  Behind the end of aligned rows the loads go to zeros: int4 11008 x 4096 at M = 16 / 32 12.5 / 14.8 us
+// -> 12.7 / 14.8, bf16 2624 x 8300 at M = 32 16.0 -> 16.0.  (Zeros put in place of what was loaded took up to 7 %, branches around
 // the products up to 15 %, the bytes moved as for unaligned rows 4 %: int4 30 x 2304 x 16192.)
 enum End {
     ON_CHUNK,   // with a chunk
@@ -685,7 +690,7 @@ static int launch_chunk(dim3 grid, const SkinnyArgs& s, hipStream_t st) {
     constexpr int lds = (2 * 8 * XD * 1024) > (8 * NP * 16 * 64 * 4) ? (2 * 8 * XD * 1024) : (8 * NP * 16 * 64 * 4);  // two buffers of x, later the reduction scratch
     void (*kern)(const SkinnyArgs) = skinny_chunk_kernel<WK, NP, FPW, XD, WIN, ON_CHUNK>;
     if constexpr (WK != 3) {  // (int8 x takes this kernel only if K fills its chunks: skinny_i8_eligible)
-        if (!s.x_vec_ok || s.K % (WK == 2 ? 256 : (WK == 0 ? 64 : 128))) kern = skinny_chunk_kernel<WK, NP, FPW, XD, WIN, ANYWHERE>;
+        if (!s.x_rows || s.K % (WK == 2 ? 256 : (WK == 0 ? 64 : 128))) kern = skinny_chunk_kernel<WK, NP, FPW, XD, WIN, ANYWHERE>;
         else if (s.K * 2 % chunk_row_bytes(WK, FPW)) kern = skinny_chunk_kernel<WK, NP, FPW, XD, WIN, IN_CHUNK>;
     }
     hipLaunchKernelGGL(kern, grid, dim3(512), lds, st, s);
@@ -701,7 +706,7 @@ enum Rows {
 // Over bf16 weights a load behind the end of a wavefront's share of K reads zero_fragment, in the first two forms.  (Zeros put in
 // place of the load's result took 1 to 8 % of the call, and the choice of address takes up to 5 % where nothing is repeated, hence
 // the third: 8 x 4096 x 11008 20.0 us, 20.5 with zeros behind the load, 20.7 with the address; 32 x 512 x 4096 4.3, 4.7 and 4.5.
-// Where loads are repeated: 8 x 320 x 4096 3.5 -> 3.7, 6 x 2600 x 4096 7.7 -> 7.7, 4 x 9600 x 2048 13.8 -> 13.4.)
+// Where loads are repeated: 8 x 320 x 4096 3.5 -> 3.6, 6 x 2600 x 4096 7.7 -> 7.8, 4 x 9600 x 2048 13.8 -> 13.3.)
 
 // ---- streaming variant for the smallest M -----------------------------------------------------------
 // When the activations fit in LDS the kernel is organised around one goal: have every byte of the
@@ -1531,6 +1536,19 @@ static StreamKernel stream_pair_kernel_for(int nfrag, bool whole) {
     return one ? skinny_stream_kernel<WK, 2, true, ANY_ROWS> : skinny_stream_kernel<WK, 2, false, ANY_ROWS>;
 }
 
+// Aligned rows of a K that ends inside the last group of fragments: whether K is so short that the general kernel, which reads x
+// beside the weights and has no barrier in front of them, is the faster one.  us, general / staged: bf16 6 x 72 x 15840 3.8 / 4.6,
+// 6 x 296 x 2144 3.4 / 3.7, 6 x 488 x 2144 3.8 / 3.7, 32 x 296 x 2144 4.0 / 4.3, 32 x 360 4.4 / 4.3; int8 weights 6 x 296 x 2144 3.7 / 4.2,
+// 6 x 808 4.2 / 4.4, 4 x 1192 5.4 / 5.2, 32 x 488 4.8 / 5.2, 32 x 552 5.4 / 5.2; int4 6 x 200 x 2144 3.7 / 4.3, 20 x 552 x 7673 4.8 / 5.1, 32 x 552 6.1 / 5.7 (with
+// panels for more than one workgroup per CU the staged form is ahead at any K: 6 x 200 x 15840 6.3 / 5.7).  Gate/up pairs: bf16
+// 6 x 200 x 15360 5.1 / 7.2, 6 x 488 6.9 / 8.0, 6 x 552 x 4288 6.1 / 5.8, 32 x 360 x 4288 6.0 / 6.0; int8 weights, whose two-panel form holds few
+// loads, 4 x 1000 x 4288 6.4 / 9.2, 4 x 2984 10.5 / 11.4, 4 x 4488 14.3 / 14.3; int4 6 x 200 x 4288 5.4 / 6.2, 6 x 808 6.8 / 7.0, 32 x 552 8.4 / 7.8.
+static bool short_tail(int wk, bool pairs, int M, int nfrag, int panels) {
+    if (pairs) return nfrag <= (wk == 0 ? (M <= 16 ? 32 : 22) : (wk == 1 ? 128 : (M <= 16 ? 16 : 8)));
+    if (wk == 2) return panels <= num_cus() && nfrag <= (M <= 16 ? 10 : 8);
+    return nfrag <= (M <= 16 ? (wk == 1 && M <= 8 ? 32 : 24) : (wk == 0 ? 20 : 16));
+}
+
 // wk: weights are bf16 (0), int8 (1) or int4 (2); 3: int8 weights and int8 activations
 int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int K, int N, int n0, int n1,
                   const Epilogue& ep, hipStream_t st, const SplitRequest* rq) {
@@ -1549,8 +1567,8 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
     s.npanels = (N + 31) / 32;
     s.n0 = n0;
     s.n1 = n1;
-    s.x_vec_ok = ((reinterpret_cast<uintptr_t>(x) & 15) == 0) && ((ldx & 15) == 0);
-    s.x_direct = s.x_vec_ok && row_bytes % 16 == 0;
+    const bool aligned = ((reinterpret_cast<uintptr_t>(x) & 15) == 0) && ((ldx & 15) == 0);
+    s.x_rows = aligned ? (row_bytes % 16 == 0 ? 2 : 1) : 0;
     s.xpitch = s.nfrag * fragment_x_bytes(wk);
     s.ep = ep;
     s.ws_part = nullptr;
@@ -1587,15 +1605,17 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
         hipLaunchKernelGGL(stream_kernel_for<3>(s.nfrag, s.xpitch == row_bytes, &unused), dim3(panels), dim3(512), stream_lds_bytes(zoff + s.xpitch, 1), st, s, zoff);
         return check_hip(hipGetLastError(), "skinny_stream_kernel launch");
     }
+    // whether x goes through LDS at all (int8 x always does)
+    const bool staged = row_bytes >= 16 && !(aligned && K % (wk == 0 ? 64 : (wk == 1 ? 128 : 256)) && short_tail(wk, pairs, M, s.nfrag, panels));
     if (wk == 2) {
         // int4 weights: the streaming kernel if x fits in LDS, else the chunked one
         if (pairs && (panels & 1)) return set_error(MMX_E_INVALID, "SILU_GATE needs an even number of 32-column panels");
         const int zoff = (M * s.xpitch + 1023) & ~1023;
         const int xb = zoff + s.xpitch;
-        if (row_bytes >= 16 && xb <= 46 * 1024) {
+        if (staged && xb <= 46 * 1024) {
             note_kernel(pairs ? "skinny_stream_w4_gateup" : "skinny_stream_w4");
             const int per_wave = (s.nfrag + 7) / 8;
-            const bool fills = s.x_direct && s.xpitch == row_bytes;
+            const bool fills = s.x_rows == 2 && s.xpitch == row_bytes;
             StreamKernel kern;  // (register sets sized to the share of K, as for the other weight types)
             if (pairs) kern = stream_pair_kernel_for<2>(s.nfrag, fills);  // gate and up panels side by side
             else if (per_wave <= 4) kern = fills ? skinny_stream_kernel<2, 1, true, WHOLE_ROWS, 4> : skinny_stream_kernel<2, 1, true, ANY_ROWS, 4>;
@@ -1606,12 +1626,12 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
             hipLaunchKernelGGL(kern, dim3(panels / np), dim3(512), stream_lds_bytes(xb, np), st, s, zoff);
             return check_hip(hipGetLastError(), "skinny_stream_kernel launch");
         }
-        if (pairs) {  // x too large for LDS: the general kernel
+        if (pairs) {  // the general kernel
             note_kernel("skinny_w4_gateup");
             hipLaunchKernelGGL((skinny_kernel<2, 2>), dim3(panels / 2), dim3(512), 0, st, s);
             return check_hip(hipGetLastError(), "skinny_kernel launch");
         }
-        if (row_bytes >= 16) {
+        if (staged) {
             // x too large for LDS: through LDS chunk by chunk (two buffers of 16 or 32 rows x 1 KiB)
             const int ksl4 = (rq && rq->ws && rq->k_splits == 0) ? chunk_slices(true, M, s.nfrag, panels, rq->ws_bytes) : 1;
             if (ksl4 > 1) {  // few panels, a workspace at hand: K in slices as for the other weight types
@@ -1632,7 +1652,7 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
         hipLaunchKernelGGL((skinny_kernel<2, 1>), dim3(panels), dim3(512), 0, st, s);
         return check_hip(hipGetLastError(), "skinny_kernel launch");
     }
-    const bool whole = K % (w8 ? 128 : 64) == 0 && s.x_vec_ok;  // K fills 128-byte groups of the weights, aligned rows of x
+    const bool whole = K % (w8 ? 128 : 64) == 0 && aligned;  // K fills 128-byte groups of the weights, aligned rows of x
     int zero_off = (M * s.xpitch + 1023) & ~1023;
     int xbytes = zero_off + s.xpitch;  // x, a gap up to the next KiB, one row of zeros
     if (whole && !w8 && !pairs && M >= 2 && M <= 4 && xbytes > 46 * 1024 && xbytes <= 128 * 1024 &&
@@ -1721,7 +1741,7 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
     // be resident): 80 KiB of x each (4096 x 11008 int8 GEMV at M = 5-8: 13.0-13.4 -> 11.5-12.0 us against the chunked
     // form; with one workgroup per CU, M = 12-16, it loses: 16.6-17.7 against 13.7-14.5 us).
     const bool bigx = !pairs && xbytes > 46 * 1024 && xbytes <= 80 * 1024;
-    const bool fills = s.x_direct && s.xpitch == row_bytes;  // (WHOLE_ROWS)
+    const bool fills = s.x_rows == 2 && s.xpitch == row_bytes;  // (WHOLE_ROWS)
     int stream_index = 0;
     const StreamKernel stream_kernel = w8 ? stream_kernel_for<1>(s.nfrag, fills, &stream_index) : stream_kernel_for<0>(s.nfrag, fills, &stream_index);
     if (bigx) {
@@ -1729,7 +1749,7 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
         const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(stream_kernel), 80 * 1024, attr_done[w8 ? 1 : 0][stream_index]);
         if (rc) return rc;
     }
-    if (row_bytes >= 16 && (xbytes <= 46 * 1024 || bigx)) {
+    if (staged && (xbytes <= 46 * 1024 || bigx)) {
         // the activations fit in LDS: streaming variant
         if (pairs && (panels & 1)) return set_error(MMX_E_INVALID, "SILU_GATE needs an even number of 32-column panels");
         note_kernel(pairs ? (w8 ? "skinny_stream_w8_gateup" : "skinny_stream_bf16_gateup") : (w8 ? "skinny_stream_w8" : "skinny_stream_bf16"));
@@ -1756,7 +1776,7 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
             if constexpr (!(W8 && NP == 2)) {
                 if (halves) {  // (the rolling window holds fewer registers where two accumulator pairs need them)
                     int unused;
-                    hipLaunchKernelGGL((half_kernel_for<W8, NP>(s.nfrag, s.xpitch == row_bytes && s.x_direct, &unused)), dim3(2 * grid), dim3(256), xbytes, st, s, zero_off);
+                    hipLaunchKernelGGL((half_kernel_for<W8, NP>(s.nfrag, s.xpitch == row_bytes && s.x_rows == 2, &unused)), dim3(2 * grid), dim3(256), xbytes, st, s, zero_off);
                     return;
                 }
             }
@@ -1787,7 +1807,7 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
         return check_hip(hipGetLastError(), "skinny_stream_kernel launch");
     }
     // K split of the chunked kernel (a workspace at hand, the library left to choose)
-    const int ksl = (row_bytes >= 16 && !pairs && wk <= 1 && rq && rq->ws && rq->k_splits == 0)
+    const int ksl = (staged && !pairs && wk <= 1 && rq && rq->ws && rq->k_splits == 0)
                         ? chunk_slices(w8, M, s.nfrag, panels, rq->ws_bytes) : 1;
     if (whole && !w8 && !pairs && M <= 8 && ksl == 1) {
         // aligned, x too large for LDS, few rows, plain bf16 weights: every lane reads its own part of x
@@ -1796,7 +1816,7 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
         hipLaunchKernelGGL((skinny_direct_kernel<false, 1>), dim3(panels), dim3(512), 0, st, s);
         return check_hip(hipGetLastError(), "skinny_direct_kernel launch");
     }
-    if (row_bytes >= 16 && !(pairs && w8)) {
+    if (staged && !(pairs && w8)) {
         // x too large for LDS, many rows: x goes through LDS chunk by chunk
         if (pairs && (panels & 1)) return set_error(MMX_E_INVALID, "SILU_GATE needs an even number of 32-column panels");
         note_kernel(pairs ? "skinny_chunk_bf16_gateup" : (w8 ? "skinny_chunk_w8" : "skinny_chunk_bf16"));

@@ -1,7 +1,7 @@
 """The decode kernels (M <= 32) at a K that ends inside the last fragments of the packed weights, and with rows of x of any
 length and alignment, against the oracle: every form that stages x (streaming, half panels, chunks with and without a K
 split, two panels at a time, gate/up pairs), remainders of 1 element to one less than a fragment; and that the general
-kernel is not what ran."""
+kernel is what ran for short rows that are aligned, and there alone."""
 import numpy as np
 import pytest
 import torch
@@ -41,11 +41,17 @@ def _operands(po, kind, M, K, N, seed):
 KW = {"bf16": {}, "w8": {"b_dtype": mx.I8}, "w4": {"b_dtype": mx.I4}, "i8": {}}
 
 
+def _short_tail(kind, M, K, stride):
+    """Aligned rows of x with a K so short that the general kernel is the faster one (up to 256 panels, no gate/up pairs)."""
+    k, group, few, many = {"bf16": (16, 64, 24, 20), "w8": (32, 128, 32 if M <= 8 else 24, 16), "w4": (64, 256, 10, 8)}[kind]
+    return (2 * (K if M == 1 else stride)) % 16 == 0 and K % group != 0 and -(-K // k) <= (few if M <= 16 else many)
+
+
 @pytest.mark.parametrize("M", [1, 4, 7, 32])
 @pytest.mark.parametrize("K", [8, 9, 15, 17, 63, 65, 96, 190, 1000, 1088, 1337])
 @pytest.mark.parametrize("kind", ["bf16", "w8", "w4", "i8"])
 def test_x_in_lds(po, kind, K, M):
-    """Short x: the streaming kernel, with every alignment of the rows."""
+    """Short x: the streaming kernel, with every alignment of the rows, and the general one where it is the faster one."""
     if kind == "i8":
         K = (K + 15) // 16 * 16   # (rows that are not whole 16-byte pieces go to the tile kernels)
     N = 100
@@ -54,7 +60,9 @@ def test_x_in_lds(po, kind, K, M):
     for pad in ((-K * es % 16) // es + 16 // es, 0, 3):
         C = torch.zeros((M, N), dtype=torch.int32 if kind == "i8" else torch.float32, device="cuda")
         mx.gemm(_in_nan((dev if kind == "i8" else dev_bf16)(x), pad), packed, N, mx.Epilogue(C), **KW[kind])
-        if kind != "i8" or pad != 3 or M == 1:
+        if kind != "i8" and _short_tail(kind, M, K, K + pad):
+            assert mx.last_kernel() == f"skinny_{kind}", mx.last_kernel()
+        elif kind != "i8" or pad != 3 or M == 1:
             if (M + 1) * K * es <= 40000:
                 assert mx.last_kernel().startswith(f"skinny_stream_{kind}"), mx.last_kernel()
             assert mx.last_kernel() not in ("skinny_bf16", "skinny_w8", "skinny_w4")
