@@ -13,6 +13,7 @@
 // us a launch, best of the tile kernels -> this: bf16 40 x 1024 x 1024 8.1 -> 4.0, 900 x 1600 x 256 9.2 -> 4.8, 512 x 1024 x 1024
 // 8.3 -> 5.2, 256 x 4096 x 4096 17.9 -> 16.4, 40 x 8192 x 1024 (four slices) 15.8 -> 7.0; gate/up pairs 100 x 1024 x 2 x 2048
 // 13.3 -> 6.0; int8 weights 256 x 1024 x 1024 10.7 -> 4.3; int8 256 x 2048 x 2048 8.5 -> 5.2.
+#include <cmath>
 #include <type_traits>
 
 #include "common.hpp"
@@ -346,25 +347,34 @@ namespace {
 struct Form {
     int mb, np, nw, per_cu;  // per_cu: workgroups that a CU holds
     float us_per_kib;        // pulled by one CU
+    // Over int8 weights (stages of fewer bytes, and the conversion) the chosen form's estimate is held against the tile kernels' times
+    // e^x, x = w8[0] + w8[1] ln(stages of a slice / 64) + w8[2] ln(workgroups on the busiest CU) + w8[3] ln(MB of A x MB of B / 400)
+    // + w8[4] with slices: fitted to 307 shapes near the line, on which the estimate was 7 to 16 % off, and is 4 to 9 so.
+    float w8[5];
 };
-constexpr Form FORMS[4] = {{1, 1, 8, 2, 0.0079f}, {1, 2, 8, 1, 0.0093f}, {2, 2, 8, 1, 0.0105f}, {2, 2, 4, 2, 0.0109f}};
+constexpr Form FORMS[4] = {{1, 1, 8, 2, 0.0079f, {0.81f, -0.19f, -0.22f, 0.18f, 0.0f}},
+                           {1, 2, 8, 1, 0.0093f, {0.50f, -0.15f, -0.185f, 0.135f, -0.10f}},
+                           {2, 2, 8, 1, 0.0105f, {0.39f, -0.255f, -0.10f, 0.115f, -0.045f}},
+                           {2, 2, 4, 2, 0.0109f, {0.46f, -0.245f, -0.27f, 0.12f, -0.095f}}};
 
-// The form is taken where its estimate is below this share of the tile kernels'.  Over 817 shapes, most of them near the line, both
-// estimates are 1.17 too small on average, within 9 and 10 %.  With the tile kernels' margin for a K split counted in theirs, and a
-// share of 0.9, 26 of the shapes were more than 3 % slower than on the tile kernels, up to 22 % (int8 weights 895 x 9760 x 1792
-// 51 -> 63 us), and 99 that could have been faster stayed there; now 12, up to 17 %, all of a K beyond 4800, and 88.
-constexpr float WIN = 0.93f;
+// The form is taken where its estimate is below this share of the tile kernels'.  Over 800 shapes whose two estimates are within 0.6 to
+// 1.35 of each other small tiles are taken on 594, at 0.77 of the tile kernels' time on average, 10 of them more than 3 % slower (at most
+// 14 %).  Without the corrections for int8 weights, here and in the tile kernels' estimate, and a share of 0.93, 119 of 700 such shapes
+// stayed with the tile kernels though small tiles were more than 3 % faster (up to 1.5 times), 52 with them; with the margin that a K split has
+// to win by counted in the tile kernels' estimate, int8 weights 895 x 9760 x 1792 went from 51 to 63 us.
+constexpr float WIN = 0.95f;
 
 struct WaveRingPlan {
     int form, slices;
     float us;
+    int on_cu;  // workgroups on the busiest CU
 };
 
 WaveRingPlan choose_form(int type, int M, int K, int Ncols, bool pairs, int k_splits, size_t ws_bytes) {
     const int cus = num_cus(), es = type == I8 ? 1 : 2, bs = type == BF16 ? 2 : 1;
     const int stages = (int)(((int64_t)K * es + 127) / 128), panels = (Ncols + 31) / 32;
-    const float mb_read = ((float)M * K * es + (float)K * Ncols * bs) * 1e-6f;
-    WaveRingPlan best = {-1, 1, 1e30f};
+    const float mb_a = (float)M * K * es * 1e-6f, mb_b = (float)K * Ncols * bs * 1e-6f, mb_read = mb_a + mb_b;
+    WaveRingPlan best = {-1, 1, 1e30f, 0};
     for (int f = 0; f < 4; f++) {
         const Form& c = FORMS[f];
         if (pairs && c.np != 2) continue;
@@ -380,8 +390,13 @@ WaveRingPlan choose_form(int type, int M, int K, int Ncols, bool pairs, int k_sp
             const float pull = on_cu * kib * c.us_per_kib, memory = 0.134f * mb_read;
             const float us = 2.5f + (pull > memory ? pull + 0.3f * memory : memory + 0.3f * pull) + 1.4f * (rounds - 1) +
                              (S > 1 ? 1.8f : 0.0f) + 0.43f * c.mb * c.np * on_cu;
-            if (us < best.us) best = {f, S, us};
+            if (us < best.us) best = {f, S, us, on_cu};
         }
+    }
+    if (type == W8 && best.form >= 0) {
+        const float* const w = FORMS[best.form].w8;
+        best.us *= expf(w[0] + w[1] * logf((stages + best.slices - 1) / best.slices * (1.0f / 64)) + w[2] * logf((float)best.on_cu) +
+                        w[3] * logf(mb_a * mb_b * (1.0f / 400)) + (best.slices > 1 ? w[4] : 0.0f));
     }
     return best;
 }
