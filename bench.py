@@ -34,8 +34,8 @@ PEAK_HBM_GBS = 8000.0       # MI355X HBM3E
 MEASURED_TRAFFIC = {
     "gemm_bf16_256x192_ring8w_out_bf16": {"bytes": (81709.6 * 2.000 + 27535.0 * 1.000) * 1024, "source": "mm_amx_amd/csrc/gemm_tile.hpp",
                                           "sha": "0f698a79075577e5"},
-    "skinny_stream_w8": {"bytes": (22137.1 * 2.000 + 21.5 * 1.000) * 1024, "source": "mm_amx_amd/csrc/skinny.hip", "sha": "fd882609fab96e73"},
-    "skinny_resident_w8_pair": {"bytes": (22616.5 * 2.000 + 344.0 * 1.000) * 1024, "source": "mm_amx_amd/csrc/skinny.hip", "sha": "fd882609fab96e73"},
+    "skinny_stream_w8": {"bytes": (22154.3 * 2.000 + 21.5 * 1.000) * 1024, "source": "mm_amx_amd/csrc/skinny.hip", "sha": "eac742926c040d29"},
+    "skinny_resident_w8_pair": {"bytes": (22616.5 * 2.000 + 344.0 * 1.000) * 1024, "source": "mm_amx_amd/csrc/skinny.hip", "sha": "eac742926c040d29"},
 }
 
 

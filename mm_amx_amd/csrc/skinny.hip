@@ -501,8 +501,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 
 // Read in place of what lies behind the end of K, where a repeat of its end would meet zeros on the other side of a product:
 // zero times an infinity is NaN.  (hidden: its address is computed then and not loaded from a table, 0.2 us of a small launch;
-// not const: the compiler would know what a load gives and choose behind it instead, see Rows.)
-__device__ __attribute__((visibility("hidden"))) __align__(1024) char zero_fragment[2048];
+// not const: the compiler would know what a load gives and choose behind it instead, where the loads then wait.)
+__device__ __attribute__((visibility("hidden"))) __align__(16) char zero_piece[16];
 
 // ---- chunked variant for aligned operands whose x does not fit in LDS, many rows (8 < M <= 32) ------
 // K is walked in chunks of 8*FPW fragments; in a chunk every wave multiplies FPW fragments of each
@@ -596,7 +596,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     do {                                                                                                       \
         _Pragma("unroll") for (int t = 0; t < XD; t++) {                                                       \
             if constexpr (END == IN_CHUNK)                                                                     \
-                xr[J][t] = *reinterpret_cast<const u32x4*>((C) * RB + xcol[t] < row_bytes ? xsrc[t] + (C) * RB + xcol[t] : zero_fragment); \
+                xr[J][t] = *reinterpret_cast<const u32x4*>((C) * RB + xcol[t] < row_bytes ? xsrc[t] + (C) * RB + xcol[t] : zero_piece); \
             else                                                                                               \
                 xr[J][t] = fetch16_in_row(xsrc[t], (C) * RB + xcol[t], row_bytes);                             \
         }                                                                                                      \
@@ -703,10 +703,19 @@ enum Rows {
     WHOLE_ROWS,  // rows of x are aligned and fill their last fragment
     NO_REPEATS,  // and the wavefronts' batches of loads hold their shares of K exactly (bf16 weights)
 };
-// Over bf16 weights a load behind the end of a wavefront's share of K reads zero_fragment, in the first two forms.  (Zeros put in
-// place of the load's result took 1 to 8 % of the call, and the choice of address takes up to 5 % where nothing is repeated, hence
-// the third: 8 x 4096 x 11008 20.0 us, 20.5 with zeros behind the load, 20.7 with the address; 32 x 512 x 4096 4.3, 4.7 and 4.5.
-// Where loads are repeated: 8 x 320 x 4096 3.5 -> 3.6, 6 x 2600 x 4096 7.7 -> 7.8, 4 x 9600 x 2048 13.8 -> 13.3.)
+// Over bf16 weights a load behind the end of a wavefront's share of K has to give zeros (a weight of an earlier fragment there may be
+// infinite), so the loads are buffer loads with the share as their range: behind it they give zeros and touch nothing.  us, a fragment
+// repeated / an address of zeros chosen per load / ranges: gate/up pairs 3 x 3200 x 4992 9.71 / 10.64 / 9.47, 1 x 1088 x 9728 9.19 / - / 7.60;
+// 3 x 3584 x 384 5.34 / 5.55 / 5.29, 4 x 7808 x 256 8.93 / 9.42 / 8.71; 3 x 256 x 608 3.28 / - / 3.37.  (Zeros chosen behind the load: 1 to 8 %.)
+// Where nothing is repeated ranges are 2 to 3 % behind at a short K (18 x 1536 x 10752 9.64 / - / 9.92), hence the third form.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t share_of_panel(const char* panel, int first, int most, int end, int bytes) {
+    const int left = end - first, n = left < most ? (left > 0 ? left : 0) : most;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(panel) + (int64_t)first * bytes, 0, n * bytes, 0x00020000);
+}
+__device__ __forceinline__ u32x4 load_of_share(__amdgpu_buffer_rsrc_t share, int at) {
+    constexpr int AUX_NT = 2;  // cache policy operand: as MMX_WLOAD
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(share, at, 0, AUX_NT));
+}
 
 // ---- streaming variant for the smallest M -----------------------------------------------------------
 // When the activations fit in LDS the kernel is organised around one goal: have every byte of the
@@ -724,7 +733,7 @@ enum Rows {
 template <int WK, int NP, bool ONE, int ROWS, int UW = 0>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void skinny_stream_kernel(const SkinnyArgs s, int zero_off) {
     constexpr bool W8 = WK == 1, W4 = WK == 2, I8A = WK == 3;  // 3: int8 weights AND int8 activations, int32 sums
-    constexpr bool WHOLE = ROWS != ANY_ROWS, ZEROS = WK == 0 && ROWS != NO_REPEATS;
+    constexpr bool WHOLE = ROWS != ANY_ROWS, RANGED = WK == 0 && ROWS != NO_REPEATS;
     // 4: int8 weights and ONE row of x without the matrix cores: every lane owns one column and half of a fragment's
     // k, v_dot2_f32_bf16 on the converted pairs, and one cross-lane add at the end.  Kept as the measured
     // counterpart of WK = 1 (option "decode_valu"); the post-op is the same code.
@@ -762,16 +771,18 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
         for (int v = 0; v < 16; v++) acc[p][v] = 0;
 
     // wave w multiplies fragments [w*per_wave, (w+1)*per_wave); indices past the end are clamped for the
-    // load (over bf16 weights: to zeros) and paired with the zero row of x
+    // load (over bf16 weights it gives zeros) and paired with the zero row of x
     const int per_wave = (s.nfrag + 7) / 8;
     const int f_begin = wave * per_wave;
     const int f_last = s.nfrag - 1;
     const char* wbase[NP];
+    __amdgpu_buffer_rsrc_t share[NP];
 #pragma unroll
     for (int p = 0; p < NP; p++) {
         int panel = panel_first + p;
         panel = (panel < panel_end && panel < s.npanels) ? panel : s.npanels - 1;  // columns past n1 are never stored
-        wbase[p] = s.Wp + (int64_t)panel * s.panel_stride + (ZEROS ? 0 : lane * 16);
+        wbase[p] = s.Wp + (int64_t)panel * s.panel_stride + lane * 16;
+        if constexpr (RANGED) share[p] = share_of_panel(s.Wp + (int64_t)panel * s.panel_stride, f_begin, per_wave, s.nfrag, 1024);
     }
     const char* zrow = xs + zero_off;
     const char* xrow = (VALU || l32 < s.M) ? xs + (VALU ? 0 : l32) * pitch : zrow;
@@ -782,12 +793,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 #define MMX_REQUEST(BT, UU)                                                                                     \
     do {                                                                                                        \
         int f_ = f_begin + (BT) * U + (UU);                                                                     \
-        const bool valid_ = (f_ - f_begin) < per_wave && f_ <= f_last; /* scalar */                             \
         f_ = f_ < f_last ? f_ : f_last;                                                                         \
         _Pragma("unroll") for (int p = 0; p < NP; p++) {                                                        \
-            const char* at_ = wbase[p] + (int64_t)f_ * 1024;                                                    \
-            if constexpr (ZEROS) at_ = (valid_ ? at_ : zero_fragment) + lane * 16;                              \
-            w[p][UU] = MMX_WLOAD(at_);                                                                          \
+            if constexpr (RANGED) w[p][UU] = load_of_share(share[p], ((BT) * U + (UU)) * 1024 + lane * 16);     \
+            else w[p][UU] = MMX_WLOAD(wbase[p] + (int64_t)f_ * 1024);                                           \
         }                                                                                                       \
     } while (0)
 #define MMX_MULTIPLY(BT, UU)                                                                                    \
@@ -1212,7 +1221,7 @@ __global__ __launch_bounds__(1024) void skinny_resident_pair_kernel(const Skinny
 template <bool W8, int NP, bool ONE, int ROWS, int U>  // U: loads per panel per wave in flight at once (1 KiB each)
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void skinny_half_kernel(const SkinnyArgs s, int zero_off) {
     constexpr int NW = 4;
-    constexpr bool WHOLE = ROWS != ANY_ROWS, ZEROS = !W8 && ROWS != NO_REPEATS;
+    constexpr bool WHOLE = ROWS != ANY_ROWS, RANGED = !W8 && ROWS != NO_REPEATS;
     __shared__ float red[NW][NP][16][64];
     extern __shared__ __attribute__((aligned(1024))) char xs[];  // [M][xpitch], then at zero_off a row of zeros
 
@@ -1252,18 +1261,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
         for (int v = 0; v < 16; v++) acc[p][0][v] = acc[p][1][v] = 0.0f;
 
     // wave w multiplies the fragment pairs [w*per_wave, (w+1)*per_wave); indices past the end are clamped
-    // for the load (over bf16 weights: to zeros) and paired with the zero row of x
+    // for the load (over bf16 weights it gives zeros) and paired with the zero row of x
     const int npairs = s.nfrag >> 1;
     const int per_wave = (npairs + NW - 1) / NW;
     const int u_begin = wave * per_wave;
     const int u_last = npairs - 1;
     const char* wbase[NP];
+    __amdgpu_buffer_rsrc_t share[NP];
     const int wlane = (l32 >> 4) * 1024 + (g32 * 32 + 16 * half + (l32 & 15)) * 16;
 #pragma unroll
     for (int p = 0; p < NP; p++) {
         int panel = panel_first + p;
         panel = (panel < panel_end && panel < s.npanels) ? panel : s.npanels - 1;  // columns past n1 are never stored
-        wbase[p] = s.Wp + (int64_t)panel * s.panel_stride + (ZEROS ? 0 : wlane);
+        wbase[p] = s.Wp + (int64_t)panel * s.panel_stride + wlane;
+        if constexpr (RANGED) share[p] = share_of_panel(s.Wp + (int64_t)panel * s.panel_stride, u_begin, per_wave, npairs, 2048);
     }
     const char* zrow = xs + zero_off;
     const char* xrow = l32 < s.M ? xs + l32 * pitch : zrow;
@@ -1272,12 +1283,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 #define MMX_REQUEST(BT, UU)                                                                                     \
     do {                                                                                                        \
         int u_ = u_begin + (BT) * U + (UU);                                                                     \
-        const bool valid_ = (u_ - u_begin) < per_wave && u_ <= u_last; /* scalar */                             \
         u_ = u_ < u_last ? u_ : u_last;                                                                         \
         _Pragma("unroll") for (int p = 0; p < NP; p++) {                                                        \
-            const char* at_ = wbase[p] + (int64_t)u_ * 2048;                                                    \
-            if constexpr (ZEROS) at_ = (valid_ ? at_ : zero_fragment) + wlane;                                  \
-            w[p][UU] = MMX_WLOAD(at_);                                                                          \
+            if constexpr (RANGED) w[p][UU] = load_of_share(share[p], ((BT) * U + (UU)) * 2048 + wlane);         \
+            else w[p][UU] = MMX_WLOAD(wbase[p] + (int64_t)u_ * 2048);                                           \
         }                                                                                                       \
     } while (0)
 #define MMX_MULTIPLY(BT, UU)                                                                                    \
@@ -1327,6 +1336,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
             for (int u = 0; u < U; u++) {
                 MMX_MULTIPLY(bt, u);
                 MMX_REQUEST(bt + 1, u);
+                // (x may be read ahead; left alone, the compiler puts off a batch's requests until all of the one before is multiplied)
+                if constexpr (RANGED) __builtin_amdgcn_sched_barrier(0x106);
             }
         }
 #pragma unroll
