@@ -175,3 +175,16 @@ def test_int8_with_a_count_of_slices_is_refused_as_ever(po):
     mx.gemm(dev(x), packed, N, mx.Epilogue(C))
     assert mx.last_kernel() == "skinny_stream_i8", mx.last_kernel()
     assert np.array_equal(host_bits(C), ref)
+
+
+@pytest.mark.parametrize("M,K,want", [(6, 1000, "skinny_stream_bf16_gateup"), (6, 1408, "skinny_stream_bf16_gateup"), (3, 3200, "skinny_half_bf16_gateup")])
+def test_infinite_weights_at_the_end_of_k_of_gate_up_pairs(M, K, want):
+    """As above for pairs: infinite weights of `up` in the last column, behind a finite gate."""
+    N = 64
+    gate, up = (torch.ones((N, K), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    up[:, K - 1] = float("inf")
+    C = torch.zeros((M, N), dtype=torch.float32, device="cuda")
+    x = torch.full((M, K), 2.0 ** -12, dtype=torch.bfloat16, device="cuda")
+    mx.gemm(x, mx.repack_gate_up(gate, up), 2 * N, mx.Epilogue(C, mx.PP_SILU_GATE))
+    assert mx.last_kernel().startswith(want), mx.last_kernel()
+    assert torch.isinf(C).all(), mx.last_kernel()
