@@ -577,7 +577,7 @@ def probe_read(buf, workgroups, kib_in_flight, sink, waves=8, blocked=False):
 
 def matvec(A, b, out=None):
     """c[M] = A[M,K] · b[K]; bf16 (c fp32) or int8 (c int32)."""
-    if _native is not None and type(out) is torch.Tensor and out.is_cuda:  # as in gemm()
+    if _native is not None and _initialised and type(out) is torch.Tensor:  # as in gemm()
         device = _current_device()
         rc = _native.matvec(A, b, out, device, _raw_stream(device)) if device in _initialised else None
         if rc is not None:
