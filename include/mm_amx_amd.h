@@ -109,6 +109,11 @@ int mmx_repack_gate_up(const void* w_gate, const void* w_up, int64_t ldw_bytes, 
  * absmax_scratch is a device uint32 the call uses as scratch. */
 int mmx_quantize_weights(const void* W, int64_t ldw_bytes, int rows, int cols, void* Wq, int64_t ldq_bytes,
                          float* scales_out, uint32_t* absmax_scratch, void* stream);
+/* The same with a scratch of scratch_bytes (contents do not matter before, and mean nothing after): from
+ * MMX_QUANTIZE_SCRATCH_BYTES on the maxima need no clearing launch and no atomics. */
+#define MMX_QUANTIZE_SCRATCH_BYTES 4096
+int mmx_quantize_weights_scratch(const void* W, int64_t ldw_bytes, int rows, int cols, void* Wq, int64_t ldq_bytes,
+                                 float* scales_out, uint32_t* scratch, size_t scratch_bytes, void* stream);
 
 /* The quantising half of repackB_1xL<int8_t, L> (weight_compression/fc16m.cpp:61-99), the way fc16m makes its int8
  * weights (:123, :630-649 with quantize_i8_scale, :51): q = trunc(bf16_rne(float(w) * scale)) per element - the
@@ -118,6 +123,9 @@ int mmx_quantize_weights(const void* W, int64_t ldw_bytes, int rows, int cols, v
  * replaced by mmx_repack_b on Wq, and the kernels' per-tensor dequant scale is 1 / scale (:280). */
 int mmx_quantize_weights_scaled(const void* W, int64_t ldw_bytes, int rows, int cols, float scale, void* Wq,
                                 int64_t ldq_bytes, void* stream);
+/* mmx_repack_b of that result (transpose = 0: W is [K, N]) in one pass, without the matrix of bytes in between; packed
+ * receives mmx_packed_b_bytes(MMX_I8, K, N) bytes. */
+int mmx_quantize_pack_scaled(const void* W, int64_t ldw_bytes, int K, int N, float scale, void* packed, void* stream);
 
 /* int4 weight compression.  The reference only times a stand-in that copies bytes
  * (weight_compression/wcompress.hpp:90-134, README.md:216-244: "we haven't found efficient instructions to

@@ -308,13 +308,8 @@ inline PackedB<T> repackB_1xL(const tensor2D<bfloat16>& Bi, float scale = 1.0f, 
         check(mmx_repack_b(MMX_BF16, Bi.data, Bi.stride, K, N, 0, p.data, stream), "repackB_1xL");
         return p;
     }
-    void* q = nullptr;  // the quantised matrix in source order, between the two kernels only
-    const size_t qbytes = static_cast<size_t>(K) * static_cast<size_t>(N);
-    check_hip(hipMalloc(&q, qbytes > 0 ? qbytes : 1), "repackB_1xL: hipMalloc");
-    std::shared_ptr<void> hold(q, [](void* x) { (void)hipFree(x); });
-    check(mmx_quantize_weights_scaled(Bi.data, Bi.stride, K, N, scale, q, N, stream), "repackB_1xL: quantise");
-    check(mmx_repack_b(MMX_I8, q, N, K, N, 0, p.data, stream), "repackB_1xL: pack");
-    check_hip(hipStreamSynchronize(stream), "repackB_1xL");  // (the temporary is freed on return)
+    check(mmx_quantize_pack_scaled(Bi.data, Bi.stride, K, N, scale, p.data, stream), "repackB_1xL");
+    check_hip(hipStreamSynchronize(stream), "repackB_1xL");
     return p;
 }
 
@@ -494,9 +489,9 @@ struct Matmul<bfloat16, int8_t, float> {
         if (!constB || !internalBI8) {
             tensor2D<int8_t> Wq(matB.dims[0], matB.dims[1]);
             device_vector<float> scales(2);
-            device_vector<uint32_t> scratch(1);
-            check(mmx_quantize_weights(matB.data, matB.stride, matB.dims[0], matB.dims[1], Wq.data, Wq.stride, scales.data,
-                                       scratch.data, stream),
+            device_vector<uint32_t> scratch(MMX_QUANTIZE_SCRATCH_BYTES / 4);
+            check(mmx_quantize_weights_scratch(matB.data, matB.stride, matB.dims[0], matB.dims[1], Wq.data, Wq.stride, scales.data,
+                                               scratch.data, MMX_QUANTIZE_SCRATCH_BYTES, stream),
                   "Matmul<bf16,int8>: quantize");
             internalBI8 = repackB_1x2(Wq, transposeB, stream);
             check_hip(hipStreamSynchronize(stream), "Matmul<bf16,int8>: sync");  // Wq and scales are read back / freed

@@ -17,7 +17,8 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB_PATH = os.environ.get("MMX_LIB_PATH") or os.path.join(_HERE, "libmm_amx_amd.so")
 
 EXPORTS = ["mmx_last_error", "mmx_init", "mmx_packed_b_bytes", "mmx_repack_b", "mmx_repack_gate_up",
-           "mmx_quantize_weights", "mmx_quantize_weights_scaled", "mmx_quantize_pack_int4", "mmx_dequant_packed", "mmx_gemm", "mmx_gemm_splitk",
+           "mmx_quantize_weights", "mmx_quantize_weights_scratch", "mmx_quantize_weights_scaled", "mmx_quantize_pack_scaled",
+           "mmx_quantize_pack_int4", "mmx_dequant_packed", "mmx_gemm", "mmx_gemm_splitk",
            "mmx_gemm_splitk_static", "mmx_gemm_workspace_bytes", "mmx_gemm_unpacked_workspace_bytes", "mmx_gemm_unpacked",
            "mmx_gemm_u8_scratch_bytes", "mmx_gemm_u8", "mmx_matvec_u8", "mmx_matvec", "mmx_mlp", "mmx_mlp_splitk", "mmx_set_tile",
            "mmx_set_option", "mmx_last_kernel"]
@@ -26,6 +27,7 @@ BENCH_EXPORTS = ["mmx_time_gemm", "mmx_probe_mfma", "mmx_probe_read"]
 
 # a workspace of this size serves every shape when the library chooses the K split itself (include/mm_amx_amd.h)
 WORKSPACE_BYTES = (64 << 20) + (16 << 10)
+QUANTIZE_SCRATCH_BYTES = 4096  # MMX_QUANTIZE_SCRATCH_BYTES
 
 
 class MmxError(RuntimeError):
@@ -61,7 +63,8 @@ def _host_module(l):
         return None
     _host_call.bind(*(C.cast(f, C.c_void_p).value for f in (
         l.mmx_gemm_splitk, l.mmx_gemm_workspace_bytes, l.mmx_gemm_unpacked, l.mmx_gemm_unpacked_workspace_bytes, l.mmx_matvec,
-        l.mmx_packed_b_bytes, l.mmx_repack_b, l.mmx_quantize_weights, l.mmx_quantize_weights_scaled, l.mmx_quantize_pack_int4)))
+        l.mmx_packed_b_bytes, l.mmx_repack_b, l.mmx_quantize_weights_scratch, l.mmx_quantize_weights_scaled, l.mmx_quantize_pack_int4,
+        l.mmx_quantize_pack_scaled)))
     return _host_call
 
 
@@ -82,6 +85,9 @@ def lib():
         l.mmx_repack_gate_up.argtypes = [C.c_void_p, C.c_void_p, C.c_int64, C.c_int, C.c_int, C.c_void_p, C.c_void_p]
         l.mmx_quantize_weights.argtypes = [C.c_void_p, C.c_int64, C.c_int, C.c_int, C.c_void_p, C.c_int64, C.c_void_p,
                                            C.c_void_p, C.c_void_p]
+        l.mmx_quantize_weights_scratch.argtypes = [C.c_void_p, C.c_int64, C.c_int, C.c_int, C.c_void_p, C.c_int64, C.c_void_p,
+                                                   C.c_void_p, C.c_size_t, C.c_void_p]
+        l.mmx_quantize_pack_scaled.argtypes = [C.c_void_p, C.c_int64, C.c_int, C.c_int, C.c_float, C.c_void_p, C.c_void_p]
         l.mmx_quantize_weights_scaled.argtypes = [C.c_void_p, C.c_int64, C.c_int, C.c_int, C.c_float, C.c_void_p, C.c_int64,
                                                   C.c_void_p]
         l.mmx_quantize_pack_int4.argtypes = [C.c_void_p, C.c_int64, C.c_int, C.c_int, C.c_int, C.c_void_p, C.c_void_p,
@@ -265,9 +271,9 @@ def quantize_weights(W):
         raise MmxError("W must be bf16")
     Wq = torch.empty(W.shape, dtype=torch.int8, device=W.device)
     scales = torch.empty(2, dtype=torch.float32, device=W.device)
-    scratch = torch.empty(1, dtype=torch.int32, device=W.device)
-    _check(lib().mmx_quantize_weights(W.data_ptr(), _row_stride_bytes(W), W.shape[0], W.shape[1], Wq.data_ptr(),
-                                      _row_stride_bytes(Wq), scales.data_ptr(), scratch.data_ptr(), _stream()))
+    scratch = torch.empty(QUANTIZE_SCRATCH_BYTES // 4, dtype=torch.int32, device=W.device)
+    _check(lib().mmx_quantize_weights_scratch(W.data_ptr(), _row_stride_bytes(W), W.shape[0], W.shape[1], Wq.data_ptr(),
+                                              _row_stride_bytes(Wq), scales.data_ptr(), scratch.data_ptr(), QUANTIZE_SCRATCH_BYTES, _stream()))
     return Wq, scales
 
 
@@ -285,6 +291,21 @@ def quantize_weights_scaled(W, scale):
     _check(lib().mmx_quantize_weights_scaled(W.data_ptr(), _row_stride_bytes(W), W.shape[0], W.shape[1], float(scale),
                                              Wq.data_ptr(), _row_stride_bytes(Wq), _stream()))
     return Wq
+
+
+def quantize_pack_scaled(W, scale):
+    """repack_b(quantize_weights_scaled(W, scale)) for W [K,N] in one pass over W."""
+    if _native is not None and _initialised:
+        made = _made(_native.quantize_pack_scaled, W, float(scale))
+        if made is not None:
+            return made
+    _dev(W, "W")
+    if W.dtype != torch.bfloat16 or W.dim() != 2:
+        raise MmxError("W must be a 2-D bf16 tensor")
+    K, N = W.shape
+    packed = torch.empty(packed_b_bytes(I8, K, N), dtype=torch.uint8, device=W.device)
+    _check(lib().mmx_quantize_pack_scaled(W.data_ptr(), _row_stride_bytes(W), K, N, float(scale), packed.data_ptr(), _stream()))
+    return packed
 
 
 def quantize_pack_int4(W, transpose=False):

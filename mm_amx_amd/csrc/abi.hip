@@ -90,7 +90,8 @@ int launch_gemm_x8(bool a_unsigned, bool b_unsigned, const void* A, int64_t lda,
 int launch_matvec_x8(bool a_unsigned, bool b_unsigned, const void* A, int64_t lda, const void* b, void* c, int M, int K, hipStream_t st);
 int launch_repack_gate_up(const void* wg, const void* wu, int64_t ldw, int K, int N, void* out, hipStream_t st);
 int launch_quantize(const void* W, int64_t ldw, int rows, int cols, void* Wq, int64_t ldq, float* scales_out,
-                    uint32_t* scratch, hipStream_t st);
+                    uint32_t* scratch, int words, hipStream_t st);
+int launch_scale_trunc_pack(const void* W, int64_t ldw, int K, int N, float scale, void* packed, hipStream_t st);
 int launch_quantize_scale_trunc(const void* W, int64_t ldw, int rows, int cols, float scale, void* Wq, int64_t ldq, hipStream_t st);
 int launch_dequant_packed(const void* in, int K, int N, void* out, hipStream_t st);
 int probe_mfma(bool i8, int random_operands, int iters, void* scratch, hipStream_t st, float* rate_out, float* mhz_out);
@@ -285,13 +286,29 @@ int mmx_repack_gate_up(const void* w_gate, const void* w_up, int64_t ldw_bytes, 
 
 int mmx_quantize_weights(const void* W, int64_t ldw_bytes, int rows, int cols, void* Wq, int64_t ldq_bytes, float* scales_out,
                          uint32_t* absmax_scratch, void* stream) {
-    if (!W || !Wq || !scales_out || !absmax_scratch) return set_error(MMX_E_INVALID, "mmx_quantize_weights: NULL pointer");
+    return mmx_quantize_weights_scratch(W, ldw_bytes, rows, cols, Wq, ldq_bytes, scales_out, absmax_scratch, sizeof(uint32_t), stream);
+}
+
+int mmx_quantize_weights_scratch(const void* W, int64_t ldw_bytes, int rows, int cols, void* Wq, int64_t ldq_bytes, float* scales_out,
+                                 uint32_t* scratch, size_t scratch_bytes, void* stream) {
+    if (!W || !Wq || !scales_out || !scratch) return set_error(MMX_E_INVALID, "mmx_quantize_weights: NULL pointer");
     if (rows <= 0 || cols <= 0 || ldw_bytes < (int64_t)cols * 2 || ldq_bytes < cols)
         return set_error(MMX_E_INVALID, "mmx_quantize_weights: bad shape or stride");
     if ((ldw_bytes & 1) || (reinterpret_cast<uintptr_t>(W) & 1) || (reinterpret_cast<uintptr_t>(scales_out) & 3) ||
-        (reinterpret_cast<uintptr_t>(absmax_scratch) & 3))
-        return set_error(MMX_E_INVALID, "mmx_quantize_weights: W, scales_out or absmax_scratch is not aligned to its element size");
-    return launch_quantize(W, ldw_bytes, rows, cols, Wq, ldq_bytes, scales_out, absmax_scratch, static_cast<hipStream_t>(stream));
+        (reinterpret_cast<uintptr_t>(scratch) & 3))
+        return set_error(MMX_E_INVALID, "mmx_quantize_weights: W, scales_out or the scratch is not aligned to its element size");
+    if (scratch_bytes < sizeof(uint32_t)) return set_error(MMX_E_INVALID, "mmx_quantize_weights: %zu bytes of scratch", scratch_bytes);
+    const int words = scratch_bytes < MMX_QUANTIZE_SCRATCH_BYTES || num_cus() > (int)(MMX_QUANTIZE_SCRATCH_BYTES / 4) ? 1 : (int)(MMX_QUANTIZE_SCRATCH_BYTES / 4);
+    return launch_quantize(W, ldw_bytes, rows, cols, Wq, ldq_bytes, scales_out, scratch, words, static_cast<hipStream_t>(stream));
+}
+
+int mmx_quantize_pack_scaled(const void* W, int64_t ldw_bytes, int K, int N, float scale, void* packed, void* stream) {
+    if (!W || !packed) return set_error(MMX_E_INVALID, "mmx_quantize_pack_scaled: NULL pointer");
+    if (K <= 0 || N <= 0 || ldw_bytes < (int64_t)N * 2) return set_error(MMX_E_INVALID, "mmx_quantize_pack_scaled: bad shape or stride");
+    if ((ldw_bytes & 1) || (reinterpret_cast<uintptr_t>(W) & 1))
+        return set_error(MMX_E_INVALID, "mmx_quantize_pack_scaled: W is not aligned to its element size");
+    if (reinterpret_cast<uintptr_t>(packed) & 15) return set_error(MMX_E_INVALID, "mmx_quantize_pack_scaled: packed buffer must be 16-byte aligned");
+    return launch_scale_trunc_pack(W, ldw_bytes, K, N, scale, packed, static_cast<hipStream_t>(stream));
 }
 
 int mmx_quantize_weights_scaled(const void* W, int64_t ldw_bytes, int rows, int cols, float scale, void* Wq, int64_t ldq_bytes,

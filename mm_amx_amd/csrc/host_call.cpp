@@ -29,9 +29,10 @@ unpacked_need_fn call_unpacked_need = nullptr;
 matvec_fn call_matvec = nullptr;
 decltype(&mmx_packed_b_bytes) call_packed_bytes = nullptr;
 decltype(&mmx_repack_b) call_repack = nullptr;
-decltype(&mmx_quantize_weights) call_quantize = nullptr;
+decltype(&mmx_quantize_weights_scratch) call_quantize = nullptr;
 decltype(&mmx_quantize_weights_scaled) call_quantize_scaled = nullptr;
 decltype(&mmx_quantize_pack_int4) call_quantize_int4 = nullptr;
+decltype(&mmx_quantize_pack_scaled) call_quantize_pack_scaled = nullptr;
 
 struct Leave {};  // not a regular call
 
@@ -278,9 +279,9 @@ PyObject* quantize(PyObject*, PyObject* const* a, Py_ssize_t count) {
         if (!unlocked([&] {
                 Wq = make({W.rows, W.cols}, at::kChar, *W.t);
                 scales = make({2}, at::kFloat, *W.t);
-                scratch = make({1}, at::kInt, *W.t);
+                scratch = make({MMX_QUANTIZE_SCRATCH_BYTES / 4}, at::kInt, *W.t);
                 rc = call_quantize(W.data, W.ld, W.rows, W.cols, Wq.mutable_data_ptr(), W.cols, static_cast<float*>(scales.mutable_data_ptr()),
-                                   static_cast<uint32_t*>(scratch.mutable_data_ptr()), stream);
+                                   static_cast<uint32_t*>(scratch.mutable_data_ptr()), MMX_QUANTIZE_SCRATCH_BYTES, stream);
             })) throw Leave();
         return rc ? PyLong_FromLong(rc) : Py_BuildValue("(NN)", THPVariable_Wrap(Wq), THPVariable_Wrap(scales));
     } catch (...) {
@@ -309,6 +310,27 @@ PyObject* quantize_scaled(PyObject*, PyObject* const* a, Py_ssize_t count) {
     }
 }
 
+// quantize_pack_scaled(W, scale, device, stream) -> packed
+PyObject* quantize_pack_scaled(PyObject*, PyObject* const* a, Py_ssize_t count) {
+    if (count != 4 || !call_quantize_pack_scaled) Py_RETURN_NONE;
+    try {
+        int device, rc = 0;
+        if (!whole_number(a[2], 0, 1 << 20, device) || !PyFloat_CheckExact(a[1])) throw Leave();
+        const Matrix W = matrix(a[0], device);
+        if (W.t->scalar_type() != at::kBFloat16) throw Leave();
+        const float scale = (float)PyFloat_AS_DOUBLE(a[1]);
+        void* const stream = stream_of(a[3]);
+        at::Tensor out;
+        if (!unlocked([&] {
+                out = make({(int64_t)call_packed_bytes(MMX_I8, W.rows, W.cols)}, at::kByte, *W.t);
+                rc = call_quantize_pack_scaled(W.data, W.ld, W.rows, W.cols, scale, out.mutable_data_ptr(), stream);
+            })) throw Leave();
+        return rc ? PyLong_FromLong(rc) : THPVariable_Wrap(out);
+    } catch (...) {
+        Py_RETURN_NONE;
+    }
+}
+
 // quantize_pack_int4(W, transpose, device, stream) -> (packed, deq)
 PyObject* quantize_pack_int4(PyObject*, PyObject* const* a, Py_ssize_t count) {
     if (count != 4 || !call_quantize_int4) Py_RETURN_NONE;
@@ -331,11 +353,11 @@ PyObject* quantize_pack_int4(PyObject*, PyObject* const* a, Py_ssize_t count) {
     }
 }
 
-// bind(addresses of the ten entry points, in the order below)
+// bind(addresses of the eleven entry points, in the order below)
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t count) {
-    constexpr int ENTRIES = 10;
+    constexpr int ENTRIES = 11;
     if (count != ENTRIES) {
-        PyErr_SetString(PyExc_TypeError, "bind takes ten addresses");
+        PyErr_SetString(PyExc_TypeError, "bind takes eleven addresses");
         return nullptr;
     }
     void* at[ENTRIES];
@@ -353,12 +375,13 @@ PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t count) {
     set(call_quantize);
     set(call_quantize_scaled);
     set(call_quantize_int4);
+    set(call_quantize_pack_scaled);
     Py_RETURN_NONE;
 }
 
 #define METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {METHOD(gemm), METHOD(gemm_unpacked), METHOD(matvec), METHOD(repack), METHOD(quantize), METHOD(quantize_scaled),
-                         METHOD(quantize_pack_int4), METHOD(bind), {nullptr, nullptr, 0, nullptr}};
+                         METHOD(quantize_pack_int4), METHOD(quantize_pack_scaled), METHOD(bind), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_call", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace

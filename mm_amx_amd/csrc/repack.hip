@@ -252,12 +252,14 @@ int launch_repack_gate_up(const void* wg, const void* wu, int64_t ldw, int K, in
 // ---- per-tensor weight compression ---------------------------------------------------------------
 __global__ void zero_u32_kernel(uint32_t* p) { *p = 0u; }
 
-// All three kernels of this section stream bf16 and are bound by memory: a lane takes 16 bytes (8 weights) at a time, four
-// such loads in flight.  A matrix whose rows
-// follow each other without a gap is walked as one row (the host passes rows = 1).
+// All three kernels of this section stream bf16 and are bound by memory: a lane takes 16 bytes (8 weights) at a time.  A matrix
+// whose rows follow each other without a gap is walked as one row (the host passes rows = 1).
 // (11008 x 4096 weights: two bytes per load and a 64-bit division per weight took 217 us for the maxima and 65 for the
-// quantisation; now 18 us, 5.1 TB/s read, and 25 us, 5.5 TB/s read and written; the scaled form 68 -> 30.)
-//   ROWS = false: blockIdx.y walks the rows, a lane's four loads lie along a row.
+// quantisation.)
+//   ROWS = false: blockIdx.y walks the rows, one load at a time: 4 MB of loads are in flight over the chip, which is what memory
+//   takes; with four loads in a row maxima, quantisation and packing took, launch to launch, 66.3 us for 11008 x 4096, 13.9 for
+//   1184 x 4160 and 19.7 for 3000 x 3000, now 61.4, 12.6 and 17.7 (two loads: 61.4, 13.5, 18.2; nontemporal loads and stores, twice
+//   as many workgroups, and quantising from the end that was read last are level or behind).
 //   ROWS = true, for rows with gaps that are too short to fill the four loads of a workgroup: 2^row_log2 lanes share a row, a
 //   lane's four loads are of four rows.  (Maxima and quantisation of rows with gaps, a row at a time -> shared out: 1000000 x 8
 //   4252 -> 17 us, 131072 x 128 518 -> 20, 16384 x 1024 67 -> 19, 4096 x 4096 31 -> 20, 4096 x 8192 46 -> 31.)
@@ -281,22 +283,20 @@ __device__ __forceinline__ void for_each_8_weights(const char* __restrict__ W, i
         const int64_t step = (int64_t)gridDim.x * THREADS;
         for (int r = blockIdx.y; r < rows; r += gridDim.y) {
             const char* const row = W + (int64_t)r * ldw;
-            for (int64_t i0 = (int64_t)blockIdx.x * THREADS + threadIdx.x; i0 * 8 < cols; i0 += step * QUANT_UNR) {
-                u32x4 v[QUANT_UNR];
-                if ((i0 + (QUANT_UNR - 1) * step) * 8 + 8 <= cols) {
-#pragma unroll
-                    for (int u = 0; u < QUANT_UNR; u++) v[u] = load16<2>(row + (i0 + u * step) * 16);
-#pragma unroll
-                    for (int u = 0; u < QUANT_UNR; u++) f(r, (i0 + u * step) * 8, v[u]);
-                } else {
-#pragma unroll
-                    for (int u = 0; u < QUANT_UNR; u++) {
-                        if ((i0 + u * step) * 8 >= cols) break;
-                        u32x4 w[1];
-                        load16_rows<2>(w, (i0 + u * step) * 16, cols * 2, [&](int) { return row; }, [&](int) { return true; });
-                        f(r, (i0 + u * step) * 8, w[0]);
-                    }
-                }
+            const int64_t first = (int64_t)blockIdx.x * THREADS + threadIdx.x, len = cols * 2;
+            if (len < 16) {  // (uniform)
+                u32x4 v[1];
+                load16_rows<2, SHORT_ROW>(v, first * 16, len, [&](int) { return row; }, [&](int) { return true; });
+                if (first * 8 < cols) f(r, first * 8, v[0]);
+                continue;
+            }
+            // One load instruction for the whole wavefront: with the row's last lane in a branch of its own, its load, into the
+            // same registers as the other lanes' load still in flight, delivered wrong bytes now and then.
+            for (int64_t i = first; i * 8 < cols; i += step) {
+                const int64_t at = i * 16, last = len - 16, from = at < last ? at : last;
+                u32x4 v = load16<2>(row + from);
+                if (from < at) v = settle16_in_row(v, (int)(at - from), 16);
+                f(r, i * 8, v);
             }
         }
     }
@@ -314,11 +314,12 @@ __device__ __forceinline__ void store_8_bytes(char* row, int64_t c, int64_t cols
     }
 }
 
-// max |w| over the matrix: the bit pattern of a non-negative float orders like an unsigned integer.  The workgroups'
-// atomics all meet at one address and take 10 ns each there, so there is one workgroup per CU, of 16 wavefronts (2048
-// workgroups of four: 4096 x 4096 weights in 27 us instead of 10).
+// max |w| over the matrix: the bit pattern of a non-negative float orders like an unsigned integer.
+// WORDS: every workgroup leaves its maximum in a word of its own, and the quantising kernel's workgroups take the largest.  Without
+// (a scratch of one word) the workgroups' atomics all meet at one address, cleared by a launch before, and take 10 ns each there, so
+// there is one workgroup per CU, of 16 wavefronts (2048 workgroups of four: 4096 x 4096 weights in 27 us instead of 10).
 constexpr int ABSMAX_THREADS = 1024;
-template <bool ROWS>
+template <bool ROWS, bool WORDS>
 __global__ __launch_bounds__(ABSMAX_THREADS) void absmax_kernel(const char* __restrict__ W, int64_t ldw, int rows, int64_t cols, int row_log2,
                                                                 uint32_t* out) {
     uint32_t m = 0;
@@ -340,15 +341,33 @@ __global__ __launch_bounds__(ABSMAX_THREADS) void absmax_kernel(const char* __re
     if (threadIdx.x == 0) {
 #pragma unroll
         for (int w = 1; w < ABSMAX_THREADS / 64; w++) m = of_wave[w] > m ? of_wave[w] : m;
-        if (m > __hip_atomic_load(out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(out, m);
+        if constexpr (WORDS) out[blockIdx.y * gridDim.x + blockIdx.x] = m;
+        else if (m > __hip_atomic_load(out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(out, m);
     }
 }
 
-// q = sat8(rne(w * (127/max))) (include/kernels_amx.hpp:508-523); scales_out = {127/max, max/127}
+// q = sat8(rne(w * (127/max))) (include/kernels_amx.hpp:508-523); scales_out = {127/max, max/127}; the maximum is that of `words` words
 template <bool ROWS>
 __global__ __launch_bounds__(256) void quantize_kernel(const char* __restrict__ W, int64_t ldw, int rows, int64_t cols, int row_log2,
-                                                       char* __restrict__ Wq, int64_t ldq, const uint32_t* absmax_bits, float* scales_out) {
-    const float amax = u2f(*absmax_bits);
+                                                       char* __restrict__ Wq, int64_t ldq, const uint32_t* __restrict__ absmax_bits, int words,
+                                                       float* __restrict__ scales_out) {
+    uint32_t bits;
+    if (words == 1) {
+        bits = *absmax_bits;
+    } else {
+        bits = 0;
+        for (int i = threadIdx.x; i < words; i += 256) bits = absmax_bits[i] > bits ? absmax_bits[i] : bits;
+        for (int off = 32; off > 0; off >>= 1) {
+            const uint32_t o = __shfl_xor(bits, off);
+            bits = o > bits ? o : bits;
+        }
+        __shared__ uint32_t of_wave[4];
+        if ((threadIdx.x & 63) == 0) of_wave[threadIdx.x >> 6] = bits;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < 4; w++) bits = of_wave[w] > bits ? of_wave[w] : bits;
+    }
+    const float amax = u2f(bits);
     const float q = 127 / amax;
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
         scales_out[0] = q;
@@ -369,39 +388,40 @@ static void one_row(int64_t ldw, int64_t ldq, int& rows, int64_t& cols) {
     if (ldw == cols * 2 && ldq == cols) cols *= rows, rows = 1;
 }
 
-// How the kernels above walk a matrix: QUANT_UNR loads per lane at a time, by at most `most` workgroups; with `spread` one load
-// per lane while there are fewer than two workgroups for every CU (a lane that works through four runs of eight weights by itself took 3.8 us
-// for 300 x 100, 3.3 with one; not for the maxima, whose workgroups cost an atomic each).  Rows with gaps that do not fill the
-// loads of one workgroup are shared out (ROWS): the fewest lanes, a power of two, that cover a row.
+// How the kernels above walk a matrix, by at most `most` workgroups.  Rows with gaps that are shorter than QUANT_UNR loads of a
+// workgroup are shared out (ROWS): the fewest lanes, a power of two, that cover a row, and QUANT_UNR rows per lane at a time; with
+// `spread` one while there are fewer than two workgroups for every CU (not for the maxima).
 struct QuantWalk {
     bool by_rows;
     int row_log2;
     dim3 grid;
 };
 static QuantWalk quantize_walk(int rows, int64_t cols, int threads, int most, bool spread) {
-    auto blocks = [&](int64_t n, int64_t per_load, int64_t others) {
-        const int64_t x = (n + per_load * QUANT_UNR - 1) / (per_load * QUANT_UNR), x1 = (n + per_load - 1) / per_load;
-        return spread && x * others < 2 * num_cus() ? (x1 < 2 * num_cus() ? x1 : 2 * num_cus()) : (x < most ? x : most);
-    };
     if (rows > 1 && cols < (int64_t)threads * 8 * QUANT_UNR) {
         int log2 = 0;
         while ((8 << log2) < cols && (1 << log2) < threads) log2++;
-        return {true, log2, dim3((unsigned)blocks(rows, threads >> log2, 1))};
+        const int64_t x1 = (rows + (threads >> log2) - 1) / (threads >> log2), x = (x1 + QUANT_UNR - 1) / QUANT_UNR;
+        return {true, log2, dim3((unsigned)(spread && x < 2 * num_cus() ? (x1 < 2 * num_cus() ? x1 : 2 * num_cus()) : (x < most ? x : most)))};
     }
-    const int gx = (int)blocks(cols, threads * 8, rows), gy = most / gx;
+    const int64_t x = (cols + (int64_t)threads * 8 - 1) / ((int64_t)threads * 8);
+    const int gx = (int)(x < most ? x : most), gy = most / gx;
     return {false, 0, dim3((unsigned)gx, (unsigned)(rows < gy ? rows : gy))};
 }
 
+// scratch: words > 1 means that many, at least as many as there are CUs
 int launch_quantize(const void* W, int64_t ldw, int rows, int cols_in, void* Wq, int64_t ldq, float* scales_out,
-                    uint32_t* scratch, hipStream_t st) {
+                    uint32_t* scratch, int words, hipStream_t st) {
     int64_t cols = cols_in;
     one_row(ldw, ldq, rows, cols);
     const QuantWalk m = quantize_walk(rows, cols, ABSMAX_THREADS, num_cus(), false), q = quantize_walk(rows, cols, 256, 2048, true);
-    hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, st, scratch);
-    hipLaunchKernelGGL(m.by_rows ? absmax_kernel<true> : absmax_kernel<false>, m.grid, dim3(ABSMAX_THREADS), 0, st, static_cast<const char*>(W),
-                       ldw, rows, cols, m.row_log2, scratch);
+    const int used = words > 1 ? (int)(m.grid.x * m.grid.y) : 1;
+    if (used > words) return set_error(MMX_E_INVALID, "quantize: %d words of scratch, %d needed", words, used);
+    if (words == 1) hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, st, scratch);
+    const auto absmax = words == 1 ? (m.by_rows ? absmax_kernel<true, false> : absmax_kernel<false, false>)
+                                   : (m.by_rows ? absmax_kernel<true, true> : absmax_kernel<false, true>);
+    hipLaunchKernelGGL(absmax, m.grid, dim3(ABSMAX_THREADS), 0, st, static_cast<const char*>(W), ldw, rows, cols, m.row_log2, scratch);
     hipLaunchKernelGGL(q.by_rows ? quantize_kernel<true> : quantize_kernel<false>, q.grid, dim3(256), 0, st, static_cast<const char*>(W), ldw,
-                       rows, cols, q.row_log2, static_cast<char*>(Wq), ldq, scratch, scales_out);
+                       rows, cols, q.row_log2, static_cast<char*>(Wq), ldq, scratch, used, scales_out);
     return check_hip(hipGetLastError(), "quantize kernels launch");
 }
 
@@ -436,6 +456,84 @@ int launch_quantize_scale_trunc(const void* W, int64_t ldw, int rows, int cols_i
     hipLaunchKernelGGL(q.by_rows ? quantize_scale_trunc_kernel<true> : quantize_scale_trunc_kernel<false>, q.grid, dim3(256), 0, st,
                        static_cast<const char*>(W), ldw, rows, cols, q.row_log2, scale, static_cast<char*>(Wq), ldq);
     return check_hip(hipGetLastError(), "quantize_scale_trunc_kernel launch");
+}
+
+// The same conversion and mmx_repack_b of its result in one pass over W [K, N]: every weight is read once and leaves as a byte of its
+// fragment, where quantising to a matrix of bytes and packing that moved each byte twice more, in a launch of its own.  A wavefront
+// takes 64 columns x 128 of k, the two 4 KiB units that repack_cols_kernel<1> makes of bytes: a lane reads 16 rows of 8 columns (a
+// load covers 8 whole lines), converts, transposes its 16 x 8 bytes in registers, and the wavefront's slots leave through LDS as
+// whole fragments.  Bound by memory (K x N, device time of the two launches -> of this one: 576 x 8640 8.1 + 3.9 -> 5.8 us, 800 x 9504
+// 10.9 + 5.5 -> 9.9; 4096 x 11008 27.1, 5.0 TB/s).
+__device__ __forceinline__ uint32_t scale_trunc_x4(uint32_t w01, uint32_t w23, float scale) {
+    const float w[4] = {u2f(w01 << 16), u2f(w01 & 0xffff0000u), u2f(w23 << 16), u2f(w23 & 0xffff0000u)};
+    uint32_t b[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        int i;  // (the instruction saturates and makes NaN 0, which the C++ conversion leaves undefined)
+        asm("v_cvt_i32_f32 %0, %1" : "=v"(i) : "v"(from_bf16(to_bf16(w[e] * scale))));
+        b[e] = (uint32_t)(i < -128 ? -128 : (i > 127 ? 127 : i)) & 0xffu;
+    }
+    return b[0] | b[1] << 8 | b[2] << 16 | b[3] << 24;
+}
+
+template <RowLength LEN>
+__global__ __launch_bounds__(64) void scale_trunc_pack_kernel(const char* __restrict__ W, int64_t ldw, int K, int N, float scale,
+                                                              char* __restrict__ out, int kunits, int npanels) {
+    __shared__ __attribute__((aligned(16))) u32x4 slots[512];
+    const int lane = threadIdx.x, ng = lane & 7, kg = lane >> 3;
+    const int ku = blockIdx.x % kunits, pg = blockIdx.x / kunits;
+    const int n = pg * 64 + ng * 8, k = ku * 128 + kg * 16;
+    u32x4 row[16];
+    if (pg * 64 + 64 <= N && ku * 128 + 128 <= K) {
+#pragma unroll
+        for (int e = 0; e < 16; e++) row[e] = load16<2>(W + (int64_t)(k + e) * ldw + (int64_t)n * 2);
+    } else {
+        load16_rows<2, LEN>(row, (int64_t)n * 2, (int64_t)N * 2, [&](int e) { return W + (int64_t)(k + e) * ldw; },
+                            [&](int e) { return k + e < K; });
+    }
+    auto put = [&](int j, u32x4 slot) {  // the slot of column n + j
+        const int col = ng * 8 + j;
+        const int at = ((col >> 5) * 4 + (kg >> 1)) * 64 + (kg & 1) * 32 + (col & 31);
+        slots[at ^ (((at >> 4) ^ (at >> 8)) & 15)] = slot;
+    };
+#pragma unroll
+    for (int h = 0; h < 2; h++) {  // four columns at a time
+        u32x4 s[4];
+#pragma unroll
+        for (int p = 0; p < 4; p++) {
+            uint32_t q[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) q[e] = scale_trunc_x4(row[4 * p + e][2 * h], row[4 * p + e][2 * h + 1], scale);
+            const uint32_t ab01 = __builtin_amdgcn_perm(q[1], q[0], 0x05010400u), ab23 = __builtin_amdgcn_perm(q[1], q[0], 0x07030602u);
+            const uint32_t xy01 = __builtin_amdgcn_perm(q[3], q[2], 0x05010400u), xy23 = __builtin_amdgcn_perm(q[3], q[2], 0x07030602u);
+            s[0][p] = __builtin_amdgcn_perm(xy01, ab01, 0x05040100u);
+            s[1][p] = __builtin_amdgcn_perm(xy01, ab01, 0x07060302u);
+            s[2][p] = __builtin_amdgcn_perm(xy23, ab23, 0x05040100u);
+            s[3][p] = __builtin_amdgcn_perm(xy23, ab23, 0x07060302u);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) put(4 * h + j, s[j]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < 2; p++) {
+        if (pg * 2 + p >= npanels) break;
+        char* const o = out + ((int64_t)(pg * 2 + p) * kunits + ku) * 4096 + lane * 16;
+#pragma unroll
+        for (int f = 0; f < 4; f++) {
+            const int at = (p * 4 + f) * 64 + lane;
+            *reinterpret_cast<u32x4*>(o + f * 1024) = slots[at ^ (((at >> 4) ^ (at >> 8)) & 15)];
+        }
+    }
+}
+
+int launch_scale_trunc_pack(const void* W, int64_t ldw, int K, int N, float scale, void* packed, hipStream_t st) {
+    const int kunits = (K + 127) / 128, npanels = (N + 31) / 32;
+    const int64_t blocks = (int64_t)((npanels + 1) / 2) * kunits;
+    if (blocks > 0x7fffffff) return set_error(MMX_E_INVALID, "weight matrix too large to pack in one launch");
+    hipLaunchKernelGGL(N < 8 ? scale_trunc_pack_kernel<SHORT_ROW> : scale_trunc_pack_kernel<LONG_ROW>, dim3((unsigned)blocks), dim3(64), 0, st,
+                       static_cast<const char*>(W), ldw, K, N, scale, static_cast<char*>(packed), kunits, npanels);
+    return check_hip(hipGetLastError(), "scale_trunc_pack_kernel launch");
 }
 
 // ---- packed int8 -> packed bf16 (exact) -------------------------------------------------------------

@@ -90,7 +90,7 @@ def repackB_1xL(Bi, dtype=torch.bfloat16, L_=2, scale=1.0):
             raise L.MmxError("repackB_1xL: a scale is for the int8 form only")
         return L.repack_b(Bi)
     if dtype == torch.int8:
-        return L.repack_b(L.quantize_weights_scaled(Bi, float(scale)))
+        return L.quantize_pack_scaled(Bi, float(scale))
     raise L.MmxError("repackB_1xL: T is bfloat16 or int8")
 
 

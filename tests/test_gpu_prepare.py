@@ -52,6 +52,40 @@ def test_quantisers_row_ends_and_gaps(po, rows, cols, gap):
     assert np.array_equal(host_bits(mx.quantize_weights_scaled(wide[:, :cols], 1234.5)), po.quantize_scale_trunc(W, 1234.5))
 
 
+@pytest.mark.parametrize("K", [1, 15, 16, 127, 128, 129, 300])
+@pytest.mark.parametrize("N", [1, 7, 8, 9, 31, 33, 64, 65, 130])
+def test_scaled_pack_is_quantised_then_packed(po, K, N):
+    """One pass over W against the two it stands for, at the edges of its units (64 columns x 128 of k), rows of any alignment."""
+    rng = np.random.default_rng(K * 1000 + N)
+    W = rng.integers(0, 65536, (K, N)).astype(np.uint16)  # any weight: infinite, NaN and denormal ones among them
+    wide = torch.full((K, N + 3), float("nan"), dtype=torch.bfloat16, device="cuda")
+    wide[:, 1:N + 1] = dev_bf16(W)
+    for scale in (30.0, 0.0, float("inf")):
+        want = po.repack(po.quantize_scale_trunc(W, scale), layout="mfma")
+        for B in (dev_bf16(W), wide[:, 1:N + 1]):
+            assert np.array_equal(host_bits(mx._lib.quantize_pack_scaled(B, scale)).view(np.uint8), want.view(np.uint8))
+
+
+def test_scaled_pack_of_every_bf16(po):
+    W = np.arange(65536).astype(np.uint16).reshape(512, 128)
+    for scale in (1.0, 127.0, 1e-3, 1e30, -2.5):
+        want = po.repack(po.quantize_scale_trunc(W, scale), layout="mfma")
+        assert np.array_equal(host_bits(mx.repackB_1xL(dev_bf16(W), torch.int8, 2, scale)).view(np.uint8), want.view(np.uint8))
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (300, 100), (4096, 1024), (70, 8193)])
+def test_quantisers_scratch_of_one_word(po, rows, cols):
+    """mmx_quantize_weights with the one word that its signature promises, filled with ones before the call."""
+    L, C = mx._lib, mx._lib.C
+    W = po.f32_to_bf16((np.random.default_rng(rows).standard_normal((rows, cols)) * 0.02).astype(np.float32))
+    Wd, got = dev_bf16(W), torch.empty((rows, cols), dtype=torch.int8, device="cuda")
+    scales, word = torch.empty(2, device="cuda"), torch.full((3,), -1, dtype=torch.int32, device="cuda")
+    assert L.lib().mmx_quantize_weights(Wd.data_ptr(), cols * 2, rows, cols, got.data_ptr(), cols, scales.data_ptr(), word.data_ptr() + 4, L._stream()) == 0
+    want, dq, q = po.quantize_weights(W)
+    assert np.array_equal(host_bits(got), want) and host_bits(scales).tolist() == [np.float32(q), np.float32(dq)]
+    assert host_bits(word)[[0, 2]].tolist() == [-1, -1]
+
+
 @pytest.mark.parametrize("rows,cols", [(1000000, 8), (131072, 128), (16384, 1024)])
 def test_gaps_between_short_rows_cost_little(rows, cols):
     """With a gap as long as the row up to twice the lines are read.  A workgroup to a row took 25 times as long as without
