@@ -24,8 +24,7 @@ int launch_gemm_tiles_bf16(const void* A, int64_t lda, const void* Bp, int M, in
 
 // What the plan for this shape is estimated to take, in us, for operands the ring pipeline takes: a line fitted to the shapes of
 // the small tiles' rule (15 % rms; gate/up pairs take 1.19 times as long as the products of their size, and products over int8
-// weights 1.1 times what the line gives, with and without a K split, 307 shapes, 5 % rms; a K tail, whose loads are a trip to memory
-// of their own, is not priced).
+// weights 1.1 times what the line gives, with and without a K split, 307 shapes, 5 % rms).
 float plan_us(int elesz, bool w8, int M, int K, int Ncols, uint32_t steps, const SplitRequest& rq_in) {
     const int64_t kbytes = (int64_t)K * elesz;
     const bool pairs = (steps & MMX_PP_SILU_GATE) != 0;
@@ -41,7 +40,7 @@ size_t plan_workspace_bytes(int elesz, bool w8, int M, int K, int Ncols, uint32_
     if (kbytes % 128 && (k_splits > 1 || kbytes < 128)) return 0;  // (a forced split of a K with a tail is refused)
     const SplitRequest rq = {k_splits, reinterpret_cast<char*>(256), ~(size_t)0};
     if (steps & MMX_PP_SILU_GATE) return 0;
-    const Plan p = choose_plan(M, Ncols, (int)(kbytes / 128), false, w8, kbytes % 128 ? 4 : 2, rq, elesz == 1);
+    const Plan p = choose_plan(M, Ncols, (int)((kbytes + 127) / 128), false, w8, kbytes % 128 ? 4 : 2, rq, elesz == 1);
     if (p.S <= 1) return 0;
     const size_t tiles = (size_t)((M + p.t.bm - 1) / p.t.bm) * ((Ncols + p.t.bn - 1) / p.t.bn);
     return WS_COUNTER_BYTES + tiles * p.S * p.t.bm * p.t.bn * 4;

@@ -18,7 +18,8 @@
 //           issued from inline asm into rings of LDS slots (A in whole 128-byte lines per row, B in
 //           half-stages of two fragments per panel), hand-scheduled against the MFMAs (see the
 //           comment at the pipeline);
-//   MODE 4  MODE 2 for a K that does not fill its last 128 bytes: whole k-iterations as there, the rest in a step of its own;
+//   MODE 4  MODE 2 for a K that does not fill its last 128 bytes, which are one more k-iteration: A through buffer loads,
+//           whose range gives zeros behind the end of a row;
 //   MODE 0  global -> VGPR -> LDS with 16-byte loads, two LDS stages, rows past M clamped to the
 //           last row: the fallback when A or the packed weights are too large for the 32-bit
 //           offsets MODE 2 addresses with, and a tested alternative;
@@ -182,7 +183,7 @@ struct Ring {
 // wave issues at under half the rate the SIMD executes them (ring pipeline only).
 template <typename TIn, int BM, int BN, int MODE, typename TOut, int SMAX, int NW = 4>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4, NW / 4))) void gemm_kernel(const GemmArgs g) {
-    static_assert(NW == 4 || (NW == 8 && MODE == 2), "eight wavefronts exist for the ring pipeline only");
+    static_assert(NW == 4 || (NW == 8 && (MODE == 2 || MODE == 4)), "eight wavefronts exist for the ring pipeline only");
     constexpr int NT = NW * 64;  // threads
     constexpr bool RING = MODE == 2 || MODE == 4;
     using MF = Mfma<TIn>;
@@ -421,6 +422,37 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
         const uint32_t lds_wave = __builtin_amdgcn_readfirstlane(
             (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)(smem + wave * 1024));
         const int last_hs = 2 * nk - 1, last_st = nk - 1;
+        // MODE 4.  A is read through a buffer descriptor (the rows' k from this slice on).  Of the last stage the 16-byte chunks that
+        // lie behind the end of their row are given an offset out of its range, which loads zeros; a lane's chunk is the same in all its
+        // loads.  A chunk that the row ends in is loaded whole (behind the last row the range ends, at the next whole dword, which
+        // cannot leave its page) and settle_last() zeroes the rest of it in LDS, once the stage is there.  In a step of its own behind
+        // the loop the tail was one more trip to memory, and only four tiles had the registers for it; before -> now: bf16
+        // 2000 x 1032 x 8000 69 -> 39.5 us, 2048 x 8160 x 8192 345 -> 214, 1500 x 4104 x 11008 191 -> 181, 700 x 520 x 3000 10.1 -> 9.8,
+        // int8 1000 x 1088 x 4096 11.7 -> 11.3, an MLP 600 x 2080 x 4160 76 -> 63.  (As the only way to load A this costs a K
+        // without a tail 1 to 6 %, 391 x 1024 x 3001 9.8 -> 10.4, and switching lanes off around its loads 9 %: the small tiles
+        // are bound by how fast a wavefront issues.)
+        constexpr uint32_t OUT_OF_RANGE = 0xFFFF0000u;  // (the host keeps A below that)
+        const i32x4 a_rsrc = {(int)(uint32_t)(uintptr_t)a_base, (int)((uint32_t)((uintptr_t)a_base >> 32) & 0xFFFFu),
+                              (int)(uint32_t)((((int64_t)(g.M - 1) * g.lda + g.kbytes + 3) & ~(int64_t)3) - (int64_t)kt0 * 128), 0x00020000};
+        const uint32_t k_left = (uint32_t)(g.kbytes - kt0 * 128);  // bytes of a row from this slice on
+        const uint32_t chunk_at = (uint32_t)(((tid & 7) ^ ((tid >> 4) & 7)) * 16);
+        const uint32_t out_of_last = chunk_at + (uint32_t)last_st * 128u < k_left ? 0u : OUT_OF_RANGE;
+        auto beyond = [&](int st) __attribute__((always_inline)) { return out_of_last & ~(uint32_t)((st - last_st) >> 31); };  // (st <= last_st)
+        const bool ends_in_chunk = (k_left & 15) && (kt0 + nk == g.nk);
+        auto settle_last = [&](int aslot) __attribute__((always_inline)) {  // (every wave is past the barrier that the stage is complete behind)
+            if (tid < BM) {
+                const int in_last = (int)(k_left - (uint32_t)last_st * 128u), keep = in_last & 15;
+                u32x4* const at = reinterpret_cast<u32x4*>(smem + aslot * A_ST + tid * 128 + (((in_last >> 4) ^ ((tid >> 1) & 7)) * 16));
+                u32x4 v = *at;
+#pragma unroll
+                for (int d = 0; d < 4; d++) {
+                    const int n = keep - 4 * d;  // bytes of this dword that stay
+                    v[d] = n >= 4 ? v[d] : (n <= 0 ? 0u : v[d] & ((1u << (8 * n)) - 1u));
+                }
+                *at = v;
+            }
+            __syncthreads();
+        };
 
         using std::integral_constant;
         typedef integral_constant<int, 0> c0;
@@ -444,6 +476,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
             uint32_t m0B, m0A;   // LDS destinations of this wave's B chunk 0 / A round 0
             const char* srcB;    // global sources (the lane offsets are boff / aoff)
             const char* srcA;
+            uint32_t kA, outA;   // MODE 4: bytes of K before the stage; OUT_OF_RANGE in a lane whose chunk of it is behind the end of the row, else 0
             uint32_t rdA, rdB;   // LDS byte offsets of this lane's first A / B fragment
         };
         // k-step KS (0/1) of half-stage h = 2 st + PAR; as/nas = A slot of this / the next stage, bs = B slot.
@@ -468,8 +501,15 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
             } else if constexpr (PART == 2) {
                 int st = (w + 1) >> 1;
                 st = st < last_st ? st : last_st;
-                n.srcA = a_base + (int64_t)st * 128;
-                asm volatile("" : "+s"(n.srcA));
+                if constexpr (MODE == 4) {
+                    n.kA = (uint32_t)st * 128u;
+                    n.outA = beyond(st);
+                    asm volatile("" : "+s"(n.kA));
+                    asm volatile("" : "+v"(n.outA));
+                } else {
+                    n.srcA = a_base + (int64_t)st * 128;
+                    asm volatile("" : "+s"(n.srcA));
+                }
             } else {
                 // A operand of k-step s (0..3 within the stage): position (2 s + g32) ^ ((row >> 1) & 7) of the row
                 if constexpr (KS == 0) {  // reads k-step 1 of this half-stage
@@ -491,6 +531,13 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
                 asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                              :
                              : "s"(kp.m0B), "v"(off), "s"(kp.srcB), "n"(Q * NT * 16)
+                             : "memory", "scc");
+            } else if constexpr (MODE == 4) {
+                const uint32_t off = aoff[HALF][Q - B_IT2] | kp.outA;
+                const i32x4 rsrc = a_rsrc;
+                asm volatile("s_add_u32 m0, %0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                             :
+                             : "s"(kp.m0A), "v"(off), "s"(rsrc), "s"(kp.kA), "n"((Q - B_IT2) * NT * 16)
                              : "memory", "scc");
             } else {
                 const uint32_t off = aoff[HALF][Q - B_IT2];
@@ -557,6 +604,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
             KParams kp;
             kp.m0A = lds_wave;
             kp.srcA = a_base;
+            kp.kA = 0;
+            kp.outA = beyond(0);
             static_for<0, A_IT2>([&](auto it_c) { dma(integral_constant<int, B_IT2 + decltype(it_c)::value>{}, c0{}, kp); });
             static_for<0, R>([&](auto w_c) {
                 constexpr int W = decltype(w_c)::value;
@@ -568,6 +617,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
                 kp.m0A = lds_wave + (((W + 1) >> 1) % RA) * A_ST + HALF * (BM / 2) * 128;
                 kp.srcB = b_base + (int64_t)hs * BP_HS;
                 kp.srcA = a_base + (int64_t)st * 128;
+                kp.kA = (uint32_t)st * 128u;
+                kp.outA = beyond(st);
                 static_for<0, (W < R - 1 ? NL : H)>([&](auto q_c) { dma(q_c, integral_constant<int, HALF>{}, kp); });
             });
         }
@@ -576,6 +627,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
         asm volatile("s_waitcnt vmcnt(%0)" : : "n"((R - 2) * NL + H) : "memory");  // window 0 and all before it have landed
         __syncthreads();
         MMX_STAMP(2);
+        if (MODE == 4 && ends_in_chunk && last_st == 0) settle_last(0);
         {
             const char* sA = smem + a_x0;
             const char* sB = smem + b_frag_off;
@@ -604,6 +656,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
             // (R-2) younger ones may still be in flight
             asm volatile("s_waitcnt vmcnt(%0)" : : "n"((R - 2) * NL) : "memory");
             __syncthreads();
+            if constexpr (MODE == 4 && PAR == 1)
+                if (__builtin_expect(ends_in_chunk && h + 1 == 2 * last_st, 0)) settle_last(nas);  // (the next k-step reads the last stage)
             __builtin_amdgcn_sched_barrier(0);
             // k-step 1: read k-step 0 of the next half-stage; first group of the loads of window h+R
             const int nbs = bs + 1 < R ? bs + 1 : 0;
@@ -631,61 +685,6 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
         } else {
             if (wave_u < NCLS0) ring(std::integral_constant<int, 0>{});
             else ring(std::integral_constant<int, 1>{});
-        }
-        // MODE 4: the part of K behind the last whole k-iteration, once: A through registers (its rows end inside the 128
-        // bytes) and the weights, whose padding is there, into the first slots of the rings; then four k-steps.  The trip to
-        // memory is not hidden behind anything, but it is one: the masked pipeline, which this replaces for aligned rows,
-        // waits for one per k-iteration (bf16 1064 x 3544 x 786 62 -> 27 us, 64 x 4104 x 4096 52 -> 14).  (A mode of its own:
-        // behind this branch the compiler keeps the accumulators twice, which the largest tiles have no registers for.)
-        if constexpr (MODE == 4) {
-            if (SMAX == 1 || kt0 + nk == g.nk) {
-                constexpr int AC = BM * 8 / NT, BC = (BN / 32) * (BP_IT / 16);
-                u32x4 ta[AC], tb[(BC + NT - 1) / NT];
-#pragma unroll
-                for (int it = 0; it < AC; it++) {
-                    const int row = (it * NT + tid) >> 3, chunk = (tid & 7) ^ ((row >> 1) & 7);
-                    const int grow = m0 + row < g.M ? m0 + row : g.M - 1;
-                    ta[it] = fetch16_in_row(g.A + (int64_t)grow * g.lda, g.nk * 128 + chunk * 16, g.kbytes);
-                }
-#pragma unroll
-                for (int it = 0; it < (BC + NT - 1) / NT; it++) {
-                    const int c = it * NT + tid;
-                    int panel = panel0 + c / (BP_IT / 16);
-                    panel = panel < g.npanels ? panel : g.npanels - 1;
-                    if (BC % NT == 0 || c < BC)
-                        tb[it] = *reinterpret_cast<const u32x4*>(g.Bp + (int64_t)panel * g.panel_stride + (int64_t)g.nk * BP_IT + (c % (BP_IT / 16)) * 16);
-                }
-                __syncthreads();  // every wave has finished with the rings (and its own re-fetched slots have landed)
-#pragma unroll
-                for (int it = 0; it < AC; it++)
-                    *reinterpret_cast<u32x4*>(smem + (it * NT + tid) * 16) =
-                        settle16_in_row(ta[it], g.nk * 128 + ((tid & 7) ^ ((((it * NT + tid) >> 3) >> 1) & 7)) * 16, g.kbytes);
-#pragma unroll
-                for (int it = 0; it < (BC + NT - 1) / NT; it++) {
-                    const int c = it * NT + tid, in = c % (BP_IT / 16);
-                    if (BC % NT == 0 || c < BC)
-                        *reinterpret_cast<u32x4*>(smem + B0 + (in / (BP_HS / 16)) * BH + (c / (BP_IT / 16)) * BP_HS + (in % (BP_HS / 16)) * 16) = tb[it];
-                }
-                __syncthreads();
-#pragma unroll
-                for (int s = 0; s < 4; s++) {
-                    const int chunk = W8 ? 4 * (s >> 1) + 2 * g32 + (s & 1) : 2 * s + g32;
-                    const char* sA = smem + (wm * WM + l32) * 128 + ((chunk ^ ((l32 >> 1) & 7)) * 16);
-                    const char* sB = smem + B0 + (s >> 1) * BH + wn * NJ * BP_HS + lane * 16;
-#pragma unroll
-                    for (int i = 0; i < MI; i++) fa[0][i] = *reinterpret_cast<const frag*>(sA + i * 32 * 128);
-#pragma unroll
-                    for (int j = 0; j < NJ; j++) {
-                        if constexpr (W8) {
-                            const u32x4 raw = *reinterpret_cast<const u32x4*>(sB + j * BP_HS);
-                            fb[0][j] = (s & 1) ? s8x8_to_bf16(raw[2], raw[3]) : s8x8_to_bf16(raw[0], raw[1]);
-                        } else {
-                            fb[0][j] = *reinterpret_cast<const frag*>(sB + j * BP_HS + (s & 1) * 1024);
-                        }
-                    }
-                    mma(fa[0], fb[0]);
-                }
-            }
         }
     } else {
     fetch(kt0);
@@ -1082,7 +1081,6 @@ static inline Plan choose_plan(int M, int Ncols, int nk, bool need_pairs, bool w
         if (wide_only && c.bn == 64) continue;                      // (no 64-column tile for int8 weights under bf16 A)
         if (need_pairs && c.bm == 64) continue;                     // (the 64-row tile stores no gate/up pairs)
         if (mode == 3 && !(c.bm == 128 && c.bn == 128)) continue;   // the masked path exists for one tile shape
-        if (mode == 4 && !((c.bm == 256 && c.bn == 192) || (c.bm <= 128 && c.bn <= 128))) continue;  // (the tiles of MODE 4)
         if (mode != 2 && mode != 4 && (c.bn == 64 || c.bm == 64)) continue;  // the 64-wide and 64-row tiles exist for the ring pipeline only
         const int tiles = ((M + c.bm - 1) / c.bm) * ((Ncols + c.bn - 1) / c.bn);
         for (int S = 1; S <= KSPLIT_MAX; S++) {
@@ -1157,8 +1155,12 @@ template <typename TIn, typename TOut>
 static int launch_tiles(const GemmArgs& g, TileCfg t, int mode, int grid, hipStream_t st) {
     if (g.ksplit > 1 && mode != 2 && mode != 4) return set_error(MMX_E_UNSUPPORTED, "the K split needs the ring pipeline (16-byte aligned rows of A)");
     if (mode == 3) return MMX_LAUNCH(TIn, 128, 128, 3, TOut, 1);  // the masked path exists for one tile shape
-    if (mode == 4) {  // a K tail: four tiles cover the range (the K split's code costs an unsplit launch nothing measurable)
-        if (t.bm == 256 && t.bn == 192) return MMX_LAUNCH(TIn, 256, 192, 4, TOut, 1);
+    if (mode == 4) {  // a K tail (the K split's code costs an unsplit launch nothing measurable)
+        constexpr int NW256 = Mfma<TIn>::W8 ? 4 : 8;
+        if (t.bm == 256 && t.bn == 256) return launch_cfg<TIn, 256, 256, 4, TOut, 1, NW256>(g, grid, st);
+        if (t.bm == 256 && t.bn == 192) return launch_cfg<TIn, 256, 192, 4, TOut, 1, NW256>(g, grid, st);
+        if (t.bm == 128 && t.bn == 256) return MMX_LAUNCH(TIn, 128, 256, 4, TOut, KSPLIT_MAX);
+        if (t.bm == 128 && t.bn == 192) return MMX_LAUNCH(TIn, 128, 192, 4, TOut, KSPLIT_MAX);
         if (t.bm == 64 && t.bn == 128) return MMX_LAUNCH(TIn, 64, 128, 4, TOut, KSPLIT_MAX);
         if constexpr (!Mfma<TIn>::W8) {
             if (t.bm == 128 && t.bn == 64) return MMX_LAUNCH(TIn, 128, 64, 4, TOut, 1);
@@ -1214,8 +1216,7 @@ static inline int prepare_gemm(GemmArgs& g, TileCfg& t, int& mode, int elesz, co
     mode = fast_ok ? load_mode() : 3;
     if (mode == 2 && g.kbytes % 128) mode = 4;
     // modes 2 and 4 address A through 32-bit per-thread offsets
-    if ((mode == 2 || mode == 4) && ((int64_t)M * lda >= ((int64_t)1 << 32) - 4096 || g.panel_stride >= ((int64_t)1 << 28))) mode = mode == 4 ? 3 : 0;
-    if (mode == 4) g.nk = g.kbytes / 128;
+    if ((mode == 2 || mode == 4) && ((int64_t)M * lda >= (int64_t)0xFFFF0000 || g.panel_stride >= ((int64_t)1 << 28))) mode = mode == 4 ? 3 : 0;
     SplitRequest use = rq;
     if ((mode != 2 && mode != 4) || pairs || (mode == 4 && rq.k_splits > 1)) {
         if (rq.k_splits > 1)

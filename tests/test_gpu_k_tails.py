@@ -93,6 +93,45 @@ def test_k_tail_behind_a_k_split(po, kind, K, tile):
         check_float_parity(host_bits(C), ref, mx.last_kernel())
 
 
+@pytest.mark.parametrize("tile", ["256x256", "128x256", "128x192"], indirect=True)
+@pytest.mark.parametrize("K", [65, 72, 191, 200, 1096])
+@pytest.mark.parametrize("kind", ["bf16", "w8", "i8"])
+def test_k_tail_wide_tiles(po, kind, K, tile):
+    """One k-iteration before the tail and many, tails of whole 16-byte pieces and not, more than one tile each way; and gate/up pairs."""
+    M, N = 270, 576
+    rng = np.random.default_rng(K)
+    if kind == "i8":
+        K *= 2
+    W = rng.integers(-127, 128, (K, N)).astype(np.int8)
+    if kind == "i8":
+        A = rng.integers(-127, 128, (M, K)).astype(np.int8)
+        up, ref, kw, odt = dev, po.gemm_i8(A, W), {}, torch.int32
+    else:
+        A = po.f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32))
+        if kind == "bf16":
+            W = po.f32_to_bf16((rng.standard_normal((K, N)) * 0.05).astype(np.float32))
+        ref = po.gemm_bf16(A, W if kind == "bf16" else po.f32_to_bf16(W.astype(np.float32)))
+        up, kw, odt = dev_bf16, ({} if kind == "bf16" else {"b_dtype": mx.I8}), torch.float32
+    es = 1 if kind == "i8" else 2
+    x = _in_nan(up(A), (-K * es % 16) // es + 16 // es)  # (rows 16-byte aligned, NaN or 77 behind them)
+    packed = mx.repack_b((dev_bf16 if kind == "bf16" else dev)(W))
+    C = torch.zeros((M, N), dtype=odt, device="cuda")
+    mx.gemm(x, packed, N, mx.Epilogue(C), **kw)
+    assert f"_{tile}_ring" in mx.last_kernel(), mx.last_kernel()
+    if kind == "i8":
+        assert np.array_equal(host_bits(C), ref), mx.last_kernel()
+        return
+    check_float_parity(host_bits(C), ref, f"{kind} K={K} {mx.last_kernel()}")
+    if tile != "128x192":  # gate and up panels in turn; silu within 2^-14 as below
+        scale = 1.0 if kind == "bf16" else 2.0 ** -10
+        h = torch.zeros((M, N // 2), dtype=torch.float32, device="cuda")
+        mx.gemm(x, packed, N, mx.Epilogue(h, mx.PP_SILU_GATE | (mx.PP_DEQUANT if kind == "w8" else 0), deq_scale=scale), **kw)
+        assert f"_{tile}_ring" in mx.last_kernel(), mx.last_kernel()
+        g, u = (np.concatenate([ref[:, n:n + 32] for n in range(32 * i, N, 64)], axis=1).astype(np.float64) * scale for i in (0, 1))
+        want = g / (1.0 + np.exp(-g)) * u
+        assert np.linalg.norm(host_bits(h).astype(np.float64) - want) <= 2.0 ** -13 * np.linalg.norm(want), mx.last_kernel()
+
+
 @pytest.mark.parametrize("kind,M,K,pad", [("bf16", 64, 4100, 4), ("bf16", 64, 4100, 0), ("w8", 64, 4100, 4), ("i8", 64, 8201, 7),
                                           ("i8", 16, 8256, 0), ("i8", 16, 8320, 0), ("bf16", 16, 8200, 0)])
 def test_the_plan_does_not_depend_on_earlier_calls(kind, M, K, pad):
