@@ -81,6 +81,7 @@ bool unpacked_takes(int M, int K, int N, int64_t lda, int64_t ldb, int transpose
 size_t unpacked_workspace_bytes(int M, int K, int N, int transpose);
 int launch_unpacked(const void* A, int64_t lda, const void* B, int64_t ldb, int transpose, int M, int K, int N, const Epilogue& ep, char* ws,
                     size_t ws_bytes, hipStream_t st);
+int launch_align_rows(const void* A, int64_t lda, int M, int row_bytes, void* out, int pitch, hipStream_t st);
 int launch_repack(int elesz, const void* B, int64_t ldb, int K, int N, int transpose, void* out, hipStream_t st, int flip);
 size_t u8_scratch_bytes(bool a_unsigned, int M, int K, int n1);
 int launch_gemm_x8(bool a_unsigned, bool b_unsigned, const void* A, int64_t lda, const void* Bp, int M, int K, int N, int n0, int n1,
@@ -170,6 +171,21 @@ static int make_epilogue(const mmx_epilogue* in, int a_dtype, int b_dtype, int M
     return MMX_OK;
 }
 
+// Dense rows of A that are not whole 16-byte pieces, and so not aligned, went to the masked pipeline, which waits for memory in every
+// k-iteration and has one tile shape.  Where a workspace is at hand they are copied there first, aligned and padded with zeros to whole
+// k-iterations, and the call goes on as one of that shape.  us, masked -> copied and multiplied (two launches, 6.8 us of host time):
+// bf16 40 x 1001 x 1024 19.1 -> 7.4, 100 x 5001 x 4096 72 -> 17, 800 x 5001 x 9654 236 -> 97, 1600 x 2234 x 9654 126 -> 77; int8
+// 200 x 4001 x 4096 34 -> 14; int8 weights 800 x 1001 x 1024 20.3 -> 10.7.  Of 174 shapes (40 to 1600 rows, K 257 to 5001, 256 to 9654
+// columns) the copy loses on 7 of short rows (up to 1024 bytes) with much to multiply, at most 1.12 (800 x 515 x 4096 int8 11.1 / 12.4, 200 x 257 x 9654
+// bf16 10.0 / 10.9), and on one behind that line (int8 weights 800 x 515 x 4096 15.2 / 15.6); short rows with little are ahead (40 x 257 x 256 8.8 / 6.6).
+// (Dense rows: the workspace query, which knows K but not the stride, foresees them, so that a first call takes the same way.)
+static int copied_pitch(int es, int K) { return (int)(((int64_t)K * es + 127) / 128 * 128); }
+static bool copy_pays(int es, int M, int K, int Ncols) {
+    const int64_t row = (int64_t)K * es;
+    return row % 16 && (int64_t)M * copied_pitch(es, K) <= (int64_t)(WS_STANDARD_BYTES / 2) &&
+           (row > 1024 || (row >= 512 && (int64_t)M * K * Ncols <= 100000000));
+}
+
 static int gemm_dispatch(int a_dtype, int b_dtype, const void* A, int64_t lda_bytes, const void* Bpacked, int M, int K,
                          int N, int n0, int n1, const mmx_epilogue* ep_in, const SplitRequest& rq, hipStream_t st) {
     if (!A || !Bpacked) return set_error(MMX_E_INVALID, "mmx_gemm: NULL operand");
@@ -199,6 +215,20 @@ static int gemm_dispatch(int a_dtype, int b_dtype, const void* A, int64_t lda_by
     if (i8 && skinny_i8_eligible(A, lda_bytes, M, K, rq.k_splits) && forced_tile().bm == 0)
         return launch_skinny(3, A, lda_bytes, Bpacked, M, K, N, n0, n1, ep, st, &rq);
     if (w4) return set_error(MMX_E_UNSUPPORTED, "mmx_gemm: bf16 x int4-weight is a decode path (M <= 32)");
+    if (lda_bytes == (int64_t)K * esa && rq.ws && rq.k_splits == 0 && forced_tile().bm == 0 && load_mode() == 2 && copy_pays(esa, M, K, n1 - n0)) {
+        const int pitch = copied_pitch(esa, K);
+        const size_t bytes = (size_t)M * pitch, room = rq.ws_bytes & ~(size_t)255;
+        if (room >= WS_COUNTER_BYTES + bytes) {  // (at the end of the workspace: the slices of the call itself take the front)
+            char* const copy = rq.ws + ((room - bytes) & ~(size_t)255);
+            rc = launch_align_rows(A, lda_bytes, M, K * esa, copy, pitch, st);
+            if (rc) return rc;
+            const SplitRequest rest = {0, rq.ws, (size_t)(copy - rq.ws)};
+            // (padded with zeros up to the same k as the packed weights)
+            rc = gemm_dispatch(a_dtype, b_dtype, copy, pitch, Bpacked, M, pitch / esa, N, n0, n1, ep_in, rest, st);
+            strncat(g_kernel, "_rows_copied", sizeof g_kernel - 1 - strlen(g_kernel));
+            return rc;
+        }
+    }
     if (rq.k_splits <= 1 && forced_tile().bm == 0 && load_mode() == 2) {  // small tiles, where they promise to be faster
         SplitRequest any = {rq.ws ? rq.k_splits : 1, rq.ws, rq.ws_bytes};
         rc = launch_wave_ring(i8 ? 3 : (w8 ? 1 : 0), A, lda_bytes, Bpacked, M, K, N, n0, n1, ep, rq, plan_us(esa, w8, M, K, n1 - n0, ep.steps, any), st);
@@ -382,7 +412,10 @@ size_t mmx_gemm_workspace_bytes(int a_dtype, int b_dtype, int M, int K, int N, i
         const SplitRequest any = {k_splits, reinterpret_cast<char*>(256), ~(size_t)0};
         const int64_t need = wave_ring_workspace_bytes(i8 ? 3 : (w8 ? 1 : 0), M, K, n1 - n0, (steps & MMX_PP_SILU_GATE) != 0, k_splits,
                                                        plan_us(i8 ? 1 : 2, w8, M, K, n1 - n0, steps, any));
-        if (need >= 0) return (size_t)need;
+        if (need > 0) return (size_t)need;
+        const int es = i8 ? 1 : 2;
+        const size_t slices = need < 0 ? plan_workspace_bytes(es, w8, M, K, n1 - n0, steps, k_splits) : 0;
+        return slices == 0 && k_splits == 0 && copy_pays(es, M, K, n1 - n0) ? WS_COUNTER_BYTES + (size_t)M * copied_pitch(es, K) + 256 : slices;
     }
     return plan_workspace_bytes(i8 ? 1 : 2, w8, M, K, n1 - n0, steps, k_splits);
 }

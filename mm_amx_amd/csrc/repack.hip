@@ -249,6 +249,30 @@ int launch_repack_gate_up(const void* wg, const void* wu, int64_t ldw, int K, in
     return launch_repack_rows<2, true>(wg, wu, ldw, K, N, 2 * N / 32, out, st, 0);
 }
 
+// Rows of any alignment and length (16 bytes and more) to rows of `pitch` bytes, a multiple of 128, zero behind their end.
+__global__ __launch_bounds__(256) void align_rows_kernel(const char* __restrict__ A, int64_t lda, int pieces, int row_bytes, char* __restrict__ out, int per_row) {
+    constexpr int UNR = 4;
+    const int i0 = blockIdx.x * (256 * UNR) + threadIdx.x;
+    u32x4 v[UNR];
+    int at[UNR];
+#pragma unroll
+    for (int u = 0; u < UNR; u++) {
+        const int i = i0 + u * 256 < pieces ? i0 + u * 256 : pieces - 1, m = i / per_row;
+        at[u] = (i - m * per_row) * 16;
+        v[u] = fetch16_in_row(A + (int64_t)m * lda, at[u], row_bytes);
+    }
+#pragma unroll
+    for (int u = 0; u < UNR; u++)
+        if (i0 + u * 256 < pieces) *reinterpret_cast<u32x4*>(out + (int64_t)(i0 + u * 256) * 16) = settle16_in_row(v[u], at[u], row_bytes);
+}
+
+int launch_align_rows(const void* A, int64_t lda, int M, int row_bytes, void* out, int pitch, hipStream_t st) {
+    const int pieces = M * (pitch / 16);  // (the caller's workspace bounds it)
+    hipLaunchKernelGGL(align_rows_kernel, dim3((pieces + 1023) / 1024), dim3(256), 0, st, static_cast<const char*>(A), lda, pieces, row_bytes,
+                       static_cast<char*>(out), pitch / 16);
+    return check_hip(hipGetLastError(), "align_rows_kernel launch");
+}
+
 // ---- per-tensor weight compression ---------------------------------------------------------------
 __global__ void zero_u32_kernel(uint32_t* p) { *p = 0u; }
 

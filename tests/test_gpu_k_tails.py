@@ -191,3 +191,65 @@ def test_a_tail_is_one_trip_to_memory():
         took[K] = call_us(lambda: mx.gemm(A, packed, N, ep))
         assert "masked" in mx.last_kernel()
     assert took[40] <= 1.2 * took[64], took
+
+
+@pytest.mark.parametrize("M,K,N", [(33, 513, 64), (40, 1001, 257), (130, 1999, 96), (300, 2234, 700), (64, 5003, 40)])
+@pytest.mark.parametrize("kind", ["bf16", "w8", "i8"])
+def test_dense_rows_that_are_not_whole_pieces(po, kind, M, K, N):
+    """Copied to the workspace first: an infinity (127s) in one row stays in that row, the workspace ends with the copy and its counters
+    are zero afterwards; a smaller one, or none, leaves the call to the masked pipeline."""
+    rng = np.random.default_rng(K)
+    W = rng.integers(-127, 128, (K, N)).astype(np.int8)
+    if kind == "i8":
+        A = rng.integers(-127, 128, (M, K)).astype(np.int8)
+        A[3] = 127
+        ref, up, kw, odt, es = po.gemm_i8(A, W), dev, {}, torch.int32, 1
+    else:
+        A = po.f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32))
+        if kind == "bf16":
+            W = po.f32_to_bf16((rng.standard_normal((K, N)) * 0.05).astype(np.float32))
+        ref, up, kw, odt, es = po.gemm_bf16(A, W if kind == "bf16" else po.f32_to_bf16(W.astype(np.float32))), dev_bf16, \
+            ({} if kind == "bf16" else {"b_dtype": mx.I8}), torch.float32, 2
+    packed, x = mx.repack_b((dev_bf16 if kind == "bf16" else dev)(W)), up(A)
+    if kind != "i8":
+        x[3, 0] = float("inf")
+    others = np.arange(M) != 3
+    room = (16 << 10) + (M + 1) * ((K * es + 127) // 128 * 128) + (8 << 20)
+    ws = torch.zeros(room + 64, dtype=torch.uint8, device="cuda")
+    ws[room:] = 0xA5
+    for how in ("stream", "given", "small", "none"):
+        C = torch.full((M + 1, N + 3), -7, dtype=odt, device="cuda")
+        extra = {"stream": {}, "given": {"ws": ws[:room]}, "small": {"ws": ws[:16 << 10]}, "none": {"k_splits": 1}}[how]
+        mx.gemm(x, packed, N, mx.Epilogue(C[:M, :N]), **kw, **extra)
+        assert mx.last_kernel().endswith("_rows_copied") == (how in ("stream", "given")), (how, mx.last_kernel())
+        got = host_bits(C)
+        assert (got[M] == -7).all() and (got[:, N:] == -7).all()
+        if kind == "i8":
+            assert np.array_equal(got[:M, :N], ref), (how, mx.last_kernel())
+        else:
+            assert not np.isfinite(got[3, :N]).any()
+            check_float_parity(got[:M, :N][others], ref[others], f"{how} {mx.last_kernel()}")
+    assert not ws[:16 << 10].any().item() and (ws[room:] == 0xA5).all().item()
+
+
+def test_dense_rows_replay_from_a_graph():
+    """Copy and product in a captured graph, new rows before each replay."""
+    M, K, N = 200, 1335, 384
+    x = torch.zeros((M, K), dtype=torch.bfloat16, device="cuda")
+    packed, C = mx.repack_b(torch.randn((K, N), device="cuda").to(torch.bfloat16)), torch.zeros((M, N), device="cuda")
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        mx.gemm(x, packed, N, mx.Epilogue(C))
+        assert mx.last_kernel().endswith("_rows_copied")
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            mx.gemm(x, packed, N, mx.Epilogue(C))
+    for seed in range(3):
+        x.copy_(torch.randn((M, K), device="cuda", generator=torch.Generator(device="cuda").manual_seed(seed)).to(torch.bfloat16))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        eager = torch.zeros((M, N), device="cuda")
+        mx.gemm(x, packed, N, mx.Epilogue(eager))
+        assert torch.equal(C, eager), seed
