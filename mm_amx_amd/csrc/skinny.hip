@@ -1560,6 +1560,26 @@ static bool short_tail(int wk, bool pairs, int M, int nfrag, int panels) {
     return nfrag <= (M <= 16 ? (wk == 1 && M <= 8 ? 32 : 24) : (wk == 0 ? 20 : 16));
 }
 
+// The most bytes of x (with its row of zeros) with which a single-panel launch takes the streaming kernel; with more it takes the
+// chunked one, which loads every chunk of x and waits at a barrier per chunk, a chain that its few loads in flight do not hide.  slices:
+// of K, that the chunked kernel would have with a workspace (not whether there is one: it decides nothing else here).  us, chunked -> streaming, weights rotated over 500 MB:
+//   156 KiB, one workgroup on a CU, with panels for more than a third of the CUs and no more than all of them: M x K x N bf16
+//   16 x 2432 x 4800 8.9 -> 7.8, 24 x 1984 x 4800 9.0 -> 7.1, 16 x 4544 x 8000 15.4 -> 15.4; int8 weights 12 x 4544 x 4800 10.7 -> 8.6,
+//   32 x 1984 x 8000 9.3 -> 7.8; int4 4 x 8192 x 4800 13.1 -> 8.9, 8 x 8000 x 8000 13.7 -> 10.7; int8 x 8 x 6144 x 4800 12.0 -> 7.9,
+//   24 x 2048 x 8000 6.7 -> 6.0.  Not over a short int4 K (11 x 4416 x 8000 9.5 / 10.4).  With fewer panels slices put the idle CUs to
+//   work (int8 weights 4 x 9024 x 1280 9.2 / 10.8, int4 6 x 8192 x 1280 8.0 / 9.0); where there are slices for up to half of the CUs
+//   they are ahead over a deep bf16 K (16 x 4544 x 2880 10.1 / 11.2; 24 x 1984 7.9 -> 6.7) and over int4 with more than 4 rows
+//   (6 x 10624 x 2880 11.7 / 11.7; 2 rows 11.7 -> 10.3), and the other types gain up to 1.24 and lose at most 0.4 us (int8 x 32 x 4096 x 2880
+//   8.1 / 8.4).
+//   More panels than CUs: 80 KiB, two workgroups on a CU, over bf16 and int8 weights; over a deep int4 K with up to 4 rows 84 KiB
+//   (2 x 8192 x 11200 18.6 -> 13.9, 4 x 8192 x 8960 17.8 -> 14.7, 4 x 5440 x 8960 13.2 / 13.3); int8 x 24 x 2048 x 12800 8.5 / 8.8.
+static int stream_x_limit(int wk, int M, int K, int nfrag, int panels, int slices) {
+    const int cus = num_cus();
+    if (panels <= cus && 3 * panels > cus && (wk != 2 || nfrag >= 80) &&
+        (slices == 1 || 2 * panels > cus || (wk == 2 ? M <= 4 : (wk != 0 || K <= 2560)))) return 156 * 1024;
+    return wk <= 1 ? 80 * 1024 : (wk == 2 && panels > cus && M <= 4 && nfrag >= 96 ? 84 * 1024 : 46 * 1024);
+}
+
 // wk: weights are bf16 (0), int8 (1) or int4 (2); 3: int8 weights and int8 activations
 int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int K, int N, int n0, int n1,
                   const Epilogue& ep, hipStream_t st, const SplitRequest* rq) {
@@ -1592,29 +1612,41 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
         s.stamps = reinterpret_cast<uint64_t*>(rq->ws + WS_COUNTER_BYTES + ((size_t)96 << 20));
 #endif
     const bool pairs = (ep.steps & MMX_PP_SILU_GATE) != 0;
+    // K slices that the chunked kernel would take (a workspace at hand, the library left to choose)
+    const int ksl = !pairs && rq && rq->ws && rq->k_splits == 0 ? chunk_slices(wk != 0, M, s.nfrag, panels, rq->ws_bytes) : 1;
+    const int x_limit = pairs ? 46 * 1024 : stream_x_limit(wk, M, K, s.nfrag, panels, chunk_slices(wk != 0, M, s.nfrag, panels, ~(size_t)0));
+    // the streaming kernel, its limit of LDS raised where x needs it
+    auto launch_stream = [&](StreamKernel kern, std::atomic<uint64_t>& raised, int lds, int zoff) {
+        if (lds > 64 * 1024) {
+            const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), 156 * 1024, raised);
+            if (rc) return rc;
+        }
+        hipLaunchKernelGGL(kern, dim3(panels), dim3(512), lds, st, s, zoff);
+        return check_hip(hipGetLastError(), "skinny_stream_kernel launch");
+    };
     if (wk == 3) {
         // int8 activations x int8 weights (int32 sums): the caller has checked skinny_i8_eligible and uses the tile
         // kernel otherwise
         const int zoff = (M * s.xpitch + 1023) & ~1023;
-        if (zoff + s.xpitch > 46 * 1024) {  // x does not fit in LDS: through LDS chunk by chunk (32 rows x 256 bytes per buffer)
+        if (zoff + s.xpitch > x_limit) {  // through LDS chunk by chunk (32 rows x 256 bytes per buffer)
             // (few panels, a workspace at hand: K in slices as for bf16 activations; int32 sums, the same bits in any order)
-            const int ksl3 = (rq && rq->ws && rq->k_splits == 0) ? chunk_slices(true, M, s.nfrag, panels, rq->ws_bytes) : 1;
-            if (ksl3 > 1) {
+            if (ksl > 1) {
                 s.ws_cnt = reinterpret_cast<uint32_t*>(rq->ws);
                 s.ws_part = rq->ws + WS_COUNTER_BYTES;
-                s.kslices = ksl3;
+                s.kslices = ksl;
                 char name_[40];
-                snprintf(name_, sizeof name_, "skinny_chunk_i8_ksplit%d", ksl3);
+                snprintf(name_, sizeof name_, "skinny_chunk_i8_ksplit%d", ksl);
                 note_kernel(name_);
-                return launch_chunk<3, 1, 1, 1, 6>(dim3(panels, ksl3), s, st);
+                return launch_chunk<3, 1, 1, 1, 6>(dim3(panels, ksl), s, st);
             }
             note_kernel("skinny_chunk_i8");
             return launch_chunk<3, 1, 1, 1>(dim3(panels), s, st);
         }
         note_kernel("skinny_stream_i8");
-        int unused;
-        hipLaunchKernelGGL(stream_kernel_for<3>(s.nfrag, s.xpitch == row_bytes, &unused), dim3(panels), dim3(512), stream_lds_bytes(zoff + s.xpitch, 1), st, s, zoff);
-        return check_hip(hipGetLastError(), "skinny_stream_kernel launch");
+        static std::atomic<uint64_t> raised[2 * STREAM_KERNELS];
+        int index;
+        const StreamKernel kern = stream_kernel_for<3>(s.nfrag, s.xpitch == row_bytes, &index);
+        return launch_stream(kern, raised[index], stream_lds_bytes(zoff + s.xpitch, 1), zoff);
     }
     // whether x goes through LDS at all (int8 x always does)
     const bool staged = row_bytes >= 16 && !(aligned && K % (wk == 0 ? 64 : (wk == 1 ? 128 : 256)) && short_tail(wk, pairs, M, s.nfrag, panels));
@@ -1623,19 +1655,23 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
         if (pairs && (panels & 1)) return set_error(MMX_E_INVALID, "SILU_GATE needs an even number of 32-column panels");
         const int zoff = (M * s.xpitch + 1023) & ~1023;
         const int xb = zoff + s.xpitch;
-        if (staged && xb <= 46 * 1024) {
+        if (staged && xb <= x_limit) {
             note_kernel(pairs ? "skinny_stream_w4_gateup" : "skinny_stream_w4");
             const int per_wave = (s.nfrag + 7) / 8;
             const bool fills = s.x_rows == 2 && s.xpitch == row_bytes;
-            StreamKernel kern;  // (register sets sized to the share of K, as for the other weight types)
-            if (pairs) kern = stream_pair_kernel_for<2>(s.nfrag, fills);  // gate and up panels side by side
-            else if (per_wave <= 4) kern = fills ? skinny_stream_kernel<2, 1, true, WHOLE_ROWS, 4> : skinny_stream_kernel<2, 1, true, ANY_ROWS, 4>;
-            else if (per_wave <= 6) kern = fills ? skinny_stream_kernel<2, 1, true, WHOLE_ROWS, 6> : skinny_stream_kernel<2, 1, true, ANY_ROWS, 6>;
-            else if (per_wave <= 8) kern = fills ? skinny_stream_kernel<2, 1, true, WHOLE_ROWS> : skinny_stream_kernel<2, 1, true, ANY_ROWS>;
-            else kern = fills ? skinny_stream_kernel<2, 1, false, WHOLE_ROWS> : skinny_stream_kernel<2, 1, false, ANY_ROWS>;
-            const int np = pairs ? 2 : 1;
-            hipLaunchKernelGGL(kern, dim3(panels / np), dim3(512), stream_lds_bytes(xb, np), st, s, zoff);
-            return check_hip(hipGetLastError(), "skinny_stream_kernel launch");
+            if (pairs) {  // gate and up panels side by side
+                hipLaunchKernelGGL(stream_pair_kernel_for<2>(s.nfrag, fills), dim3(panels / 2), dim3(512), stream_lds_bytes(xb, 2), st, s, zoff);
+                return check_hip(hipGetLastError(), "skinny_stream_kernel launch");
+            }
+            // (register sets sized to the share of K, as for the other weight types)
+            static const StreamKernel list[2][4] = {
+                {skinny_stream_kernel<2, 1, true, ANY_ROWS, 4>, skinny_stream_kernel<2, 1, true, ANY_ROWS, 6>,
+                 skinny_stream_kernel<2, 1, true, ANY_ROWS>, skinny_stream_kernel<2, 1, false, ANY_ROWS>},
+                {skinny_stream_kernel<2, 1, true, WHOLE_ROWS, 4>, skinny_stream_kernel<2, 1, true, WHOLE_ROWS, 6>,
+                 skinny_stream_kernel<2, 1, true, WHOLE_ROWS>, skinny_stream_kernel<2, 1, false, WHOLE_ROWS>}};
+            static std::atomic<uint64_t> raised[2][4];
+            const int i = per_wave <= 4 ? 0 : (per_wave <= 6 ? 1 : (per_wave <= 8 ? 2 : 3));
+            return launch_stream(list[fills][i], raised[fills][i], stream_lds_bytes(xb, 1), zoff);
         }
         if (pairs) {  // the general kernel
             note_kernel("skinny_w4_gateup");
@@ -1644,16 +1680,15 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
         }
         if (staged) {
             // x too large for LDS: through LDS chunk by chunk (two buffers of 16 or 32 rows x 1 KiB)
-            const int ksl4 = (rq && rq->ws && rq->k_splits == 0) ? chunk_slices(true, M, s.nfrag, panels, rq->ws_bytes) : 1;
-            if (ksl4 > 1) {  // few panels, a workspace at hand: K in slices as for the other weight types
+            if (ksl > 1) {  // few panels, a workspace at hand: K in slices as for the other weight types
                 s.ws_cnt = reinterpret_cast<uint32_t*>(rq->ws);
                 s.ws_part = rq->ws + WS_COUNTER_BYTES;
-                s.kslices = ksl4;
+                s.kslices = ksl;
                 char name_[40];
-                snprintf(name_, sizeof name_, "skinny_chunk_w4_ksplit%d", ksl4);
+                snprintf(name_, sizeof name_, "skinny_chunk_w4_ksplit%d", ksl);
                 note_kernel(name_);
-                if (M <= 16) return launch_chunk<2, 1, 1, 2, 3>(dim3(panels, ksl4), s, st);
-                return launch_chunk<2, 1, 1, 4, 2>(dim3(panels, ksl4), s, st);
+                if (M <= 16) return launch_chunk<2, 1, 1, 2, 3>(dim3(panels, ksl), s, st);
+                return launch_chunk<2, 1, 1, 4, 2>(dim3(panels, ksl), s, st);
             }
             note_kernel("skinny_chunk_w4");
             if (M <= 16) return launch_chunk<2, 1, 1, 2>(dim3(panels), s, st);
@@ -1751,13 +1786,13 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
     // The streaming form needs all of x in LDS and at least two workgroups per CU (344 panels of N = 11008 must all
     // be resident): 80 KiB of x each (4096 x 11008 int8 GEMV at M = 5-8: 13.0-13.4 -> 11.5-12.0 us against the chunked
     // form; with one workgroup per CU, M = 12-16, it loses: 16.6-17.7 against 13.7-14.5 us).
-    const bool bigx = !pairs && xbytes > 46 * 1024 && xbytes <= 80 * 1024;
+    const bool bigx = !pairs && xbytes > 46 * 1024 && xbytes <= x_limit;
     const bool fills = s.x_rows == 2 && s.xpitch == row_bytes;  // (WHOLE_ROWS)
     int stream_index = 0;
     const StreamKernel stream_kernel = w8 ? stream_kernel_for<1>(s.nfrag, fills, &stream_index) : stream_kernel_for<0>(s.nfrag, fills, &stream_index);
     if (bigx) {
         static std::atomic<uint64_t> attr_done[2][3 * STREAM_KERNELS];
-        const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(stream_kernel), 80 * 1024, attr_done[w8 ? 1 : 0][stream_index]);
+        const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(stream_kernel), 156 * 1024, attr_done[w8 ? 1 : 0][stream_index]);
         if (rc) return rc;
     }
     if (staged && (xbytes <= 46 * 1024 || bigx)) {
@@ -1817,10 +1852,7 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
         }
         return check_hip(hipGetLastError(), "skinny_stream_kernel launch");
     }
-    // K split of the chunked kernel (a workspace at hand, the library left to choose)
-    const int ksl = (staged && !pairs && wk <= 1 && rq && rq->ws && rq->k_splits == 0)
-                        ? chunk_slices(w8, M, s.nfrag, panels, rq->ws_bytes) : 1;
-    if (whole && !w8 && !pairs && M <= 8 && ksl == 1) {
+    if (whole && !w8 && !pairs && M <= 8 && !(staged && ksl > 1)) {
         // aligned, x too large for LDS, few rows, plain bf16 weights: every lane reads its own part of x
         // (measured: for int8 weights and for gate/up pairs the chunked kernel below is faster at these M too)
         note_kernel("skinny_direct_bf16");

@@ -95,6 +95,26 @@ def test_x_through_lds_in_chunks_and_half_panels(po, kind, M, K, N, splits, want
         check_float_parity(host_bits(C), ref, f"{kind} {M}x{K}x{N} pad={pad} {mx.last_kernel()}")
 
 
+# the largest x that each rule takes, the next larger one, few and many panels, K that fills its fragments and not
+@pytest.mark.parametrize("kind,M,K,N,stream", [
+    ("bf16", 32, 2400, 4800, True), ("bf16", 32, 2424, 4800, False), ("bf16", 24, 1990, 2900, True), ("bf16", 24, 2624, 2900, False),
+    ("bf16", 16, 4544, 8192, True), ("w8", 16, 4544, 4807, True), ("w8", 31, 2450, 2900, True), ("w8", 31, 2496, 2900, False), ("w8", 8, 7360, 1280, False),
+    ("w4", 13, 5632, 4800, True), ("w4", 8, 5100, 4800, True), ("w4", 8, 5056, 4800, False), ("w4", 4, 6913, 2900, True), ("w4", 5, 6913, 2900, False),
+    ("w4", 4, 8192, 8300, True), ("w4", 3, 6000, 8300, False),
+    ("i8", 32, 4096, 4800, True), ("i8", 32, 4864, 4800, False), ("i8", 16, 4608, 1280, False), ("i8", 24, 2048, 8300, False)])
+def test_long_x_in_lds(po, kind, M, K, N, stream):
+    x, packed, ref = _operands(po, kind, M, K, N, K + M)
+    for pad in ((8, 1) if kind != "i8" else (16, 0)):
+        C = torch.zeros((M, N), dtype=torch.int32 if kind == "i8" else torch.float32, device="cuda")
+        pad += -K % 8 if pad == 8 else 0
+        mx.gemm(_in_nan((dev if kind == "i8" else dev_bf16)(x), pad), packed, N, mx.Epilogue(C), **KW[kind])
+        assert mx.last_kernel().startswith(f"skinny_{'stream' if stream else 'chunk'}_{kind}"), mx.last_kernel()
+        if kind == "i8":
+            assert np.array_equal(host_bits(C), ref), mx.last_kernel()
+        else:
+            check_float_parity(host_bits(C), ref, f"{kind} {M}x{K}x{N} pad={pad} {mx.last_kernel()}")
+
+
 @pytest.mark.parametrize("M,K", [(3, 200), (2, 2104), (16, 2104), (32, 1001)])
 @pytest.mark.parametrize("kind", ["bf16", "w8", "w4"])
 def test_gate_up(po, kind, M, K):
