@@ -1663,14 +1663,27 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
                 hipLaunchKernelGGL(stream_pair_kernel_for<2>(s.nfrag, fills), dim3(panels / 2), dim3(512), stream_lds_bytes(xb, 2), st, s, zoff);
                 return check_hip(hipGetLastError(), "skinny_stream_kernel launch");
             }
-            // (register sets sized to the share of K, as for the other weight types)
-            static const StreamKernel list[2][4] = {
-                {skinny_stream_kernel<2, 1, true, ANY_ROWS, 4>, skinny_stream_kernel<2, 1, true, ANY_ROWS, 6>,
-                 skinny_stream_kernel<2, 1, true, ANY_ROWS>, skinny_stream_kernel<2, 1, false, ANY_ROWS>},
-                {skinny_stream_kernel<2, 1, true, WHOLE_ROWS, 4>, skinny_stream_kernel<2, 1, true, WHOLE_ROWS, 6>,
-                 skinny_stream_kernel<2, 1, true, WHOLE_ROWS>, skinny_stream_kernel<2, 1, false, WHOLE_ROWS>}};
-            static std::atomic<uint64_t> raised[2][4];
-            const int i = per_wave <= 4 ? 0 : (per_wave <= 6 ? 1 : (per_wave <= 8 ? 2 : 3));
+            // Register sets sized to the share of K, as for the other weight types; past 8 fragments the rolling window in the batch
+            // with the fewest repeats, the larger at equal ones.  Unpacking bounds these calls, and a repeat costs as much as a
+            // fragment: in batches of 8 alone 1 x 4416 x 11008 (9 to a wavefront) took 12.9 us, 9.3 in 10; 5888 (12) 12.8 -> 10.5 in 6;
+            // 8704 (17) 17.0 -> 13.4 in 6; 9984 (20) 17.3 -> 15.9 in 10; 4 x 4416 x 4800 8.3 -> 6.7.
+            constexpr int FORMS = 7;
+            static const StreamKernel list[2][FORMS] = {
+                {skinny_stream_kernel<2, 1, true, ANY_ROWS, 4>, skinny_stream_kernel<2, 1, true, ANY_ROWS, 6>, skinny_stream_kernel<2, 1, true, ANY_ROWS>,
+                 skinny_stream_kernel<2, 1, false, ANY_ROWS, 10>, skinny_stream_kernel<2, 1, false, ANY_ROWS>, skinny_stream_kernel<2, 1, false, ANY_ROWS, 7>,
+                 skinny_stream_kernel<2, 1, false, ANY_ROWS, 6>},
+                {skinny_stream_kernel<2, 1, true, WHOLE_ROWS, 4>, skinny_stream_kernel<2, 1, true, WHOLE_ROWS, 6>, skinny_stream_kernel<2, 1, true, WHOLE_ROWS>,
+                 skinny_stream_kernel<2, 1, false, WHOLE_ROWS, 10>, skinny_stream_kernel<2, 1, false, WHOLE_ROWS>, skinny_stream_kernel<2, 1, false, WHOLE_ROWS, 7>,
+                 skinny_stream_kernel<2, 1, false, WHOLE_ROWS, 6>}};
+            static std::atomic<uint64_t> raised[2][FORMS];
+            constexpr int batch[FORMS] = {4, 6, 8, 10, 8, 7, 6};
+            int i = per_wave <= 4 ? 0 : (per_wave <= 6 ? 1 : 2);
+            if (per_wave > 8) {
+                auto repeats = [per_wave](int u) { return (per_wave + u - 1) / u * u - per_wave; };
+                i = 3;
+                for (int t = 4; t < FORMS; t++)
+                    if (repeats(batch[t]) < repeats(batch[i])) i = t;
+            }
             return launch_stream(list[fills][i], raised[fills][i], stream_lds_bytes(xb, 1), zoff);
         }
         if (pairs) {  // the general kernel

@@ -101,6 +101,9 @@ def test_x_through_lds_in_chunks_and_half_panels(po, kind, M, K, N, splits, want
     ("bf16", 16, 4544, 8192, True), ("w8", 16, 4544, 4807, True), ("w8", 31, 2450, 2900, True), ("w8", 31, 2496, 2900, False), ("w8", 8, 7360, 1280, False),
     ("w4", 13, 5632, 4800, True), ("w4", 8, 5100, 4800, True), ("w4", 8, 5056, 4800, False), ("w4", 4, 6913, 2900, True), ("w4", 5, 6913, 2900, False),
     ("w4", 4, 8192, 8300, True), ("w4", 3, 6000, 8300, False),
+    # (int4 shares of 9 to 21 fragments: every batch of the rolling window, with repeats and without)
+    ("w4", 2, 4417, 100, True), ("w4", 1, 5120, 100, True), ("w4", 1, 5700, 100, True), ("w4", 1, 6300, 100, True), ("w4", 1, 7168, 100, True),
+    ("w4", 1, 7681, 100, True), ("w4", 1, 8705, 100, True), ("w4", 1, 9984, 100, True), ("w4", 1, 10689, 100, True),
     ("i8", 32, 4096, 4800, True), ("i8", 32, 4864, 4800, False), ("i8", 16, 4608, 1280, False), ("i8", 24, 2048, 8300, False)])
 def test_long_x_in_lds(po, kind, M, K, N, stream):
     x, packed, ref = _operands(po, kind, M, K, N, K + M)
