@@ -1533,14 +1533,16 @@ static StreamKernel stream_kernel_for(int nfrag, bool whole, int* index) {
     *index = i + (whole ? 0 : STREAM_KERNELS);
     return whole ? stream_kernel_at<WK, WHOLE_ROWS>(i) : stream_kernel_at<WK, ANY_ROWS>(i);
 }
-// Gate/up pairs: batches of 8 fragments per panel, 4 over int4 weights.
+// Gate/up pairs: batches of 8 fragments per panel, 4 over int4 weights.  *index: the kernel's place in a list of six
 template <int WK>
-static StreamKernel stream_pair_kernel_for(int nfrag, bool whole) {
+static StreamKernel stream_pair_kernel_for(int nfrag, bool whole, int* index) {
     constexpr int U = WK == 2 ? 4 : 8;
     const int per_wave = (nfrag + 7) / 8;
     const bool one = per_wave <= U;
+    *index = (whole ? 2 : 0) + one;
     if constexpr (WK == 0) {
-        if (whole && nfrag == 8 * per_wave && per_wave % U == 0)
+        if (whole && nfrag == 8 * per_wave && per_wave % U == 0) *index = 4 + one;
+        if (*index >= 4)
             return one ? skinny_stream_kernel<0, 2, true, NO_REPEATS> : skinny_stream_kernel<0, 2, false, NO_REPEATS>;
     }
     if (whole) return one ? skinny_stream_kernel<WK, 2, true, WHOLE_ROWS> : skinny_stream_kernel<WK, 2, false, WHOLE_ROWS>;
@@ -1558,6 +1560,14 @@ static bool short_tail(int wk, bool pairs, int M, int nfrag, int panels) {
     if (pairs) return nfrag <= (wk == 0 ? (M <= 16 ? 32 : 22) : (wk == 1 ? 128 : (M <= 16 ? 16 : 8)));
     if (wk == 2) return panels <= num_cus() && nfrag <= (M <= 16 ? 10 : 8);
     return nfrag <= (M <= 16 ? (wk == 1 && M <= 8 ? 32 : 24) : (wk == 0 ? 20 : 16));
+}
+
+// The same for gate/up pairs over bf16 weights, one workgroup on a CU: M x K x 2 N 12 x 1984 x 6400 11.3 -> 9.7, 21 x 3264 x 7936 18.8 -> 15.4,
+// 28 x 1984 x 10752 14.2 -> 11.7, 32 x 1024 x 4096 8.3 -> 7.4, 16 x 2432 x 16000 16.2 -> 15.8; a deep K with pairs for more than half of
+// the CUs is the chunked kernel's, which walks the panels side by side (16 x 4096 x 10752 20.0 / 21.0, x 16000 23.3 / 30.6; x 7936
+// 18.9 -> 18.1), and so are more pairs than CUs (21 x 1984 x 22016 21.3 / 22.5).
+static int stream_pair_x_limit(int wk, int nfrag, int panels) {
+    return wk == 0 && panels <= 2 * num_cus() && (nfrag < 224 || panels <= num_cus()) ? 156 * 1024 : 46 * 1024;
 }
 
 // The most bytes of x (with its row of zeros) with which a single-panel launch takes the streaming kernel; with more it takes the
@@ -1614,7 +1624,7 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
     const bool pairs = (ep.steps & MMX_PP_SILU_GATE) != 0;
     // K slices that the chunked kernel would take (a workspace at hand, the library left to choose)
     const int ksl = !pairs && rq && rq->ws && rq->k_splits == 0 ? chunk_slices(wk != 0, M, s.nfrag, panels, rq->ws_bytes) : 1;
-    const int x_limit = pairs ? 46 * 1024 : stream_x_limit(wk, M, K, s.nfrag, panels, chunk_slices(wk != 0, M, s.nfrag, panels, ~(size_t)0));
+    const int x_limit = pairs ? stream_pair_x_limit(wk, s.nfrag, panels) : stream_x_limit(wk, M, K, s.nfrag, panels, chunk_slices(wk != 0, M, s.nfrag, panels, ~(size_t)0));
     // the streaming kernel, its limit of LDS raised where x needs it
     auto launch_stream = [&](StreamKernel kern, std::atomic<uint64_t>& raised, int lds, int zoff) {
         if (lds > 64 * 1024) {
@@ -1660,7 +1670,8 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
             const int per_wave = (s.nfrag + 7) / 8;
             const bool fills = s.x_rows == 2 && s.xpitch == row_bytes;
             if (pairs) {  // gate and up panels side by side
-                hipLaunchKernelGGL(stream_pair_kernel_for<2>(s.nfrag, fills), dim3(panels / 2), dim3(512), stream_lds_bytes(xb, 2), st, s, zoff);
+                int unused;
+                hipLaunchKernelGGL(stream_pair_kernel_for<2>(s.nfrag, fills, &unused), dim3(panels / 2), dim3(512), stream_lds_bytes(xb, 2), st, s, zoff);
                 return check_hip(hipGetLastError(), "skinny_stream_kernel launch");
             }
             // Register sets sized to the share of K, as for the other weight types; past 8 fragments the rolling window in the batch
@@ -1808,7 +1819,7 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
         const int rc = ensure_dynamic_lds(reinterpret_cast<const void*>(stream_kernel), 156 * 1024, attr_done[w8 ? 1 : 0][stream_index]);
         if (rc) return rc;
     }
-    if (staged && (xbytes <= 46 * 1024 || bigx)) {
+    if (staged && xbytes <= x_limit) {
         // the activations fit in LDS: streaming variant
         if (pairs && (panels & 1)) return set_error(MMX_E_INVALID, "SILU_GATE needs an even number of 32-column panels");
         note_kernel(pairs ? (w8 ? "skinny_stream_w8_gateup" : "skinny_stream_bf16_gateup") : (w8 ? "skinny_stream_w8" : "skinny_stream_bf16"));
@@ -1821,7 +1832,7 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
         const int wg_per_cu = (160 * 1024 / lds_wg) < 4 ? (160 * 1024 / lds_wg) : 4;
         const int64_t unit_bytes = (int64_t)s.nfrag * 512 * (pairs ? 2 : 1);
         const int force = decode_halves();  // -1: by the rule above, 0: never, 1: for every M <= 4 (tests pin the path with it)
-        const bool halves = M <= 4 && !bigx && !(pairs && w8) && force != 0 &&
+        const bool halves = M <= 4 && xbytes <= 46 * 1024 && !(pairs && w8) && force != 0 &&
                             (force == 1 || (2 * units <= 2 * num_cus() * wg_per_cu && unit_bytes >= (pairs ? 128 : (w8 ? 160 : 80)) * 1024));
         if (halves) {  // (fragments in pairs)
             s.nfrag = (s.nfrag + 1) & ~1;
@@ -1829,6 +1840,7 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
             zero_off = (M * s.xpitch + 1023) & ~1023;
             xbytes = zero_off + s.xpitch;
         }
+        int rc = MMX_OK;
         auto stream = [&](auto w8_c, auto np_c, int grid) {
             constexpr bool W8 = decltype(w8_c)::value;
             constexpr int NP = decltype(np_c)::value;
@@ -1840,7 +1852,13 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
                 }
             }
             StreamKernel kern = stream_kernel;
-            if constexpr (NP == 2) kern = stream_pair_kernel_for<W8 ? 1 : 0>(s.nfrag, fills);
+            if constexpr (NP == 2) {
+                static std::atomic<uint64_t> raised[6];
+                int index;
+                kern = stream_pair_kernel_for<W8 ? 1 : 0>(s.nfrag, fills, &index);
+                if (xbytes > 64 * 1024) rc = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), 156 * 1024, raised[index]);
+                if (rc) return;
+            }
             hipLaunchKernelGGL(kern, dim3(grid), dim3(512), stream_lds_bytes(xbytes, NP), st, s, zero_off);
         };
         if (halves) note_kernel(pairs ? "skinny_half_bf16_gateup" : (w8 ? "skinny_half_w8" : "skinny_half_bf16"));
@@ -1863,6 +1881,7 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
             else if (w8) stream(integral_constant<bool, true>{}, integral_constant<int, 1>{}, panels);
             else stream(integral_constant<bool, false>{}, integral_constant<int, 1>{}, panels);
         }
+        if (rc) return rc;
         return check_hip(hipGetLastError(), "skinny_stream_kernel launch");
     }
     if (whole && !w8 && !pairs && M <= 8 && !(staged && ksl > 1)) {

@@ -138,6 +138,23 @@ def test_gate_up(po, kind, M, K):
     assert np.linalg.norm(got - want) <= 2.0 ** -13 * np.linalg.norm(want), mx.last_kernel()
 
 
+# the largest x with one workgroup on a CU and the next one; x that LDS holds twice; K that fills the batches, its fragments, and neither
+@pytest.mark.parametrize("M,K,N,stream", [(28, 1344, 96, True), (17, 1001, 96, True), (32, 2400, 96, True), (32, 2424, 96, False), (16, 4096, 4096, True),
+                                          (16, 4096, 4160, False), (4, 7000, 96, True), (9, 2049, 8192, True), (9, 2688, 8224, False)])
+def test_gate_up_over_a_long_x(M, K, N, stream):
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x = torch.randn((M, K), device="cuda", generator=g).to(torch.bfloat16)
+    w = (torch.randn((2, N, K), device="cuda", generator=g) * K ** -0.5).to(torch.bfloat16)
+    packed = mx.repack_gate_up(w[0], w[1])
+    a, b = (x.double() @ v.double().t() for v in w)
+    for pad in (-K % 8 + 8, 5):
+        h = torch.zeros((M, N), dtype=torch.float32, device="cuda")
+        mx.gemm(_in_nan(x, pad), packed, 2 * N, mx.Epilogue(h, mx.PP_SILU_GATE))
+        assert mx.last_kernel() == f"skinny_{'stream' if stream else 'chunk'}_bf16_gateup", mx.last_kernel()
+        want = a / (1.0 + torch.exp(-a)) * b  # silu within 2^-14, and twice that for the roundings around it
+        assert (h.double() - want).norm() <= 2.0 ** -13 * want.norm(), mx.last_kernel()
+
+
 @pytest.mark.parametrize("kind,M,K,N,splits,want", [
     ("bf16", 12, 2600, 64, 0, "skinny_stream_bf16"),
     ("w8", 12, 2600, 64, 0, "skinny_stream_w8"),
