@@ -203,7 +203,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
     constexpr int A_BYTES = BM * 128, B_BYTES = BN / 32 * BP_IT, STAGE = A_BYTES + B_BYTES;
     constexpr int A_IT = BM / 32, B_IT = BN * (BP_IT / 32) / 4096;  // 16-byte chunks per thread per stage
 
-    extern __shared__ __attribute__((aligned(16))) char smem[];
+    extern __shared__ __attribute__((aligned(1024))) char smem[];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -463,8 +463,13 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
         // A operand of k-step s = 2 PAR + KS of a stage: chunk 2 s + g32 of the row; under int8 fragments (16
         // consecutive k per lane) chunk 4 PAR + 2 g32 + KS.  Chunks sit at position chunk ^ ((row >> 1) & 7).
         constexpr int KS1 = W8 ? 1 : 2;  // chunk distance from k-step 0 to k-step 1 of a half-stage
-        const int a_x0 = (wm * WM + l32) * 128 + (((W8 ? 2 * g32 : g32) ^ ((l32 >> 1) & 7)) * 16);
-        const int b_frag_off = B0 + wn * NJ * BP_HS + lane * 16;
+        // (Byte addresses of LDS, with which the main loop reads: from pointers into smem every read had an addition of its own.  That and
+        // the places of a window's loads worked out once per half-stage, not for each group of them: 130 -> 110 instructions a k-iteration of
+        // the 128x64 tile; int8 512 x 4096 x 4096 16.5 -> 15.9 us, bf16 300 x 992 x 6144 11.6 -> 11.2, int8 weights 1500 x 1088 x 2048 16.2 -> 15.3,
+        // 907 x 5888 x 7776 85.6 -> 83.2; the tiles with many products per k-step level.)
+        const int lds0 = (int)(uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+        const int a_x0 = lds0 + (wm * WM + l32) * 128 + (((W8 ? 2 * g32 : g32) ^ ((l32 >> 1) & 7)) * 16);
+        const int b_frag_off = lds0 + B0 + wn * NJ * BP_HS + lane * 16;
         u32x4 braw[W8 ? NJ : 1];  // int8 fragments as read from LDS: each feeds both k-steps of its half-stage
 
         // Everything a k-step needs besides its operands: where its LDS reads come from and where its
@@ -554,8 +559,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
         auto kstep = [&](const frag (&ca)[MI], const frag (&cb)[NJ], frag (&na)[MI], frag (&nb)[NJ], const KParams& kp,
                          auto q0_c, auto q1_c, auto half_c, auto ks_c, auto&& prep) {
             constexpr int Q0 = decltype(q0_c)::value, Q1 = decltype(q1_c)::value, KS = decltype(ks_c)::value;
-            const char* sA = smem + kp.rdA;
-            const char* sB = smem + kp.rdB;
+            using lds_frag = __attribute__((address_space(3))) const frag;
+            using lds_u32x4 = __attribute__((address_space(3))) const u32x4;
+            const uint32_t sA = kp.rdA, sB = kp.rdB;
             static_for<0, MN>([&](auto t_c) {
                 constexpr int t = decltype(t_c)::value;
                 acc[t / NJ][t % NJ] = MF::run(cb[t % NJ], ca[t / NJ], acc[t / NJ][t % NJ]);
@@ -563,11 +569,11 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
                     constexpr int rd = decltype(rd_c)::value;
                     if constexpr (rd < NJ) {
                         if constexpr (!W8) {
-                            nb[rd] = *reinterpret_cast<const frag*>(sB + rd * BP_HS);
+                            nb[rd] = *reinterpret_cast<lds_frag*>(sB + rd * BP_HS);
                         } else if constexpr (KS == 1) {  // next: k-step 0 of the next half-stage - fetch its int8 fragment
-                            braw[rd] = *reinterpret_cast<const u32x4*>(sB + rd * BP_HS);
+                            braw[rd] = *reinterpret_cast<lds_u32x4*>(sB + rd * BP_HS);
                         }
-                    } else if constexpr (rd < NJ + MI) na[rd - NJ] = *reinterpret_cast<const frag*>(sA + (rd - NJ) * 32 * 128);
+                    } else if constexpr (rd < NJ + MI) na[rd - NJ] = *reinterpret_cast<lds_frag*>(sA + (rd - NJ) * 32 * 128);
                 });
                 // int8 fragments -> the next k-step's bf16 operands, one dword (two weights, three instructions) at a time
                 // and spread over the k-step's MFMA slots: a wave issues in order, and a whole fragment's conversion in
@@ -629,8 +635,8 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
         MMX_STAMP(2);
         if (MODE == 4 && ends_in_chunk && last_st == 0) settle_last(0);
         {
-            const char* sA = smem + a_x0;
-            const char* sB = smem + b_frag_off;
+            const char* sA = smem + (a_x0 - lds0);
+            const char* sB = smem + (b_frag_off - lds0);
 #pragma unroll
             for (int i = 0; i < MI; i++) fa[0][i] = *reinterpret_cast<const frag*>(sA + i * 32 * 128);
 #pragma unroll
@@ -667,7 +673,15 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW / 4,
                 nas_n = nas + 1 < RA ? nas + 1 : 0;
             }
             kstep(fa[1], fb[1], fa[0], fb[0], kpb, c0{}, cH{}, integral_constant<int, (PAR + R + 1) & 1>{}, c1{},
-                  [&](auto part_c) { prepare(part_c, kpa, integral_constant<int, 1 - PAR>{}, c0{}, h + 1, as_n, nas_n, nbs); });
+                  [&](auto part_c) {
+                      if constexpr (decltype(part_c)::value == 0) {  // its second group of loads is of the same window: same places
+                          const uint32_t rdA = kpa.rdA, rdB = kpa.rdB;
+                          kpa = kpb;
+                          kpa.rdA = rdA, kpa.rdB = rdB;
+                      } else if constexpr (decltype(part_c)::value == 3) {
+                          prepare(part_c, kpa, integral_constant<int, 1 - PAR>{}, c0{}, h + 1, as_n, nas_n, nbs);
+                      }
+                  });
         };
         int as = 0, bs = 0;
         for (int st = 0; st <= last_st; st++) {
