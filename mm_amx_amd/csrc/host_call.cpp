@@ -245,6 +245,43 @@ Matrix matrix(PyObject* o, int device) {
     return {&t, ld, (int)t.size(0), (int)t.size(1), t.mutable_data_ptr()};
 }
 
+// gemm_packing(A, B, transpose, ws, device, stream, C, steps, bias, deq, deq_per_oc, q, q_per_oc) -> packed: a B that is used once, where the
+// library would have it packed first
+PyObject* gemm_packing(PyObject*, PyObject* const* a, Py_ssize_t count) {
+    if (count != 13 || !call_unpacked_need || !call_repack || !call_gemm) Py_RETURN_NONE;
+    try {
+        int device, rc = 0;
+        if (!whole_number(a[4], 0, 1 << 20, device) || !PyBool_Check(a[2])) throw Leave();
+        const int transpose = a[2] == Py_True;
+        const Matrix A = matrix(a[0], device), B = matrix(a[1], device);
+        const int M = A.rows, K = A.cols, N = transpose ? B.rows : B.cols;
+        if (A.t->scalar_type() != at::kBFloat16 || B.t->scalar_type() != at::kBFloat16 || (transpose ? B.cols : B.rows) != K) throw Leave();
+        if (call_unpacked_need(MMX_BF16, M, K, N, A.ld, B.ld, transpose) >= 0) throw Leave();
+        const mmx_epilogue e = epilogue_of(a + 6, device, M, N);
+        if (e.steps & MMX_PP_SILU_GATE) throw Leave();
+        void* ws = nullptr;
+        size_t ws_bytes = 0;
+        if (a[3] != Py_None) {
+            const at::Tensor& w = tensor_on(a[3], device);
+            if (w.scalar_type() != at::kByte || !w.is_contiguous()) throw Leave();
+            ws = w.mutable_data_ptr();
+            ws_bytes = (size_t)w.numel();
+        } else if (call_need(MMX_BF16, MMX_BF16, M, K, N, 0, N, e.steps, 0)) {
+            throw Leave();  // (it is made outside)
+        }
+        void* const stream = stream_of(a[5]);
+        at::Tensor out;
+        if (!unlocked([&] {
+                out = make({(int64_t)call_packed_bytes(MMX_BF16, K, N)}, at::kByte, *B.t);
+                rc = call_repack(MMX_BF16, B.data, B.ld, K, N, transpose, out.mutable_data_ptr(), stream);
+                if (!rc) rc = call_gemm(MMX_BF16, MMX_BF16, A.data, A.ld, out.mutable_data_ptr(), M, K, N, 0, N, &e, ws ? 0 : 1, ws, ws_bytes, stream);
+            })) throw Leave();
+        return rc ? PyLong_FromLong(rc) : THPVariable_Wrap(out);
+    } catch (...) {
+        Py_RETURN_NONE;
+    }
+}
+
 // repack(B, transpose, device, stream) -> packed
 PyObject* repack(PyObject*, PyObject* const* a, Py_ssize_t count) {
     if (count != 4 || !call_repack) Py_RETURN_NONE;
@@ -380,7 +417,7 @@ PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t count) {
 }
 
 #define METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {METHOD(gemm), METHOD(gemm_unpacked), METHOD(matvec), METHOD(repack), METHOD(quantize), METHOD(quantize_scaled),
+PyMethodDef methods[] = {METHOD(gemm), METHOD(gemm_unpacked), METHOD(gemm_packing), METHOD(matvec), METHOD(repack), METHOD(quantize), METHOD(quantize_scaled),
                          METHOD(quantize_pack_int4), METHOD(quantize_pack_scaled), METHOD(bind), {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_call", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -120,9 +120,13 @@ class Matmul:
             raise L.MmxError(f"Matmul: K = {K} must be at least {kstep}")
         n0 = 0 if n0 is None else n0
         n1 = N if n1 is None else n1
-        if not self.constB and not self.weight_int8 and n0 == 0 and n1 == N and L.gemm_unpacked(matA, matB, self.transposeB, ppkernel.descriptor()):
-            self.internalB = None  # read where it lay: nothing was packed
-            return
+        ep = None
+        if not self.constB and not self.weight_int8 and n0 == 0 and n1 == N:
+            ep = ppkernel.descriptor()
+            done, packed = L.gemm_once(matA, matB, self.transposeB, ep)
+            if done:
+                self.internalB = packed  # None: read where it lay, nothing was packed
+                return
         if not self.constB or self.internalB is None:
             if self.weight_int8:
                 if matB.dtype != torch.bfloat16:
@@ -141,7 +145,7 @@ class Matmul:
             # the int8 fragments are converted between LDS and the MFMA operand at every M (:1447-1497); no bf16 copy
             L.gemm(matA, self.internalB, N, ppkernel.descriptor(), b_dtype=L.I8, n0=n0, n1=n1)
         else:
-            L.gemm(matA, self.internalB, N, ppkernel.descriptor(), n0=n0, n1=n1)
+            L.gemm(matA, self.internalB, N, ep or ppkernel.descriptor(), n0=n0, n1=n1)
 
 
 class MatmulVector:

@@ -159,6 +159,31 @@ def test_unpacked(monkeypatch, M, K, N, trans, taken):
             L.gemm_unpacked(x[:, :-1], B, trans, mx.Epilogue(torch.zeros((M, N), device="cuda")))
 
 
+@pytest.mark.parametrize("M,K,N,trans", [(300, 288, 1440, True), (700, 96, 201, True), (300, 200, 70, False), (300, 8192, 64, True)])
+def test_packed_and_used_once(monkeypatch, M, K, N, trans):
+    """Where the library would have B packed first both launches are one native call, on any rows and columns; what it cannot say is left
+    to the Python form: a workspace that the stream does not have yet, operands that do not fit together."""
+    x, B, bias = _bf(M, K + 3)[:, :K], _bf(N, K) if trans else _bf(K, N), torch.randn(N, device="cuda")
+    op = mx.Matmul(False, trans)
+
+    def call():
+        y = torch.zeros((M, N + 3), device="cuda")
+        op(x, B, ppkernel=mx.BiasGeluStore(y[:, :N], mx.Steps.BIAS, bias))
+        return y
+    mx.workspace()
+    (native, python), answers = _both(monkeypatch, call)
+    assert native[1] == python[1] and np.array_equal(native[0], python[0])
+    assert answers[0] is None and isinstance(answers[1], torch.Tensor) and len(answers) == 2, answers
+    assert torch.equal(op.internalB, mx.repack_b(B, transpose=trans))
+    needs = mx.gemm_workspace_bytes(mx.BF16, mx.BF16, M, K, N) > 0
+    L.release_workspaces()
+    watch = _Watch(_host_call)
+    monkeypatch.setattr(L, "_native", watch)
+    assert np.array_equal(host_bits(call()), native[0]) and isinstance(watch.answers[1], torch.Tensor) == (not needs), watch.answers
+    with pytest.raises(L.MmxError, match="differ"):
+        L.gemm_once(x[:, :-1], B, trans, mx.Epilogue(torch.zeros((M, N), device="cuda")))
+
+
 @pytest.mark.parametrize("kind", ["bf16", "i8"])
 def test_matvec(monkeypatch, kind):
     M, K = 100, 96
