@@ -32,10 +32,10 @@ PEAK_HBM_GBS = 8000.0       # MI355X HBM3E
 # when the kernel that ran is the one profiled AND its source is the one that was profiled (first 16 hex digits of
 # the SHA-256 of the kernel's source file): after a change of the kernel the figure reads null until it is re-measured.
 MEASURED_TRAFFIC = {
-    "gemm_bf16_256x192_ring8w_out_bf16": {"bytes": (81709.6 * 2.000 + 27535.0 * 1.000) * 1024, "source": "mm_amx_amd/csrc/gemm_tile.hpp",
-                                          "sha": "0f698a79075577e5"},
-    "skinny_stream_w8": {"bytes": (22154.3 * 2.000 + 21.5 * 1.000) * 1024, "source": "mm_amx_amd/csrc/skinny.hip", "sha": "eac742926c040d29"},
-    "skinny_resident_w8_pair": {"bytes": (22616.5 * 2.000 + 344.0 * 1.000) * 1024, "source": "mm_amx_amd/csrc/skinny.hip", "sha": "eac742926c040d29"},
+    "gemm_bf16_256x192_ring8w_out_bf16": {"bytes": (81715.0 * 2.000 + 27588.4 * 1.000) * 1024, "source": "mm_amx_amd/csrc/gemm_tile.hpp",
+                                          "sha": "b3c87ac688e7db2f"},
+    "skinny_stream_w8": {"bytes": (22154.3 * 2.000 + 21.5 * 1.000) * 1024, "source": "mm_amx_amd/csrc/skinny.hip", "sha": "9a41beeeda6595f6"},
+    "skinny_resident_w8_pair": {"bytes": (22611.0 * 2.000 + 344.0 * 1.000) * 1024, "source": "mm_amx_amd/csrc/skinny.hip", "sha": "9a41beeeda6595f6"},
 }
 
 

@@ -1807,8 +1807,8 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
             return check_hip(hipGetLastError(), "skinny_resident_kernel launch");
         }
     }
-    // The streaming form needs all of x in LDS and at least two workgroups per CU (344 panels of N = 11008 must all
-    // be resident): 80 KiB of x each (4096 x 11008 int8 GEMV at M = 5-8: 13.0-13.4 -> 11.5-12.0 us against the chunked
+    // The streaming form needs all of x in LDS and, with more panels than CUs, two workgroups per CU (344 panels of N = 11008 must all
+    // be resident): 80 KiB of x each (stream_x_limit; 4096 x 11008 int8 GEMV at M = 5-8: 13.0-13.4 -> 11.5-12.0 us against the chunked
     // form; with one workgroup per CU, M = 12-16, it loses: 16.6-17.7 against 13.7-14.5 us).
     const bool bigx = !pairs && xbytes > 46 * 1024 && xbytes <= x_limit;
     const bool fills = s.x_rows == 2 && s.xpitch == row_bytes;  // (WHOLE_ROWS)
