@@ -134,3 +134,23 @@ def test_rows_that_end_inside_16_bytes_are_one_trip_to_memory():
         call = (mx.I8, B.data_ptr(), N, 512, N, 0, out.data_ptr(), torch.cuda.current_stream().cuda_stream)
         took[N] = call_us(lambda: mx.lib().mmx_repack_b(*call), n=50)
     assert took[3001] <= 1.7 * took[3008], took
+
+
+@pytest.mark.parametrize("K", [257, 2048, 2049, 4096, 4100, 8192, 8191, 8200, 12288, 12289])
+@pytest.mark.parametrize("N", [1, 8, 41])
+def test_int4_weights_read_once(po, K, N):
+    """[N, K] held in registers, 2, 4, 8 or 12 fragments a wavefront, and the first K that is not: rows at any address, columns that
+    do not fill a group, infinities, NaN and a column of zeros."""
+    rng = np.random.default_rng(K + N)
+    W = (rng.standard_normal((K, N)) * 0.05).astype(np.float32)
+    W[K - 1, N - 1] = 3.0  # (the largest of its column in the last place)
+    if N > 8:
+        W[:, 2], W[5, 3], W[K - 2, 4] = 0.0, np.inf, np.nan
+    W = po.f32_to_bf16(W)
+    q, deq = po.quantize_int4(W)
+    wide = torch.full((N + 1, K + 3), float("nan"), dtype=torch.bfloat16, device="cuda")
+    Wt = wide[1:, 1:K + 1]
+    Wt.copy_(dev_bf16(np.ascontiguousarray(W.T)))
+    packed, deq_gpu = mx.quantize_pack_int4(Wt, transpose=True)
+    assert np.array_equal(host_bits(deq_gpu).view(np.uint32), deq.view(np.uint32))
+    assert np.array_equal(host_bits(packed), po.pack_int4(q))
