@@ -476,37 +476,34 @@ def gemm_unpacked(A, B, transpose, ep):
     and does nothing, where packing B first is faster or the only way (repack_b, gemm): also for a call that wants K slices
     while the stream is being captured into a graph and has no workspace.  Such a first call is packed and not split, so its
     sums can differ in the last bits from an eager call's; call the shape once eagerly before capturing to have the same."""
-    return _unpacked_natively(A, B, transpose, ep) or _unpacked(A, B, transpose, ep)
+    if _native is not None and type(ep) is Epilogue:  # as in gemm()
+        device = _current_device()
+        stream = _raw_stream(device)
+        rc = _native.gemm_unpacked(A, B, transpose, _workspaces.get((device, stream)), device, stream,
+                                   ep.C, ep.steps, ep.bias, ep.deq, ep.deq_oc, ep.q, ep.q_oc)
+        if rc is not None:
+            _check(rc)
+            return True
+    return _unpacked(A, B, transpose, ep)
 
 
 def gemm_once(A, B, transpose, ep):
     """gemm_unpacked(), and where that would return False the packing and the product of a regular call: returns (whether C has been
     computed, the packed weights if B was packed for it)."""
-    if _unpacked_natively(A, B, transpose, ep):
-        return True, None
     if _native is not None and type(ep) is Epilogue:  # the query, the packing and the product took 13.3 us of host time for 696 x 288 x 1440, 8.5 on the device
         device = _current_device()
         stream = _raw_stream(device)
-        packed = _native.gemm_packing(A, B, transpose, _workspaces.get((device, stream)), device, stream,
-                                      ep.C, ep.steps, ep.bias, ep.deq, ep.deq_oc, ep.q, ep.q_oc)
+        args = (A, B, transpose, _workspaces.get((device, stream)), device, stream, ep.C, ep.steps, ep.bias, ep.deq, ep.deq_oc, ep.q, ep.q_oc)
+        rc = _native.gemm_unpacked(*args)
+        if rc is not None:
+            _check(rc)
+            return True, None
+        packed = _native.gemm_packing(*args)
         if packed is not None:
             if type(packed) is int:
                 _check(packed)
             return True, packed
     return _unpacked(A, B, transpose, ep), None
-
-
-def _unpacked_natively(A, B, transpose, ep):
-    if _native is None or type(ep) is not Epilogue:  # as in gemm()
-        return False
-    device = _current_device()
-    stream = _raw_stream(device)
-    rc = _native.gemm_unpacked(A, B, transpose, _workspaces.get((device, stream)), device, stream,
-                               ep.C, ep.steps, ep.bias, ep.deq, ep.deq_oc, ep.q, ep.q_oc)
-    if rc is None:
-        return False
-    _check(rc)
-    return True
 
 
 def _unpacked(A, B, transpose, ep):
