@@ -1562,32 +1562,63 @@ static bool short_tail(int wk, bool pairs, int M, int nfrag, int panels) {
     return nfrag <= (M <= 16 ? (wk == 1 && M <= 8 ? 32 : 24) : (wk == 0 ? 20 : 16));
 }
 
-// The same for gate/up pairs over bf16 weights, one workgroup on a CU: M x K x 2 N 12 x 1984 x 6400 11.3 -> 9.7, 21 x 3264 x 7936 18.8 -> 15.4,
-// 28 x 1984 x 10752 14.2 -> 11.7, 32 x 1024 x 4096 8.3 -> 7.4, 16 x 2432 x 16000 16.2 -> 15.8; a deep K with pairs for more than half of
-// the CUs is the chunked kernel's, which walks the panels side by side (16 x 4096 x 10752 20.0 / 21.0, x 16000 23.3 / 30.6; x 7936
-// 18.9 -> 18.1), and so are more pairs than CUs (21 x 1984 x 22016 21.3 / 22.5).
-static int stream_pair_x_limit(int wk, int nfrag, int panels) {
-    return wk == 0 && panels <= 2 * num_cus() && (nfrag < 224 || panels <= num_cus()) ? 156 * 1024 : 46 * 1024;
+// How long an x the streaming kernel takes, in bytes with its row of zeros; a longer one goes to the chunked kernel, which loads every
+// chunk of x and waits at a barrier per chunk, a chain that its few loads in flight do not hide.  The lines below lie where the two meet on
+// 2400 calls (M x K x N, us, chunked / streaming, weights rotated over 500 MB); what they leave behind is at most 1.2 % slower than the other way.
+//   rows: as s.x_rows.  Rows that are not whole aligned 16-byte pieces (not 2) are moved into place one by one on their way to LDS, by every
+//   workgroup, which is what a long x then spends its time on.
+// Gate/up pairs over bf16 weights: all of x in LDS, one workgroup on a CU (12 x 1984 x 2 3200 11.3 / 9.7, 21 x 3264 x 2 3968 18.8 / 15.4), with
+// panels for no more than all of the CUs whatever K and the rows are; with up to twice as many over whole rows, but not
+//   - over a deep K, where the chunked kernel walks gate and up side by side (16 x 4096 x 2 8000 23.3 / 30.6);
+//   - where a panel takes a multiple of 128 KiB (K 1985 to 2048), so that the workgroups' streams meet in the same memory channels
+//     (16 x 2048 x 2 7328 13.1 / 15.2, 30 x 2048 x 2 7712 15.0 / 16.2, 31 x 1990 x 2 8000 15.8 / 18.7);
+//   - for up to 16 rows with panels for more than 5/3 of the CUs (13 x 2304 x 2 8032 14.6 / 15.0, 15 x 1536 x 2 7008 10.6 / 10.8; 18 x 2304 x 2 8192 16.1 / 15.5).
+//   (Other rows with more panels than CUs: 27 x 2683 x 2 8160 19.3 / 21.4, 14 x 3047 x 2 6880 17.4 / 18.4.)
+static int stream_pair_x_limit(int wk, int M, int nfrag, int panels, int rows) {
+    const int cus = num_cus();
+    if (wk != 0 || panels > 2 * cus) return 46 * 1024;
+    if (panels > cus && (rows != 2 || nfrag >= 224 || (nfrag + 3) / 4 % 32 == 0 || (M <= 16 && 3 * panels > 5 * cus))) return 46 * 1024;
+    return 156 * 1024;
 }
 
-// The most bytes of x (with its row of zeros) with which a single-panel launch takes the streaming kernel; with more it takes the
-// chunked one, which loads every chunk of x and waits at a barrier per chunk, a chain that its few loads in flight do not hide.  slices:
-// of K, that the chunked kernel would have with a workspace (not whether there is one: it decides nothing else here).  us, chunked -> streaming, weights rotated over 500 MB:
-//   156 KiB, one workgroup on a CU, with panels for more than a third of the CUs and no more than all of them: M x K x N bf16
-//   16 x 2432 x 4800 8.9 -> 7.8, 24 x 1984 x 4800 9.0 -> 7.1, 16 x 4544 x 8000 15.4 -> 15.4; int8 weights 12 x 4544 x 4800 10.7 -> 8.6,
-//   32 x 1984 x 8000 9.3 -> 7.8; int4 4 x 8192 x 4800 13.1 -> 8.9, 8 x 8000 x 8000 13.7 -> 10.7; int8 x 8 x 6144 x 4800 12.0 -> 7.9,
-//   24 x 2048 x 8000 6.7 -> 6.0.  Not over a short int4 K (11 x 4416 x 8000 9.5 / 10.4).  With fewer panels slices put the idle CUs to
-//   work (int8 weights 4 x 9024 x 1280 9.2 / 10.8, int4 6 x 8192 x 1280 8.0 / 9.0); where there are slices for up to half of the CUs
-//   they are ahead over a deep bf16 K (16 x 4544 x 2880 10.1 / 11.2; 24 x 1984 7.9 -> 6.7) and over int4 with more than 4 rows
-//   (6 x 10624 x 2880 11.7 / 11.7; 2 rows 11.7 -> 10.3), and the other types gain up to 1.24 and lose at most 0.4 us (int8 x 32 x 4096 x 2880
-//   8.1 / 8.4).
-//   More panels than CUs: 80 KiB, two workgroups on a CU, over bf16 and int8 weights; over a deep int4 K with up to 4 rows 84 KiB
-//   (2 x 8192 x 11200 18.6 -> 13.9, 4 x 8192 x 8960 17.8 -> 14.7, 4 x 5440 x 8960 13.2 / 13.3); int8 x 24 x 2048 x 12800 8.5 / 8.8.
-static int stream_x_limit(int wk, int M, int K, int nfrag, int panels, int slices) {
-    const int cus = num_cus();
-    if (panels <= cus && 3 * panels > cus && (wk != 2 || nfrag >= 80) &&
-        (slices == 1 || 2 * panels > cus || (wk == 2 ? M <= 4 : (wk != 0 || K <= 2560)))) return 156 * 1024;
-    return wk <= 1 ? 80 * 1024 : (wk == 2 && panels > cus && M <= 4 && nfrag >= 96 ? 84 * 1024 : 46 * 1024);
+// One panel.  slices: of K, that the chunked kernel would have with a workspace (not whether there is one: it decides nothing else
+// here); fills: K fills its last fragment too.
+//   More panels than CUs: 80 KiB, two workgroups on a CU, over bf16 and int8 weights, 46 over the others; over a deep int4 K with up to 4
+//   rows 84 KiB (2 x 8192 x 11200 18.6 / 13.9, 4 x 8192 x 8960 17.8 / 14.7); int8 x 24 x 2048 x 12800 8.5 / 8.8.
+//   Up to a third of the CUs: the same; slices put the idle CUs to work (int8 weights 4 x 9024 x 1280 9.2 / 10.8, int4 6 x 8192 x 1280 8.0 / 9.0).
+//   In between all of x, 156 KiB, one workgroup on a CU: bf16 16 x 2432 x 4800 8.9 / 7.8; int8 weights 12 x 4544 x 4800 10.7 / 8.6; int4
+//   4 x 8192 x 4800 13.1 / 8.9, 8 x 8000 x 8000 13.7 / 10.7; int8 x 8 x 6144 x 4800 12.0 / 7.9; but not
+//   - over a short int4 K (11 x 4416 x 8000 9.5 / 10.4);
+//   - over rows that are not whole pieces, except up to 10 of them over int4 weights (4 x 8931 x 6176 0.61 of the chunked time, 11 x 5101 x 6304
+//     10.6 / 11.7) and over the others where there are no slices and panels for no more than 3/4 of the CUs (bf16 8 x 5291 x 6464 0.92, int8
+//     weights 6 x 8921 x 6144 0.78; 27 x 2559 x 7264 12.2 / 14.3, int8 weights 9 x 6375 x 7680 14.4 / 15.8; with slices bf16 31 x 2301 x 4032 9.1 / 12.4,
+//     int8 weights 14 x 4861 x 3680 9.7 / 12.9);
+//   - with slices for up to half of the CUs: nothing over a deep bf16 K (16 x 4544 x 2880 10.1 / 11.2), int4 with more than 4 rows (6 x 10624 x 2880
+//     11.7 / 11.7) and a K that does not fill its fragments (int8 weights 15 x 3240 x 3808 8.5 / 9.5), and of the rest what LDS serves without
+//     rows in the same banks and without many repeated loads in the last batch: bf16 112 KiB (27 x 2432 x 2784, 133 KiB, 8.6 / 9.0), 84
+//     where K is a multiple of 256 (32 x 1792 x 4000 8.0 / 8.4); int8 weights 120 (31 x 2432 x 3520, 152 KiB, 8.6 / 9.5) but none of
+//     13 to 15 fragments to a wavefront, which are loaded as 16, or more than 38 (13 x 3840 x 3264 8.4 / 8.8, 4 x 10944 x 3712 13.6 / 14.3);
+//     int8 x 108 with 15 to 32 fragments to a wavefront, 84 with others up to 40 (31 x 4864 x 3456, 152 KiB, 8.7 / 9.6, 31 x 2816 x 3584 7.3 / 7.7,
+//     13 x 10496 x 3232 11.7 / 12.5; 24 x 3840 x 3680 7.8 / 7.4);
+//   - with slices at all, int8 weights and more than 38 fragments to a wavefront (3 x 10496 x 4128 13.6 / 14.1);
+//   - with panels for more than 7/8 of the CUs: bf16 up to 8 rows (6 x 8064 x 8000 22.5 / 23.7 where every lane reads its own part of x, 6 x 6400 x 7968
+//     19.1 / 18.1) and int8 weights in 17 fragments to a wavefront, 20 loads of which 3 are repeats (15 x 4352 x 8064 11.1 / 11.7).
+static int stream_x_limit(int wk, int M, int K, int nfrag, int panels, int slices, int rows, bool fills) {
+    const int cus = num_cus(), usual = (wk <= 1 ? 80 : 46) * 1024, all = 156 * 1024, per_wave = (nfrag + 7) / 8;
+    if (panels > cus) return wk == 2 && M <= 4 && nfrag >= 96 ? 84 * 1024 : usual;
+    if (3 * panels <= cus || (wk == 2 && nfrag < 80)) return usual;
+    const bool few = slices > 1 && 2 * panels <= cus;
+    if (wk == 2) return few ? (M <= 4 ? all : usual) : (rows == 2 || M <= 10 ? all : usual);
+    if (rows != 2) return slices == 1 && M <= 10 && 4 * panels <= 3 * cus ? all : usual;
+    if (few) {
+        if (!fills) return usual;
+        if (wk == 0) return K > 2560 ? usual : (K % 256 ? 112 : 84) * 1024;
+        if (wk == 1) return (per_wave >= 13 && per_wave <= 15) || per_wave > 38 ? usual : 120 * 1024;
+        return per_wave > 40 ? usual : (per_wave >= 15 && per_wave <= 32 ? 108 : 84) * 1024;
+    }
+    if (wk == 1 && slices > 1 && per_wave > 38) return usual;
+    if (8 * panels > 7 * cus && ((wk == 0 && M <= 8) || (wk == 1 && per_wave == 17))) return usual;
+    return all;
 }
 
 // wk: weights are bf16 (0), int8 (1) or int4 (2); 3: int8 weights and int8 activations
@@ -1624,7 +1655,9 @@ int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int
     const bool pairs = (ep.steps & MMX_PP_SILU_GATE) != 0;
     // K slices that the chunked kernel would take (a workspace at hand, the library left to choose)
     const int ksl = !pairs && rq && rq->ws && rq->k_splits == 0 ? chunk_slices(wk != 0, M, s.nfrag, panels, rq->ws_bytes) : 1;
-    const int x_limit = pairs ? stream_pair_x_limit(wk, s.nfrag, panels) : stream_x_limit(wk, M, K, s.nfrag, panels, chunk_slices(wk != 0, M, s.nfrag, panels, ~(size_t)0));
+    const int x_limit = pairs ? stream_pair_x_limit(wk, M, s.nfrag, panels, s.x_rows)
+                              : stream_x_limit(wk, M, K, s.nfrag, panels, chunk_slices(wk != 0, M, s.nfrag, panels, ~(size_t)0), s.x_rows,
+                                               s.xpitch == row_bytes);
     // the streaming kernel, its limit of LDS raised where x needs it
     auto launch_stream = [&](StreamKernel kern, std::atomic<uint64_t>& raised, int lds, int zoff) {
         if (lds > 64 * 1024) {

@@ -95,23 +95,38 @@ def test_x_through_lds_in_chunks_and_half_panels(po, kind, M, K, N, splits, want
         check_float_parity(host_bits(C), ref, f"{kind} {M}x{K}x{N} pad={pad} {mx.last_kernel()}")
 
 
-# the largest x that each rule takes, the next larger one, few and many panels, K that fills its fragments and not
+# The largest x that each rule takes, the next larger one, few and many panels, K that fills its fragments and not.  stream: whether the
+# streaming kernel is the faster one, WHOLE: over rows that are whole aligned 16-byte pieces only (over others, chunked and streaming, us:
+# bf16 31 x 2301 x 4032 9.1 / 12.4, int8 weights 14 x 4861 x 3680 9.7 / 12.9).
+WHOLE = "whole rows"
+
+
 @pytest.mark.parametrize("kind,M,K,N,stream", [
-    ("bf16", 32, 2400, 4800, True), ("bf16", 32, 2424, 4800, False), ("bf16", 24, 1990, 2900, True), ("bf16", 24, 2624, 2900, False),
-    ("bf16", 16, 4544, 8192, True), ("w8", 16, 4544, 4807, True), ("w8", 31, 2450, 2900, True), ("w8", 31, 2496, 2900, False), ("w8", 8, 7360, 1280, False),
-    ("w4", 13, 5632, 4800, True), ("w4", 8, 5100, 4800, True), ("w4", 8, 5056, 4800, False), ("w4", 4, 6913, 2900, True), ("w4", 5, 6913, 2900, False),
+    ("bf16", 32, 2400, 4800, WHOLE), ("bf16", 32, 2424, 4800, False), ("bf16", 24, 1990, 2900, False), ("bf16", 24, 2624, 2900, False),
+    ("bf16", 16, 4544, 8192, WHOLE), ("w8", 16, 4544, 4807, WHOLE), ("w8", 31, 2450, 2900, False), ("w8", 31, 2496, 2900, False), ("w8", 8, 7360, 1280, False),
+    ("w4", 13, 5632, 4800, WHOLE), ("w4", 8, 5100, 4800, True), ("w4", 8, 5056, 4800, False), ("w4", 4, 6913, 2900, True), ("w4", 5, 6913, 2900, False),
     ("w4", 4, 8192, 8300, True), ("w4", 3, 6000, 8300, False),
     # (int4 shares of 9 to 21 fragments: every batch of the rolling window, with repeats and without)
     ("w4", 2, 4417, 100, True), ("w4", 1, 5120, 100, True), ("w4", 1, 5700, 100, True), ("w4", 1, 6300, 100, True), ("w4", 1, 7168, 100, True),
     ("w4", 1, 7681, 100, True), ("w4", 1, 8705, 100, True), ("w4", 1, 9984, 100, True), ("w4", 1, 10689, 100, True),
-    ("i8", 32, 4096, 4800, True), ("i8", 32, 4864, 4800, False), ("i8", 16, 4608, 1280, False), ("i8", 24, 2048, 8300, False)])
+    ("i8", 32, 4096, 4800, True), ("i8", 32, 4864, 4800, False), ("i8", 16, 4608, 1280, False), ("i8", 24, 2048, 8300, False),
+    # (rows that are not whole pieces: up to 10, panels for up to 3/4 of the CUs)
+    ("bf16", 10, 5005, 6100, True), ("bf16", 11, 5005, 6100, False), ("bf16", 10, 5005, 6150, False), ("w8", 9, 5853, 6100, True), ("w4", 11, 5101, 6300, False),
+    # (slices for up to half of the CUs)
+    ("bf16", 25, 2112, 2900, WHOLE), ("bf16", 27, 2432, 2900, False), ("bf16", 30, 1536, 2900, False), ("w8", 12, 4480, 2900, WHOLE), ("w8", 12, 4528, 2900, False),
+    ("w8", 13, 3840, 2900, False), ("w8", 4, 10944, 2900, False), ("i8", 22, 4352, 2900, True), ("i8", 26, 4864, 2900, False), ("i8", 6, 10240, 2900, True),
+    ("i8", 13, 10496, 2900, False),
+    # (and for more; panels for nearly all CUs)
+    ("w8", 4, 9728, 4128, WHOLE), ("w8", 3, 10496, 4128, False), ("bf16", 6, 8064, 8000, False), ("w8", 15, 4352, 8064, False), ("w8", 15, 4608, 8064, WHOLE)])
 def test_long_x_in_lds(po, kind, M, K, N, stream):
     x, packed, ref = _operands(po, kind, M, K, N, K + M)
+    es = 1 if kind == "i8" else 2
     for pad in ((8, 1) if kind != "i8" else (16, 0)):
         C = torch.zeros((M, N), dtype=torch.int32 if kind == "i8" else torch.float32, device="cuda")
         pad += -K % 8 if pad == 8 else 0
         mx.gemm(_in_nan((dev if kind == "i8" else dev_bf16)(x), pad), packed, N, mx.Epilogue(C), **KW[kind])
-        assert mx.last_kernel().startswith(f"skinny_{'stream' if stream else 'chunk'}_{kind}"), mx.last_kernel()
+        streams = (K * es % 16 == 0 and pad != 1) if stream is WHOLE else stream
+        assert mx.last_kernel().startswith((f"skinny_stream_{kind}",) if streams else (f"skinny_chunk_{kind}", f"skinny_direct_{kind}")), mx.last_kernel()
         if kind == "i8":
             assert np.array_equal(host_bits(C), ref), mx.last_kernel()
         else:
@@ -138,9 +153,12 @@ def test_gate_up(po, kind, M, K):
     assert np.linalg.norm(got - want) <= 2.0 ** -13 * np.linalg.norm(want), mx.last_kernel()
 
 
-# the largest x with one workgroup on a CU and the next one; x that LDS holds twice; K that fills the batches, its fragments, and neither
+# The largest x with one workgroup on a CU and the next one; x that LDS holds twice; K that fills the batches, its fragments, and neither;
+# more panels than CUs, where panels 128 KiB apart (K 1985 to 2048) are the chunked kernel's (16 x 2048 x 2 7328 13.1 / 15.2 us)
 @pytest.mark.parametrize("M,K,N,stream", [(28, 1344, 96, True), (17, 1001, 96, True), (32, 2400, 96, True), (32, 2424, 96, False), (16, 4096, 4096, True),
-                                          (16, 4096, 4160, False), (4, 7000, 96, True), (9, 2049, 8192, True), (9, 2688, 8224, False)])
+                                          (16, 4096, 4160, False), (4, 7000, 96, True), (9, 2049, 8192, True), (12, 2049, 8192, False), (9, 2688, 8224, False), (18, 2304, 8192, WHOLE),
+                                          (16, 2304, 6816, WHOLE), (16, 2304, 6848, False), (20, 2048, 4608, False), (20, 1990, 4608, False),
+                                          (20, 1984, 4608, WHOLE), (20, 2048, 4096, True)])
 def test_gate_up_over_a_long_x(M, K, N, stream):
     g = torch.Generator(device="cuda").manual_seed(K)
     x = torch.randn((M, K), device="cuda", generator=g).to(torch.bfloat16)
@@ -150,7 +168,8 @@ def test_gate_up_over_a_long_x(M, K, N, stream):
     for pad in (-K % 8 + 8, 5):
         h = torch.zeros((M, N), dtype=torch.float32, device="cuda")
         mx.gemm(_in_nan(x, pad), packed, 2 * N, mx.Epilogue(h, mx.PP_SILU_GATE))
-        assert mx.last_kernel() == f"skinny_{'stream' if stream else 'chunk'}_bf16_gateup", mx.last_kernel()
+        streams = (K % 8 == 0 and pad != 5) if stream is WHOLE else stream
+        assert mx.last_kernel() == f"skinny_{'stream' if streams else 'chunk'}_bf16_gateup", mx.last_kernel()
         want = a / (1.0 + torch.exp(-a)) * b  # silu within 2^-14, and twice that for the roundings around it
         assert (h.double() - want).norm() <= 2.0 ** -13 * want.norm(), mx.last_kernel()
 
