@@ -34,8 +34,8 @@ PEAK_HBM_GBS = 8000.0       # MI355X HBM3E
 MEASURED_TRAFFIC = {
     "gemm_bf16_256x192_ring8w_out_bf16": {"bytes": (81715.8 * 2.000 + 27420.5 * 1.000) * 1024, "source": "mm_amx_amd/csrc/gemm_tile.hpp",
                                           "sha": "ff3404236ca7fb7d"},
-    "skinny_stream_w8": {"bytes": (22154.3 * 2.000 + 21.5 * 1.000) * 1024, "source": "mm_amx_amd/csrc/skinny.hip", "sha": "9a41beeeda6595f6"},
-    "skinny_resident_w8_pair": {"bytes": (22611.0 * 2.000 + 344.0 * 1.000) * 1024, "source": "mm_amx_amd/csrc/skinny.hip", "sha": "9a41beeeda6595f6"},
+    "skinny_stream_w8": {"bytes": (22137.2 * 2.000 + 21.5 * 1.000) * 1024, "source": "mm_amx_amd/csrc/skinny.hip", "sha": "16d953824b6381ca"},
+    "skinny_resident_w8_pair": {"bytes": (22611.0 * 2.000 + 344.0 * 1.000) * 1024, "source": "mm_amx_amd/csrc/skinny.hip", "sha": "16d953824b6381ca"},
 }
 
 

@@ -177,14 +177,15 @@ int mmx_gemm(int a_dtype, int b_dtype, const void* A, int64_t lda_bytes, const v
  *             suffices for k_splits = 0; with less, the choice is restricted to what fits).  Its first 16 KiB are
  *             arrival counters: zero them once after allocation; every call leaves them zero.  Calls that share
  *             a workspace must not overlap in time (different streams need different workspaces).  With k_splits = 0
- *             dense rows of A (lda_bytes = K * sizeof(T), more than 32) that are not whole 16-byte pieces are also
- *             copied to its end, aligned, where that is the faster way and it has room: two launches.
+ *             dense rows of A (lda_bytes = K * sizeof(T); more than 32 of bf16, any number of int8) that are not
+ *             whole 16-byte pieces are also copied to its end, aligned, where that is the faster way and it
+ *             has room: two launches.
  * With workspace = NULL this is mmx_gemm. */
 int mmx_gemm_splitk(int a_dtype, int b_dtype, const void* A, int64_t lda_bytes, const void* Bpacked, int M, int K,
                     int N, int n0, int n1, const mmx_epilogue* ep, int k_splits, void* workspace,
                     size_t workspace_bytes, void* stream);
-/* Workspace the call above would use for this shape (0 if it would neither split nor copy A; where it would split, the
- * slices' share only, beside which a copy has room in the 64 MiB + 16 KiB).  steps = the post-op steps.  For decode
+/* Workspace the call above would use for this shape (0 if it would neither split nor copy A).  With this much it makes the same
+ * choices, and so the same sums, as with 64 MiB + 16 KiB, whatever the stride of A is.  steps = the post-op steps.  For decode
  * shapes (M <= 32) the figure is an upper bound: it looks at the number of panels and the length of K only, and a launch
  * whose x fits in LDS, or whose K or alignment takes another kernel, does not split after all.  The answer depends on the
  * device's CU count: call mmx_init first. */

@@ -61,20 +61,20 @@ int ensure_dynamic_lds(const void* kernel, int bytes, std::atomic<uint64_t>& don
 }
 
 
-size_t skinny_workspace_bytes(int wk, int M, int K, int n0, int n1);
+size_t skinny_workspace_bytes(int wk, int M, int K, int n0, int n1, size_t most);
 int launch_gemm_tiles_bf16(const void* A, int64_t lda, const void* Bp, int M, int K, int N, int n0, int n1,
                            const Epilogue& ep, const SplitRequest& rq, hipStream_t st);
 int launch_gemm_tiles_i8(const void* A, int64_t lda, const void* Bp, int M, int K, int N, int n0, int n1,
                          const Epilogue& ep, const SplitRequest& rq, hipStream_t st);
 int launch_gemm_tiles_w8(const void* A, int64_t lda, const void* Bp, int M, int K, int N, int n0, int n1,
                          const Epilogue& ep, const SplitRequest& rq, hipStream_t st);
-size_t plan_workspace_bytes(int elesz, bool w8, int M, int K, int Ncols, uint32_t steps, int k_splits);
+size_t plan_workspace_bytes(int elesz, bool w8, int M, int K, int Ncols, uint32_t steps, int k_splits, size_t most);
 bool skinny_i8_eligible(const void* x, int64_t ldx, int M, int K, int k_splits);
 int launch_skinny(int wk, const void* x, int64_t ldx, const void* Wp, int M, int K, int N, int n0, int n1,
                   const Epilogue& ep, hipStream_t st, const SplitRequest* rq);
 int launch_wave_ring(int type, const void* A, int64_t lda, const void* Bp, int M, int K, int N, int n0, int n1, const Epilogue& ep,
                      const SplitRequest& rq, float tiles_us, hipStream_t st);
-int64_t wave_ring_workspace_bytes(int type, int M, int K, int Ncols, bool pairs, int k_splits, float tiles_us);
+int64_t wave_ring_workspace_bytes(int type, int M, int K, int Ncols, bool pairs, int k_splits, size_t most, float tiles_us);
 float plan_us(int elesz, bool w8, int M, int K, int Ncols, uint32_t steps, const SplitRequest& rq);
 bool unpacked_can(int M, int K, int N, int64_t lda, int64_t ldb, int transpose);
 bool unpacked_takes(int M, int K, int N, int64_t lda, int64_t ldb, int transpose);
@@ -178,7 +178,8 @@ static int make_epilogue(const mmx_epilogue* in, int a_dtype, int b_dtype, int M
 // 200 x 4001 x 4096 34 -> 14; int8 weights 800 x 1001 x 1024 20.3 -> 10.7.  Of 174 shapes (40 to 1600 rows, K 257 to 5001, 256 to 9654
 // columns) the copy loses on 7 of short rows (up to 1024 bytes) with much to multiply, at most 1.12 (800 x 515 x 4096 int8 11.1 / 12.4, 200 x 257 x 9654
 // bf16 10.0 / 10.9), and on one behind that line (int8 weights 800 x 515 x 4096 15.2 / 15.6); short rows with little are ahead (40 x 257 x 256 8.8 / 6.6).
-// (Dense rows: the workspace query, which knows K but not the stride, foresees them, so that a first call takes the same way.)
+// (Dense rows: the workspace query, which knows K but not the stride, counts them in, so that a first call takes the same way.)
+static size_t round256(size_t n) { return (n + 255) & ~(size_t)255; }
 static int copied_pitch(int es, int K) { return (int)(((int64_t)K * es + 127) / 128 * 128); }
 static bool copy_pays(int es, int M, int K, int Ncols) {
     const int64_t row = (int64_t)K * es;
@@ -250,6 +251,25 @@ static int signed_gemm_i32(const void* A, int64_t lda, const void* Bp, int M, in
     e.ldc_bytes = ldacc_bytes;
     const SplitRequest none = {1, nullptr, 0};
     return gemm_dispatch(MMX_I8, MMX_I8, A, lda, Bp, M, K, N, n0, n1, &e, none, st);
+}
+
+// Bytes of a workspace of `most` that the K slices of a call would take (0: none); rows of A aligned where its K can be.
+static size_t slices_workspace_bytes(int a_dtype, int b_dtype, int M, int K, int N, int n0, int n1, uint32_t steps, int k_splits, size_t most) {
+    const bool bf = a_dtype == MMX_BF16 && b_dtype == MMX_BF16, i8 = a_dtype == MMX_I8 && b_dtype == MMX_I8;
+    const bool w8 = a_dtype == MMX_BF16 && b_dtype == MMX_I8;
+    const bool w4 = a_dtype == MMX_BF16 && b_dtype == MMX_I4;
+    // int8 activations that the decode kernels do not take, by K or by a forced tile, go to the tile kernels at any M
+    const bool i8_tiles = i8 && M > 0 && K > 0 && (forced_tile().bm != 0 || !skinny_i8_eligible(nullptr, 0, M, K, k_splits));
+    if (M > 0 && M <= 32 && !i8_tiles && (bf || w8 || i8 || w4) && K > 0 && N > 0 && n0 >= 0 && n1 <= N && n0 < n1)
+        return k_splits == 0 && !(steps & MMX_PP_SILU_GATE) ? skinny_workspace_bytes(i8 ? 3 : (w4 ? 2 : (w8 ? 1 : 0)), M, K, n0, n1, most) : 0;
+    if ((!bf && !i8 && !w8) || (M <= 32 && !i8_tiles) || K <= 0 || N <= 0 || n0 < 0 || n1 > N || n0 >= n1 || k_splits < 0) return 0;
+    if (k_splits <= 1 && forced_tile().bm == 0 && load_mode() == 2) {
+        const SplitRequest any = {k_splits, reinterpret_cast<char*>(256), most};
+        const int64_t need = wave_ring_workspace_bytes(i8 ? 3 : (w8 ? 1 : 0), M, K, n1 - n0, (steps & MMX_PP_SILU_GATE) != 0, k_splits, most,
+                                                       plan_us(i8 ? 1 : 2, w8, M, K, n1 - n0, steps, any));
+        if (need >= 0) return (size_t)need;
+    }
+    return plan_workspace_bytes(i8 ? 1 : 2, w8, M, K, n1 - n0, steps, k_splits, most);
 }
 
 }  // namespace mmx
@@ -400,24 +420,18 @@ int mmx_gemm_splitk_static(int a_dtype, int b_dtype, const void* A, int64_t lda_
 }
 
 size_t mmx_gemm_workspace_bytes(int a_dtype, int b_dtype, int M, int K, int N, int n0, int n1, uint32_t steps, int k_splits) {
-    const bool bf = a_dtype == MMX_BF16 && b_dtype == MMX_BF16, i8 = a_dtype == MMX_I8 && b_dtype == MMX_I8;
-    const bool w8 = a_dtype == MMX_BF16 && b_dtype == MMX_I8;
-    const bool w4 = a_dtype == MMX_BF16 && b_dtype == MMX_I4;
-    // int8 activations that the decode kernels do not take, by K or by a forced tile, go to the tile kernels at any M
-    const bool i8_tiles = i8 && M > 0 && K > 0 && (forced_tile().bm != 0 || !skinny_i8_eligible(nullptr, 0, M, K, k_splits));
-    if (M > 0 && M <= 32 && !i8_tiles && (bf || w8 || i8 || w4) && K > 0 && N > 0 && n0 >= 0 && n1 <= N && n0 < n1)
-        return k_splits == 0 && !(steps & MMX_PP_SILU_GATE) ? skinny_workspace_bytes(i8 ? 3 : (w4 ? 2 : (w8 ? 1 : 0)), M, K, n0, n1) : 0;
-    if ((!bf && !i8 && !w8) || (M <= 32 && !i8_tiles) || K <= 0 || N <= 0 || n0 < 0 || n1 > N || n0 >= n1 || k_splits < 0) return 0;
-    if (k_splits <= 1 && forced_tile().bm == 0 && load_mode() == 2) {
-        const SplitRequest any = {k_splits, reinterpret_cast<char*>(256), ~(size_t)0};
-        const int64_t need = wave_ring_workspace_bytes(i8 ? 3 : (w8 ? 1 : 0), M, K, n1 - n0, (steps & MMX_PP_SILU_GATE) != 0, k_splits,
-                                                       plan_us(i8 ? 1 : 2, w8, M, K, n1 - n0, steps, any));
-        if (need > 0) return (size_t)need;
-        const int es = i8 ? 1 : 2;
-        const size_t slices = need < 0 ? plan_workspace_bytes(es, w8, M, K, n1 - n0, steps, k_splits) : 0;
-        return slices == 0 && k_splits == 0 && copy_pays(es, M, K, n1 - n0) ? WS_COUNTER_BYTES + (size_t)M * copied_pitch(es, K) + 256 : slices;
-    }
-    return plan_workspace_bytes(i8 ? 1 : 2, w8, M, K, n1 - n0, steps, k_splits);
+    const size_t slices = slices_workspace_bytes(a_dtype, b_dtype, M, K, N, n0, n1, steps, k_splits, ~(size_t)0);
+    const int es = elesz_of(a_dtype);
+    const bool tiles = (M > 32 || a_dtype == MMX_I8) && (a_dtype == MMX_BF16 || a_dtype == MMX_I8) && (b_dtype == MMX_I8 || b_dtype == a_dtype);
+    if (!tiles || M <= 0 || K <= 0 || N <= 0 || n0 < 0 || n1 > N || n0 >= n1 || k_splits != 0 || forced_tile().bm != 0 || load_mode() != 2 ||
+        !copy_pays(es, M, K, n1 - n0)) return slices;
+    // dense rows are copied, and the call goes on as one of their pitch beside the copy: what it then chooses beside one in a workspace of the
+    // standard size has to fit, or a workspace of this size would have other slices, and so other sums
+    const int pitch = copied_pitch(es, K);
+    const size_t copy = round256((size_t)M * pitch);
+    const size_t rest = slices_workspace_bytes(a_dtype, b_dtype, M, pitch / es, N, n0, n1, steps, 0, WS_STANDARD_BYTES - copy);
+    const size_t copied = round256(rest > WS_COUNTER_BYTES ? rest : WS_COUNTER_BYTES) + copy;
+    return copied > slices ? copied : slices;  // (A may have aligned rows of this K too)
 }
 
 int64_t mmx_gemm_unpacked_workspace_bytes(int dtype, int M, int K, int N, int64_t lda_bytes, int64_t ldb_bytes, int transpose) {

@@ -33,12 +33,12 @@ float plan_us(int elesz, bool w8, int M, int K, int Ncols, uint32_t steps, const
     return (pairs ? 1.2f : (w8 ? 1.1f : 1.0f)) * (1.3f + 0.0004f * choose_plan(M, Ncols, (int)((kbytes + 127) / 128), pairs, w8, kbytes % 128 ? 4 : 2, rq, elesz == 1).cycles);
 }
 
-// Bytes of workspace the plan for this shape would use (0: no K split), assuming operands the ring pipeline takes: rows of
+// Bytes of a workspace of `most` that the plan for this shape would use (0: no K split), assuming operands the ring pipeline takes: rows of
 // any K can be aligned through their stride, so this is an upper bound for those that are not.
-size_t plan_workspace_bytes(int elesz, bool w8, int M, int K, int Ncols, uint32_t steps, int k_splits) {
+size_t plan_workspace_bytes(int elesz, bool w8, int M, int K, int Ncols, uint32_t steps, int k_splits, size_t most) {
     const int64_t kbytes = (int64_t)K * elesz;
     if (kbytes % 128 && (k_splits > 1 || kbytes < 128)) return 0;  // (a forced split of a K with a tail is refused)
-    const SplitRequest rq = {k_splits, reinterpret_cast<char*>(256), ~(size_t)0};
+    const SplitRequest rq = {k_splits, reinterpret_cast<char*>(256), most};
     if (steps & MMX_PP_SILU_GATE) return 0;
     const Plan p = choose_plan(M, Ncols, (int)((kbytes + 127) / 128), false, w8, kbytes % 128 ? 4 : 2, rq, elesz == 1);
     if (p.S <= 1) return 0;

@@ -1425,10 +1425,10 @@ static int fragments(int wk, int K) {
 }
 static int fragment_x_bytes(int wk) { return wk == 2 ? 128 : (wk == 1 ? 64 : 32); }
 
-// Bytes of workspace a decode launch of this shape can use (0: it takes no K split)
-size_t skinny_workspace_bytes(int wk, int M, int K, int n0, int n1) {
+// Bytes of a workspace of `most` that a decode launch of this shape can use (0: it takes no K split)
+size_t skinny_workspace_bytes(int wk, int M, int K, int n0, int n1, size_t most) {
     const int panels = ((n1 + 31) >> 5) - (n0 >> 5);
-    const int S = chunk_slices(wk != 0, M, fragments(wk, K), panels, ~(size_t)0);
+    const int S = chunk_slices(wk != 0, M, fragments(wk, K), panels, most);
     return S > 1 ? WS_COUNTER_BYTES + (size_t)panels * S * 4096 : 0;
 }
 

@@ -458,9 +458,9 @@ int launch_wave_ring(int type, const void* A, int64_t lda, const void* Bp, int M
 // Bytes of workspace the call above can use (0: no slices), or -1 if it would leave the call to the tile kernels.  Rows are counted in
 // whole 64s: an upper bound, and one answer for counts of rows in the same 64 that get the same form and slices.  (Rows of A that
 // are not aligned go to the masked pipeline there, which takes no slices.)
-int64_t wave_ring_workspace_bytes(int type, int M, int K, int Ncols, bool pairs, int k_splits, float tiles_us) {
+int64_t wave_ring_workspace_bytes(int type, int M, int K, int Ncols, bool pairs, int k_splits, size_t most, float tiles_us) {
     if (!wave_ring_can(type, K, true)) return -1;
-    const WaveRingPlan p = choose_form(type, M, K, Ncols, pairs, k_splits, ~(size_t)0);
+    const WaveRingPlan p = choose_form(type, M, K, Ncols, pairs, k_splits, most);
     if (p.form < 0 || p.us >= WIN * tiles_us) return -1;
     const Form& c = FORMS[p.form];
     if (p.slices == 1) return 0;

@@ -103,12 +103,16 @@ def test_no_automatic_workspace_is_larger_than_the_standard_one(lib):
 
 
 def test_the_workspace_query_covers_every_call_that_splits(lib):
-    """The query knows K but not the stride of A's rows: rows of any K can be 16-byte aligned, and such rows are split."""
+    """The query knows K but not the stride of A's rows: rows of any K can be 16-byte aligned, and such rows are split; dense ones are copied
+    first, and the call that is made of the copy is split beside it."""
     import mm_amx_amd._lib as L
     need = lib.mmx_gemm_workspace_bytes
     need.restype = C.c_size_t
     for a, b, K in ((L.BF16, L.BF16, 4100), (L.BF16, L.I8, 4099), (L.I8, L.I8, 8199)):
-        assert need(a, b, 64, K, 256, 0, 256, 0, 0) == need(a, b, 64, K + 16 - K % 16, 256, 0, 256, 0, 0) > 0
+        es, pitch = (1 if a == L.I8 else 2), (K * (1 if a == L.I8 else 2) + 127) // 128 * 128
+        assert need(a, b, 64, K, 256, 0, 256, 0, 0) == need(a, b, 64, pitch // es, 256, 0, 256, 0, 0) + 64 * pitch
+        assert need(a, b, 64, K, 256, 0, 256, 0, 0) > need(a, b, 64, K + 16 - K % 16, 256, 0, 256, 0, 0) > 0
+        assert need(a, b, 64, K, 256, 0, 256, 0, 2) == need(a, b, 64, K, 256, 0, 256, 0, 1) == 0  # (no copy where the slices are not the library's choice)
     # int8 rows that the decode kernels do not take (K no multiple of 128) go to the tile kernels at any M
     assert need(L.I8, L.I8, 16, 8256, 256, 0, 256, 0, 0) == need(L.I8, L.I8, 33, 8256, 256, 0, 256, 0, 0) > 0
 

@@ -232,6 +232,48 @@ def test_dense_rows_that_are_not_whole_pieces(po, kind, M, K, N):
     assert not ws[:16 << 10].any().item() and (ws[room:] == 0xA5).all().item()
 
 
+# few rows and many, slices of every kind of kernel that the copy goes on to and none, a column range; int8 down to one row (the decode kernels)
+@pytest.mark.parametrize("kind,M,K,N,n0,n1", [("bf16", 40, 1001, 1024, 0, 1024), ("bf16", 100, 5001, 1000, 0, 1000), ("bf16", 300, 2234, 700, 64, 601), ("bf16", 64, 9001, 512, 0, 512),
+                                              ("bf16", 500, 9001, 1100, 0, 1100), ("bf16", 700, 700, 900, 0, 900), ("w8", 64, 4099, 256, 0, 256), ("w8", 300, 8001, 2000, 0, 2000),
+                                              ("i8", 64, 8199, 256, 0, 256), ("i8", 400, 3333, 1000, 0, 1000), ("i8", 1, 4001, 300, 0, 300), ("i8", 17, 9990, 640, 0, 640),
+                                              ("i8", 32, 515, 1000, 32, 1000), ("i8", 32, 7999, 640, 0, 640)])
+def test_the_workspace_query_is_enough(po, kind, M, K, N, n0, n1):
+    """Dense rows of an odd K with a workspace of just the size that the query names: the kernel and the bits are those of the standard
+    workspace, and what lies behind it stays; with 256 bytes less the copy or a slice does not fit, and the result is right all the same."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    x = torch.randint(-127, 128, (M, K), device="cuda", generator=g, dtype=torch.int8)
+    W = torch.randint(-127, 128, (K, N), device="cuda", generator=g, dtype=torch.int8)
+    if kind != "i8":
+        x = x.to(torch.bfloat16)
+    packed = mx.repack_b(W if kind != "bf16" else W.to(torch.bfloat16))
+    # (products of whole numbers below 2^24 in every partial sum of int8; of bf16 the sums are compared to the precision of 32 bits)
+    want = (x.double() @ W.double())[:, n0:n1]
+    types, es = (mx.I8 if kind == "i8" else mx.BF16, mx.BF16 if kind == "bf16" else mx.I8), 1 if kind == "i8" else 2
+    need = mx.gemm_workspace_bytes(*types, M, K, N, n0=n0, n1=n1)
+    pitch = (K * es + 127) // 128 * 128
+    beside = max(16 << 10, mx.gemm_workspace_bytes(*types, M, pitch // es, N, n0=n0, n1=n1))
+    tight = M > 32 and need < beside + M * pitch + 512  # (not where aligned rows of this K take more, for slices)
+    assert (16 << 10) < need <= mx._lib.WORKSPACE_BYTES
+    answers = []
+    for size in (mx._lib.WORKSPACE_BYTES, need, need - 256):
+        ws = torch.zeros(mx._lib.WORKSPACE_BYTES + 4096, dtype=torch.uint8, device="cuda")
+        ws[size:] = 0xA5
+        C = torch.zeros((M, N), dtype=torch.int32 if kind == "i8" else torch.float32, device="cuda")
+        mx.gemm(x, packed, N, mx.Epilogue(C), b_dtype=types[1], n0=n0, n1=n1, ws=ws[:size])
+        answers.append((mx.last_kernel(), C))
+        assert (ws[size:] == 0xA5).all().item() and not ws[:16 << 10].any().item(), (size, mx.last_kernel())
+        if kind == "i8":
+            assert torch.equal(C[:, n0:n1].double(), want), (size, mx.last_kernel())
+        else:  # 32-bit sums of K products, in any order
+            assert ((C[:, n0:n1].double() - want).abs() <= K * 2.0 ** -24 * (x.double().abs() @ W.double().abs())[:, n0:n1]).all(), (size, mx.last_kernel())
+        assert not C[:, :n0].any().item() and not C[:, n1:].any().item()
+    assert answers[0][0].endswith("_rows_copied") and answers[1][0] == answers[0][0], [a[0] for a in answers]
+    assert not tight or answers[2][0] != answers[0][0], [a[0] for a in answers]
+    assert torch.equal(answers[0][1], answers[1][1])
+    if kind == "i8" and M <= 32:  # (the decode kernels take the copy where x fits in LDS or its rows are whole chunks)
+        assert answers[0][0].startswith("skinny_") == (M * pitch <= 45 << 10 or pitch % 256 == 0), answers[0][0]
+
+
 def test_dense_rows_replay_from_a_graph():
     """Copy and product in a captured graph, new rows before each replay."""
     M, K, N = 200, 1335, 384
