@@ -175,14 +175,19 @@ static int make_epilogue(const mmx_epilogue* in, int a_dtype, int b_dtype, int M
 // k-iteration and has one tile shape.  Where a workspace is at hand they are copied there first, aligned and padded with zeros to whole
 // k-iterations, and the call goes on as one of that shape.  us, masked -> copied and multiplied (two launches, 6.8 us of host time):
 // bf16 40 x 1001 x 1024 19.1 -> 7.4, 100 x 5001 x 4096 72 -> 17, 800 x 5001 x 9654 236 -> 97, 1600 x 2234 x 9654 126 -> 77; int8
-// 200 x 4001 x 4096 34 -> 14; int8 weights 800 x 1001 x 1024 20.3 -> 10.7.  Of 174 shapes (40 to 1600 rows, K 257 to 5001, 256 to 9654
-// columns) the copy loses on 7 of short rows (up to 1024 bytes) with much to multiply, at most 1.12 (800 x 515 x 4096 int8 11.1 / 12.4, 200 x 257 x 9654
-// bf16 10.0 / 10.9), and on one behind that line (int8 weights 800 x 515 x 4096 15.2 / 15.6); short rows with little are ahead (40 x 257 x 256 8.8 / 6.6).
+// 200 x 4001 x 4096 34 -> 14; int8 weights 800 x 1001 x 1024 20.3 -> 10.7; int8 down to one row, where the copy is a decode call 1 x 6081 x 422 35 -> 9.0,
+// 17 x 555 x 8767 8.4 -> 7.8, 32 x 1347 x 8246 15.2 -> 10.3.  Not short rows (up to 1024 bytes) with much to multiply (800 x 515 x 4096 int8 11.1 / 12.4,
+// 200 x 257 x 9654 bf16 10.0 / 10.9; with little 40 x 257 x 256 8.8 / 6.6), and not many rows of up to 1700 bytes where the masked kernel has one nearly
+// full round of its 128 x 128 tiles (int8 1867 x 1109 x 2103 15.5 / 18.8, int8 weights 1917 x 669 x 1952 15.7 / 16.8, bf16 2014 x 577 x 1372 14.2 / 15.0;
+// fewer rows int8 994 x 1297 x 2276 16.1 / 14.5).  On 600 shapes (1 to 2040 rows, rows of 512 to 16000 bytes) what is copied is at most 1.03
+// times the masked time (int8 weights 967 x 571 x 2228 13.3 / 13.7).
 // (Dense rows: the workspace query, which knows K but not the stride, counts them in, so that a first call takes the same way.)
 static size_t round256(size_t n) { return (n + 255) & ~(size_t)255; }
 static int copied_pitch(int es, int K) { return (int)(((int64_t)K * es + 127) / 128 * 128); }
 static bool copy_pays(int es, int M, int K, int Ncols) {
     const int64_t row = (int64_t)K * es;
+    const int64_t tiles = (int64_t)((M + 127) / 128) * ((Ncols + 127) / 128), cus = num_cus();
+    if (25 * tiles > 13 * cus && tiles <= cus && row <= 1700 && 10 * row <= 11 * (int64_t)M) return false;
     return row % 16 && (int64_t)M * copied_pitch(es, K) <= (int64_t)(WS_STANDARD_BYTES / 2) &&
            (row > 1024 || (row >= 512 && (int64_t)M * K * Ncols <= 100000000));
 }
