@@ -314,8 +314,9 @@ __device__ __forceinline__ void for_each_8_weights(const char* __restrict__ W, i
                 if (first * 8 < cols) f(r, first * 8, v[0]);
                 continue;
             }
-            // One load instruction for the whole wavefront: with the row's last lane in a branch of its own, its load, into the
-            // same registers as the other lanes' load still in flight, delivered wrong bytes now and then.
+            // One load instruction for the whole wavefront, the row's end in it.  (A draft that loaded the end in a branch of its own gave
+            // wrong bytes now and then on the GPU.  Why is not known: compiled again, that form waits for both loads before
+            // either is used, and its offsets stay in the row.)
             for (int64_t i = first; i * 8 < cols; i += step) {
                 const int64_t at = i * 16, last = len - 16, from = at < last ? at : last;
                 u32x4 v = load16<2>(row + from);
@@ -882,23 +883,12 @@ __global__ __launch_bounds__(QUANT4_WAVES * 64) void quant4_pack_kernel(const ch
             if (n0 + c < N) {
                 const char* const row = W + (int64_t)(n0 + c) * ldw;
                 for (int k = lane * 8; k < K; k += 512 * UNR) {
+                    // (past the end of the row its last 16 bytes, which a maximum may meet twice: one load instruction for the whole wavefront)
                     u32x4 v[UNR];
-                    if (k + 512 * (UNR - 1) + 8 <= K) {
 #pragma unroll
-                        for (int u = 0; u < UNR; u++) v[u] = load16<2>(row + (int64_t)(k + 512 * u) * 2);
-                    } else {
-#pragma unroll
-                        for (int u = 0; u < UNR; u++) {
-                            v[u] = u32x4{0u, 0u, 0u, 0u};
-                            if (k + 512 * u + 8 <= K) v[u] = load16<2>(row + (int64_t)(k + 512 * u) * 2);
-                        }
-#pragma unroll
-                        for (int u = 0; u < UNR; u++)
-                            if (k + 512 * u < K && k + 512 * u + 8 > K) {
-                                u32x4 w[1];
-                                load16_rows<2>(w, (int64_t)(k + 512 * u) * 2, (int64_t)K * 2, [&](int) { return row; }, [&](int) { return true; });
-                                v[u] = w[0];
-                            }
+                    for (int u = 0; u < UNR; u++) {
+                        const int from = k + 512 * u < K - 8 ? k + 512 * u : K - 8;
+                        v[u] = load16<2>(row + (int64_t)from * 2);
                     }
 #pragma unroll
                     for (int u = 0; u < UNR; u++)

@@ -154,3 +154,21 @@ def test_int4_weights_read_once(po, K, N):
     packed, deq_gpu = mx.quantize_pack_int4(Wt, transpose=True)
     assert np.array_equal(host_bits(deq_gpu).view(np.uint32), deq.view(np.uint32))
     assert np.array_equal(host_bits(packed), po.pack_int4(q))
+
+
+@pytest.mark.parametrize("K", [12290, 12295, 12296, 12297, 14336, 14337, 14343, 14344, 16383])
+@pytest.mark.parametrize("N", [1, 33])
+def test_int4_weights_of_a_deep_k(po, K, N):
+    """[N, K] that is read twice (K > 12288): rows that end anywhere in a lane's 16 bytes and in a lane's four loads, a largest weight at
+    their end, infinities around them that take no part."""
+    rng = np.random.default_rng(K + N)
+    W = (rng.standard_normal((K, N)) * 0.05).astype(np.float32)
+    W[K - 1 - np.arange(N) % 9, np.arange(N)] = 2.0 + np.arange(N)
+    W = po.f32_to_bf16(W)
+    q, deq = po.quantize_int4(W)
+    wide = torch.full((N + 2, K + 3), float("inf"), dtype=torch.bfloat16, device="cuda")
+    Wt = wide[1:N + 1, 1:K + 1]
+    Wt.copy_(dev_bf16(np.ascontiguousarray(W.T)))
+    packed, deq_gpu = mx.quantize_pack_int4(Wt, transpose=True)
+    assert np.array_equal(host_bits(deq_gpu).view(np.uint32), deq.view(np.uint32))
+    assert np.array_equal(host_bits(packed), po.pack_int4(q))
