@@ -294,7 +294,7 @@ inline PackedB<T> repackB_1x2(const tensor2D<T>& Bi, bool transpose = false, hip
 // becomes int8_t(w * scale), the bf16 product rounded to nearest even and then truncated toward zero (:80-81; saturated
 // here where the reference's conversion is undefined).  L = 1..4 tiles of 16 columns side by side only orders the
 // reference's cache layout: its preconditions are kept (K a multiple of 32, N of 16 L), the result is this library's
-// fragment order.
+// fragment order.  In stream order, like repackB_1x2: nothing is waited for.
 template <typename T, int L>
 inline PackedB<T> repackB_1xL(const tensor2D<bfloat16>& Bi, float scale = 1.0f, hipStream_t stream = nullptr) {
     static_assert(L >= 1 && L <= 4, "L = 1 ... 4");
@@ -309,7 +309,6 @@ inline PackedB<T> repackB_1xL(const tensor2D<bfloat16>& Bi, float scale = 1.0f, 
         return p;
     }
     check(mmx_quantize_pack_scaled(Bi.data, Bi.stride, K, N, scale, p.data, stream), "repackB_1xL");
-    check_hip(hipStreamSynchronize(stream), "repackB_1xL");
     return p;
 }
 

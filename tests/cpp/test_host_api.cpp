@@ -257,6 +257,27 @@ static void test_repack_1xL(int M, int K, int N) {
     EXPECT(throws([&] { repackB_1xL<int8_t, 2>(Bodd, scale); }), "N = %d is not a multiple of 32: no error", N + 16);
 }
 
+// both forms are in stream order: they return while the stream is still busy with what was queued before (200 packings of
+// 268 MB of weights, 20 ms)
+static void test_repack_1xL_does_not_wait() {
+    std::printf("  repackB_1xL does not wait for the stream\n");
+    const int K = 8192, N = 16384;
+    tensor2D<bfloat16> B(K, N), W(512, 352);
+    PackedB<bfloat16> Bp = repackB_1x2(B);  // (its code is loaded now)
+    PackedB<int8_t> first = repackB_1xL<int8_t, 2>(W, 100.0f);
+    check_hip(hipDeviceSynchronize(), "sync");
+    auto busy = [&](const char* what, auto&& pack) {
+        for (int i = 0; i < 200; i++) check(mmx_repack_b(MMX_BF16, B.data, B.stride, K, N, 0, Bp.data, nullptr), "mmx_repack_b");
+        auto p = pack();
+        const hipError_t state = hipStreamQuery(nullptr);
+        (void)hipGetLastError();  // (not ready is an error to the runtime)
+        EXPECT(state == hipErrorNotReady, "%s returned after the stream had drained (%d)", what, static_cast<int>(state));
+        check_hip(hipDeviceSynchronize(), "sync");
+    };
+    busy("the bf16 form", [&] { return repackB_1xL<bfloat16, 2>(W); });
+    busy("the int8 form", [&] { return repackB_1xL<int8_t, 2>(W, 100.0f); });
+}
+
 // ---- MatmulW4: int4 weight compression inside the op (no reference counterpart beyond a timing stand-in) ----
 static void test_matmul_weight_int4(int M, int K, int N) {
     std::printf("  MatmulW4 (weights compressed to int4 per output channel) M=%d K=%d N=%d\n", M, K, N);
@@ -565,6 +586,7 @@ int main() {
         test_matmul_weight_int8(24, 8192, 256);   // decode with few panels: K walked in slices through the stream's workspace
         test_repack_1xL(2, 2560, 192);            // fc16m.cpp:749
         test_repack_1xL(16, 512, 352);
+        test_repack_1xL_does_not_wait();
         test_matmul_weight_int4(1, 4096, 352);
         test_matmul_weight_int4(7, 300, 77);
         test_matvec(901, 80);  // main.cpp:884
