@@ -266,11 +266,12 @@ const char* mmx_last_kernel(void);
  * 2 (default) direct HBM->LDS loads in a hand-scheduled ring pipeline, 0 through registers (the
  * fallback for operands beyond 32-bit offsets).  Rows of A that are not 16-byte aligned use a masked
  * kernel whatever this is set to, as does a K that does not fill its last 128 bytes if this is 0 or K is shorter than
- * that (otherwise the ring pipeline finishes it in a step of its own).  "decode_halves": whether the streaming decode
+ * that (otherwise it is one more k-iteration of the ring pipeline).  "decode_halves": whether the streaming decode
  * kernel for M <= 4 splits every 32-column panel over two workgroups — -1 (default) where that fills the
  * CUs better, 0 never, 1 always while x takes at most 46 KiB of LDS (the two forms add the partial sums in
- * different orders).  "waves": 8 (default) lets the 256x192 tile kernel run as eight wavefronts per
- * workgroup, 4 keeps the four-wavefront form (same results).  "decode_valu": whether the
+ * different orders).  "waves": 8 (default) lets the 256-row tile kernels over bf16 and int8 operands run as
+ * eight wavefronts per workgroup, 4 keeps the four-wavefront form (same results); a K that does not fill its last
+ * 128 bytes has the default's form only.  "decode_valu": whether the
  * streaming decode kernel at M = 1 over int8-compressed weights uses v_dot2_f32_bf16 and a cross-lane add
  * instead of the matrix cores — -1 (default) where at most one workgroup per CU is launched (it is the faster form
  * there), 0 never, 1 always; the two forms agree to fp32 summation order.  "decode_resident": whether a decode
