@@ -172,3 +172,21 @@ def test_int4_weights_of_a_deep_k(po, K, N):
     packed, deq_gpu = mx.quantize_pack_int4(Wt, transpose=True)
     assert np.array_equal(host_bits(deq_gpu).view(np.uint32), deq.view(np.uint32))
     assert np.array_equal(host_bits(packed), po.pack_int4(q))
+
+
+@pytest.mark.parametrize("gap", [0, 5])
+@pytest.mark.parametrize("rows,cols", [(1, 1), (300, 100), (4096, 1024), (70, 8193), (5, 40000), (3000, 2500)])
+def test_quantisers_scratch_of_4_kib(po, rows, cols, gap):
+    """A word for every workgroup of the maxima, filled with ones before the call (a NaN, the largest pattern of all, were it read), and
+    the words on both sides of it."""
+    L, n = mx._lib, mx._lib.QUANTIZE_SCRATCH_BYTES // 4
+    W = po.f32_to_bf16((np.random.default_rng(rows).standard_normal((rows, cols)) * 0.02).astype(np.float32))
+    wide = torch.full((rows, cols + gap), float("nan"), dtype=torch.bfloat16, device="cuda")
+    wide[:, :cols] = dev_bf16(W)
+    got = torch.empty((rows, cols), dtype=torch.int8, device="cuda")
+    scales, words = torch.empty(2, device="cuda"), torch.full((n + 2,), -1, dtype=torch.int32, device="cuda")
+    assert L.lib().mmx_quantize_weights_scratch(wide.data_ptr(), (cols + gap) * 2, rows, cols, got.data_ptr(), cols, scales.data_ptr(),
+                                                words.data_ptr() + 4, 4 * n, L._stream()) == 0
+    want, dq, q = po.quantize_weights(W)
+    assert np.array_equal(host_bits(got), want) and host_bits(scales).tolist() == [np.float32(q), np.float32(dq)]
+    assert host_bits(words)[[0, n + 1]].tolist() == [-1, -1]
