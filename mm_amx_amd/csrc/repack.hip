@@ -283,10 +283,12 @@ __global__ void zero_u32_kernel(uint32_t* p) { *p = 0u; }
 //   ROWS = false: blockIdx.y walks the rows, one load at a time: 4 MB of loads are in flight over the chip, which is what memory
 //   takes; with four loads in a row maxima, quantisation and packing took, launch to launch, 66.3 us for 11008 x 4096, 13.9 for
 //   1184 x 4160 and 19.7 for 3000 x 3000, now 61.4, 12.6 and 17.7 (two loads: 61.4, 13.5, 18.2; nontemporal loads and stores, twice
-//   as many workgroups, and quantising from the end that was read last are level or behind).
+//   as many workgroups, and quantising from the end that was read last are level or behind).  Rows with gaps that are walked like this by
+//   the quantiser (from 8192 columns) or by both (from 32768), maxima and quantisation, launch to launch: 4096 x 8192 31.9 -> 29.8,
+//   4096 x 11008 43.8 -> 39.5, 11008 x 8200 104 -> 97, 512 x 32768 21.9 -> 19.5, 4 x 100000 12.9 -> 10.3.
 //   ROWS = true, for rows with gaps that are too short to fill the four loads of a workgroup: 2^row_log2 lanes share a row, a
 //   lane's four loads are of four rows.  (Maxima and quantisation of rows with gaps, a row at a time -> shared out: 1000000 x 8
-//   4252 -> 17 us, 131072 x 128 518 -> 20, 16384 x 1024 67 -> 19, 4096 x 4096 31 -> 20, 4096 x 8192 46 -> 31.)
+//   4252 -> 17 us, 131072 x 128 518 -> 20, 16384 x 1024 67 -> 18, 4096 x 4096 31 -> 18; the maxima alone 4096 x 8192 46 -> 31, both kernels.)
 constexpr int QUANT_UNR = 4;
 
 template <int THREADS, bool ROWS, typename F>
