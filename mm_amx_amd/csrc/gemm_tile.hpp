@@ -1078,7 +1078,7 @@ struct Plan {
 // shader cycles of the busiest CU: rounds of resident workgroups x (prologue + main loop + epilogue
 // [+ parking and combining partial sums]).  The main loop takes the longer of MFMA issue (BM*BN/32 cycles
 // per k-iteration of 128 bytes, at the measured issue efficiency of the shape) and of pulling its
-// (BM + BN) * 128 bytes per k-iteration through the CU's L2 -> L1 path (about 48 bytes per cycle).
+// (BM + BN) * 128 bytes per k-iteration through the CU's L2 -> L1 path.
 // A K split is considered where the slices of all tiles are resident at once.
 static inline Plan choose_plan(int M, int Ncols, int nk, bool need_pairs, bool wide_only, int mode, const SplitRequest& rq, bool int8_a = false) {
     static const struct { int bm, bn; float eff; } cand[] = {
@@ -1086,8 +1086,9 @@ static inline Plan choose_plan(int M, int Ncols, int nk, bool need_pairs, bool w
         {64, 128, 0.27f}};  // (64 rows: two MFMAs per k-step and wave leave the loads nothing to hide behind: 940 cycles per k-iteration)
     const TileCfg f = forced_tile();
     const int cus = num_cus();
-    // measured: a CU takes 36.6 bytes per clock from L2 with all CUs pulling; parking a 64 KiB partial tile and counting
-    // takes 5.5k cycles, adding one in 2.9k
+    // The price of pulling as it was measured when the prices were fitted to each other, 36.6 bytes per clock with all CUs pulling (the main loop
+    // has become shorter since: 128x64 tiles 41.7, 128x128 38.8, 64 k-iterations of int8 21.5k -> 18.85k cycles; over 110 products of 33 to 2048
+    // rows what is picked is 1.35 % behind the best tile); parking a 64 KiB partial tile and counting takes 5.5k cycles, adding one in 2.9k
     const float l1_bytes_per_clk = 36.6f, ws_bytes_per_clk = 22.5f;
     float best = 1e30f;
     Plan pick = {{128, 128}, 1, best};
